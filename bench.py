@@ -172,7 +172,7 @@ def roofline(prof, plastic, tsize, workload, precision):
     rows, bx, by = prof["march_rows"], prof["bx"], prof["by"]
     shape = ("march%d" % rows) if rows else ("tile%dx%d" % (bx, by))
     traffic, src = measured_traffic(workload, precision, shape)
-    kernel = ("k_godunov_march (interior strips of 58 x %d)" % rows) if rows else \
+    kernel = ("k_godunov_step (interior strips of 58 x %d, and the boundary pieces)" % rows) if rows else \
         ("k_godunov_interior (interior tiles %dx%d)" % (bx, by))
     return {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": achieved / HBM_PEAK_GBS, "traffic": traffic, "traffic_source": src,

@@ -187,9 +187,9 @@ int tmk_level_run(tmk_level *lev, int nsteps, double time, double dt);
 int tmk_level_run_timed(tmk_level *lev, int nsteps, double time, double dt, double *ms);
 /* nsteps eager level steps (host-supplied times, no graph) bracketed by HIP
  * events on the level's stream; *ms_per_step = mean elapsed time per step.  A step
- * of a single-box level is the fused update (one launch over the interior tiles and,
- * concurrently on a side stream, one over the tiles that meet the domain boundary
- * or the fault) plus the clock advance. */
+ * of a single-box level is the fused update: one launch where it marches
+ * (tmk_set_march), else one over the interior tiles and, concurrently on a side stream,
+ * one over the tiles that meet the domain boundary or the fault, plus the clock advance. */
 int tmk_level_profile(tmk_level *lev, int nsteps, double time, double dt, double *ms_per_step);
 
 /* Per-kernel timing of level steps.  Measurement aid with no counterpart in the
@@ -197,11 +197,12 @@ int tmk_level_profile(tmk_level *lev, int nsteps, double time, double dt, double
  * (eagerly where capture or event timing inside a graph is unavailable; in_graph says
  * which).  Each launch is bracketed by HIP events on the stream it runs on: the
  * interior-tile update on the level's stream, the boundary-tile update on the side
- * stream.  Reports means in ms. */
+ * stream.  A level that marches updates both in one launch, reported as the interior one
+ * (ms_boundary 0).  Reports means in ms. */
 typedef struct {
     double ms_step;      /* whole step (both update launches, exchanges, clock) */
     double ms_interior;  /* interior-tile update launch */
-    double ms_boundary;  /* boundary-tile update launch (0 when there is none) */
+    double ms_boundary;  /* boundary-tile update launch (0 when there is none of its own) */
     long long cells_interior, cells_boundary; /* valid cells each launch updates */
     int tiles_interior, tiles_boundary;
     int in_graph;        /* 1: timed inside a replayed graph; 0: eager steps */
@@ -357,7 +358,8 @@ int tmk_set_tile(tmk_ctx *ctx, int bx, int by);
  * one wavefront per strip and side marching up the rows with no LDS (mode II, PPM with primitive
  * limiting; other numerics keep the tile kernels); the cells along the domain boundary run the
  * general kernel.  0 = the tile kernels of tmk_set_tile.  Results are those of the tile kernels
- * (bit-identical in FP64).  New contexts start at 32 rows. */
+ * (bit-identical in FP64).  New contexts start at 32 rows, a nominal height: until a height is set
+ * here or by tmk_level_set_update_shape, each launch takes one that suits its size. */
 int tmk_set_march(tmk_ctx *ctx, int rows);
 
 /* A level's own update shape (no reference counterpart; levels start with their context's):

@@ -1,0 +1,86 @@
+"""The one-launch level step (k_godunov_step) at the sizes where its boundary pieces and strips can
+go wrong: domains of a few cells (no interior at all), bands that end in pieces of one cell, pieces
+of exactly 23 cells, boxes whose edges cut the bands, free surfaces; and the strip height a launch
+takes when none was set.
+
+Slip weakening has no transcendental function, so FP64 is bit-identical to the oracle on every
+cell and face.  FP32 bulk is held to the 1e-5 of the other FP32 tests over a few steps.
+"""
+import numpy as np
+import pytest
+
+import tmo
+from tetemoko_amd import capi, scenarios
+
+pytestmark = pytest.mark.gpu
+
+G = scenarios.GHOST
+NSTEPS = 4
+
+
+def _case(nx, ny, boxes, bc, precision, plastic=False, march=None):
+    cfg = scenarios.config_c0(seed=3, nx=nx, ny=ny, dx=100.0)
+    cfg["bc"] = bc
+    if plastic:
+        cfg.update(plasticity=1, p_mu=0.6, p_beta=0.3, p_eta=0.03 * scenarios.G_MPA, p_b=1.0)
+    U, B = scenarios.level_arrays(cfg)
+    scenarios.perturb(U, seed=nx * 1000 + ny, amp_v=1.0, amp_s=5.0)
+    dt = scenarios.dt_of(cfg)
+    Ur, Br = U.copy(), B.copy()
+    assert tmo.level_steps(tmo.OracleParams(cfg), Ur, Br, 0.0, dt, NSTEPS) == 0
+    ctx = capi.Context(cfg, precision)
+    if march is not None:
+        ctx.set_march(march)
+    lev = capi.Level(ctx, boxes)
+    for k, b in enumerate(boxes):
+        lev.upload(k, scenarios.box_view(U, b), scenarios.box_bview(B, b) if b[1] == 0 else None)
+    lev.run(NSTEPS, 0.0, dt)
+    lev.sync()
+    Ug, Bg = np.full_like(U, np.nan), np.full_like(B, np.nan)
+    for k, (x0, y0, x1, y1) in enumerate(boxes):
+        ub = scenarios.box_view(U, boxes[k])
+        bb = scenarios.box_bview(B, boxes[k]) if y0 == 0 else None
+        lev.download(k, ub, bb)
+        Ug[:, y0 + G:y1 + G + 1, x0 + G:x1 + G + 1] = ub[:, G:-G, G:-G]
+        if bb is not None:
+            Bg[:, x0 + G:x1 + G + 1] = bb[:, G:-G]
+    lev.close()
+    ctx.close()
+    s = (slice(None), slice(G, -G), slice(G, -G))
+    return Ug[s], Ur[s], Bg[:, G:-G], Br[:, G:-G]
+
+
+LAYOUTS = {
+    "5x6": (5, 6, None),              # no cell's stencil lies inside the domain
+    "7x7": (7, 7, None),              # one interior cell
+    "24x8": (24, 8, None),            # a row band of 23 + 1 cells
+    "23x29": (23, 29, None),          # row pieces of exactly 23, column pieces of 23
+    "30x75": (30, 75, None),
+    "65x31": (65, 31, None),          # a strip of 58 and one of 1
+    "52x40 cut": (52, 40, [(0, 0, 23, 0), (24, 0, 51, 0), (0, 1, 51, 1), (0, 2, 22, 39), (23, 2, 51, 39)]),
+    "52x40 boxes": (52, 40, scenarios.split_boxes(52, 40, 16)),
+}
+
+
+@pytest.mark.parametrize("bc", [(0, 0, 0, 0), (1, 0, 0, 1)])
+@pytest.mark.parametrize("precision", [capi.PREC_FP64, capi.PREC_FP32_BULK])
+@pytest.mark.parametrize("layout", list(LAYOUTS))
+def test_small_domains_and_cut_bands(layout, precision, bc):
+    nx, ny, boxes = LAYOUTS[layout]
+    Ug, Ur, Bg, Br = _case(nx, ny, boxes or [(0, 0, nx - 1, ny - 1)], bc, precision, plastic=nx > 50)
+    if precision == capi.PREC_FP64:
+        assert np.array_equal(Ug, Ur) and np.array_equal(Bg, Br)
+        return
+    scale = np.maximum(np.abs(Ur).reshape(22, -1).max(axis=1), 1e-300)
+    err = np.abs(Ug - Ur).reshape(22, -1).max(axis=1) / scale
+    assert np.all(err <= 1e-5), err
+
+
+@pytest.mark.parametrize("nx,ny", [(64, 40), (300, 150), (1500, 700)])
+def test_chosen_strip_height_changes_nothing(nx, ny):
+    """The height a launch chooses by its size gives the state of a height set by hand (FP32 bulk:
+    a cell's arithmetic does not depend on it)."""
+    boxes = scenarios.split_boxes(nx, ny, 250)
+    a = _case(nx, ny, boxes, (0, 0, 0, 0), capi.PREC_FP32_BULK)
+    b = _case(nx, ny, boxes, (0, 0, 0, 0), capi.PREC_FP32_BULK, march=5)
+    assert np.array_equal(a[0], b[0]) and np.array_equal(a[2], b[2])

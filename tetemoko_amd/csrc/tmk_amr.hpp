@@ -76,11 +76,12 @@ struct AvgFace {
 // clocks, as LinElastLevelGodunov::step computes it (LinElastLevelGodunov.cpp:234-258):
 // alpha = (t - tCoarseOld) / (tCoarseNew - tCoarseOld), snapped to 0 or 1 within
 // 0.04 dt / ref_ratio.  Returns false when alpha lies outside [0, 1].
-__device__ __forceinline__ bool amr_alpha(const Scen& fine, const Scen& crs, int r, double& alpha)
+// fpar, cpar: the clock parities of the fine level's next step and of the coarse level's
+__device__ __forceinline__ bool amr_alpha(const Scen& fine, const Scen& crs, int fpar, int cpar, int r, double& alpha)
 {
-    const double tn = crs.time;
+    const double tn = crs.time[cpar];
     const double to = tn - crs.dt;
-    double a = (fine.time - to) / (tn - to);
+    double a = (fine.time[fpar] - to) / (tn - to);
     const double eps = 0.04 * fine.dt / (double)r;
     if (fabs(a) < eps) a = 0.0;
     if (fabs(1.0 - a) < eps) a = 1.0;
@@ -104,8 +105,8 @@ __device__ __forceinline__ T time_interp(T o, T n, double alpha)
 template <typename T>
 __global__ void k_amr_fill_state(const CfCell* __restrict__ cells, int ncells, const int* __restrict__ comps,
                                  int ncomp, const Patch<T>* __restrict__ fine, const Patch<T>* __restrict__ cold,
-                                 const Patch<T>* __restrict__ cnew, const Scen* fscen, const Scen* cscen, int r,
-                                 double alpha_fixed)
+                                 const Patch<T>* __restrict__ cnew, const Scen* fscen, const Scen* cscen, int fpar,
+                                 int cpar, int r, double alpha_fixed)
 {
     // component-major: the lanes of a wave fill neighbouring ghost cells of one plane, whose
     // coarse neighbourhoods overlap
@@ -114,7 +115,7 @@ __global__ void k_amr_fill_state(const CfCell* __restrict__ cells, int ncells, c
     const int e = (int)(t % ncells), c = comps[t / ncells];
     const CfCell cc = cells[e];
     double alpha = alpha_fixed;
-    if (alpha_fixed < 0.0 && !amr_alpha(fscen[cc.m], cscen[cc.m], r, alpha)) {
+    if (alpha_fixed < 0.0 && !amr_alpha(fscen[cc.m], cscen[cc.m], fpar, cpar, r, alpha)) {
         report(&((Scen*)fscen)[cc.m].err, TMK_E_AMR_TIME);
         return;
     }
@@ -156,7 +157,7 @@ __global__ void k_amr_fill_state(const CfCell* __restrict__ cells, int ncells, c
 template <typename T>
 __global__ void k_amr_fill_fault(const CfFace* __restrict__ faces, int nfaces, int nb, const Patch<T>* __restrict__ fine,
                                  const Patch<T>* __restrict__ cold, const Patch<T>* __restrict__ cnew,
-                                 const Scen* fscen, const Scen* cscen, int r, double alpha_fixed)
+                                 const Scen* fscen, const Scen* cscen, int fpar, int cpar, int r, double alpha_fixed)
 {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= nfaces * nb) return;
@@ -164,7 +165,7 @@ __global__ void k_amr_fill_fault(const CfFace* __restrict__ faces, int nfaces, i
     const CfFace f = faces[e];
     if (c >= fine[f.dpatch].bnb) return;  // members of a batch may have different fault laws
     double alpha = alpha_fixed;
-    if (alpha_fixed < 0.0 && !amr_alpha(fscen[f.m], cscen[f.m], r, alpha)) return;
+    if (alpha_fixed < 0.0 && !amr_alpha(fscen[f.m], cscen[f.m], fpar, cpar, r, alpha)) return;
     double v[3];
 #pragma unroll
     for (int k = 0; k < 3; ++k) {

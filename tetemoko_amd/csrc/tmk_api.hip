@@ -24,15 +24,14 @@
 
 #include "tmk_kernels.hpp"
 #include "tmk_interior.hpp"
-#include "tmk_march.hpp"
+#include "tmk_step.hpp"
 #include "tmk_amr.hpp"
 
 #ifndef TMK_DEFAULT_BY_F64
 #define TMK_DEFAULT_BY_F64 8
 #endif
-// strip rows of the row-marching interior update for new contexts (measured on the 8192 x 4096
-// and 4096 x 2048 rate-and-state levels: 32 rows is within 3 % of the best of 16 ... 256 for FP32
-// bulk and FP64 on both)
+// nominal strip rows of the row-marching interior update for new contexts; a launch whose levels
+// have set no height of their own takes march_height's
 #ifndef TMK_DEFAULT_MARCH_ROWS
 #define TMK_DEFAULT_MARCH_ROWS 32
 #endif
@@ -45,8 +44,8 @@ namespace tmk {
 #define TMK_DECLARE_EXTERN(T, NS, BX, BY, PK) \
     extern template __global__ void k_godunov_interior<T, NS, BX, BY, PK>(const KArgs<T>);
 TMK_ALL_UPDATE_KERNELS(TMK_DECLARE_EXTERN, float)
-extern template __global__ void k_godunov_march<float, PK_PPM_PRIM, true>(const KArgs<float>);
-extern template __global__ void k_godunov_march<float, PK_PPM_PRIM, false>(const KArgs<float>);
+extern template __global__ void k_godunov_step<float, true>(const KArgs<float>);
+extern template __global__ void k_godunov_step<float, false>(const KArgs<float>);
 extern template __global__ void k_godunov_bnd<float, 2, PK_RUNTIME>(const KArgs<float>);
 extern template __global__ void k_godunov_bnd<float, 3, PK_RUNTIME>(const KArgs<float>);
 extern template __global__ void k_godunov_bnd<float, 2, PK_PPM_PRIM>(const KArgs<float>);
@@ -273,18 +272,20 @@ void make_tiles(const tmk_box& v, int patch, int tx, int ty, std::vector<Tile>& 
 }
 
 // Workgroup g runs on XCD g % 8.  Give each XCD a contiguous band of the tile
-// list so that halos shared by neighbouring tiles stay in that XCD's L2.
-void xcd_order(std::vector<Tile>& t)
+// list so that halos shared by neighbouring tiles stay in that XCD's L2.  each: the consecutive
+// tiles of the list that one workgroup takes.
+void xcd_order(std::vector<Tile>& t, size_t each = 1)
 {
     const size_t nx = 8, n = t.size();
     if (n < 64) return;
-    const size_t per = (n + nx - 1) / nx;
+    const size_t per = ((n + each - 1) / each + nx - 1) / nx;
     std::vector<Tile> o;
     o.reserve(n);
-    for (size_t g = 0; g < per * nx; ++g) {
-        const size_t src = (g % nx) * per + g / nx;
-        if (src < n) o.push_back(t[src]);
-    }
+    for (size_t g = 0; g < per * nx; ++g)
+        for (size_t k = 0; k < each; ++k) {
+            const size_t src = ((g % nx) * per + g / nx) * each + k;
+            if (src < n) o.push_back(t[src]);
+        }
     t.swap(o);
 }
 
@@ -299,10 +300,11 @@ bool tile_interior_host(const Tile& t, const DevParams& P, int bx, int by)
 // The cells of rectangle r within 3 of the domain's edges, whose stencils need the boundary
 // conditions, form bands at most 3 cells thick: the rows below and above r's core (full width)
 // and the columns left and right of it.  band_split passes them to put as boundary pieces --
-// (BND_BX - 2) x (BND_BY - 2) along a row band, the transpose along a column band -- and returns
+// (bw - 2) x (bh - 2) along a row band, the transpose along a column band -- and returns
 // the core, the cells whose +-3 stencil lies inside the domain (empty when there are none).
+// bw, bh: the workgroup of a piece along a row band.
 template <typename Put>
-Tile band_split(const Tile& r, const DevParams& P, Put put)
+Tile band_split(const Tile& r, const DevParams& P, Put put, int bw = BND_BX, int bh = BND_BY)
 {
     Tile c = r;
     c.x0 = std::max(r.x0, P.dlo[0] + 3);
@@ -310,7 +312,7 @@ Tile band_split(const Tile& r, const DevParams& P, Put put)
     c.y0 = std::max(r.y0, P.dlo[1] + 3);
     c.y1 = std::min(r.y1, P.dhi[1] - 3);
     auto pieces = [&](int x0, int y0, int x1, int y1, bool col) {
-        const int pw = col ? BND_BY - 2 : BND_BX - 2, ph = col ? BND_BX - 2 : BND_BY - 2;
+        const int pw = col ? bh - 2 : bw - 2, ph = col ? bw - 2 : bh - 2;
         for (int py = y0; py <= y1; py += ph)
             for (int px = x0; px <= x1; px += pw) {
                 Tile t;
@@ -324,7 +326,7 @@ Tile band_split(const Tile& r, const DevParams& P, Put put)
     };
     if (c.x0 > c.x1 || c.y0 > c.y1) {
         // no core: r lies in a band (or the domain is under 7 cells across)
-        pieces(r.x0, r.y0, r.x1, r.y1, r.x1 - r.x0 + 1 <= BND_BY - 2 && r.y1 - r.y0 + 1 > BND_BY - 2);
+        pieces(r.x0, r.y0, r.x1, r.y1, r.x1 - r.x0 + 1 <= bh - 2 && r.y1 - r.y0 + 1 > bh - 2);
         c.x1 = c.x0 - 1;
         return c;
     }
@@ -363,12 +365,13 @@ int partition_tiles(std::vector<Tile>& t, F is_interior, G params, bool xcd = tr
 }
 
 // Row-marching partition of one rectangle of an island (r.patch: its descriptor): the core in
-// strips of MARCH_COLS x rows for k_godunov_march, the bands in boundary pieces (fault-row
+// strips of MARCH_COLS x rows for the marching step, the bands in boundary pieces (fault-row
 // pieces apart).
 void march_rect(const Tile& r, const DevParams& P, int rows, std::vector<Tile>& strips, std::vector<Tile>& bf,
                 std::vector<Tile>& bo)
 {
-    const Tile c = band_split(r, P, [&](const Tile& p) { (p.y0 == P.dlo[1] ? bf : bo).push_back(p); });
+    const Tile c = band_split(r, P, [&](const Tile& p) { (p.y0 == P.dlo[1] ? bf : bo).push_back(p); },
+                              STEP_BX, STEP_BY);
     if (tile_empty(c)) return;
     for (int y = c.y0; y <= c.y1; y += rows)
         for (int x = c.x0; x <= c.x1; x += MARCH_COLS) {
@@ -380,6 +383,48 @@ void march_rect(const Tile& r, const DevParams& P, int rows, std::vector<Tile>& 
             t.y1 = std::min(y + rows - 1, c.y1);
             strips.push_back(t);
         }
+}
+
+// Strip height of a launch over rectangles (their domains' parameters: params(r)) whose levels have
+// set none.  A wavefront marches rows + 3 rows (the two before its strip, and the first loads), and a
+// SIMD issues for its share of the wavefronts in turn, so a launch takes about ceil(wavefronts / 1024
+// SIMDs) (rows + 3) row times: short strips where the launch does not fill the chip (a 400 x 200 FP64
+// level: 32 rows 59 us per step, 4 rows 19; 1024 x 512: 65, 6 rows 49), tall ones where they repeat
+// less work (4096 x 2048: 48 rows 545 us, 16 rows 579, 6 rows 657).  FP32 moves half the bytes per
+// row and is bound by memory before issue, where tall strips cost: the halos that neighbouring strips
+// share drift out of L2 as their wavefronts drift apart.  With plasticity 8 rows stay the best up to
+// the largest level (4096 x 2048: 266 us, 16 rows 286, 32 rows 305), without it 12 to 16 (228; 8 rows
+// 239, 32 rows 239).
+template <typename P>
+int march_height(const std::vector<Tile>& rects, P params, bool fp32, bool plast)
+{
+    static const int heights[] = {4, 6, 8, 12, 16, 24, 32, 48};
+    const int most = !fp32 ? 48 : plast ? 8 : 16;
+    int best = heights[0];
+    double least = 0.0;
+    for (int rows : heights) {
+        if (rows > most) break;
+        long long strips = 0, lines = 0;
+        int tallest = 0;
+        for (const Tile& r : rects) {
+            const DevParams& p = params(r);
+            const long long w = std::min(r.x1, p.dhi[0] - 3) - std::max(r.x0, p.dlo[0] + 3) + 1;
+            const int h = std::min(r.y1, p.dhi[1] - 3) - std::max(r.y0, p.dlo[1] + 3) + 1;
+            if (w <= 0 || h <= 0) continue;
+            const long long cols = (w + MARCH_COLS - 1) / MARCH_COLS;
+            strips += cols * ((h + rows - 1) / rows);
+            lines += cols * h;
+            tallest = std::max(tallest, std::min(h, rows));
+        }
+        if (strips == 0) return rows;
+        const double mean = (double)lines / (double)strips + 3.0;
+        const double cost = std::max((double)((2 * strips + 1023) / 1024) * mean, tallest + 3.0);
+        if (least == 0.0 || cost < least) {
+            least = cost;
+            best = rows;
+        }
+    }
+    return best;
 }
 
 // state planes that sweeps read with a stencil (double-buffered); the others
@@ -405,7 +450,7 @@ int stencil_mask(int ns)
 struct Group {
     size_t tsize = 8;
     int ns = 2, bx = 32, by = 16;
-    int march = 0;                 // > 0: interior strips of this many rows run k_godunov_march
+    int march = 0;                 // > 0: interior strips of this many rows (k_godunov_step)
     bool any_plast = true;         // some member has plasticity (the march variant with lam, gam)
     int xcd = 1;                   // interior tiles / strips in XCD bands (the first member's choice)
     int pk = PK_RUNTIME;  // predictor kind the kernel is specialised for (all members agree)
@@ -467,6 +512,7 @@ struct tmk_ctx {
     int bx = 32, by = 16;
     bool antiplane = true;
     int march = TMK_DEFAULT_MARCH_ROWS;  // strip rows of the row-marching interior update (0: tile kernels)
+    bool march_auto = true;              // the launch chooses the height (march_height)
     void* noalloc_scratch = nullptr;  // this device's scratch array (tmk_patch_update_state_noalloc)
 };
 
@@ -500,6 +546,7 @@ struct tmk_level {
     size_t tsize = 8;
     int bx = 32, by = 16;         // update tile (the context's at creation; tmk_level_set_update_shape)
     int march = 0;                // strip rows of the row-marching update (0: tile kernels)
+    bool march_auto = false;      // no height set: the launch chooses it (march_height)
     int xcd = 1;                  // interior tiles / strips in XCD bands (0: row-major order)
     std::vector<Island> isl;
     std::vector<int> box_isl;     // island of each box
@@ -794,6 +841,7 @@ extern "C" int tmk_set_march(tmk_ctx* c, int rows)
 {
     if (!c || rows < 0 || rows > 65536) return TMK_E_ARG;
     c->march = rows;
+    c->march_auto = false;
     return TMK_OK;
 }
 
@@ -850,7 +898,7 @@ static int launch_bnd_t(hipStream_t st, const KArgs<T>& a)
     if (a.ntiles == 0) return TMK_OK;
     const void* k = (const void*)k_godunov_bnd<T, NS, PK>;
     if (shm > 64 * 1024) (void)hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
-    hipLaunchKernelGGL((k_godunov_bnd<T, NS, PK>), dim3(a.ntiles), dim3(BND_BX * BND_BY), shm, st, a);
+    hipLaunchKernelGGL((k_godunov_bnd<T, NS, PK>), dim3(a.ntiles), dim3(BND_NT), shm, st, a);
     return hipGetLastError() == hipSuccess ? TMK_OK : TMK_E_HIP;
 }
 
@@ -897,24 +945,28 @@ static int timer_mark(const StepTimers* tm, hipStream_t s, int k)
     return hipEventRecord(e, s) == hipSuccess ? TMK_OK : TMK_E_HIP;
 }
 
-// the fused update of one step over a tile list [interior | boundary]: the boundary launch runs
-// on `side` (forked from and joined back into st by events; captured graphs keep the fork), the
-// interior launch on st
-// the interior strips of the row-marching partition (grid: two one-wavefront workgroups per strip);
-// plast: some scenario of the launch has plasticity (the variant that reads and writes lam, gam)
+// one step of a group that marches, in one launch: its boundary pieces, its interior strips and its
+// clocks; plast: some scenario of the launch has plasticity (the variant that reads and writes lam, gam)
 template <typename T>
-static int launch_march(hipStream_t st, const KArgs<T>& a, bool plast)
+static int launch_step(hipStream_t st, const KArgs<T>& a, bool plast, const StepTimers* tm)
 {
+    int e;
+    if ((e = timer_mark(tm, st, 0))) return e;
+    const dim3 grid((unsigned)(a.ntiles - a.nint + (2 * a.nint + STEP_WAVES - 1) / STEP_WAVES));
     if (plast && a.plastic)
-        hipLaunchKernelGGL((k_godunov_march<T, PK_PPM_PRIM, true>), dim3(2 * a.ntiles), dim3(64), 0, st, a);
+        hipLaunchKernelGGL((k_godunov_step<T, true>), grid, dim3(STEP_NT), 0, st, a);
     else
-        hipLaunchKernelGGL((k_godunov_march<T, PK_PPM_PRIM, false>), dim3(2 * a.ntiles), dim3(64), 0, st, a);
-    return hipGetLastError() == hipSuccess ? TMK_OK : TMK_E_HIP;
+        hipLaunchKernelGGL((k_godunov_step<T, false>), grid, dim3(STEP_NT), 0, st, a);
+    if (hipGetLastError() != hipSuccess) return TMK_E_HIP;
+    return timer_mark(tm, st, 1);
 }
 
+// the update of one step over a tile list [interior | boundary] by the tile kernels: the boundary
+// launch runs on `side` (forked from and joined back into st by events; captured graphs keep the
+// fork), the interior launch on st
 template <typename T>
 static int launch_update(hipStream_t st, hipStream_t side, hipEvent_t fork, hipEvent_t join, int ns, int pk, int bx,
-                         int by, KArgs<T> a, int nint, const StepTimers* tm, int march = 0, bool plast = true)
+                         int by, KArgs<T> a, int nint, const StepTimers* tm)
 {
     const int nbnd = a.ntiles - nint;
     const Tile* tiles = a.tiles;
@@ -937,11 +989,7 @@ static int launch_update(hipStream_t st, hipStream_t side, hipEvent_t fork, hipE
         KArgs<T> b = a;
         b.ntiles = nint;
         if ((e = timer_mark(tm, st, 0))) return e;
-        if (march > 0) {
-            if ((e = launch_march<T>(st, b, plast))) return e;
-        } else if ((e = launch_tiles<T>(st, ns, pk, bx, by, b))) {
-            return e;
-        }
+        if ((e = launch_tiles<T>(st, ns, pk, bx, by, b))) return e;
         if ((e = timer_mark(tm, st, 1))) return e;
     }
     if (split) {
@@ -962,8 +1010,11 @@ static int group_enqueue_step_t(Group& G, hipStream_t st, const StepTimers* tm =
     a.tiles = G.tiles_dev;
     a.ntiles = G.ntiles;
     a.plastic = G.plastic;
-    int e = launch_update<T>(st, G.side, G.ev_fork, G.ev_join, G.ns, G.pk, G.bx, G.by, a, G.nint, tm, G.march,
-                             G.any_plast);
+    a.par = G.g;
+    a.nint = G.nint;
+    a.nscen = G.nscen;
+    int e = G.march > 0 ? launch_step<T>(st, a, G.any_plast, tm)
+                        : launch_update<T>(st, G.side, G.ev_fork, G.ev_join, G.ns, G.pk, G.bx, G.by, a, G.nint, tm);
     if (e) return e;
     const Patch<T>* pn = (const Patch<T>*)G.patches_dev[G.g];  // its out planes hold the new state
     if (G.nrects > 0) {
@@ -975,10 +1026,12 @@ static int group_enqueue_step_t(Group& G, hipStream_t st, const StepTimers* tm =
         hipLaunchKernelGGL(k_bexchange<T>, dim3(G.nbrects), dim3(64), 0, st, pn, G.brects_dev, G.nbrects);
         if (hipGetLastError() != hipSuccess) return TMK_E_HIP;
     }
-    hipLaunchKernelGGL(k_advance_time, dim3((G.nscen + 63) / 64), dim3(64), 0, st, G.scen_dev, G.nscen);
-    if (hipGetLastError() != hipSuccess) return TMK_E_HIP;
+    if (G.march <= 0) {  // the marching step advances the clocks itself
+        hipLaunchKernelGGL(k_advance_time, dim3((G.nscen + 63) / 64), dim3(64), 0, st, G.scen_dev, G.nscen, G.g);
+        if (hipGetLastError() != hipSuccess) return TMK_E_HIP;
+    }
     if (G.stations) {
-        hipLaunchKernelGGL(k_station_record<T>, dim3(1), dim3(256), 0, st, pn, G.scen_dev, *G.stations);
+        hipLaunchKernelGGL(k_station_record<T>, dim3(1), dim3(256), 0, st, pn, G.scen_dev, G.g ^ 1, *G.stations);
         if (hipGetLastError() != hipSuccess) return TMK_E_HIP;
     }
     G.g ^= 1;
@@ -1099,9 +1152,13 @@ static int group_build_t(Group& G, const std::vector<tmk_level*>& mem, const std
         // strips of levels with flux registers hold at most 63 rows (the kernel's face masks)
         bool fluxes = false;
         for (const Patch<T>& p : pts[0]) fluxes = fluxes || p.F[0] || p.F[1];
+        auto params = [&](const Tile& t) -> const DevParams& { return sc[patch_scen[t.patch]].P; };
+        bool chosen = false;  // some member's level has a height of its own
+        for (tmk_level* L : mem) chosen = chosen || !L->march_auto;
+        if (!chosen) G.march = march_height(tiles, params, sizeof(T) == sizeof(float), G.plastic && G.any_plast);
         const int rows = fluxes ? std::min(G.march, 63) : G.march;
-        for (const Tile& r : tiles) march_rect(r, sc[patch_scen[r.patch]].P, rows, strips, bf, bo);
-        if (G.xcd) xcd_order(strips);
+        for (const Tile& r : tiles) march_rect(r, params(r), rows, strips, bf, bo);
+        if (G.xcd) xcd_order(strips, STEP_WAVES / 2);
         G.nint = (int)strips.size();
         tiles.swap(strips);
         tiles.insert(tiles.end(), bf.begin(), bf.end());
@@ -1393,6 +1450,9 @@ static int patch_update_t(tmk_ctx* c, tmk_box valid, double* U, tmk_box ub, doub
         a.tiles = (const Tile*)(meta + off_t);
         a.ntiles = ntiles;
         a.plastic = 0;  // updateState does not include the plastic return
+        a.par = 0;
+        a.nint = nint;
+        a.nscen = 1;
         // the anti-plane planes are skipped only when background and data are zero there
         int ns = 3;
         if (!c->antiplane) {
@@ -1854,6 +1914,7 @@ extern "C" int tmk_level_create(tmk_ctx* c, int nboxes, const tmk_box* boxes, tm
     L->bx = c->bx;
     L->by = c->by;
     L->march = c->march;
+    L->march_auto = c->march_auto;
     L->ns = c->antiplane ? 3 : 2;
     L->tsize = c->precision == TMK_PREC_FP64 ? sizeof(double) : sizeof(float);
     L->bytes = level_bytes(c->precision, c->hp.fault_kind, c->hp.domain, nboxes, boxes);
@@ -2301,7 +2362,8 @@ extern "C" int tmk_level_profile_kernels(tmk_level* L, int nsteps, double time, 
     if (e) return e;
     hipStream_t st = L->ctx->stream;
     Group& G = L->own;
-    const bool has_bnd = G.ntiles > G.nint, has_int = G.nint > 0;
+    // a marching step is one launch, marked as the interior one
+    const bool has_int = G.march > 0 || G.nint > 0, has_bnd = G.march <= 0 && G.ntiles > G.nint;
     double sum[3] = {0, 0, 0};
     // The steps as one captured graph, replayed once, so that the launches run as in
     // tmk_level_run; each mark is a one-lane kernel reading the constant-rate wall clock.
@@ -2413,6 +2475,7 @@ extern "C" int tmk_level_set_update_shape(tmk_level* L, int march_rows, int bx, 
     if (!tile_ok(bx, by)) return TMK_E_ARG;
     HIPCHK(hipStreamSynchronize(L->ctx->stream));
     L->march = march_rows;
+    L->march_auto = false;
     if (bx != L->bx || by != L->by) {
         L->bx = bx;
         L->by = by;
@@ -2510,6 +2573,7 @@ extern "C" int tmk_level_autotune(tmk_level* L, double time, double dt, int nste
     LevelSnapshot snap;
     if ((e = snap.take(L, st))) return e;
     const int march0 = L->march, bx0 = L->bx, by0 = L->by, xcd0 = L->xcd;
+    const bool auto0 = L->march_auto;
     std::vector<std::array<int, 3>> cand;
     if (L->ns == 2 && pred_kind(c->P) == PK_PPM_PRIM)
         for (int rows : kTuneMarch) cand.push_back({rows, bx0, by0});
@@ -2557,6 +2621,7 @@ extern "C" int tmk_level_autotune(tmk_level* L, double time, double dt, int nste
     L->time = time;
     if (e || best < 0) {
         (void)tmk_level_set_update_shape(L, march0, bx0, by0);
+        L->march_auto = auto0;
         (void)tmk_level_set_tile_order(L, xcd0);
         return e ? e : e2;
     }
@@ -2609,7 +2674,7 @@ static int batch_detach_all(tmk_batch* B)
     for (size_t m = 0; m < B->members.size(); ++m) {
         tmk_level* L = B->members[m];
         L->cur = B->phase[m] ^ B->grp.g;
-        L->time = sc[m].time;
+        L->time = sc[m].time[B->grp.g];
         if (sc[m].err) L->own_built = false;
         B->phase[m] = L->cur;
     }
@@ -3329,7 +3394,7 @@ static int amr_detach(tmk_amr* A)
         for (size_t m = 0; m < A->mem.size(); ++m) {
             tmk_level* L = A->mem[m]->L[l];
             L->cur = a.phase[m] ^ a.grp.g;
-            L->time = sc[m].time;
+            L->time = sc[m].time[a.grp.g];
             if (sc[m].err && !A->mem[m]->err) A->mem[m]->err = sc[m].err;
         }
         a.grp.reset();
@@ -3602,13 +3667,13 @@ static int amr_advance_t(tmk_amr* A, int l)
         if (a.ncells > 0) {
             hipLaunchKernelGGL(k_amr_fill_state<T>, amr_grid((long long)a.ncells * a.ncomps), dim3(256), 0, st,
                                (const CfCell*)a.cells.p, a.ncells, (const int*)a.comps.p, a.ncomps, fine, cold, cnew,
-                               G.scen_dev, GC.scen_dev, A->r, -1.0);
+                               G.scen_dev, GC.scen_dev, G.g, GC.g, A->r, -1.0);
             HIPCHK(hipGetLastError());
         }
         if (a.nfaces > 0) {
             hipLaunchKernelGGL(k_amr_fill_fault<T>, amr_grid((long long)a.nfaces * TMK_NBDRY_RS), dim3(256), 0, st,
                                (const CfFace*)a.faces.p, a.nfaces, TMK_NBDRY_RS, fine, cold, cnew, G.scen_dev,
-                               GC.scen_dev, A->r, -1.0);
+                               GC.scen_dev, G.g, GC.g, A->r, -1.0);
             HIPCHK(hipGetLastError());
         }
     }
@@ -4143,13 +4208,13 @@ static int level_regrid_t(tmk_level* N, tmk_level* O, tmk_level* C, int r)
     if (!cells.empty()) {
         hipLaunchKernelGGL(k_amr_fill_state<T>, amr_grid((long long)cells.size() * TMK_NCOMP), dim3(256), 0, st,
                            (const CfCell*)dcells.p, (int)cells.size(), (const int*)dcomps.p, TMK_NCOMP, tN, tC, tC,
-                           (const Scen*)nullptr, (const Scen*)nullptr, r, 1.0);
+                           (const Scen*)nullptr, (const Scen*)nullptr, 0, 0, r, 1.0);
         HIPCHK(hipGetLastError());
     }
     if (!faces.empty()) {
         hipLaunchKernelGGL(k_amr_fill_fault<T>, amr_grid((long long)faces.size() * nb), dim3(256), 0, st,
                            (const CfFace*)dfaces.p, (int)faces.size(), nb, tN, tC, tC, (const Scen*)nullptr,
-                           (const Scen*)nullptr, r, 1.0);
+                           (const Scen*)nullptr, 0, 0, r, 1.0);
         HIPCHK(hipGetLastError());
     }
     if (!rects.empty()) {

@@ -7,7 +7,7 @@
 // contraction.  tmk_api.hip declares these instantiations extern and launches them.
 #include "tmk_kernels.hpp"
 #include "tmk_interior.hpp"
-#include "tmk_march.hpp"
+#include "tmk_step.hpp"
 
 namespace tmk {
 
@@ -19,7 +19,7 @@ template __global__ void k_godunov_bnd<float, 2, PK_RUNTIME>(const KArgs<float>)
 template __global__ void k_godunov_bnd<float, 3, PK_RUNTIME>(const KArgs<float>);
 template __global__ void k_godunov_bnd<float, 2, PK_PPM_PRIM>(const KArgs<float>);
 template __global__ void k_godunov_bnd<float, 3, PK_PPM_PRIM>(const KArgs<float>);
-template __global__ void k_godunov_march<float, PK_PPM_PRIM, true>(const KArgs<float>);
-template __global__ void k_godunov_march<float, PK_PPM_PRIM, false>(const KArgs<float>);
+template __global__ void k_godunov_step<float, true>(const KArgs<float>);
+template __global__ void k_godunov_step<float, false>(const KArgs<float>);
 
 }  // namespace tmk

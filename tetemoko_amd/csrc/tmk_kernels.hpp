@@ -58,7 +58,9 @@ struct StateVec {
 // boxes of several scenarios can share one launch
 struct Scen {
     DevParams P;
-    double time;  // time at the start of the current step
+    // time at the start of the current step, by the parity of the launch: a step's launch reads
+    // time[par] and writes time[par ^ 1], so one launch can both use the clock and advance it
+    double time[2];
     double dt;
     // step constants, evaluated on the host with the expressions the update uses:
     // dt/dx, -(1/2) dt/dx (transverse correction), -dt/dx (flux difference), and in FP32
@@ -71,7 +73,7 @@ struct Scen {
 // host: the clock and step constants of a scenario
 __host__ inline void scen_set_clock(Scen& s, double time, double dt)
 {
-    s.time = time;
+    s.time[0] = s.time[1] = time;
     s.dt = dt;
     s.dtdx = dt / s.P.dx;
     s.hdtdx = -(1.0 / 2.0) * dt / s.P.dx;
@@ -107,6 +109,9 @@ struct KArgs {
     const Tile* tiles;
     int ntiles;
     int plastic;   // 0: skip the Drucker-Prager return even if the scenario enables it
+    int par;       // clock parity of this launch (Scen::time)
+    int nint;      // k_godunov_step: tiles [0, nint) are interior strips, the rest boundary pieces
+    int nscen;     // k_godunov_step: the scenarios whose clocks it advances
 };
 
 __device__ __forceinline__ void report(int* err, int code)
@@ -397,12 +402,95 @@ __device__ __forceinline__ void update_cell(const KArgs<T>& a, const Patch<T>& p
     }
 }
 
+// the half-step fault solve of face i: its face states, and the half step's psi (rate-and-state) or
+// slip total (slip weakening), the only fault data of the half step that the final solve reads
+template <typename T, int NS>
+__device__ __forceinline__ double fault_half(const Patch<T>& pt, const DevParams& P, int i, double dt,
+                                             const FaultIn& fin, FaultOut& fo, int* errp)
+{
+    const size_t bi = (size_t)(i - pt.blo0);
+    const size_t bp = (size_t)pt.bnx;
+    if (P.fault_kind == 0) {
+        const double psi = gmem(pt.bin)[bi + 10 * bp];
+        rs_fault(P, i, psi, fin, fo);
+        // RSSETBND into the half-step copy (RSIBC.cpp:325-333): only psi is consumed
+        const double Vx = fo.vx[0] - fo.vx[1];
+        const double Vz = NS == 3 ? fo.vz[0] - fo.vz[1] : 0.0;
+        const double V = sqrt(Vx * Vx + Vz * Vz);
+        const double half = rs_psi_update(P, i, psi, V, 0.5 * dt);
+        if (isnan(half)) report(errp, TMK_E_PSI_NAN);
+        return half;
+    }
+    const double slip = gmem(pt.bin)[bi + 7 * bp];
+    sw_fault(P, i, slip, fin, fo);
+    const double Vx = fo.vx[0] - fo.vx[1];
+    const double Vz = NS == 3 ? fo.vz[0] - fo.vz[1] : 0.0;
+    const double V = sqrt(Vx * Vx + Vz * Vz);
+    return slip + (0.5 * dt) * V;
+}
+
+// the final fault solve of face i from the half step's state, and its new fault data
+template <typename T, int NS>
+__device__ __forceinline__ void fault_final(const Patch<T>& pt, const DevParams& P, int i, double time, double dt,
+                                            double half, const FaultIn& fin, FaultOut& fo, int* errp)
+{
+    const size_t bi = (size_t)(i - pt.blo0);
+    const size_t bp = (size_t)pt.bnx;
+    const __attribute__((address_space(1))) double* B = gmem(pt.bin);
+    __attribute__((address_space(1))) double* Bo = gmem(pt.bout);
+    const double tnew = time + dt;
+    if (P.fault_kind == 0) {
+        rs_fault(P, i, half, fin, fo);
+        // RSSETBND final (RSIBCF.ChF:61-151) on m_bdryData
+        const double x = (i + 0.5) * P.dx - P.x0;
+        double tau_xy_0 = P.nsig * gaussianfunc(P.r0, x);
+        if (P.f_tau) tau_xy_0 = tau_xy_0 + face_val(P.f_tau, P, i, 0.0);
+        const double Vx = fo.vx[0] - fo.vx[1];
+        const double Vz = NS == 3 ? fo.vz[0] - fo.vz[1] : 0.0;
+        const double V = sqrt(Vx * Vx + Vz * Vz);
+        const double dX = B[bi + 6 * bp], dZ = B[bi + 7 * bp], dT = B[bi + 8 * bp];
+        const double RT = B[bi + 9 * bp], psi = B[bi + 10 * bp];
+        Bo[bi + 0 * bp] = Vx;
+        Bo[bi + 1 * bp] = Vz;
+        Bo[bi + 2 * bp] = V;
+        Bo[bi + 3 * bp] = fo.sxy[0] + tau_xy_0;
+        Bo[bi + 4 * bp] = (NS == 3 ? fo.syz[0] : 0.0) + 0.0;
+        Bo[bi + 6 * bp] = dX + dt * Vx;
+        Bo[bi + 7 * bp] = dZ + dt * Vz;
+        Bo[bi + 8 * bp] = dT + dt * V;
+        if (RT > tnew && V > P.rs_thr) Bo[bi + 9 * bp] = tnew;
+        else if (RT > tnew) Bo[bi + 9 * bp] = 1e10;
+        else Bo[bi + 9 * bp] = RT;
+        Bo[bi + 5 * bp] = fo.syy[0];
+        const double np = rs_psi_update(P, i, psi, V, dt);
+        if (isnan(np)) report(errp, TMK_E_PSI_NAN);
+        Bo[bi + 10 * bp] = np;
+    } else {
+        sw_fault(P, i, half, fin, fo);
+        // SWSETBND final (SWIBCF.ChF:32-72) on m_bdryData (Bout aliases Bin)
+        const double Vx = fo.vx[0] - fo.vx[1];
+        const double Vz = NS == 3 ? fo.vz[0] - fo.vz[1] : 0.0;
+        const double b5 = B[bi + 5 * bp], b6 = B[bi + 6 * bp], b7 = B[bi + 7 * bp];
+        const double b8 = B[bi + 8 * bp];
+        const double V = sqrt(Vx * Vx + Vz * Vz);
+        Bo[bi + 0 * bp] = Vx;
+        Bo[bi + 1 * bp] = Vz;
+        Bo[bi + 2 * bp] = fo.sxy[0];
+        Bo[bi + 3 * bp] = NS == 3 ? fo.syz[0] : 0.0;
+        Bo[bi + 4 * bp] = V;
+        Bo[bi + 5 * bp] = b5 + dt * Vx;
+        Bo[bi + 6 * bp] = b6 + dt * Vz;
+        Bo[bi + 7 * bp] = b7 + dt * V;
+        Bo[bi + 8 * bp] = (b8 > tnew && V > P.sw_thr) ? tnew : b8;
+    }
+}
+
 // INT: the tile is full size and its stencil (+-3 cells) lies inside the domain, so no cell of
 // it is a domain-boundary or fault cell; the body then carries no boundary code at all.
 template <typename T, int NS, int BX, int BY, int PK, bool INT>
 __device__ __forceinline__ void godunov_tile(const KArgs<T>& a, const Tile& tl, T* sm)
 {
-    constexpr int NT = BX * BY;
+    constexpr int NT = (BX * BY + 63) / 64 * 64;  // lanes (those past BX * BY hold no cell)
     constexpr int NC = 4 * NS;  // staged components per direction
     const Patch<T>& pt = a.patches[tl.patch];
     Scen& S = a.scen[pt.scen];
@@ -418,7 +506,7 @@ __device__ __forceinline__ void godunov_tile(const KArgs<T>& a, const Tile& tl, 
     const bool rowD = INT || (j >= dlo1 && j <= dhi1);
     const bool r1 = colD && rowD && lx <= tnx + 1 && ly <= tny + 1;
     const bool valid = lx >= 1 && lx <= tnx && ly >= 1 && ly <= tny;
-    const double time = S.time;
+    const double time = S.time[a.par];
     const double dt = S.dt;
     const StepConst<T> K = step_const<T>(S);
     const T dtbydx = K.dtbydx;
@@ -557,23 +645,7 @@ __device__ __forceinline__ void godunov_tile(const KArgs<T>& a, const Tile& tl, 
                     FaultIn fin;
                     fault_input<T, NS>(P, WmY, fin);
                     FaultOut fo;
-                    const size_t bi = (size_t)(i - pt.blo0);
-                    const size_t bp = (size_t)pt.bnx;
-                    if (P.fault_kind == 0) {
-                        rs_fault(P, i, gmem(pt.bin)[bi + 10 * bp], fin, fo);
-                        // RSSETBND into the half-step copy (RSIBC.cpp:325-333): only psi is consumed
-                        const double Vx = fo.vx[0] - fo.vx[1];
-                        const double Vz = NS == 3 ? fo.vz[0] - fo.vz[1] : 0.0;
-                        const double V = sqrt(Vx * Vx + Vz * Vz);
-                        tmp_state = rs_psi_update(P, i, gmem(pt.bin)[bi + 10 * bp], V, 0.5 * dt);
-                        if (isnan(tmp_state)) report(errp, TMK_E_PSI_NAN);
-                    } else {
-                        sw_fault(P, i, gmem(pt.bin)[bi + 7 * bp], fin, fo);
-                        const double Vx = fo.vx[0] - fo.vx[1];
-                        const double Vz = NS == 3 ? fo.vz[0] - fo.vz[1] : 0.0;
-                        const double V = sqrt(Vx * Vx + Vz * Vz);
-                        tmp_state = gmem(pt.bin)[bi + 7 * bp] + (0.5 * dt) * V;
-                    }
+                    tmp_state = fault_half<T, NS>(pt, P, i, dt, fin, fo, errp);
                     fault_output<T, NS>(P, fo, H1);
                 }
             } else {
@@ -671,55 +743,7 @@ __device__ __forceinline__ void godunov_tile(const KArgs<T>& a, const Tile& tl, 
                     FaultIn fin;
                     fault_input<T, NS>(P, WmY, fin);
                     FaultOut fo;
-                    const size_t bi = (size_t)(i - pt.blo0);
-                    const size_t bp = (size_t)pt.bnx;
-                    const __attribute__((address_space(1))) double* B = gmem(pt.bin);
-                    __attribute__((address_space(1))) double* Bo = gmem(pt.bout);
-                    const double tnew = time + dt;
-                    if (P.fault_kind == 0) {
-                        rs_fault(P, i, tmp_state, fin, fo);
-                        // RSSETBND final (RSIBCF.ChF:61-151) on m_bdryData
-                        const double x = (i + 0.5) * P.dx - P.x0;
-                        double tau_xy_0 = P.nsig * gaussianfunc(P.r0, x);
-                        if (P.f_tau) tau_xy_0 = tau_xy_0 + face_val(P.f_tau, P, i, 0.0);
-                        const double Vx = fo.vx[0] - fo.vx[1];
-                        const double Vz = NS == 3 ? fo.vz[0] - fo.vz[1] : 0.0;
-                        const double V = sqrt(Vx * Vx + Vz * Vz);
-                        const double dX = B[bi + 6 * bp], dZ = B[bi + 7 * bp], dT = B[bi + 8 * bp];
-                        const double RT = B[bi + 9 * bp], psi = B[bi + 10 * bp];
-                        Bo[bi + 0 * bp] = Vx;
-                        Bo[bi + 1 * bp] = Vz;
-                        Bo[bi + 2 * bp] = V;
-                        Bo[bi + 3 * bp] = fo.sxy[0] + tau_xy_0;
-                        Bo[bi + 4 * bp] = (NS == 3 ? fo.syz[0] : 0.0) + 0.0;
-                        Bo[bi + 6 * bp] = dX + dt * Vx;
-                        Bo[bi + 7 * bp] = dZ + dt * Vz;
-                        Bo[bi + 8 * bp] = dT + dt * V;
-                        if (RT > tnew && V > P.rs_thr) Bo[bi + 9 * bp] = tnew;
-                        else if (RT > tnew) Bo[bi + 9 * bp] = 1e10;
-                        else Bo[bi + 9 * bp] = RT;
-                        Bo[bi + 5 * bp] = fo.syy[0];
-                        const double np = rs_psi_update(P, i, psi, V, dt);
-                        if (isnan(np)) report(errp, TMK_E_PSI_NAN);
-                        Bo[bi + 10 * bp] = np;
-                    } else {
-                        sw_fault(P, i, tmp_state, fin, fo);
-                        // SWSETBND final (SWIBCF.ChF:32-72) on m_bdryData (Bout aliases Bin)
-                        const double Vx = fo.vx[0] - fo.vx[1];
-                        const double Vz = NS == 3 ? fo.vz[0] - fo.vz[1] : 0.0;
-                        const double b5 = B[bi + 5 * bp], b6 = B[bi + 6 * bp], b7 = B[bi + 7 * bp];
-                        const double b8 = B[bi + 8 * bp];
-                        const double V = sqrt(Vx * Vx + Vz * Vz);
-                        Bo[bi + 0 * bp] = Vx;
-                        Bo[bi + 1 * bp] = Vz;
-                        Bo[bi + 2 * bp] = fo.sxy[0];
-                        Bo[bi + 3 * bp] = NS == 3 ? fo.syz[0] : 0.0;
-                        Bo[bi + 4 * bp] = V;
-                        Bo[bi + 5 * bp] = b5 + dt * Vx;
-                        Bo[bi + 6 * bp] = b6 + dt * Vz;
-                        Bo[bi + 7 * bp] = b7 + dt * V;
-                        Bo[bi + 8 * bp] = (b8 > tnew && V > P.sw_thr) ? tnew : b8;
-                    }
+                    fault_final<T, NS>(pt, P, i, time, dt, tmp_state, fin, fo, errp);
                     fault_output<T, NS>(P, fo, F1);
                 }
             } else {
@@ -783,6 +807,7 @@ __device__ __forceinline__ bool tile_interior(const Tile& t, const DevParams& P)
 // (taller than 3) on the transposed BND_BY x BND_BX one: either way the 255 lanes cover 3 rows or
 // columns of cells and the ring around them, with no idle row.
 constexpr int BND_BX = 51, BND_BY = 5;
+constexpr int BND_NT = (BND_BX * BND_BY + 63) / 64 * 64;  // lanes of its workgroup
 
 template <typename T, int NS>
 constexpr size_t bnd_lds_elems()
@@ -790,7 +815,7 @@ constexpr size_t bnd_lds_elems()
     constexpr size_t NC = 4 * NS;
     constexpr size_t s1 = NC * BND_BY * (BND_BX + 4), s2 = NC * (BND_BY + 4) * BND_BX;
     constexpr size_t s1t = NC * BND_BX * (BND_BY + 4), s2t = NC * (BND_BX + 4) * BND_BY;
-    constexpr size_t s3 = (size_t)8 * NS * BND_BX * BND_BY;  // the exchange slots (either shape)
+    constexpr size_t s3 = (size_t)8 * NS * BND_NT;  // the exchange slots (either shape)
     constexpr size_t a = s1 > s2 ? s1 : s2, b = s1t > s2t ? s1t : s2t;
     return (a > b ? a : b) > s3 ? (a > b ? a : b) : s3;
 }
@@ -798,7 +823,7 @@ constexpr size_t bnd_lds_elems()
 // FP32: held to 128 VGPRs, 4 wavefronts per SIMD (a spill of about 20 VGPRs per lane); measured
 // 3-4 % faster in batches of serving scenarios than 145 VGPRs at 3 per SIMD
 template <typename T, int NS, int PK>
-__global__ void __launch_bounds__(BND_BX * BND_BY) __attribute__((amdgpu_waves_per_eu(sizeof(T) == sizeof(float) ? 4 : 1)))
+__global__ void __launch_bounds__(BND_NT) __attribute__((amdgpu_waves_per_eu(sizeof(T) == sizeof(float) ? 4 : 1)))
 k_godunov_bnd(const KArgs<T> a)
 {
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -885,7 +910,7 @@ struct StationDev {
 // one record per station after a level step: the new time and B[i] (1 - d) + B[i+1] d per
 // fault-data component, from the step's output fault data (ghosts exchanged)
 template <typename T>
-__global__ void k_station_record(const Patch<T>* patches, const Scen* scen, StationDev s)
+__global__ void k_station_record(const Patch<T>* patches, const Scen* scen, int par, StationDev s)
 {
     __shared__ int base;
     if (threadIdx.x == 0) base = s.count[0];
@@ -900,7 +925,7 @@ __global__ void k_station_record(const Patch<T>* patches, const Scen* scen, Stat
         const size_t i = (size_t)(s.face[k] - p.blo0), bp = (size_t)p.bnx;
         const double d = s.d[k];
         double* r = s.rec + ((size_t)b * s.n + k) * (size_t)(1 + s.nb);
-        r[0] = scen[p.scen].time;
+        r[0] = scen[p.scen].time[par];
         for (int c = 0; c < s.nb; ++c) r[1 + c] = gmem(p.bout)[i + c * bp] * (1.0 - d) + gmem(p.bout)[i + 1 + c * bp] * d;
     }
     __syncthreads();
@@ -999,10 +1024,10 @@ static __global__ void k_dilate(const unsigned char* raw, unsigned char* out, in
 }
 
 // every scenario's clock advances by its own step (AMRLevelLinElast.cpp:478, m_time += m_dt)
-static __global__ void k_advance_time(Scen* s, int n)
+static __global__ void k_advance_time(Scen* s, int n, int par)
 {
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < n) s[k].time = s[k].time + s[k].dt;
+    if (k < n) s[k].time[par ^ 1] = s[k].time[par] + s[k].dt;
 }
 
 }  // namespace tmk

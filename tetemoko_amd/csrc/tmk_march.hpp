@@ -177,28 +177,48 @@ struct MarchCarry {
     T f1v[2], f1s[2];      // final state of the lo y face of row r - 2
 };
 
-// grid: two workgroups of one wavefront per strip, side = blockIdx.x & 1 (a scalar, so every
-// plane pointer and descriptor of the side stays in scalar registers).  FP32: at least four
-// wavefronts per SIMD (at most 128 VGPRs) keep enough loads in flight to cover their latency;
-// FP64 needs about twice the registers (two wavefronts per SIMD) and is left to the compiler.
+// LDS floats of one wavefront's march: the ring, the plastic return's constants (16 floats), the
+// lanes' flux-register face masks (4 x 64)
+template <typename T, bool PL>
+struct MarchRing {
+    // FP64 without plasticity requests one row ahead into VGPRs instead (its loop reads nothing
+    // else from memory, and the ring's extra loads and LDS reads measured slower there)
+    static constexpr bool on = sizeof(T) == sizeof(float) || PL;
+    // an element is WORDS dwords, each plane row of a slot WORDS loads of one dword per lane (FP64:
+    // low words, then high words); a slot holds NPL planes (gam only with plasticity) and a row of
+    // the strip stores ROW_STORES planes (lam and gam only with plasticity).  As many slots, at most
+    // MARCH_RING, as keep the ring's operations that can be in flight at a wait -- the slot's own
+    // loads, the later slots' and the stores of RING - 1 rows -- within what the 6-bit counter holds
+    // (flux-register stores of hierarchy levels come on top)
+    static constexpr int WORDS = (int)(sizeof(T) / sizeof(float));
+    static constexpr int NPL = PL ? MARCH_RING_LOADS : MARCH_RING_LOADS - 1;
+    static constexpr int SLOT_LOADS = NPL * WORDS;
+    static constexpr int ROW_STORES = PL ? MARCH_ROW_STORES : MARCH_ROW_STORES - 2;
+    static constexpr int RING_FIT = (63 + ROW_STORES) / (SLOT_LOADS + ROW_STORES);
+    static constexpr int RING = RING_FIT < MARCH_RING ? RING_FIT : MARCH_RING;
+    static_assert(RING >= 2 && RING * SLOT_LOADS + (RING - 1) * ROW_STORES <= 63, "vmcnt counts to 63");
+    static constexpr int RING_FLOATS = (on ? RING * SLOT_LOADS : 0) * 64;
+    static constexpr int LDS_FLOATS = RING_FLOATS + 16 + 4 * 64;
+};
+
+// One side sd of strip tl, marched by one wavefront whose LDS is ring[0, LDS_FLOATS).  tl, sd and
+// ring are the same in every lane and held in scalar registers, so every plane pointer and
+// descriptor of the side stays in scalar registers.
 // PL: the launch may hold scenarios with plasticity.  Without (PL false), a row neither reads gam
 // nor writes lam and gam, and a scenario with plasticity is an error.
 template <typename T, int PK, bool PL>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(sizeof(T) == sizeof(float) ? 4 : 1)))
-k_godunov_march(const KArgs<T> a)
+__device__ __forceinline__ void march_strip(const KArgs<T>& a, const Tile& tl, const int sd, const int lane,
+                                            float* const ring)
 {
     static_assert(PK == PK_PPM_PRIM, "row marching carries PPM with primitive limiting");
-    const Tile tl = a.tiles[blockIdx.x >> 1];
     const Patch<T>& pt = a.patches[tl.patch];
     Scen& S = a.scen[pt.scen];
     const DevParams& P = S.P;
     if (!march_interior(tl, P)) {
-        if (threadIdx.x == 0 && (blockIdx.x & 1) == 0) report(&S.err, TMK_E_BOX);
+        if (lane == 0 && sd == 0) report(&S.err, TMK_E_BOX);
         return;
     }
     const Mat<T> m(P);
-    const int lane = threadIdx.x;
-    const int sd = blockIdx.x & 1;  // side of this wavefront
     const int i = tl.x0 - 3 + lane;
     const int tnx = tl.x1 - tl.x0 + 1;
     const bool valid = lane >= 3 && lane <= tnx + 2;  // column of the strip
@@ -210,7 +230,7 @@ k_godunov_march(const KArgs<T> a)
     const T rvy = sd ? rv1 : (T)1;  // velocity sign of this side in y
     const T scx = sd ? rv1 * scale : scale;
     if (!PL && P.plast && a.plastic) {
-        if (threadIdx.x == 0 && (blockIdx.x & 1) == 0) report(&S.err, TMK_E_ARG);
+        if (lane == 0 && sd == 0) report(&S.err, TMK_E_ARG);
         return;
     }
     const bool plastic = PL && P.plast && a.plastic;
@@ -242,26 +262,10 @@ k_godunov_march(const KArgs<T> a)
     const int rlast = y1 + 3;  // the last row loaded (row y1 is updated after it)
     constexpr bool f32 = sizeof(T) == sizeof(float);
     constexpr bool peel = !f32;  // the first two rows of the march as code of their own
-    // FP64 without plasticity requests one row ahead into VGPRs instead (its loop reads nothing
-    // else from memory, and the ring's extra loads and LDS reads measured slower there)
-    constexpr bool ring_fetch = f32 || PL;
-    // the ring: an element is WORDS dwords, each plane row of a slot WORDS loads of one dword per
-    // lane (FP64: low words, then high words); a slot holds NPL planes (gam only with plasticity)
-    // and a row of the strip stores ROW_STORES planes (lam and gam only with plasticity).  As many
-    // slots, at most MARCH_RING, as keep the ring's operations that can be in flight at a wait --
-    // the slot's own loads, the later slots' and the stores of RING - 1 rows -- within what the
-    // 6-bit counter holds (flux-register stores of hierarchy levels come on top)
-    constexpr int WORDS = (int)(sizeof(T) / sizeof(float));
-    constexpr int NPL = PL ? MARCH_RING_LOADS : MARCH_RING_LOADS - 1;
-    constexpr int SLOT_LOADS = NPL * WORDS;
-    constexpr int ROW_STORES = PL ? MARCH_ROW_STORES : MARCH_ROW_STORES - 2;
-    constexpr int RING_FIT = (63 + ROW_STORES) / (SLOT_LOADS + ROW_STORES);
-    constexpr int RING = RING_FIT < MARCH_RING ? RING_FIT : MARCH_RING;
-    static_assert(RING >= 2 && RING * SLOT_LOADS + (RING - 1) * ROW_STORES <= 63, "vmcnt counts to 63");
-    // one LDS object: the ring, then the plastic return's constants (PlasticConstL for FP32,
-    // PlasticConstL64 for FP64), then the lanes' flux-register face masks (below)
-    constexpr int RING_FLOATS = (ring_fetch ? RING * SLOT_LOADS : 0) * 64;
-    __shared__ float ring[RING_FLOATS + 16 + 4 * 64];
+    using R = MarchRing<T, PL>;
+    constexpr bool ring_fetch = R::on;
+    constexpr int WORDS = R::WORDS, NPL = R::NPL, SLOT_LOADS = R::SLOT_LOADS, ROW_STORES = R::ROW_STORES;
+    constexpr int RING = R::RING, RING_FLOATS = R::RING_FLOATS;
     float* const pconst = &ring[RING_FLOATS];
     if constexpr (f32) {
         if (lane < 14) pconst[lane] = lane < 7 ? P.pbg[lane] : lane < 13 ? P.pf[lane - 7] : P.fG;
