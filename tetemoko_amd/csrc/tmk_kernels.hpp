@@ -405,34 +405,37 @@ __device__ __forceinline__ void update_cell(const KArgs<T>& a, const Patch<T>& p
 // the half-step fault solve of face i: its face states, and the half step's psi (rate-and-state) or
 // slip total (slip weakening), the only fault data of the half step that the final solve reads
 template <typename T, int NS>
-__device__ __forceinline__ double fault_half(const Patch<T>& pt, const DevParams& P, int i, double dt,
+__device__ __forceinline__ void fault_load(const Patch<T>& pt, const DevParams& P, int i, FaultFace& f)
+{
+    const double s0 = gmem(pt.bin)[(size_t)(i - pt.blo0) + (size_t)(P.fault_kind == 0 ? 10 : 7) * (size_t)pt.bnx];
+    fault_face(P, i, s0, f);
+}
+
+template <typename T, int NS>
+__device__ __forceinline__ double fault_half(const DevParams& P, int i, const FaultFace& f, double dt,
                                              const FaultIn& fin, FaultOut& fo, int* errp)
 {
-    const size_t bi = (size_t)(i - pt.blo0);
-    const size_t bp = (size_t)pt.bnx;
     if (P.fault_kind == 0) {
-        const double psi = gmem(pt.bin)[bi + 10 * bp];
-        rs_fault(P, i, psi, fin, fo);
+        rs_fault(P, f, f.s0, fin, fo);
         // RSSETBND into the half-step copy (RSIBC.cpp:325-333): only psi is consumed
         const double Vx = fo.vx[0] - fo.vx[1];
         const double Vz = NS == 3 ? fo.vz[0] - fo.vz[1] : 0.0;
         const double V = sqrt(Vx * Vx + Vz * Vz);
-        const double half = rs_psi_update(P, i, psi, V, 0.5 * dt);
+        const double half = rs_psi_update(P, i, f, f.s0, V, 0.5 * dt);
         if (isnan(half)) report(errp, TMK_E_PSI_NAN);
         return half;
     }
-    const double slip = gmem(pt.bin)[bi + 7 * bp];
-    sw_fault(P, i, slip, fin, fo);
+    sw_fault(P, i, f, f.s0, fin, fo);
     const double Vx = fo.vx[0] - fo.vx[1];
     const double Vz = NS == 3 ? fo.vz[0] - fo.vz[1] : 0.0;
     const double V = sqrt(Vx * Vx + Vz * Vz);
-    return slip + (0.5 * dt) * V;
+    return f.s0 + (0.5 * dt) * V;
 }
 
 // the final fault solve of face i from the half step's state, and its new fault data
 template <typename T, int NS>
-__device__ __forceinline__ void fault_final(const Patch<T>& pt, const DevParams& P, int i, double time, double dt,
-                                            double half, const FaultIn& fin, FaultOut& fo, int* errp)
+__device__ __forceinline__ void fault_final(const Patch<T>& pt, const DevParams& P, int i, const FaultFace& f,
+                                            double time, double dt, double half, const FaultIn& fin, FaultOut& fo, int* errp)
 {
     const size_t bi = (size_t)(i - pt.blo0);
     const size_t bp = (size_t)pt.bnx;
@@ -440,20 +443,17 @@ __device__ __forceinline__ void fault_final(const Patch<T>& pt, const DevParams&
     __attribute__((address_space(1))) double* Bo = gmem(pt.bout);
     const double tnew = time + dt;
     if (P.fault_kind == 0) {
-        rs_fault(P, i, half, fin, fo);
+        // the old fault data, loaded ahead of the solve
+        const double dX = B[bi + 6 * bp], dZ = B[bi + 7 * bp], dT = B[bi + 8 * bp], RT = B[bi + 9 * bp];
+        rs_fault(P, f, half, fin, fo);
         // RSSETBND final (RSIBCF.ChF:61-151) on m_bdryData
-        const double x = (i + 0.5) * P.dx - P.x0;
-        double tau_xy_0 = P.nsig * gaussianfunc(P.r0, x);
-        if (P.f_tau) tau_xy_0 = tau_xy_0 + face_val(P.f_tau, P, i, 0.0);
         const double Vx = fo.vx[0] - fo.vx[1];
         const double Vz = NS == 3 ? fo.vz[0] - fo.vz[1] : 0.0;
         const double V = sqrt(Vx * Vx + Vz * Vz);
-        const double dX = B[bi + 6 * bp], dZ = B[bi + 7 * bp], dT = B[bi + 8 * bp];
-        const double RT = B[bi + 9 * bp], psi = B[bi + 10 * bp];
         Bo[bi + 0 * bp] = Vx;
         Bo[bi + 1 * bp] = Vz;
         Bo[bi + 2 * bp] = V;
-        Bo[bi + 3 * bp] = fo.sxy[0] + tau_xy_0;
+        Bo[bi + 3 * bp] = fo.sxy[0] + f.tau0;
         Bo[bi + 4 * bp] = (NS == 3 ? fo.syz[0] : 0.0) + 0.0;
         Bo[bi + 6 * bp] = dX + dt * Vx;
         Bo[bi + 7 * bp] = dZ + dt * Vz;
@@ -462,16 +462,15 @@ __device__ __forceinline__ void fault_final(const Patch<T>& pt, const DevParams&
         else if (RT > tnew) Bo[bi + 9 * bp] = 1e10;
         else Bo[bi + 9 * bp] = RT;
         Bo[bi + 5 * bp] = fo.syy[0];
-        const double np = rs_psi_update(P, i, psi, V, dt);
+        const double np = rs_psi_update(P, i, f, f.s0, V, dt);
         if (isnan(np)) report(errp, TMK_E_PSI_NAN);
         Bo[bi + 10 * bp] = np;
     } else {
-        sw_fault(P, i, half, fin, fo);
+        const double b5 = B[bi + 5 * bp], b6 = B[bi + 6 * bp], b8 = B[bi + 8 * bp];
+        sw_fault(P, i, f, half, fin, fo);
         // SWSETBND final (SWIBCF.ChF:32-72) on m_bdryData (Bout aliases Bin)
         const double Vx = fo.vx[0] - fo.vx[1];
         const double Vz = NS == 3 ? fo.vz[0] - fo.vz[1] : 0.0;
-        const double b5 = B[bi + 5 * bp], b6 = B[bi + 6 * bp], b7 = B[bi + 7 * bp];
-        const double b8 = B[bi + 8 * bp];
         const double V = sqrt(Vx * Vx + Vz * Vz);
         Bo[bi + 0 * bp] = Vx;
         Bo[bi + 1 * bp] = Vz;
@@ -480,7 +479,7 @@ __device__ __forceinline__ void fault_final(const Patch<T>& pt, const DevParams&
         Bo[bi + 4 * bp] = V;
         Bo[bi + 5 * bp] = b5 + dt * Vx;
         Bo[bi + 6 * bp] = b6 + dt * Vz;
-        Bo[bi + 7 * bp] = b7 + dt * V;
+        Bo[bi + 7 * bp] = f.s0 + dt * V;
         Bo[bi + 8 * bp] = (b8 > tnew && V > P.sw_thr) ? tnew : b8;
     }
 }
@@ -600,6 +599,7 @@ __device__ __forceinline__ void godunov_tile(const KArgs<T>& a, const Tile& tl, 
 
     // ---------------- stage 3: predictor face states ----------------
     Slots<T, NS> H0, H1;
+    FaultFace ff;            // of a lane on a fault face
     double tmp_state = 0.0;  // RS: psi of the half step; SW: slip-total of the half step
     {
         T cpx[2][NS], cpy[2][NS];
@@ -645,7 +645,8 @@ __device__ __forceinline__ void godunov_tile(const KArgs<T>& a, const Tile& tl, 
                     FaultIn fin;
                     fault_input<T, NS>(P, WmY, fin);
                     FaultOut fo;
-                    tmp_state = fault_half<T, NS>(pt, P, i, dt, fin, fo, errp);
+                    fault_load<T, NS>(pt, P, i, ff);
+                    tmp_state = fault_half<T, NS>(P, i, ff, dt, fin, fo, errp);
                     fault_output<T, NS>(P, fo, H1);
                 }
             } else {
@@ -743,7 +744,7 @@ __device__ __forceinline__ void godunov_tile(const KArgs<T>& a, const Tile& tl, 
                     FaultIn fin;
                     fault_input<T, NS>(P, WmY, fin);
                     FaultOut fo;
-                    fault_final<T, NS>(pt, P, i, time, dt, tmp_state, fin, fo, errp);
+                    fault_final<T, NS>(pt, P, i, ff, time, dt, tmp_state, fin, fo, errp);
                     fault_output<T, NS>(P, fo, F1);
                 }
             } else {

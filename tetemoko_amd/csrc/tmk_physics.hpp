@@ -643,6 +643,111 @@ __device__ __forceinline__ double rs_newton(const DevParams& P, double phi, doub
     return alpha * asinh(beta * V);
 }
 
+// 1 / x, to about an ulp: the hardware's estimate and two Newton steps
+__device__ __forceinline__ double fast_rcp(double x)
+{
+    double r = __builtin_amdgcn_rcp(x);
+    r = fma(fma(-x, r, 1.0), r, r);
+    return fma(fma(-x, r, 1.0), r, r);
+}
+
+// Where RSNEWTON's bracketed iteration stops, relative to the root V* it approaches: its last
+// iterate is V* (1 + d), |d| up to 1e-12 or so (it stops at |f| <= atol).  In t = V / V* the iteration
+// needs no asinh: on the range rs_solve admits, f / alpha = ln t + r (t - 1) with r = eta V* / alpha
+// to within 1 / (2 beta V)^2, so its steps are
+//   from t > e^(1 + r) a Newton step would leave the bracket below: V halves (the bracket's lower
+//   end is 0 until an iterate lies left of the root), the same number of times for any t: counted;
+//   Newton steps on t elsewhere, in l = ln t and, within 5 %, in d = t - 1, where the step is
+//   d' = (d / (1 + d) - ln(1 + d)) / (1 / (1 + d) + r), a series in d.
+// FP32 carries d to a few parts in 1e5 (each step's d' depends on the last d's relative error
+// twice over), so V comes out as the iteration's to about 1e-16.
+__device__ __forceinline__ float rs_stop(float l, float r, float falpha, float atol)
+{
+    constexpr float ln2 = 0.69314718f;
+    const float c = 1.0f + r;
+    if (l > c) l -= ln2 * ceilf((l - c) * (1.0f / ln2));
+    for (int it = 0; it < 64 && fabsf(l) > 0.05f; ++it) {
+        const float t = __builtin_amdgcn_exp2f(l * (1.0f / ln2));
+        const float q = 1.0f - (l + r * (t - 1.0f)) / (1.0f + r * t);
+        l += q > 1e-6f ? ln2 * __builtin_amdgcn_logf(q) : -ln2;
+    }
+    float d = l * (1.0f + l * (0.5f + l * (1.0f / 6.0f + l * (1.0f / 24.0f))));
+    for (int it = 0; it < 8; ++it) {
+        const float n = d * d * (0.5f - d * (2.0f / 3.0f - d * (0.75f - d * (0.8f - d * (5.0f / 6.0f)))));
+        d = -n / (1.0f / (1.0f + d) + r);
+        if (falpha * fabsf(c * d) <= atol) break;
+    }
+    return d;
+}
+
+// RSNEWTON: the root of alpha asinh(beta V) + eta V = phi (alpha = sn a, beta = exp(psi / a) / (2 V0),
+// eta = Zs / 2), solved in y = asinh(beta V): alpha y + kappa sinh(y) = phi with kappa = eta / beta.  In
+// V the root lies 20 to 50 factors of e below the bracket's top and the bracketed iteration halves its
+// way down (30 to 60 evaluations of asinh where the predictor's trace is no guess); in y the left side
+// is convex and increasing, so Newton from a guess clamped to [0, phi / alpha] (where the left side is
+// no smaller than phi) converges from any start.  The guess takes sinh y = e^y / 2: then w = phi / alpha
+// - y solves w + ln w = L = phi / alpha + ln(kappa / (2 alpha)), two Newton steps in FP32 with the
+// hardware's exp2 and log2; from there two FP64 steps reach rounding level (a step of at most 1e-7
+// leaves an error of its square, 1e-14 at most in y, the unit in the last place of y itself).  The last
+// iterate of the reference's iteration is then placed beside the root (rs_stop).
+// What bounds it: one lane per face, a chain of dependent FP64 operations.  A step of the 261 x 131
+// rate-and-state FP32 level, whose length is that of one fault piece with its two solves, fell from
+// 70 to 19.4 us (14.6 with slip weakening in place of the solves), 1024 x 512 from 76 to 25.
+// Outside the range this holds for (compression and a positive load, |psi / a| < 600, y > 15, a root
+// between 2^-80 of the bracket's top and the top) the reference's own iteration runs (rs_newton), which
+// also decides what an unordered or unreachable case returns.
+__device__ __forceinline__ double rs_solve(const DevParams& P, double phi, double psi, double sn, double c_rs_a,
+                                           double& Vio)
+{
+    const double alpha = sn * c_rs_a, q = psi / c_rs_a, eta = 0.5 * P.Zs;
+    const double Vmax = phi / P.Zs;
+    if (alpha > 0.0 && phi > 0.0 && fabs(q) < 600.0 && phi < 1e100) {
+        constexpr float ln2 = 0.69314718f;
+        const double ia = fast_rcp(alpha);
+        const double ymax = phi * ia;
+        const double E = exp(-q), k = (eta * P.rs_V0) * E;  // kappa / 2
+        const float L = (float)(ymax - q) + ln2 * __builtin_amdgcn_logf((float)(eta * P.rs_V0 * ia));
+        float w = __builtin_amdgcn_exp2f((1.0f / ln2) * fminf(L, 1.0f));
+        w = w / (1.0f + w);
+        if (L > 1.0f) w = L - ln2 * __builtin_amdgcn_logf(L);
+        if (w > 1e-20f) {
+#pragma unroll
+            for (int it = 0; it < 2; ++it) w = w * (1.0f + L - ln2 * __builtin_amdgcn_logf(w)) / (1.0f + w);
+        }
+        const double top = fmin(ymax, 690.0);
+        double y = fmin(fmax(ymax - (double)w, 0.0), top), e = 1.0, dy = 1.0;
+        for (int it = 0; it < 64; ++it) {
+            e = exp(y);
+            const double up = k * e, dn = k * fast_rcp(e);
+            const double g = fma(alpha, y, -phi) + (up - dn);
+            const double yn = fmin(fmax(fma(-g, fast_rcp(alpha + (up + dn)), y), 0.0), top);
+            dy = yn - y;
+            y = yn;
+            if (fabs(dy) <= 1e-7) break;
+        }
+        e = e * fma(dy, fma(dy, 0.5, 1.0), 1.0);  // exp(y) from exp(y - dy)
+        const double V = (P.rs_V0 * E) * (e - fast_rcp(e));
+        if (fabs(dy) <= 1e-7 && y > 15.0 && V <= Vmax && V > Vmax * 0x1p-80) {
+            // the iteration's start; from (nearly) rest its first step is taken as it is written, since
+            // asinh(beta V) is no logarithm there
+            double V1 = Vio;
+            if (V1 < 0.0 || V1 > Vmax) V1 = Vmax / 2.0;
+            const double beta = (0.5 / P.rs_V0) * fast_rcp(E);
+            if (beta * V1 < 30.0) {
+                const double x = beta * V1;
+                const double f = alpha * asinh(x) + eta * V1 - phi;
+                V1 = V1 - f / (alpha * beta / sqrt(x * x + 1.0) + eta);
+                if (V1 > Vmax) V1 = Vmax / 2.0;
+            }
+            const float l = (float)log(V1 * fast_rcp(V));
+            const double d = (double)rs_stop(l, (float)(eta * V * ia), (float)alpha, 2.220446e-12f);
+            Vio = fma(V, d, V);
+            return fma(alpha, d, alpha * y);
+        }
+    }
+    return rs_newton(P, phi, psi, sn, c_rs_a, Vio);
+}
+
 // inside state of a fault face (W- of the cell above, physical components)
 struct FaultIn {
     double vx[2], vy[2], vz[2], syy[2], sxy[2], syz[2];
@@ -656,64 +761,69 @@ __device__ __forceinline__ double ramp_of(const DevParams& P, double x)
     return fmin(1.0, fmax(0.0, (x - P.ramp_x) / P.ramp_w));
 }
 
+// what the two solves and the update of one fault face read besides the state's traces: the face's
+// parameters, its initial state variable and the terms that depend on neither the traces nor the slip
+// rate.  Gathered once per face, ahead of the solves, so that the loads' latency is not in their chain.
+struct FaultFace {
+    double s0;    // psi (rate-and-state) or slip total (slip weakening) at the step's start
+    double tau0;  // the fault's own shear load
+    double syy;   // fault-local normal stress
+    double a, b, L;  // rate-and-state a, b, L; slip weakening: static and dynamic friction, weakening slip
+    double theta;    // aging law: exp((f0 - psi) / b) at the step's start
+};
+
 // RSFAULTBCF (RSIBCF.ChF:158-323)
-__device__ __forceinline__ void rs_fault(const DevParams& P, int i, double psi, const FaultIn& in, FaultOut& o)
+__device__ __forceinline__ void rs_fault(const DevParams& P, const FaultFace& f, double psi, const FaultIn& in, FaultOut& o)
 {
     const double Zp = P.Zp, Zs = P.Zs;
-    const double x = (i + 0.5) * P.dx - P.x0;
     const double wpxy1 = -in.sxy[0] - Zs * in.vx[0];
     const double wpyy1 = -in.syy[0] - Zp * in.vy[0];
     const double wpxy2 = in.sxy[1] - Zs * in.vx[1];
     const double wpyy2 = in.syy[1] - Zp * in.vy[1];
     const double wpyz1 = 0.0, wpyz2 = 0.0;
-    double tau_xy_0 = P.nsig * gaussianfunc(P.r0, x);
-    if (P.f_tau) tau_xy_0 = tau_xy_0 + face_val(P.f_tau, P, i, 0.0);
+    const double tau_xy_0 = f.tau0;
     const double tau_yz_0 = 0.0;
     const double phi_xy = 0.5 * (wpxy2 - wpxy1) + tau_xy_0;
     const double phi_yz = 0.5 * (wpyz2 - wpyz1) + tau_yz_0;
     const double phi = sqrt(phi_xy * phi_xy + phi_yz * phi_yz);
     const double syy = -((wpyy1 - wpyy2) / 2.0);
-    const double vy = -((wpyy1 + wpyy2) / 2.0 / Zp);
+    const double vy = -divr((wpyy1 + wpyy2) / 2.0, Zp, P.iZp);
     const double dvx = in.vx[0] - in.vx[1], dvz = in.vz[0] - in.vz[1];
     double V = sqrt(dvx * dvx + dvz * dvz);
-    const double c_rs_a = face_val(P.f_a, P, i, P.rs_a) + P.ramp_a * ramp_of(P, x);
     double sn = -syy;
-    if (P.f_syy) sn = -(syy + face_val(P.f_syy, P, i, 0.0));
-    const double tau = rs_newton(P, phi, psi, sn, c_rs_a, V);
+    if (P.f_syy) sn = -(syy + f.syy);
+    const double tau = rs_solve(P, phi, psi, sn, f.a, V);
     const double sxy = (phi_xy / phi) * tau - tau_xy_0;
     const double syz = (phi_yz / phi) * tau - tau_yz_0;
     const double Vx = (phi_xy / phi) * V;
     const double Vz = (phi_yz / phi) * V;
-    const double vx1 = -((sxy + wpxy1) / Zs);
-    const double vz1 = -((syz + wpyz1) / Zs);
+    const double vx1 = -divr(sxy + wpxy1, Zs, P.iZs);
+    const double vz1 = -divr(syz + wpyz1, Zs, P.iZs);
     o.vx[0] = vx1; o.vy[0] = vy; o.vz[0] = vz1; o.syy[0] = syy; o.sxy[0] = sxy; o.syz[0] = syz;
     o.vx[1] = vx1 - Vx; o.vy[1] = vy; o.vz[1] = vz1 - Vz; o.syy[1] = syy; o.sxy[1] = sxy; o.syz[1] = syz;
 }
 
 // RSSETBND psi update (RSIBCF.ChF:125-146) and the aging-law extension
-__device__ __forceinline__ double rs_psi_update(const DevParams& P, int i, double psi, double V, double dt)
+__device__ __forceinline__ double rs_psi_update(const DevParams& P, int i, const FaultFace& f, double psi, double V,
+                                                double dt)
 {
-    const double x = (i + 0.5) * P.dx - P.x0;
-    const double c_ramp = ramp_of(P, x);
-    const double c_rs_a = face_val(P.f_a, P, i, P.rs_a) + P.ramp_a * c_ramp;
-    const double L = face_val(P.f_L, P, i, P.rs_L);
-    const double b = face_val(P.f_b, P, i, P.rs_b);
     if (P.state_law == 0) {
-        const double f = c_rs_a * asinh(V * exp(psi / c_rs_a) / (2.0 * P.rs_V0));
-        double fss = P.rs_f0 - (b - c_rs_a) * log(V / P.rs_V0);
+        const double ff = f.a * asinh(V * exp(psi / f.a) / (2.0 * P.rs_V0));
+        double fss = P.rs_f0 - (f.b - f.a) * log(V / P.rs_V0);
         if (P.rs_fexp > 0.0) {
-            const double c_rs_Vw = P.rs_Vw + P.ramp_Vw * c_ramp;
+            const double x = (i + 0.5) * P.dx - P.x0;
+            const double c_rs_Vw = P.rs_Vw + P.ramp_Vw * ramp_of(P, x);
             const double r = V / c_rs_Vw;
             const double r2 = r * r, r4 = r2 * r2, r8 = r4 * r4;
             fss = P.rs_fw + (fss - P.rs_fw) / pow(1.0 + r8, 0.125);
         }
-        return psi - dt * (V / L) * (f - fss);
+        return psi - dt * (V / f.L) * (ff - fss);
     }
-    return psi + dt * (b * P.rs_V0 / L) * (exp((P.rs_f0 - psi) / b) - V / P.rs_V0);
+    return psi + dt * (f.b * P.rs_V0 / f.L) * (f.theta - V / P.rs_V0);  // psi is the step's own (f.s0)
 }
 
 // SWFAULTBCF (SWIBCF.ChF:79-267), side 2 at IX2_* = 11+n; slip = fault slip-total
-__device__ __forceinline__ void sw_fault(const DevParams& P, int i, double slip, const FaultIn& in, FaultOut& o)
+__device__ __forceinline__ void sw_fault(const DevParams& P, int i, const FaultFace& f, double slip, const FaultIn& in, FaultOut& o)
 {
     const double Zp = P.Zp, Zs = P.Zs;
     const double x = (i + 0.5) * P.dx - P.fric_c0;
@@ -723,37 +833,56 @@ __device__ __forceinline__ void sw_fault(const DevParams& P, int i, double slip,
     const double wpxy2 = in.sxy[1] - Zs * in.vx[1];
     const double wpyy2 = in.syy[1] - Zp * in.vy[1];
     const double wpyz2 = in.syz[1] - Zs * in.vz[1];
-    double tau_0 = 0.0;
-    for (int ip = 0; ip < P.npatch; ++ip) {
-        const double valx = smoothfunc(P.sm, fabs(x - P.xc[ip]) - P.xw[ip]);
-        tau_0 = tau_0 + P.taup[ip] * valx;
-    }
-    if (P.f_tau) tau_0 = tau_0 + face_val(P.f_tau, P, i, 0.0);
+    const double tau_0 = f.tau0;
     const double ta = 0.5 * (wpxy2 - wpxy1) + tau_0;
     const double tb = 0.5 * (wpyz2 - wpyz1);
     const double tau_lock = sqrt(ta * ta + tb * tb);
     const double syy = -((wpyy1 - wpyy2) / 2.0);
-    const double vy = -((wpyy1 + wpyy2) / 2.0 / Zp);
+    const double vy = -divr((wpyy1 + wpyy2) / 2.0, Zp, P.iZp);
     const double valx = (fabs(x) >= P.fric_w0) ? 0.0 : 1.0;
-    const double fs = face_val(P.f_fs, P, i, P.fs);
-    const double fd = face_val(P.f_fd, P, i, P.fd);
-    const double dw = face_val(P.f_dc, P, i, P.dw);
-    double fric = fs * valx + (1.0 - valx) * P.outside_f;
-    fric = fric - (fric - fd) * fmin(1.0, slip / dw);
+    double fric = f.a * valx + (1.0 - valx) * P.outside_f;
+    fric = fric - (fric - f.b) * fmin(1.0, slip / f.L);
     double sn_syy = syy;
-    if (P.f_syy) sn_syy = syy + face_val(P.f_syy, P, i, 0.0);
+    if (P.f_syy) sn_syy = syy + f.syy;
     const double tau = fmin(tau_lock, -sn_syy * fric) - tau_0;
     const double phi_xy = 0.5 * (wpxy2 - wpxy1);
     const double phi_yz = 0.5 * (wpyz2 - wpyz1);
     const double phi = sqrt(phi_xy * phi_xy + phi_yz * phi_yz);
     const double sxy = (phi_xy / phi) * tau;
     const double syz = (phi_yz / phi) * tau;
-    o.vx[0] = -((sxy + wpxy1) / Zs);
-    o.vz[0] = -((syz + wpyz1) / Zs);
+    o.vx[0] = -divr(sxy + wpxy1, Zs, P.iZs);
+    o.vz[0] = -divr(syz + wpyz1, Zs, P.iZs);
     o.vy[0] = vy; o.syy[0] = syy; o.sxy[0] = sxy; o.syz[0] = syz;
-    o.vx[1] = (sxy - wpxy2) / Zs;
-    o.vz[1] = (syz - wpyz2) / Zs;
+    o.vx[1] = divr(sxy - wpxy2, Zs, P.iZs);
+    o.vz[1] = divr(syz - wpyz2, Zs, P.iZs);
     o.vy[1] = vy; o.syy[1] = syy; o.sxy[1] = sxy; o.syz[1] = syz;
+}
+
+// the fault face i, s0 its state variable
+__device__ __forceinline__ void fault_face(const DevParams& P, int i, double s0, FaultFace& f)
+{
+    f.s0 = s0;
+    f.syy = face_val(P.f_syy, P, i, 0.0);
+    if (P.fault_kind == 0) {
+        const double x = (i + 0.5) * P.dx - P.x0;
+        f.a = face_val(P.f_a, P, i, P.rs_a) + P.ramp_a * ramp_of(P, x);
+        f.b = face_val(P.f_b, P, i, P.rs_b);
+        f.L = face_val(P.f_L, P, i, P.rs_L);
+        f.tau0 = P.nsig * gaussianfunc(P.r0, x);
+        f.theta = P.state_law == 0 ? 0.0 : exp((P.rs_f0 - s0) / f.b);
+    } else {
+        const double x = (i + 0.5) * P.dx - P.fric_c0;
+        f.a = face_val(P.f_fs, P, i, P.fs);
+        f.b = face_val(P.f_fd, P, i, P.fd);
+        f.L = face_val(P.f_dc, P, i, P.dw);
+        f.theta = 0.0;
+        f.tau0 = 0.0;
+        for (int ip = 0; ip < P.npatch; ++ip) {
+            const double valx = smoothfunc(P.sm, fabs(x - P.xc[ip]) - P.xw[ip]);
+            f.tau0 = f.tau0 + P.taup[ip] * valx;
+        }
+    }
+    if (P.f_tau) f.tau0 = f.tau0 + face_val(P.f_tau, P, i, 0.0);
 }
 
 // PLASTICFLOW + INVARIANTS + YIELD (PlasticPhysicsF.ChF:74-181)

@@ -201,15 +201,17 @@ __device__ __forceinline__ void bnd_piece(const KArgs<T>& a, const Tile& tl, T* 
         }
     };
 
+    const bool yf = ly >= 1 && ly <= tny + 1 && colD && lx <= tnx + 1 && j <= dhi1 + 1;
+    const bool fault_face = yf && lo_y;
+    FaultFace ff;
+    if (fault_face && sd == 0 && pt.bin) fault_load<T, 2>(pt, P, i, ff);
     put_chars();
     __syncthreads();
     // ---------------- predictor face states ----------------
     T xv[2] = {(T)0, (T)0}, xs[2] = {(T)0, (T)0}, yv[2] = {(T)0, (T)0}, ys[2] = {(T)0, (T)0};
     double half = 0.0;  // psi or slip total of the half step
     if (lx >= 1 && lx <= tnx + 1 && rowD && ly <= tny + 1 && i <= dhi0 + 1) x_face(xv, xs);
-    const bool yf = ly >= 1 && ly <= tny + 1 && colD && lx <= tnx + 1 && j <= dhi1 + 1;
     if (yf && !lo_y) y_face(yv, ys);
-    const bool fault_face = yf && lo_y;
     if (fault_face && sd == 0) {
         if (!pt.bin) {
             report(errp, TMK_E_NO_BDRY);
@@ -217,7 +219,7 @@ __device__ __forceinline__ void bnd_piece(const KArgs<T>& a, const Tile& tl, T* 
             FaultIn fin;
             FaultOut fo;
             traces(fin);
-            half = fault_half<T, 2>(pt, P, i, dt, fin, fo, errp);
+            half = fault_half<T, 2>(P, i, ff, dt, fin, fo, errp);
             fault_states(fo, yv, ys);
         }
     }
@@ -253,7 +255,7 @@ __device__ __forceinline__ void bnd_piece(const KArgs<T>& a, const Tile& tl, T* 
         FaultIn fin;
         FaultOut fo;
         traces(fin);
-        fault_final<T, 2>(pt, P, i, S.time[a.par], dt, half, fin, fo, errp);
+        fault_final<T, 2>(pt, P, i, ff, S.time[a.par], dt, half, fin, fo, errp);
         fault_states(fo, yv, ys);
     }
     put_faces(xv, xs, yv, ys, !(fault_final_face && sd == 1));
