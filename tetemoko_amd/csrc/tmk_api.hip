@@ -1061,12 +1061,21 @@ static int group_exchange_now_t(Group& G, hipStream_t st)
     return TMK_OK;
 }
 
-// n steps; a two-step graph (parities 0 -> 1 -> 0) is captured once per group
-// layout and dt and replayed
+// n steps.  A marching step is one launch (plus the exchange and the stations where there are any),
+// enqueued as it is: back to back such launches leave no gap on the device and cost the host less
+// than the step takes, where a graph of two steps left 9 us between replays (400 x 200 slip weakening
+// FP64 16.7 -> 14.3 us per step, a first run of 400 steps 7.5 -> 6.1 ms without the capture; graphs of
+// 8 and 32 steps 14.8 and 14.3).  The tile kernels' step, two streams joined by events, is captured
+// as a two-step graph (parities 0 -> 1 -> 0) once per group layout and dt and replayed.
 static int group_run(Group& G, hipStream_t st, int nsteps)
 {
     int e;
     if (nsteps <= 0) return TMK_OK;
+    if (G.march > 0) {
+        for (int k = 0; k < nsteps; ++k)
+            if ((e = group_enqueue_step(G, st))) return e;
+        return TMK_OK;
+    }
     if (G.g != 0) {
         if ((e = group_enqueue_step(G, st))) return e;
         --nsteps;
@@ -1995,11 +2004,27 @@ extern "C" int tmk_level_destroy(tmk_level* L)
     return TMK_OK;
 }
 
-// a box's ghosted region <-> staging array (22 planes of the ghosted box, x fastest); put
-// writes the cells the box owns and the island's ghost cells, never another box's cells
+// the level's stored form of a host value and back (FP32 bulk stores U - bg)
+template <typename T>
+__device__ __forceinline__ T to_stored(double v, double bg)
+{
+    if constexpr (stores_delta<T>()) return (T)(v - bg);
+    else return v;
+}
+template <typename T>
+__device__ __forceinline__ double from_stored(T v, double bg)
+{
+    if constexpr (stores_delta<T>()) return (double)v + bg;
+    else return v;
+}
+
+// a box's ghosted region <-> staging array (22 FP64 planes of the ghosted box, x fastest); put
+// writes the cells the box owns and the island's ghost cells, never another box's cells.  The FP32
+// bulk's conversion is done here, on values already in flight: on the host it took one thread and a
+// second array, 13 of the 18 ms of a 200-step pass over a 1024 x 512 level that reads its state.
 template <typename T>
 static __global__ void k_box_put(T* u0, T* u1, T* w, const int* owner, int aunx, size_t aplane, int ox, int oy,
-                                 const T* src, int gnx, int gny, int box)
+                                 const double* src, StateVec bg, int gnx, int gny, int box)
 {
     const size_t n = (size_t)gnx * gny;
     const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -2009,7 +2034,7 @@ static __global__ void k_box_put(T* u0, T* u1, T* w, const int* owner, int aunx,
     const int o = owner[a];
     if (o != box && o != -1) return;
     for (int c = 0; c < TMK_NCOMP; ++c) {
-        const T v = src[t + c * n];
+        const T v = to_stored<T>(src[t + c * n], bg.c[c]);
         u0[a + c * aplane] = v;
         u1[a + c * aplane] = v;
         w[a + c * aplane] = v;
@@ -2036,15 +2061,16 @@ static __global__ void k_box_const(T* u0, T* u1, T* w, const int* owner, int aun
 }
 
 template <typename T>
-static __global__ void k_box_get(const T* u, const T* w, int aunx, size_t aplane, int ox, int oy, T* dst, int gnx,
-                                 int gny, int smask)
+static __global__ void k_box_get(const T* u, const T* w, int aunx, size_t aplane, int ox, int oy, double* dst,
+                                 StateVec bg, int gnx, int gny, int smask)
 {
     const size_t n = (size_t)gnx * gny;
     const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= n) return;
     const int x = (int)(t % gnx), y = (int)(t / gnx);
     const size_t a = (size_t)(x + ox) + (size_t)(y + oy) * aunx;
-    for (int c = 0; c < TMK_NCOMP; ++c) dst[t + c * n] = ((smask >> c) & 1) ? u[a + c * aplane] : w[a + c * aplane];
+    for (int c = 0; c < TMK_NCOMP; ++c)
+        dst[t + c * n] = from_stored<T>(((smask >> c) & 1) ? u[a + c * aplane] : w[a + c * aplane], bg.c[c]);
 }
 
 // fault-data row of a box (with its ghosts) <-> the island's row
@@ -2115,26 +2141,20 @@ extern "C" int tmk_level_upload(tmk_level* L, int b, const double* U, const doub
                     if (U[k + (size_t)(11 * s + cc) * plane] != 0.0) return TMK_E_ARG;
     }
     if (L->has_b[b] && !B) return TMK_E_NO_BDRY;
-    std::vector<float> tmp;
-    const void* src = U;
-    if (L->tsize == sizeof(float)) {
-        tmp.resize(nU);
-        to_stored_f32(U, tmp.data(), plane, c->P);
-        src = tmp.data();
-    }
     HIPCHK(hipStreamSynchronize(c->stream));
     int e;
-    if ((e = c->bufs[7].ensure(nU * L->tsize))) return e;
-    HIPCHK(copy_on(c->stream, c->bufs[7].p, src, nU * L->tsize, hipMemcpyHostToDevice));
+    if ((e = c->bufs[7].ensure(nU * sizeof(double)))) return e;
+    HIPCHK(copy_on(c->stream, c->bufs[7].p, U, nU * sizeof(double), hipMemcpyHostToDevice));
+    const StateVec bg = background(c->P);
     const Island& I = L->isl[L->box_isl[b]];
     const int ox = ub.lo[0] - I.abox.lo[0], oy = ub.lo[1] - I.abox.lo[1];
     const dim3 grid((unsigned)((plane + 255) / 256));
     if (L->tsize == sizeof(double))
         hipLaunchKernelGGL(k_box_put<double>, grid, dim3(256), 0, c->stream, (double*)I.u[0], (double*)I.u[1],
-                           (double*)I.w, I.owner, I.unx(), I.plane(), ox, oy, (const double*)c->bufs[7].p, gnx, gny, b);
+                           (double*)I.w, I.owner, I.unx(), I.plane(), ox, oy, (const double*)c->bufs[7].p, bg, gnx, gny, b);
     else
         hipLaunchKernelGGL(k_box_put<float>, grid, dim3(256), 0, c->stream, (float*)I.u[0], (float*)I.u[1],
-                           (float*)I.w, I.owner, I.unx(), I.plane(), ox, oy, (const float*)c->bufs[7].p, gnx, gny, b);
+                           (float*)I.w, I.owner, I.unx(), I.plane(), ox, oy, (const double*)c->bufs[7].p, bg, gnx, gny, b);
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(c->stream));
     if (L->has_b[b] && (e = level_put_fault(L, b, B))) return e;
@@ -2193,25 +2213,19 @@ extern "C" int tmk_level_download(tmk_level* L, int b, double* U, double* B)
     const size_t plane = (size_t)gnx * gny;
     const size_t nU = plane * TMK_NCOMP;
     int e;
-    if ((e = c->bufs[7].ensure(nU * L->tsize))) return e;
+    if ((e = c->bufs[7].ensure(nU * sizeof(double)))) return e;
+    const StateVec bg = background(c->P);
     const Island& I = L->isl[L->box_isl[b]];
     const int ox = ub.lo[0] - I.abox.lo[0], oy = ub.lo[1] - I.abox.lo[1];
     const dim3 grid((unsigned)((plane + 255) / 256));
     if (L->tsize == sizeof(double))
         hipLaunchKernelGGL(k_box_get<double>, grid, dim3(256), 0, st, (const double*)I.u[L->cur], (const double*)I.w,
-                           I.unx(), I.plane(), ox, oy, (double*)c->bufs[7].p, gnx, gny, stencil_mask(L->ns));
+                           I.unx(), I.plane(), ox, oy, (double*)c->bufs[7].p, bg, gnx, gny, stencil_mask(L->ns));
     else
         hipLaunchKernelGGL(k_box_get<float>, grid, dim3(256), 0, st, (const float*)I.u[L->cur], (const float*)I.w,
-                           I.unx(), I.plane(), ox, oy, (float*)c->bufs[7].p, gnx, gny, stencil_mask(L->ns));
+                           I.unx(), I.plane(), ox, oy, (double*)c->bufs[7].p, bg, gnx, gny, stencil_mask(L->ns));
     HIPCHK(hipGetLastError());
-    HIPCHK(hipStreamSynchronize(st));
-    if (L->tsize == sizeof(double)) {
-        HIPCHK(copy_on(st, U, c->bufs[7].p, nU * sizeof(double), hipMemcpyDeviceToHost));
-    } else {
-        std::vector<float> a(nU);
-        HIPCHK(copy_on(st, a.data(), c->bufs[7].p, nU * sizeof(float), hipMemcpyDeviceToHost));
-        from_stored_f32(a.data(), U, plane, c->P);
-    }
+    HIPCHK(copy_on(st, U, c->bufs[7].p, nU * sizeof(double), hipMemcpyDeviceToHost));
     if (L->has_b[b] && B) return level_get_fault(L, b, B, st);
     return TMK_OK;
 }
