@@ -18,8 +18,10 @@ G = scenarios.GHOST
 NSTEPS = 4
 
 
-def _case(nx, ny, boxes, bc, precision, plastic=False, march=None):
+def _case(nx, ny, boxes, bc, precision, plastic=False, march=None, cs=None):
     cfg = scenarios.config_c0(seed=3, nx=nx, ny=ny, dx=100.0)
+    if cs is not None:
+        cfg["cs"] = cs
     cfg["bc"] = bc
     if plastic:
         cfg.update(plasticity=1, p_mu=0.6, p_beta=0.3, p_eta=0.03 * scenarios.G_MPA, p_b=1.0)
@@ -84,3 +86,12 @@ def test_chosen_strip_height_changes_nothing(nx, ny):
     a = _case(nx, ny, boxes, (0, 0, 0, 0), capi.PREC_FP32_BULK)
     b = _case(nx, ny, boxes, (0, 0, 0, 0), capi.PREC_FP32_BULK, march=5)
     assert np.array_equal(a[0], b[0]) and np.array_equal(a[2], b[2])
+
+
+@pytest.mark.parametrize("plastic", [False, True])
+@pytest.mark.parametrize("cs", [scenarios.CS, 3013.5])
+def test_divisions_of_either_kind(cs, plastic):
+    """A shear speed whose impedance or density does not pass the check of the two-operation division
+    (tests/test_div2.py), and the one every scenario has: both bit-identical to the oracle."""
+    Ug, Ur, Bg, Br = _case(130, 70, [(0, 0, 129, 69)], (0, 0, 0, 0), capi.PREC_FP64, plastic=plastic, cs=cs)
+    assert np.array_equal(Ug, Ur) and np.array_equal(Bg, Br)

@@ -44,8 +44,8 @@ namespace tmk {
 #define TMK_DECLARE_EXTERN(T, NS, BX, BY, PK) \
     extern template __global__ void k_godunov_interior<T, NS, BX, BY, PK>(const KArgs<T>);
 TMK_ALL_UPDATE_KERNELS(TMK_DECLARE_EXTERN, float)
-extern template __global__ void k_godunov_step<float, true>(const KArgs<float>);
-extern template __global__ void k_godunov_step<float, false>(const KArgs<float>);
+extern template __global__ void k_godunov_step<float, true, false>(const KArgs<float>);
+extern template __global__ void k_godunov_step<float, false, false>(const KArgs<float>);
 extern template __global__ void k_godunov_bnd<float, 2, PK_RUNTIME>(const KArgs<float>);
 extern template __global__ void k_godunov_bnd<float, 3, PK_RUNTIME>(const KArgs<float>);
 extern template __global__ void k_godunov_bnd<float, 2, PK_PPM_PRIM>(const KArgs<float>);
@@ -452,6 +452,7 @@ struct Group {
     int ns = 2, bx = 32, by = 16;
     int march = 0;                 // > 0: interior strips of this many rows (k_godunov_step)
     bool any_plast = true;         // some member has plasticity (the march variant with lam, gam)
+    bool div2 = false;             // every member's constants divide exactly in two operations
     int xcd = 1;                   // interior tiles / strips in XCD bands (the first member's choice)
     int pk = PK_RUNTIME;  // predictor kind the kernel is specialised for (all members agree)
     Scen* scen_dev = nullptr;
@@ -665,6 +666,41 @@ extern "C" int tmk_cache_trim(void)
     return TMK_OK;
 }
 
+// RN(1/b - y) for y = RN(1/b): the remainder 1 - b y is exact in one fma
+static double recip_low(double b, double y) { return std::fma(-b, y, 1.0) / b; }
+
+// whether divr2 by b gives the IEEE quotient for every dividend.  With b and the dividend scaled to
+// 53-bit integers Y, X and the quotient next to the midpoint (2Q + 1) / 2^p (p = 53 for X >= Y, else 54),
+// 2^p X - (2Q + 1) Y = N is a nonzero integer, and the sum under divr2's last rounding, within 2^-105 of
+// a / b, can lie on the other side of the midpoint only if |N| <= 2^(p-105) X < 4.  For each such N
+// (to 6, for margin) the odd multiples (2Q + 1) in [2^53, 2^54) with (2Q + 1) Y = -N modulo 2^p give the
+// only dividends to try.  They are few: N is a multiple of Y's power of two.
+static bool div2_exact(double b)
+{
+    if (!(b > 0.0) || !std::isnormal(b)) return false;
+    int ex;
+    const unsigned long long Y = (unsigned long long)std::ldexp(std::frexp(b, &ex), 53);
+    const double y = (double)Y, yh = 1.0 / y, yl = recip_low(y, yh);
+    int k = 0;
+    while (!((Y >> k) & 1)) ++k;
+    unsigned long long inv = 1;  // the inverse of Y's odd part modulo 2^64
+    for (int it = 0; it < 6; ++it) inv *= 2 - (Y >> k) * inv;
+    for (int p = 53; p <= 54; ++p)
+        for (long long N = -6; N <= 6; ++N) {
+            if (N == 0 || k > 2 || N % (1 << k)) continue;
+            const unsigned long long M = 1ull << (p - k);
+            unsigned long long c = (unsigned long long)(-(N / (1 << k))) * inv & (M - 1);
+            for (; c < (1ull << 54); c += M) {
+                if (c < (1ull << 53) || !(c & 1)) continue;
+                const unsigned long long X = (unsigned long long)(((unsigned __int128)c * Y + (__int128)N) >> p);
+                if (X < (1ull << 52) || X >= (1ull << 53) || (X >= Y) != (p == 53)) continue;
+                const double x = (double)X;
+                if (std::fma(x, yh, x * yl) != x / y) return false;
+            }
+        }
+    return true;
+}
+
 static void fill_dev_params(const tmk_params& h, DevParams& P)
 {
     memset(&P, 0, sizeof P);
@@ -679,6 +715,10 @@ static void fill_dev_params(const tmk_params& h, DevParams& P)
     P.irho = 1.0 / P.rho;
     P.i2Zp = 0.5 * P.iZp;
     P.i2Zs = 0.5 * P.iZs;
+    P.lZp = recip_low(P.Zp, P.iZp);
+    P.lZs = recip_low(P.Zs, P.iZs);
+    P.lrho = recip_low(P.rho, P.irho);
+    P.div2 = div2_exact(P.Zp) && div2_exact(P.Zs) && div2_exact(P.rho);
     P.K = P.lam + 2.0 * h.G / 3.0;
     P.den = 2.0 * h.G + P.lam;
     P.lam2G = P.lam + 2.0 * h.G;
@@ -946,17 +986,20 @@ static int timer_mark(const StepTimers* tm, hipStream_t s, int k)
 }
 
 // one step of a group that marches, in one launch: its boundary pieces, its interior strips and its
-// clocks; plast: some scenario of the launch has plasticity (the variant that reads and writes lam, gam)
+// clocks; plast: some scenario of the launch has plasticity (the variant that reads and writes lam,
+// gam); div2: every scenario's constants divide exactly in two operations (FP64)
 template <typename T>
-static int launch_step(hipStream_t st, const KArgs<T>& a, bool plast, const StepTimers* tm)
+static int launch_step(hipStream_t st, const KArgs<T>& a, bool plast, bool div2, const StepTimers* tm)
 {
     int e;
     if ((e = timer_mark(tm, st, 0))) return e;
-    const dim3 grid((unsigned)(a.ntiles - a.nint + (2 * a.nint + STEP_WAVES - 1) / STEP_WAVES));
-    if (plast && a.plastic)
-        hipLaunchKernelGGL((k_godunov_step<T, true>), grid, dim3(STEP_NT), 0, st, a);
-    else
-        hipLaunchKernelGGL((k_godunov_step<T, false>), grid, dim3(STEP_NT), 0, st, a);
+    const dim3 grid((unsigned)(a.ntiles - a.nint + (2 * a.nint + STEP_WAVES - 1) / STEP_WAVES)), block(STEP_NT);
+    constexpr bool d = sizeof(T) == sizeof(double);
+    const bool pl = plast && a.plastic;
+    if (pl && div2 && d) hipLaunchKernelGGL((k_godunov_step<T, true, d>), grid, block, 0, st, a);
+    else if (pl) hipLaunchKernelGGL((k_godunov_step<T, true, false>), grid, block, 0, st, a);
+    else if (div2 && d) hipLaunchKernelGGL((k_godunov_step<T, false, d>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL((k_godunov_step<T, false, false>), grid, block, 0, st, a);
     if (hipGetLastError() != hipSuccess) return TMK_E_HIP;
     return timer_mark(tm, st, 1);
 }
@@ -1013,7 +1056,7 @@ static int group_enqueue_step_t(Group& G, hipStream_t st, const StepTimers* tm =
     a.par = G.g;
     a.nint = G.nint;
     a.nscen = G.nscen;
-    int e = G.march > 0 ? launch_step<T>(st, a, G.any_plast, tm)
+    int e = G.march > 0 ? launch_step<T>(st, a, G.any_plast, G.div2, tm)
                         : launch_update<T>(st, G.side, G.ev_fork, G.ev_join, G.ns, G.pk, G.bx, G.by, a, G.nint, tm);
     if (e) return e;
     const Patch<T>* pn = (const Patch<T>*)G.patches_dev[G.g];  // its out planes hold the new state
@@ -1120,7 +1163,11 @@ static int group_build_t(Group& G, const std::vector<tmk_level*>& mem, const std
     G.nb = L0->ctx->hp.fault_kind == TMK_FAULT_RS ? TMK_NBDRY_RS : TMK_NBDRY_SW;
     G.plastic = plastic;
     G.any_plast = false;
-    for (tmk_level* L : mem) G.any_plast = G.any_plast || L->ctx->P.plast;
+    G.div2 = true;
+    for (tmk_level* L : mem) {
+        G.any_plast = G.any_plast || L->ctx->P.plast;
+        G.div2 = G.div2 && L->ctx->P.div2;
+    }
     G.g = 0;
     std::vector<Scen> sc(mem.size());
     std::vector<Patch<T>> pts[2];

@@ -19,7 +19,7 @@ template __global__ void k_godunov_bnd<float, 2, PK_RUNTIME>(const KArgs<float>)
 template __global__ void k_godunov_bnd<float, 3, PK_RUNTIME>(const KArgs<float>);
 template __global__ void k_godunov_bnd<float, 2, PK_PPM_PRIM>(const KArgs<float>);
 template __global__ void k_godunov_bnd<float, 3, PK_PPM_PRIM>(const KArgs<float>);
-template __global__ void k_godunov_step<float, true>(const KArgs<float>);
-template __global__ void k_godunov_step<float, false>(const KArgs<float>);
+template __global__ void k_godunov_step<float, true, false>(const KArgs<float>);
+template __global__ void k_godunov_step<float, false, false>(const KArgs<float>);
 
 }  // namespace tmk

@@ -138,8 +138,8 @@ __device__ __forceinline__ int stage_comp(int d, int c)
 // GETFLUXF (LinElastPhysicsF.ChF:303-350) from the face state of one side, in slot form:
 // f[0]=F(vn) f[1]=F(snn) f[2]=F(vt) f[3]=F(snt) f[4]=F(s_transverse normal) f[5]=F(va) f[6]=F(sna);
 // r is the side's velocity sign in the face direction (a product with r = 1 is exact)
-template <typename T, int NS>
-__device__ __forceinline__ void face_flux_side(const Mat<T>& m, const T (&v)[NS], const T (&s)[NS], T r, T (&f)[7])
+template <typename T, int NS, bool D2>
+__device__ __forceinline__ void face_flux_side(const Mat<T, D2>& m, const T (&v)[NS], const T (&s)[NS], T r, T (&f)[7])
 {
     f[0] = -m.divrho(r * s[0]);
     f[2] = -m.divrho(r * s[1]);
@@ -152,8 +152,8 @@ __device__ __forceinline__ void face_flux_side(const Mat<T>& m, const T (&v)[NS]
     }
 }
 
-template <typename T, int NS>
-__device__ __forceinline__ void face_flux(const Mat<T>& m, const Slots<T, NS>& S, T rv, T (&f)[2][7])
+template <typename T, int NS, bool D2>
+__device__ __forceinline__ void face_flux(const Mat<T, D2>& m, const Slots<T, NS>& S, T rv, T (&f)[2][7])
 {
     face_flux_side<T, NS>(m, S.v[0], S.s[0], (T)1, f[0]);
     face_flux_side<T, NS>(m, S.v[1], S.s[1], rv, f[1]);
@@ -209,9 +209,9 @@ __device__ __forceinline__ bool register_face(unsigned a, unsigned b)
 
 // the 11 components of side sd of the face flux in direction d at index fi of the flux array
 // Fo (fp faces per component plane)
-template <typename T, int NS>
+template <typename T, int NS, bool D2>
 __device__ __forceinline__ void put_face_flux(__attribute__((address_space(1))) double* Fo, size_t fi, size_t fp,
-                                              const Mat<T>& m, int d, const T (&v)[NS], const T (&sv)[NS], T r,
+                                              const Mat<T, D2>& m, int d, const T (&v)[NS], const T (&sv)[NS], T r,
                                               int sd)
 {
     T f[7];
@@ -242,8 +242,8 @@ __device__ __forceinline__ void put_face_flux(__attribute__((address_space(1))) 
     Fo[fi + (o + 10) * fp] = 0.0;
 }
 
-template <typename T, int NS>
-__device__ __forceinline__ void store_flux_side(const Patch<T>& pt, const Mat<T>& m, int d, const T (&v)[NS],
+template <typename T, int NS, bool D2>
+__device__ __forceinline__ void store_flux_side(const Patch<T>& pt, const Mat<T, D2>& m, int d, const T (&v)[NS],
                                                 const T (&sv)[NS], T r, int i, int j, int sd)
 {
     const int fnx = pt.vhi0 - pt.vlo0 + 1 + (d == 0), fny = pt.vhi1 - pt.vlo1 + 1 + (d == 1);
@@ -258,8 +258,8 @@ __device__ __forceinline__ void store_flux_side(const Patch<T>& pt, const Mat<T>
     put_face_flux<T, NS>(gmem(pt.F[d]), fi, fp, m, d, v, sv, r, sd);
 }
 
-template <typename T, int NS>
-__device__ __forceinline__ void store_flux(const Patch<T>& pt, const Mat<T>& m, int d, const Slots<T, NS>& Fs, T rv,
+template <typename T, int NS, bool D2>
+__device__ __forceinline__ void store_flux(const Patch<T>& pt, const Mat<T, D2>& m, int d, const Slots<T, NS>& Fs, T rv,
                                            int i, int j)
 {
     store_flux_side<T, NS>(pt, m, d, Fs.v[0], Fs.s[0], (T)1, i, j, 0);
@@ -272,14 +272,36 @@ struct Faces1 {
     T xlv[NS], xls[NS], xhv[NS], xhs[NS], ylv[NS], yls[NS], yhv[NS], yhs[NS];
 };
 
+// U += dU of one side from the fluxes of a cell's four faces (face_flux_side), the in-plane components
+template <typename T>
+__device__ __forceinline__ void flux_update(T sc, const T (&fxl)[7], const T (&fxh)[7], const T (&fyl)[7],
+                                            const T (&fyh)[7], T (&u)[11])
+{
+    // dU = (0 + (Fx_hi - Fx_lo)) + (Fy_hi - Fy_lo); U += dU * (-dt/dx)
+    // x flux: vx<-F(vn) vy<-F(vt) sxx<-F(snn) syy,szz<-F(stt) sxy<-F(snt)
+    // y flux: vy<-F(vn) vx<-F(vt) syy<-F(snn) sxx,szz<-F(stt) sxy<-F(snt)
+    const T dvx_x = fxh[0] - fxl[0], dvx_y = fyh[2] - fyl[2];
+    const T dvy_x = fxh[2] - fxl[2], dvy_y = fyh[0] - fyl[0];
+    const T dsxx_x = fxh[1] - fxl[1], dsxx_y = fyh[4] - fyl[4];
+    const T dsyy_x = fxh[4] - fxl[4], dsyy_y = fyh[1] - fyl[1];
+    const T dszz_x = fxh[4] - fxl[4], dszz_y = fyh[4] - fyl[4];
+    const T dsxy_x = fxh[3] - fxl[3], dsxy_y = fyh[3] - fyl[3];
+    u[0] = u[0] + (((T)0 + dvx_x) + dvx_y) * sc;
+    u[1] = u[1] + (((T)0 + dvy_x) + dvy_y) * sc;
+    u[3] = u[3] + (((T)0 + dsxx_x) + dsxx_y) * sc;
+    u[4] = u[4] + (((T)0 + dsyy_x) + dsyy_y) * sc;
+    u[5] = u[5] + (((T)0 + dszz_x) + dszz_y) * sc;
+    u[6] = u[6] + (((T)0 + dsxy_x) + dsxy_y) * sc;
+}
+
 // New values of one side's state of a valid cell from its old values u[0..10] (side-local
 // component index) and the final states on its four faces: flux difference and
 // U += dU (-dt/dx) (LinElastPatchGodunov.cpp:117-126, LinElastPhysics.cpp:135-179), then, with
 // plastic, the Drucker-Prager return (LinElastLevelGodunov::plasticUpdate after the level step,
 // AMRLevelLinElast.cpp:476).  Changes u[0 1 3 4 5 6] (+ 2 7 8 with NS 3, + 7 8 9 10 with plastic).
 // PP: DevParams, or PlasticConstL (FP32) / PlasticConstL64 (FP64): the plastic return's constants in LDS
-template <typename T, int NS, typename PP>
-__device__ __forceinline__ void cell_update_side(const PP& P, const Mat<T>& m, double dt, T sc, bool plastic,
+template <typename T, int NS, typename PP, bool D2>
+__device__ __forceinline__ void cell_update_side(const PP& P, const Mat<T, D2>& m, double dt, T sc, bool plastic,
                                                  T ry, const Faces1<T, NS>& F, T (&u)[11])
 {
     if constexpr (regroup<T>()) {
@@ -312,21 +334,7 @@ __device__ __forceinline__ void cell_update_side(const PP& P, const Mat<T>& m, d
     face_flux_side<T, NS>(m, F.xhv, F.xhs, (T)1, fxh);
     face_flux_side<T, NS>(m, F.ylv, F.yls, ry, fyl);
     face_flux_side<T, NS>(m, F.yhv, F.yhs, ry, fyh);
-    // dU = (0 + (Fx_hi - Fx_lo)) + (Fy_hi - Fy_lo); U += dU * (-dt/dx)
-    // x flux: vx<-F(vn) vy<-F(vt) sxx<-F(snn) syy,szz<-F(stt) sxy<-F(snt)
-    // y flux: vy<-F(vn) vx<-F(vt) syy<-F(snn) sxx,szz<-F(stt) sxy<-F(snt)
-    const T dvx_x = fxh[0] - fxl[0], dvx_y = fyh[2] - fyl[2];
-    const T dvy_x = fxh[2] - fxl[2], dvy_y = fyh[0] - fyl[0];
-    const T dsxx_x = fxh[1] - fxl[1], dsxx_y = fyh[4] - fyl[4];
-    const T dsyy_x = fxh[4] - fxl[4], dsyy_y = fyh[1] - fyl[1];
-    const T dszz_x = fxh[4] - fxl[4], dszz_y = fyh[4] - fyl[4];
-    const T dsxy_x = fxh[3] - fxl[3], dsxy_y = fyh[3] - fyl[3];
-    u[0] = u[0] + (((T)0 + dvx_x) + dvx_y) * sc;
-    u[1] = u[1] + (((T)0 + dvy_x) + dvy_y) * sc;
-    u[3] = u[3] + (((T)0 + dsxx_x) + dsxx_y) * sc;
-    u[4] = u[4] + (((T)0 + dsyy_x) + dsyy_y) * sc;
-    u[5] = u[5] + (((T)0 + dszz_x) + dszz_y) * sc;
-    u[6] = u[6] + (((T)0 + dsxy_x) + dsxy_y) * sc;
+    flux_update<T>(sc, fxl, fxh, fyl, fyh, u);
     if (NS == 3) {
         const T dvz_x = fxh[5] - fxl[5], dvz_y = fyh[5] - fyl[5];
         const T dsxz_x = fxh[6] - fxl[6], dsxz_y = (T)0 - (T)0;
@@ -341,9 +349,9 @@ __device__ __forceinline__ void cell_update_side(const PP& P, const Mat<T>& m, d
 
 // U += dU of side sd of valid cell (i, j) from the final states on its four faces, then the
 // optional Drucker-Prager return (cell_update_side)
-template <typename T, int NS>
+template <typename T, int NS, bool D2>
 __device__ __forceinline__ void update_cell_side(const KArgs<T>& a, const Patch<T>& pt, const DevParams& P,
-                                                 const Mat<T>& m, double dt, T sc, int i, int j, int sd,
+                                                 const Mat<T, D2>& m, double dt, T sc, int i, int j, int sd,
                                                  const Faces1<T, NS>& F)
 {
     const T ry = sd ? (T)-1 : (T)1;
@@ -382,9 +390,9 @@ __device__ __forceinline__ void update_cell_side(const KArgs<T>& a, const Patch<
 }
 
 // both sides
-template <typename T, int NS>
+template <typename T, int NS, bool D2>
 __device__ __forceinline__ void update_cell(const KArgs<T>& a, const Patch<T>& pt, const DevParams& P,
-                                            const Mat<T>& m, double dt, T sc, int i, int j, const Slots<T, NS>& F0,
+                                            const Mat<T, D2>& m, double dt, T sc, int i, int j, const Slots<T, NS>& F0,
                                             const Slots<T, NS>& F0h, const Slots<T, NS>& F1,
                                             const Slots<T, NS>& F1h)
 {

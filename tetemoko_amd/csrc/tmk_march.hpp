@@ -174,7 +174,8 @@ struct MarchCarry {
     T h1v[2], h1s[2];      // predictor state of the lo y face of row r - 2
     T cpu[2];              // right characteristics of row r - 2's uncorrected W+ (y)
     T cpc[2];              // the same of its corrected W+
-    T f1v[2], f1s[2];      // final state of the lo y face of row r - 2
+    T f1v[2], f1s[2];      // final state of the lo y face of row r - 2 (FP32)
+    T fl[5];               // flux through the lo y face of row r - 2 (FP64)
 };
 
 // LDS floats of one wavefront's march: the ring, the plastic return's constants (16 floats), the
@@ -206,7 +207,7 @@ struct MarchRing {
 // descriptor of the side stays in scalar registers.
 // PL: the launch may hold scenarios with plasticity.  Without (PL false), a row neither reads gam
 // nor writes lam and gam, and a scenario with plasticity is an error.
-template <typename T, int PK, bool PL>
+template <typename T, int PK, bool PL, bool D2>
 __device__ __forceinline__ void march_strip(const KArgs<T>& a, const Tile& tl, const int sd, const int lane,
                                             float* const ring)
 {
@@ -218,7 +219,7 @@ __device__ __forceinline__ void march_strip(const KArgs<T>& a, const Tile& tl, c
         if (lane == 0 && sd == 0) report(&S.err, TMK_E_BOX);
         return;
     }
-    const Mat<T> m(P);
+    const Mat<T, D2> m(P);
     const int i = tl.x0 - 3 + lane;
     const int tnx = tl.x1 - tl.x0 + 1;
     const bool valid = lane >= 3 && lane <= tnx + 2;  // column of the strip
@@ -227,7 +228,11 @@ __device__ __forceinline__ void march_strip(const KArgs<T>& a, const Tile& tl, c
     const T dtbydx = K.dtbydx;
     const T scale = K.scale;
     const T rv1 = (T)-1;
-    const T rvy = sd ? rv1 : (T)1;  // velocity sign of this side in y
+    // velocity sign of this side in y: in the constants, or rvy.  FP64 without plasticity 461 -> 451 us
+    // per step of 4096 x 2048; with it the constants' registers do not fit (spills: 577 -> 797)
+    constexpr bool sgn = sizeof(T) == sizeof(double) && !PL;
+    const Mat<T, D2> my = sgn ? m.signed_for(sd) : m;
+    const T rvy = sgn ? (T)1 : sd ? rv1 : (T)1;
     const T scx = sd ? rv1 * scale : scale;
     if (!PL && P.plast && a.plastic) {
         if (lane == 0 && sd == 0) report(&S.err, TMK_E_ARG);
@@ -377,6 +382,8 @@ __device__ __forceinline__ void march_strip(const KArgs<T>& a, const Tile& tl, c
         A.xp.mv[k] = A.xp.ms[k] = A.xp.pv[k] = A.xp.ps[k] = (T)0;
         A.h1v[k] = A.h1s[k] = A.cpu[k] = A.cpc[k] = A.f1v[k] = A.f1s[k] = (T)0;
     }
+#pragma unroll
+    for (int k = 0; k < 5; ++k) A.fl[k] = (T)0;
     if constexpr (ring_fetch) {
 #pragma unroll
         for (int q = 1; q < RING; ++q) request(y0 + q);
@@ -459,7 +466,7 @@ __device__ __forceinline__ void march_strip(const KArgs<T>& a, const Tile& tl, c
             const T wv = c.w2[MQ_Y[k]], ws = c.w2[MQ_Y[2 + k]];
             const T dvm = incr(c.fy[k], wv), dvp = incr(fy1[k], wv);
             const T dsm = incr(c.fy[2 + k], ws), dsp = incr(fy1[2 + k], ws);
-            ppm_slot<T>(m, k, rvy, dtbydx, true, false, wv, ws, dvm, dvp, dsm, dsp, yp.mv[k], yp.ms[k], yp.pv[k],
+            ppm_slot<T>(my, k, rvy, dtbydx, true, false, wv, ws, dvm, dvp, dsm, dsp, yp.mv[k], yp.ms[k], yp.pv[k],
                         yp.ps[k]);
         }
         // x predictor of row r - 2: slopes and face values once per lane, neighbours by DPP
@@ -495,9 +502,9 @@ __device__ __forceinline__ void march_strip(const KArgs<T>& a, const Tile& tl, c
         // predictor state of the lo y face of row r - 2 (row r - 3's uncorrected W+, its W-)
         {
             T wmR[2];
-            left_chars_side<T, 2>(m, rvy, yp.mv, yp.ms, wmR);
-            riemann_side<T, 2>(m, rvy, c.cpu, wmR, n.h1v, n.h1s);
-            right_chars_side<T, 2>(m, rvy, yp.pv, yp.ps, n.cpu);
+            left_chars_side<T, 2>(my, rvy, yp.mv, yp.ms, wmR);
+            riemann_side<T, 2>(my, rvy, c.cpu, wmR, n.h1v, n.h1s);
+            right_chars_side<T, 2>(my, rvy, yp.pv, yp.ps, n.cpu);
         }
         // y predictor corrected with the x-face states of its cell (GETADWDXF, dir2 = x)
         {
@@ -513,9 +520,17 @@ __device__ __forceinline__ void march_strip(const KArgs<T>& a, const Tile& tl, c
         // final state of the lo y face of row r - 2 (row r - 3's corrected W+, its corrected W-)
         {
             T wmR[2];
-            left_chars_side<T, 2>(m, rvy, yp.mv, yp.ms, wmR);
-            riemann_side<T, 2>(m, rvy, c.cpc, wmR, n.f1v, n.f1s);
-            right_chars_side<T, 2>(m, rvy, yp.pv, yp.ps, n.cpc);
+            left_chars_side<T, 2>(my, rvy, yp.mv, yp.ms, wmR);
+            riemann_side<T, 2>(my, rvy, c.cpc, wmR, n.f1v, n.f1s);
+            right_chars_side<T, 2>(my, rvy, yp.pv, yp.ps, n.cpc);
+        }
+        // FP64 carries the face's flux, which the row above it reads again: the reference's flux of a face
+        // is one expression wherever it is read from (FP32 differences the face states instead)
+        T fyh[7];
+        if constexpr (!regroup<T>()) {
+            face_flux_side<T, 2>(my, n.f1v, n.f1s, rvy, fyh);
+#pragma unroll
+            for (int k = 0; k < 5; ++k) n.fl[k] = fyh[k];
         }
         const int j2 = r - 2;
         // flux registers (multi-level): the lo y face of row r - 2, the x faces of row r - 3
@@ -524,7 +539,7 @@ __device__ __forceinline__ void march_strip(const KArgs<T>& a, const Tile& tl, c
         if (flux1 && j2 >= y0 && fbit(1, j2 - y0)) {
             int ix = i - fvlo0;
             asm volatile("" : "+v"(ix));
-            put_face_flux<T, 2>(Fo1, (size_t)ix + (size_t)(j2 - fvlo1) * fvnx, (size_t)fvnx * (fvny + 1), m, 1, n.f1v,
+            put_face_flux<T, 2>(Fo1, (size_t)ix + (size_t)(j2 - fvlo1) * fvnx, (size_t)fvnx * (fvny + 1), my, 1, n.f1v,
                                 n.f1s, rvy, sd);
         }
         // row r - 3, a row of the strip: x predictor corrected with the y-face states below and
@@ -548,18 +563,6 @@ __device__ __forceinline__ void march_strip(const KArgs<T>& a, const Tile& tl, c
             }
             // update of row r - 3: every row of the strip issues exactly ROW_STORES stores (the
             // ring's waits count them)
-            Faces1<T, 2> F;
-#pragma unroll
-            for (int k = 0; k < 2; ++k) {
-                F.xlv[k] = f0v[k];
-                F.xls[k] = f0s[k];
-                F.xhv[k] = dshift<DPP_FROM_NEXT>(f0v[k]);
-                F.xhs[k] = dshift<DPP_FROM_NEXT>(f0s[k]);
-                F.ylv[k] = c.f1v[k];
-                F.yls[k] = c.f1s[k];
-                F.yhv[k] = n.f1v[k];
-                F.yhs[k] = n.f1s[k];
-            }
             // every lane runs the update (a lane outside the strip has off3 past the planes)
             T u[11];
             u[0] = c.w3[0];
@@ -570,10 +573,32 @@ __device__ __forceinline__ void march_strip(const KArgs<T>& a, const Tile& tl, c
             u[2] = u[7] = u[8] = u[9] = (T)0;
             u[5] = szz;
             u[10] = gam;
-            if constexpr (f32)
+            if constexpr (f32) {
+                Faces1<T, 2> F;
+#pragma unroll
+                for (int k = 0; k < 2; ++k) {
+                    F.xlv[k] = f0v[k];
+                    F.xls[k] = f0s[k];
+                    F.xhv[k] = dshift<DPP_FROM_NEXT>(f0v[k]);
+                    F.xhs[k] = dshift<DPP_FROM_NEXT>(f0s[k]);
+                    F.ylv[k] = c.f1v[k];
+                    F.yls[k] = c.f1s[k];
+                    F.yhv[k] = n.f1v[k];
+                    F.yhs[k] = n.f1s[k];
+                }
                 cell_update_side<T, 2>(pc, m, dt, K.sc, plastic, rvy, F, u);
-            else
-                cell_update_side<T, 2>(pc64, m, dt, K.sc, plastic, rvy, F, u);
+            } else {
+                T fxl[7], fxh[7], fyl[7];
+                face_flux_side<T, 2>(m, f0v, f0s, (T)1, fxl);
+#pragma unroll
+                for (int k = 0; k < 5; ++k) {
+                    fxh[k] = dshift<DPP_FROM_NEXT>(fxl[k]);  // the right lane's lo face
+                    fyl[k] = c.fl[k];
+                }
+                flux_update<T>(K.sc, fxl, fxh, fyl, fyh, u);
+                if (plastic)
+                    plastic_flow<T, PlasticConstL64>(pc64, (T)dt, u[3], u[4], u[5], u[6], u[7], u[8], u[9], u[10]);
+            }
 #pragma unroll
             for (int q = 0; q < 5; ++q) bst<T>(rout[q], off3, u[QC[q]]);
             bst<T>(rpw[0], off3, u[5]);

@@ -58,6 +58,8 @@ struct DevParams {
     double cs, cp, G, rho, lam, K, Zp, Zs;
     double iZp, iZs, irho;  // correctly rounded reciprocals 1/Zp, 1/Zs, 1/rho
     double i2Zp, i2Zs;      // 1/(2 Zp), 1/(2 Zs): the reciprocals halved (exact)
+    double lZp, lZs, lrho;  // RN(1/Z - RN(1/Z)): the low words of the reciprocals
+    int div2;               // Zp, Zs, rho divide exactly in two operations (div2_exact)
     // the same constants rounded to FP32 on the host, for the FP32-bulk kernels
     float frho, flam, fG, fZp, fZs, fden, flam2G, fiZp, fiZs, firho, fi2Zp, fi2Zs, fcp, fcs;
     double den;    // 2G + lam   (LinElastPhysicsF.ChF:427 form)
@@ -154,26 +156,60 @@ __device__ __forceinline__ T pick(double d, float f)
         return (T)f;
 }
 
-// elastic constants in the bulk arithmetic type
-template <typename T>
+// a / b given the reciprocal in two words, yh = RN(1/b) and yl = RN(1/b - yh): RN(a yh + RN(a yl)).
+// The sum under the last rounding is a / b to within 2^-105, so the result is the IEEE quotient
+// unless a / b lies that close to a midpoint of two floating-point numbers, which for a given b a few
+// dividends at most do (Brisebarre, Muller and Raina, IEEE Trans. Comput. 53 (2004) 1069-1072);
+// div2_exact tries those on the host, and constants that fail keep divr.  Two operations for six
+// (divr and its copysign): the sign of a zero dividend comes out by itself.  A cell side of the FP64
+// march divides 28 times; with the flux of a face computed once (march_strip) the 4096 x 2048 level
+// went from 522 to 461 us per step without plasticity and from 640 to 577 with it.
+__device__ __forceinline__ double divr2(double a, double yh, double yl) { return fma(a, yh, a * yl); }
+
+// elastic constants in the bulk arithmetic type.  D2 (FP64): the constants divide by divr2.
+template <typename T, bool D2 = false>
 struct Mat {
     T rho, lam, G, Zp, Zs, den, lam2G;
     T iZp, iZs, irho, i2Zp, i2Zs;  // reciprocals (1/(2Z) = (1/Z)/2 exactly)
+    T lZp, lZs, lrho;              // their low words (D2)
     T cp, cs;
     __device__ __forceinline__ explicit Mat(const DevParams& p)
         : rho(pick<T>(p.rho, p.frho)), lam(pick<T>(p.lam, p.flam)), G(pick<T>(p.G, p.fG)),
           Zp(pick<T>(p.Zp, p.fZp)), Zs(pick<T>(p.Zs, p.fZs)), den(pick<T>(p.den, p.fden)),
           lam2G(pick<T>(p.lam2G, p.flam2G)), iZp(pick<T>(p.iZp, p.fiZp)), iZs(pick<T>(p.iZs, p.fiZs)),
           irho(pick<T>(p.irho, p.firho)), i2Zp(pick<T>(p.i2Zp, p.fi2Zp)), i2Zs(pick<T>(p.i2Zs, p.fi2Zs)),
-          cp(pick<T>(p.cp, p.fcp)), cs(pick<T>(p.cs, p.fcs)) {}
+          lZp((T)p.lZp), lZs((T)p.lZs), lrho((T)p.lrho), cp(pick<T>(p.cp, p.fcp)), cs(pick<T>(p.cs, p.fcs)) {}
+    // the same with every constant that the velocity sign of a side multiplies carrying that sign: side
+    // 2 in y (sd = 1) then runs the expressions of side 1, and no product with the sign is left (FP64;
+    // negation is exact).  The sign goes in by integer arithmetic on uniform values: scalar registers.
+    __device__ __forceinline__ Mat signed_for(int sd) const
+    {
+        Mat o = *this;
+        const auto s = [sd](T v) {
+            return (T)__longlong_as_double(__double_as_longlong((double)v) ^ (long long)((unsigned long long)sd << 63));
+        };
+        o.rho = s(rho); o.lam = s(lam); o.G = s(G); o.Zp = s(Zp); o.Zs = s(Zs); o.lam2G = s(lam2G);
+        o.iZp = s(iZp); o.iZs = s(iZs); o.irho = s(irho); o.i2Zp = s(i2Zp); o.i2Zs = s(i2Zs);
+        o.lZp = s(lZp); o.lZs = s(lZs); o.lrho = s(lrho);
+        return o;
+    }
     __device__ __forceinline__ T Z(int k) const { return k == 0 ? Zp : Zs; }
     // x / Z(k), x / (2 Z(k)), x / rho, rounded like the division
-    __device__ __forceinline__ T divZ(T x, int k) const { return k == 0 ? divr(x, Zp, iZp) : divr(x, Zs, iZs); }
+    __device__ __forceinline__ T divZ(T x, int k) const
+    {
+        if constexpr (D2) return k == 0 ? divr2(x, iZp, lZp) : divr2(x, iZs, lZs);
+        else return k == 0 ? divr(x, Zp, iZp) : divr(x, Zs, iZs);
+    }
     __device__ __forceinline__ T div2Z(T x, int k) const
     {
-        return k == 0 ? divr(x, (T)2 * Zp, i2Zp) : divr(x, (T)2 * Zs, i2Zs);
+        if constexpr (D2) return k == 0 ? divr2(x, i2Zp, (T)0.5 * lZp) : divr2(x, i2Zs, (T)0.5 * lZs);
+        else return k == 0 ? divr(x, (T)2 * Zp, i2Zp) : divr(x, (T)2 * Zs, i2Zs);
     }
-    __device__ __forceinline__ T divrho(T x) const { return divr(x, rho, irho); }
+    __device__ __forceinline__ T divrho(T x) const
+    {
+        if constexpr (D2) return divr2(x, irho, lrho);
+        else return divr(x, rho, irho);
+    }
     __device__ __forceinline__ T i2Z(int k) const { return k == 0 ? i2Zp : i2Zs; }
 };
 
@@ -292,8 +328,8 @@ __device__ __forceinline__ void ppm_limit(T& m, T& p)
 // of v and s at the lo (m) and hi (p) faces): limiter in primitive or characteristic variables,
 // CHARANALYSISF (LinElastPhysicsF.ChF:424-447), tracing of the wave moving toward lo on the lo
 // face and toward hi on the hi face, CHARSYNTHESISF (:526-550), then W+- = increment + W.
-template <typename T>
-__device__ __forceinline__ void ppm_slot(const Mat<T>& m, int k, T rvs, T dtbydx, bool limit, bool charl, T wv, T ws,
+template <typename T, bool D2>
+__device__ __forceinline__ void ppm_slot(const Mat<T, D2>& m, int k, T rvs, T dtbydx, bool limit, bool charl, T wv, T ws,
                                          T dvm, T dvp, T dsm, T dsp, T& Wmv, T& Wms, T& Wpv, T& Wps)
 {
     if (limit && !charl) {
@@ -365,8 +401,8 @@ __device__ __forceinline__ void ppm_slot(const Mat<T>& m, int k, T rvs, T dtbydx
 constexpr int PK_RUNTIME = -1;
 constexpr int PK_PPM_PRIM = 2;
 
-template <typename T, int NS, int PK = PK_RUNTIME>
-__device__ __forceinline__ void normal_pred_side(const DevParams& P, const Mat<T>& m, int pred_rt, T rvs,
+template <typename T, int NS, int PK = PK_RUNTIME, bool D2 = false>
+__device__ __forceinline__ void normal_pred_side(const DevParams& P, const Mat<T, D2>& m, int pred_rt, T rvs,
                                                  const T (&w)[NS][2][5], int ci, int dlo, int dhi, T dtbydx,
                                                  T (&Wmv)[NS], T (&Wms)[NS], T (&Wpv)[NS], T (&Wps)[NS])
 {
@@ -462,8 +498,8 @@ __device__ __forceinline__ void normal_pred_side(const DevParams& P, const Mat<T
 }
 
 // both sides (side 2 with velocity sign rv)
-template <typename T, int NS, int PK = PK_RUNTIME>
-__device__ __forceinline__ void normal_pred(const DevParams& P, const Mat<T>& m, int pred_rt, T rv,
+template <typename T, int NS, int PK = PK_RUNTIME, bool D2 = false>
+__device__ __forceinline__ void normal_pred(const DevParams& P, const Mat<T, D2>& m, int pred_rt, T rv,
                                             const T (&w)[2][NS][2][5], int ci, int dlo, int dhi,
                                             T dtbydx, Slots<T, NS>& Wm, Slots<T, NS>& Wp)
 {
@@ -472,24 +508,24 @@ __device__ __forceinline__ void normal_pred(const DevParams& P, const Mat<T>& m,
 }
 
 // outgoing-to-the-right characteristic of a left state (RIEMANNF wxxp, LinElastPhysicsF.ChF:677-679,733-735)
-template <typename T, int NS>
-__device__ __forceinline__ void right_chars_side(const Mat<T>& m, T rvs, const T (&v)[NS], const T (&s)[NS],
+template <typename T, int NS, bool D2>
+__device__ __forceinline__ void right_chars_side(const Mat<T, D2>& m, T rvs, const T (&v)[NS], const T (&s)[NS],
                                                  T (&c)[NS])
 {
 #pragma unroll
     for (int k = 0; k < NS; ++k) c[k] = s[k] - (rvs * m.Z(k)) * v[k];
 }
 // left-moving characteristic of a right state (RIEMANNF wxxm, :681-683,738-740)
-template <typename T, int NS>
-__device__ __forceinline__ void left_chars_side(const Mat<T>& m, T rvs, const T (&v)[NS], const T (&s)[NS],
+template <typename T, int NS, bool D2>
+__device__ __forceinline__ void left_chars_side(const Mat<T, D2>& m, T rvs, const T (&v)[NS], const T (&s)[NS],
                                                 T (&c)[NS])
 {
 #pragma unroll
     for (int k = 0; k < NS; ++k) c[k] = s[k] + (rvs * m.Z(k)) * v[k];
 }
 // RIEMANNF face state from the two characteristics (:693-702, :750-759)
-template <typename T, int NS>
-__device__ __forceinline__ void riemann_side(const Mat<T>& m, T rvs, const T (&wp)[NS], const T (&wm)[NS],
+template <typename T, int NS, bool D2>
+__device__ __forceinline__ void riemann_side(const Mat<T, D2>& m, T rvs, const T (&wp)[NS], const T (&wm)[NS],
                                              T (&v)[NS], T (&s)[NS])
 {
 #pragma unroll
@@ -504,20 +540,20 @@ __device__ __forceinline__ void riemann_side(const Mat<T>& m, T rvs, const T (&w
     }
 }
 
-template <typename T, int NS>
-__device__ __forceinline__ void right_chars(const Mat<T>& m, T rv, const Slots<T, NS>& L, T (&c)[2][NS])
+template <typename T, int NS, bool D2>
+__device__ __forceinline__ void right_chars(const Mat<T, D2>& m, T rv, const Slots<T, NS>& L, T (&c)[2][NS])
 {
     right_chars_side<T, NS>(m, (T)1, L.v[0], L.s[0], c[0]);
     right_chars_side<T, NS>(m, rv, L.v[1], L.s[1], c[1]);
 }
-template <typename T, int NS>
-__device__ __forceinline__ void left_chars(const Mat<T>& m, T rv, const Slots<T, NS>& R, T (&c)[2][NS])
+template <typename T, int NS, bool D2>
+__device__ __forceinline__ void left_chars(const Mat<T, D2>& m, T rv, const Slots<T, NS>& R, T (&c)[2][NS])
 {
     left_chars_side<T, NS>(m, (T)1, R.v[0], R.s[0], c[0]);
     left_chars_side<T, NS>(m, rv, R.v[1], R.s[1], c[1]);
 }
-template <typename T, int NS>
-__device__ __forceinline__ void riemann_state(const Mat<T>& m, T rv, const T (&wp)[2][NS], const T (&wm)[2][NS],
+template <typename T, int NS, bool D2>
+__device__ __forceinline__ void riemann_state(const Mat<T, D2>& m, T rv, const T (&wp)[2][NS], const T (&wm)[2][NS],
                                               Slots<T, NS>& F)
 {
     riemann_side<T, NS>(m, (T)1, wp[0], wm[0], F.v[0], F.s[0]);
@@ -526,8 +562,8 @@ __device__ __forceinline__ void riemann_state(const Mat<T>& m, T rv, const T (&w
 
 // LINELASTOUTBCF / LINELASTFREEBCF (LinElastPhysicsF.ChF:906-1144) on the face state.
 // lohisign -1: inside chars are the left-moving wm; +1: right-moving wp.
-template <typename T, int NS>
-__device__ __forceinline__ void bc_state(const DevParams& P, const Mat<T>& m, int d, T rv, int type, int lohisign,
+template <typename T, int NS, bool D2>
+__device__ __forceinline__ void bc_state(const DevParams& P, const Mat<T, D2>& m, int d, T rv, int type, int lohisign,
                                          const T (&cin)[2][NS], Slots<T, NS>& F)
 {
 #pragma unroll
@@ -563,8 +599,8 @@ __device__ __forceinline__ void bc_state(const DevParams& P, const Mat<T>& m, in
 
 // GETADWDXF applied as W(d1) += A(d2) (WHalf(d2)[+1] - WHalf(d2)[0]) (LinElastPhysicsF.ChF:791-901,
 // LinElastPatchGodunov.cpp:408-416) on one side.  sc = -(1/2) dt/dx, times rv(d2) on side 2.
-template <typename T, int NS>
-__device__ __forceinline__ void transverse_side(const Mat<T>& m, T sc, const T (&Hlov)[NS], const T (&Hlos)[NS],
+template <typename T, int NS, bool D2>
+__device__ __forceinline__ void transverse_side(const Mat<T, D2>& m, T sc, const T (&Hlov)[NS], const T (&Hlos)[NS],
                                                 const T (&Hhiv)[NS], const T (&Hhis)[NS], T (&Wv)[NS], T (&Ws)[NS])
 {
     const T dNv = Hhiv[0] - Hlov[0], dNs = Hhis[0] - Hlos[0];
@@ -589,8 +625,8 @@ __device__ __forceinline__ void transverse_side(const Mat<T>& m, T sc, const T (
     }
 }
 
-template <typename T, int NS>
-__device__ __forceinline__ void transverse_add(const Mat<T>& m, T sc1, T sc2, const Slots<T, NS>& Hlo,
+template <typename T, int NS, bool D2>
+__device__ __forceinline__ void transverse_add(const Mat<T, D2>& m, T sc1, T sc2, const Slots<T, NS>& Hlo,
                                                const Slots<T, NS>& Hhi, Slots<T, NS>& W)
 {
     transverse_side<T, NS>(m, sc1, Hlo.v[0], Hlo.s[0], Hhi.v[0], Hhi.s[0], W.v[0], W.s[0]);

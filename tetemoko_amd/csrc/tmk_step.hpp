@@ -17,8 +17,8 @@ constexpr int STEP_BX = 25, STEP_BY = 5;
 constexpr int STEP_SLOTS = 16;  // LDS values per lane of a piece
 
 // LINELASTOUTBCF / LINELASTFREEBCF on one side's face state (bc_state for one side)
-template <typename T>
-__device__ __forceinline__ void bc_state_side(const DevParams& P, const Mat<T>& m, int d, T rvs, int sd, int type,
+template <typename T, bool D2>
+__device__ __forceinline__ void bc_state_side(const DevParams& P, const Mat<T, D2>& m, int d, T rvs, int sd, int type,
                                               int lohisign, const T (&cin)[2], T (&v)[2], T (&sv)[2])
 {
 #pragma unroll
@@ -58,13 +58,13 @@ __device__ __forceinline__ void bc_state_side(const DevParams& P, const Mat<T>& 
 // way.  The values are those of godunov_tile, by the same expressions.
 // What bounds it: the latency of one piece (a few hundred dependent operations, the fault solve's
 // Newton iterations above all); its bytes and operations are a few per cent of a level's.
-template <typename T>
+template <typename T, bool D2>
 __device__ __forceinline__ void bnd_piece(const KArgs<T>& a, const Tile& tl, T* const sm)
 {
     const Patch<T>& pt = a.patches[tl.patch];
     Scen& S = a.scen[pt.scen];
     const DevParams& P = S.P;
-    const Mat<T> m(P);
+    const Mat<T, D2> m(P);
     int* const errp = &S.err;
     const int tid = threadIdx.x;
     const int sd = __builtin_amdgcn_readfirstlane(tid >> 7);
@@ -310,7 +310,7 @@ __device__ __forceinline__ void bnd_piece(const KArgs<T>& a, const Tile& tl, T* 
 // 1.09 -> 1.05 ms (workgroups of four strip sides share their halos better than single wavefronts).
 // FP32 is held to 128 VGPRs (four wavefronts per SIMD, LDS 33 KB of 160 for each of four workgroups)
 // as the march and the boundary pieces were on their own; FP64 to 256 (two per SIMD).
-template <typename T, bool PL>
+template <typename T, bool PL, bool D2>
 __global__ void __launch_bounds__(STEP_NT)
     __attribute__((amdgpu_waves_per_eu(sizeof(T) == sizeof(float) ? 4 : 2)))
 k_godunov_step(const KArgs<T> a)
@@ -326,14 +326,14 @@ k_godunov_step(const KArgs<T> a)
             a.scen[k].time[a.par ^ 1] = a.scen[k].time[a.par] + a.scen[k].dt;
     if (b < nbnd) {
         const Tile tl = a.tiles[a.nint + b];
-        bnd_piece<T>(a, tl, reinterpret_cast<T*>(lds));
+        bnd_piece<T, D2>(a, tl, reinterpret_cast<T*>(lds));
         return;
     }
     const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int q = (STEP_WAVES / 2) * (b - nbnd) + (w >> 1);
     if (q >= a.nint) return;
     const Tile tl = a.tiles[q];
-    march_strip<T, PK_PPM_PRIM, PL>(a, tl, w & 1, (int)(threadIdx.x & 63), lds + w * MF);
+    march_strip<T, PK_PPM_PRIM, PL, D2>(a, tl, w & 1, (int)(threadIdx.x & 63), lds + w * MF);
 }
 
 }  // namespace tmk
