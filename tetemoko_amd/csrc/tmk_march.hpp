@@ -229,8 +229,9 @@ __device__ __forceinline__ void march_strip(const KArgs<T>& a, const Tile& tl, c
     const T scale = K.scale;
     const T rv1 = (T)-1;
     // velocity sign of this side in y: in the constants, or rvy.  FP64 without plasticity 461 -> 451 us
-    // per step of 4096 x 2048; with it the constants' registers do not fit (spills: 577 -> 797)
-    constexpr bool sgn = sizeof(T) == sizeof(double) && !PL;
+    // per step of 4096 x 2048; with it the constants' registers do not fit (spills: 577 -> 797).  Only
+    // with divr2: divr takes the quotient's sign from the dividend and needs positive constants.
+    constexpr bool sgn = sizeof(T) == sizeof(double) && !PL && D2;
     const Mat<T, D2> my = sgn ? m.signed_for(sd) : m;
     const T rvy = sgn ? (T)1 : sd ? rv1 : (T)1;
     const T scx = sd ? rv1 * scale : scale;

@@ -180,8 +180,8 @@ struct Mat {
           irho(pick<T>(p.irho, p.firho)), i2Zp(pick<T>(p.i2Zp, p.fi2Zp)), i2Zs(pick<T>(p.i2Zs, p.fi2Zs)),
           lZp((T)p.lZp), lZs((T)p.lZs), lrho((T)p.lrho), cp(pick<T>(p.cp, p.fcp)), cs(pick<T>(p.cs, p.fcs)) {}
     // the same with every constant that the velocity sign of a side multiplies carrying that sign: side
-    // 2 in y (sd = 1) then runs the expressions of side 1, and no product with the sign is left (FP64;
-    // negation is exact).  The sign goes in by integer arithmetic on uniform values: scalar registers.
+    // 2 in y (sd = 1) then runs the expressions of side 1, and no product with the sign is left (FP64 with
+    // D2, whose division takes either sign; negation is exact).  The sign goes in by integer arithmetic on uniform values: scalar registers.
     __device__ __forceinline__ Mat signed_for(int sd) const
     {
         Mat o = *this;
