@@ -381,6 +381,7 @@ void march_rect(const Tile& r, const DevParams& P, int rows, std::vector<Tile>& 
             t.y0 = y;
             t.x1 = std::min(x + MARCH_COLS - 1, c.x1);
             t.y1 = std::min(y + rows - 1, c.y1);
+            t.flux = 1;
             strips.push_back(t);
         }
 }
@@ -1173,6 +1174,7 @@ static int group_build_t(Group& G, const std::vector<tmk_level*>& mem, const std
     std::vector<Patch<T>> pts[2];
     std::vector<Tile> tiles;
     std::vector<CopyRect> rects, brects;
+    bool fluxes = false;  // a hierarchy level, with flux registers
     int poff = 0;
     for (size_t m = 0; m < mem.size(); ++m) {
         tmk_level* L = mem[m];
@@ -1206,7 +1208,6 @@ static int group_build_t(Group& G, const std::vector<tmk_level*>& mem, const std
         // the rectangles become interior strips, then boundary pieces (fault row first)
         std::vector<Tile> strips, bf, bo;
         // strips of levels with flux registers hold at most 63 rows (the kernel's face masks)
-        bool fluxes = false;
         for (const Patch<T>& p : pts[0]) fluxes = fluxes || p.F[0] || p.F[1];
         auto params = [&](const Tile& t) -> const DevParams& { return sc[patch_scen[t.patch]].P; };
         bool chosen = false;  // some member's level has a height of its own
@@ -1253,6 +1254,12 @@ static int group_build_t(Group& G, const std::vector<tmk_level*>& mem, const std
     G.ntiles = (int)tiles.size();
     G.nrects = (int)rects.size();
     G.nbrects = (int)brects.size();
+    if (fluxes && G.march && G.nint > 0) {
+        hipLaunchKernelGGL(k_strip_flux<T>, dim3((unsigned)G.nint), dim3(64), 0, G.side, G.tiles_dev,
+                           (const Patch<T>*)G.patches_dev[0]);
+        HIPCHK(hipGetLastError());
+        HIPCHK(hipStreamSynchronize(G.side));
+    }
     return TMK_OK;
 }
 
@@ -3039,6 +3046,7 @@ struct tmk_amr {
     hipGraphExec_t gexec = nullptr;  // two coarse steps (every level back to its parity)
     int gpar = 0;                    // level-0 group parity the graph was captured at
     Group xgrp;                      // one-level group for the exchange of an uploaded level
+    int pend = -1;                   // level whose last step's register increments are not yet enqueued
 };
 
 // offset of cell (i, j) in the plane of the island array holding box b
@@ -3237,6 +3245,11 @@ static int member_pair_lists(const AmrMember& M, int l, int r, PairLists& P)
                         if (cc.cpatch[k] < 0) return TMK_E_NESTING;
                     flags |= 16;
                 }
+                // boxes of one island share its arrays, so any one descriptor of it serves all nine cells
+                bool one = true;
+                for (int k = 0; k < 9; ++k)
+                    one = one && cc.cpatch[k] >= 0 && C->box_isl[cc.cpatch[k]] == C->box_isl[cc.cpatch[4]];
+                if (one) flags |= 32;
                 cc.flags = flags;
                 cc.coef0 = -0.5 + ((double)(i - r * ic) + 0.5) / (double)r;
                 cc.coef1 = -0.5 + ((double)(j - r * jc) + 0.5) / (double)r;
@@ -3710,55 +3723,80 @@ extern "C" int tmk_amr_create(int nlevels, tmk_level* const* levels, int ref_rat
     return TMK_OK;
 }
 
-static inline dim3 amr_grid(long long n) { return dim3((unsigned)((n + 255) / 256)); }
+static inline int amr_blocks(long long n) { return (int)((n + 255) / 256); }
 
-// AMRLevelLinElast::advance of level l for every member: coarse-fine fill, the level step
-// (update with flux capture, exchange, clock), register increments
+// one launch between two level steps: the register increments still pending and the coarse-fine fill
+// of level l (l <= 0: none)
+template <typename T>
+static int launch_between(hipStream_t st, AmrBetween<T>& a)
+{
+    a.b1 = amr_blocks((long long)a.fill.ncells * a.fill.ncomps);
+    a.b2 = a.b1 + amr_blocks((long long)a.fin.n * TMK_NCOMP);
+    a.b3 = a.b2 + amr_blocks((long long)a.fill.nfaces * a.fill.nb);
+    const int n = a.b3 + amr_blocks((long long)a.crs.n * TMK_NCOMP);
+    if (n == 0) return TMK_OK;
+    hipLaunchKernelGGL(k_amr_between<T>, dim3((unsigned)n), dim3(256), 0, st, a);
+    return hipGetLastError() == hipSuccess ? TMK_OK : TMK_E_HIP;
+}
+
+template <typename T>
+static int amr_between_t(tmk_amr* A, int l)
+{
+    AmrBetween<T> a;
+    memset(&a, 0, sizeof a);
+    if (A->pend >= 0) {
+        // increments of the step of level p: its coarse faces (the register with p + 1 starts anew) and
+        // its fine faces (the register with p - 1); flux pointers are the same at both parities
+        const int p = A->pend;
+        A->pend = -1;
+        AmrLevel& q = A->lv[p];
+        const Patch<T>* pts = (const Patch<T>*)q.grp.patches_dev[q.grp.g];
+        if (p + 1 < A->nlev && q.nreg > 0)
+            a.crs = RegInc<T>{(const RegFace*)q.regf.p, (double*)q.reg.p, pts, q.grp.scen_dev, q.nreg, A->r};
+        if (p > 0 && A->lv[p - 1].nreg > 0) {
+            AmrLevel& c = A->lv[p - 1];
+            a.fin = RegInc<T>{(const RegFace*)c.regf.p, (double*)c.reg.p, pts, q.grp.scen_dev, c.nreg, A->r};
+        }
+    }
+    if (l > 0) {
+        AmrLevel& f = A->lv[l];
+        Group &G = f.grp, &GC = A->lv[l - 1].grp;
+        CfFill<T>& F = a.fill;
+        F.cells = (const CfCell*)f.cells.p;
+        F.comps = (const int*)f.comps.p;
+        F.faces = (const CfFace*)f.faces.p;
+        F.ncells = f.ncells;
+        F.ncomps = f.ncomps;
+        F.nfaces = f.nfaces;
+        F.nb = TMK_NBDRY_RS;
+        F.fine = (const Patch<T>*)G.patches_dev[G.g];
+        F.cnew = (const Patch<T>*)GC.patches_dev[GC.g];      // state after the coarse step
+        F.cold = (const Patch<T>*)GC.patches_dev[GC.g ^ 1];  // its input: the state before
+        F.fscen = G.scen_dev;
+        F.cscen = GC.scen_dev;
+        F.fpar = G.g;
+        F.cpar = GC.g;
+        F.r = A->r;
+        F.alpha_fixed = -1.0;
+    }
+    return launch_between(A->stream, a);
+}
+
+// AMRLevelLinElast::advance of level l for every member: coarse-fine fill (with the increments of the
+// level step before), the level step (update with flux capture, exchange, clock); its register
+// increments stay pending until the next launch between steps
 template <typename T>
 static int amr_advance_t(tmk_amr* A, int l)
 {
-    AmrLevel& a = A->lv[l];
-    Group& G = a.grp;
-    hipStream_t st = A->stream;
-    if (l > 0) {
-        Group& GC = A->lv[l - 1].grp;
-        const Patch<T>* fine = (const Patch<T>*)G.patches_dev[G.g];
-        const Patch<T>* cnew = (const Patch<T>*)GC.patches_dev[GC.g];      // state after the coarse step
-        const Patch<T>* cold = (const Patch<T>*)GC.patches_dev[GC.g ^ 1];  // its input: the state before
-        if (a.ncells > 0) {
-            hipLaunchKernelGGL(k_amr_fill_state<T>, amr_grid((long long)a.ncells * a.ncomps), dim3(256), 0, st,
-                               (const CfCell*)a.cells.p, a.ncells, (const int*)a.comps.p, a.ncomps, fine, cold, cnew,
-                               G.scen_dev, GC.scen_dev, G.g, GC.g, A->r, -1.0);
-            HIPCHK(hipGetLastError());
-        }
-        if (a.nfaces > 0) {
-            hipLaunchKernelGGL(k_amr_fill_fault<T>, amr_grid((long long)a.nfaces * TMK_NBDRY_RS), dim3(256), 0, st,
-                               (const CfFace*)a.faces.p, a.nfaces, TMK_NBDRY_RS, fine, cold, cnew, G.scen_dev,
-                               GC.scen_dev, G.g, GC.g, A->r, -1.0);
-            HIPCHK(hipGetLastError());
-        }
-    }
-    const Patch<T>* pts = (const Patch<T>*)G.patches_dev[G.g];  // flux pointers are the same at both parities
-    int e = group_enqueue_step(G, st);
+    int e = amr_between_t<T>(A, l);
     if (e) return e;
+    if ((e = group_enqueue_step(A->lv[l].grp, A->stream))) return e;
     for (AmrMember* M : A->mem) {
         tmk_level* L = M->L[l];
         L->cur ^= 1;
         L->time = L->time + L->dt;
     }
-    if (l + 1 < A->nlev && a.nreg > 0) {
-        hipLaunchKernelGGL(k_amr_reg_coarse<T>, amr_grid((long long)a.nreg * TMK_NCOMP), dim3(256), 0, st,
-                           (const RegFace*)a.regf.p, a.nreg, (double*)a.reg.p, pts, (const Scen*)G.scen_dev);
-        HIPCHK(hipGetLastError());
-    }
-    if (l > 0) {
-        AmrLevel& c = A->lv[l - 1];
-        if (c.nreg > 0) {
-            hipLaunchKernelGGL(k_amr_reg_fine<T>, amr_grid((long long)c.nreg * TMK_NCOMP), dim3(256), 0, st,
-                               (const RegFace*)c.regf.p, c.nreg, (double*)c.reg.p, pts, A->r, (const Scen*)G.scen_dev);
-            HIPCHK(hipGetLastError());
-        }
-    }
+    A->pend = l;
     return TMK_OK;
 }
 
@@ -3768,31 +3806,37 @@ template <typename T>
 static int amr_post_t(tmk_amr* A, int l)
 {
     if (l + 1 >= A->nlev) return TMK_OK;
+    int e = amr_between_t<T>(A, 0);  // the last fine step's increments
+    if (e) return e;
     AmrLevel& a = A->lv[l];
-    Group& G = a.grp;
-    Group& GF = A->lv[l + 1].grp;
-    hipStream_t st = A->stream;
-    const Patch<T>* cur = (const Patch<T>*)G.patches_dev[G.g];
-    const Patch<T>* fcur = (const Patch<T>*)GF.patches_dev[GF.g];
-    const int r = A->r;
-    if (a.nrcells > 0) {
-        hipLaunchKernelGGL(k_amr_reflux<T>, amr_grid((long long)a.nrcells * TMK_NCOMP), dim3(256), 0, st,
-                           (const RefluxCell*)a.rcells.p, a.nrcells, (const double*)a.reg.p,
-                           (const double*)a.rscale.p, a.nreg, cur);
+    Group &G = a.grp, &GF = A->lv[l + 1].grp;
+    AmrPost<T> p;
+    memset(&p, 0, sizeof p);
+    p.rcells = (const RefluxCell*)a.rcells.p;
+    p.reg = (const double*)a.reg.p;
+    p.scale = (const double*)a.rscale.p;
+    p.avgc = (const AvgCell*)a.avgc.p;
+    p.comps = (const int*)a.acomps.p;
+    p.avgf = (const AvgFace*)a.avgf.p;
+    p.crs = (const Patch<T>*)G.patches_dev[G.g];
+    p.fine = (const Patch<T>*)GF.patches_dev[GF.g];
+    p.nrcells = a.nrcells;
+    p.nreg = a.nreg;
+    p.navgc = a.navgc;
+    p.ncomps = a.nacomps;
+    p.navgf = a.navgf;
+    p.nb = TMK_NBDRY_RS;
+    p.r = A->r;
+    p.scale_state = 1.0 / (A->r * A->r);
+    p.scale_fault = 1.0 / A->r;
+    p.b1 = amr_blocks((long long)a.navgc * a.nacomps);
+    p.b2 = p.b1 + amr_blocks((long long)a.nrcells * TMK_NCOMP);
+    const int n = p.b2 + amr_blocks((long long)a.navgf * TMK_NBDRY_RS);
+    if (n > 0) {
+        hipLaunchKernelGGL(k_amr_post<T>, dim3((unsigned)n), dim3(256), 0, A->stream, p);
         HIPCHK(hipGetLastError());
     }
-    if (a.navgc > 0) {
-        hipLaunchKernelGGL(k_amr_avg_state<T>, amr_grid((long long)a.navgc * a.nacomps), dim3(256), 0, st,
-                           (const AvgCell*)a.avgc.p, a.navgc, (const int*)a.acomps.p, a.nacomps, cur, fcur, r,
-                           1.0 / (r * r));
-        HIPCHK(hipGetLastError());
-    }
-    if (a.navgf > 0) {
-        hipLaunchKernelGGL(k_amr_avg_fault<T>, amr_grid((long long)a.navgf * TMK_NBDRY_RS), dim3(256), 0, st,
-                           (const AvgFace*)a.avgf.p, a.navgf, TMK_NBDRY_RS, cur, fcur, r, 1.0 / r);
-        HIPCHK(hipGetLastError());
-    }
-    return group_exchange_now_t<T>(G, st);
+    return group_exchange_now_t<T>(G, A->stream);
 }
 
 template <typename T>
@@ -3808,6 +3852,7 @@ static int amr_time_step_t(tmk_amr* A, int l)
 
 static int amr_time_step(tmk_amr* A)
 {
+    A->pend = -1;
     return A->mem[0]->L[0]->tsize == sizeof(double) ? amr_time_step_t<double>(A, 0) : amr_time_step_t<float>(A, 0);
 }
 
@@ -4266,17 +4311,21 @@ static int level_regrid_t(tmk_level* N, tmk_level* O, tmk_level* C, int r)
     const Patch<T>* tN = (const Patch<T>*)dN.p;
     const Patch<T>* tC = (const Patch<T>*)dC.p;
     const int nb = N->ctx->hp.fault_kind == TMK_FAULT_RS ? TMK_NBDRY_RS : TMK_NBDRY_SW;
-    if (!cells.empty()) {
-        hipLaunchKernelGGL(k_amr_fill_state<T>, amr_grid((long long)cells.size() * TMK_NCOMP), dim3(256), 0, st,
-                           (const CfCell*)dcells.p, (int)cells.size(), (const int*)dcomps.p, TMK_NCOMP, tN, tC, tC,
-                           (const Scen*)nullptr, (const Scen*)nullptr, 0, 0, r, 1.0);
-        HIPCHK(hipGetLastError());
-    }
-    if (!faces.empty()) {
-        hipLaunchKernelGGL(k_amr_fill_fault<T>, amr_grid((long long)faces.size() * nb), dim3(256), 0, st,
-                           (const CfFace*)dfaces.p, (int)faces.size(), nb, tN, tC, tC, (const Scen*)nullptr,
-                           (const Scen*)nullptr, 0, 0, r, 1.0);
-        HIPCHK(hipGetLastError());
+    {
+        AmrBetween<T> a;
+        memset(&a, 0, sizeof a);
+        a.fill.cells = (const CfCell*)dcells.p;
+        a.fill.comps = (const int*)dcomps.p;
+        a.fill.faces = (const CfFace*)dfaces.p;
+        a.fill.ncells = (int)cells.size();
+        a.fill.ncomps = TMK_NCOMP;
+        a.fill.nfaces = (int)faces.size();
+        a.fill.nb = nb;
+        a.fill.fine = tN;
+        a.fill.cold = a.fill.cnew = tC;
+        a.fill.r = r;
+        a.fill.alpha_fixed = 1.0;
+        if ((e = launch_between(st, a))) return e;
     }
     if (!rects.empty()) {
         hipLaunchKernelGGL(k_exchange<T>, dim3((unsigned)rects.size()), dim3(128), 0, st, (const Patch<T>*)dX.p,

@@ -100,6 +100,7 @@ __device__ __forceinline__ StepConst<T> step_const(const Scen& S)
 struct Tile {
     int patch;
     int x0, y0, x1, y1;  // valid cells of this tile (inclusive)
+    int flux;            // marching strips of a hierarchy level: 0 when no face of the strip carries a register flux
 };
 
 template <typename T>

@@ -202,6 +202,53 @@ struct MarchRing {
     static constexpr int LDS_FLOATS = RING_FLOATS + 16 + 4 * 64;
 };
 
+// The faces of strip tl that carry a register flux, from the level's face masks (Patch::fmask): bit
+// j - y0 of m0 for this lane's lo x face on row j, of m1 for its lo y face (row y1 + 1 too).  One mask
+// byte is loaded per row, four rows at a time; the left neighbour's comes by a lane shift and the lower
+// one's from the row before.
+template <typename T>
+__device__ __forceinline__ void march_faces(const Patch<T>& pt, const Tile& tl, int lane, unsigned long long& m0,
+                                            unsigned long long& m1)
+{
+    const __attribute__((address_space(1))) unsigned char* mk = gmem(pt.fmask);
+    const int tnx = tl.x1 - tl.x0 + 1, y0 = tl.y0, rows = tl.y1 - tl.y0 + 1;
+    const int mw = pt.vhi0 - pt.vlo0 + 3;  // the masks cover the descriptor's valid box grown by one
+    const int i = tl.x0 - 3 + min(max(lane, 2), tnx + 3);
+    const size_t at = (size_t)(i - pt.vlo0 + 1) + (size_t)(y0 - pt.vlo1 + 1) * mw;
+    unsigned below = mk[at - mw];
+    for (int k = 0; k <= rows; k += 4) {
+        unsigned b[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) b[q] = mk[at + (size_t)min(k + q, rows) * mw];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const unsigned left = (unsigned)__builtin_amdgcn_update_dpp(0, (int)b[q], DPP_FROM_PREV, 0xF, 0xF, true);
+            if (k + q < rows && register_face(left, b[q])) m0 |= 1ull << (k + q);
+            if (k + q <= rows && register_face(below, b[q])) m1 |= 1ull << (k + q);
+            below = b[q];
+        }
+    }
+    if (lane < 3 || lane > tnx + 3) m0 = 0;
+    if (lane < 3 || lane > tnx + 2) m1 = 0;
+}
+
+// marks the strips tiles[0, n) of a hierarchy level that touch a face of its registers (one wavefront
+// per strip); run once when the launch's tables are built.  Few strips do: the others no longer build
+// face masks or test them on every row (the lens hierarchy's finest level 116 -> 103 us per step)
+template <typename T>
+__global__ void __launch_bounds__(64) k_strip_flux(Tile* tiles, const Patch<T>* patches)
+{
+    const Tile tl = tiles[blockIdx.x];
+    const Patch<T>& pt = patches[tl.patch];
+    unsigned long long m0 = 0, m1 = 0;
+    bool any = pt.F[0] || pt.F[1];
+    if (any && pt.fmask) {
+        march_faces(pt, tl, (int)threadIdx.x, m0, m1);
+        any = __any((m0 | m1) != 0);
+    }
+    if (threadIdx.x == 0) tiles[blockIdx.x].flux = any;
+}
+
 // One side sd of strip tl, marched by one wavefront whose LDS is ring[0, LDS_FLOATS).  tl, sd and
 // ring are the same in every lane and held in scalar registers, so every plane pointer and
 // descriptor of the side stays in scalar registers.
@@ -261,7 +308,9 @@ __device__ __forceinline__ void march_strip(const KArgs<T>& a, const Tile& tl, c
     // the loop's first stores the compiler could only read them again with vector loads, each
     // waiting for every request in flight
     const int ulo1 = __builtin_amdgcn_readfirstlane(pt.ulo1);
-    const bool flux0 = pt.F[0] != nullptr, flux1 = pt.F[1] != nullptr;
+    // most strips of a hierarchy level touch no face of its registers (k_strip_flux marks those that do):
+    // the others run as a single level's
+    const bool flux0 = tl.flux && pt.F[0] != nullptr, flux1 = tl.flux && pt.F[1] != nullptr;
     auto row_off = [=](int j) { return col + (unsigned)(j - ulo1) * rowb; };
     const int y0 = tl.y0, y1 = tl.y1;
 
@@ -307,20 +356,15 @@ __device__ __forceinline__ void march_strip(const KArgs<T>& a, const Tile& tl, c
         return;
     }
     if (flux0 || flux1) {
-        unsigned long long m0 = 0, m1 = 0;
+        unsigned long long m0 = 0, m1 = 0;  // (march_faces)
         const bool lx = flux0 && lane >= 3 && lane <= tnx + 3, ly = flux1 && valid;
         if (!pt.fmask) {
             m0 = lx ? ~0ull : 0ull;
             m1 = ly ? ~0ull : 0ull;
-        } else if (lx || ly) {
-            const __attribute__((address_space(1))) unsigned char* mk = gmem(pt.fmask);
-            const int mw = fvnx + 2;  // the masks cover the descriptor's valid box grown by one
-            for (int j = y0; j <= y1 + 1; ++j) {
-                const size_t q = (size_t)(i - fvlo0 + 1) + (size_t)(j - fvlo1 + 1) * mw;
-                const unsigned b = mk[q];
-                if (lx && j <= y1 && register_face(mk[q - 1], b)) m0 |= 1ull << (j - y0);
-                if (ly && register_face(mk[q - mw], b)) m1 |= 1ull << (j - y0);
-            }
+        } else {
+            march_faces(pt, tl, lane, m0, m1);
+            if (!lx) m0 = 0;
+            if (!ly) m1 = 0;
         }
         fsel[lane] = (unsigned)m0;
         fsel[64 + lane] = (unsigned)(m0 >> 32);
