@@ -186,7 +186,8 @@ struct Mat {
     {
         Mat o = *this;
         const auto s = [sd](T v) {
-            return (T)__longlong_as_double(__double_as_longlong((double)v) ^ (long long)((unsigned long long)sd << 63));
+            return (T)__builtin_bit_cast(
+                double, __builtin_bit_cast(unsigned long long, (double)v) ^ ((unsigned long long)sd << 63));
         };
         o.rho = s(rho); o.lam = s(lam); o.G = s(G); o.Zp = s(Zp); o.Zs = s(Zs); o.lam2G = s(lam2G);
         o.iZp = s(iZp); o.iZs = s(iZs); o.irho = s(irho); o.i2Zp = s(i2Zp); o.i2Zs = s(i2Zs);
