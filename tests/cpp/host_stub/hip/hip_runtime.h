@@ -13,6 +13,7 @@ using std::max;
 using std::min;
 using std::isnan;
 static inline double __builtin_amdgcn_rcp(double x) { return (double)(1.0f / (float)1.0f) / x * (1.0 + 1e-7); }
+static inline float __builtin_amdgcn_rcpf(float x) { return (1.0f / x) * (1.0f + 1e-7f); }
 static inline float __builtin_amdgcn_exp2f(float x) { return exp2f(x); }
 static inline float __builtin_amdgcn_logf(float x) { return log2f(x); }
 static inline float __builtin_amdgcn_fmed3f(float a, float b, float c) { return std::max(std::min(a, b), std::min(std::max(a, b), c)); }

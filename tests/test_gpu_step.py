@@ -95,3 +95,19 @@ def test_divisions_of_either_kind(cs, plastic):
     (tests/test_div2.py), and the one every scenario has: both bit-identical to the oracle."""
     Ug, Ur, Bg, Br = _case(130, 70, [(0, 0, 129, 69)], (0, 0, 0, 0), capi.PREC_FP64, plastic=plastic, cs=cs)
     assert np.array_equal(Ug, Ur) and np.array_equal(Bg, Br)
+
+
+@pytest.mark.parametrize("plastic", [False, True])
+@pytest.mark.parametrize("nx,ny", [(64, 17), (65, 40), (121, 30), (122, 9)])
+def test_fp32_march_no_further_off_than_the_tiles(nx, ny, plastic):
+    """The FP32 march carries characteristics, the tile kernels (march=0) face states: at strips of 58
+    columns and of one, the march is no further from the oracle than they are.  Both accumulate some 30
+    roundings of 2^-24 a step that do not depend on one another, so the largest errors of the two differ
+    by less than a factor of 2, up to one rounding a step."""
+    boxes = [(0, 0, nx - 1, ny - 1)]
+    errs = []
+    for march in (6, 0):
+        Ug, Ur, _, _ = _case(nx, ny, boxes, (0, 1, 0, 0), capi.PREC_FP32_BULK, plastic=plastic, march=march)
+        scale = np.maximum(np.abs(Ur).reshape(22, -1).max(axis=1), 1e-300)
+        errs.append(np.abs(Ug - Ur).reshape(22, -1).max(axis=1) / scale)
+    assert np.all(errs[0] <= 2.0 * errs[1] + NSTEPS * 2.0 ** -24), errs

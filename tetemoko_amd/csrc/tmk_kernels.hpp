@@ -327,7 +327,7 @@ __device__ __forceinline__ void cell_update_side(const PP& P, const Mat<T, D2>& 
             u[7] = fma(kg, xv2, u[7]);
             u[8] = fma(kg, ry * yv2, u[8]);
         }
-        if (plastic) plastic_flow_delta<T, PP>(P, (T)dt, u[3], u[4], u[5], u[6], u[7], u[8], u[9], u[10]);
+        if (plastic) plastic_flow_delta<T, NS, PP>(P, (T)dt, u[3], u[4], u[5], u[6], u[7], u[8], u[9], u[10]);
         return;
     }
     T fxl[7], fxh[7], fyl[7], fyh[7];
@@ -859,7 +859,7 @@ __global__ void k_plastic(const DevParams P, T* U, int ulo0, int ulo1, int unx, 
         T sxy = U[u + (o + 6) * plane], sxz = U[u + (o + 7) * plane], syz = U[u + (o + 8) * plane];
         T lam = U[u + (o + 9) * plane], gam = U[u + (o + 10) * plane];
         if constexpr (stores_delta<T>())
-            plastic_flow_delta<T, DevParams>(P, (T)dt, sxx, syy, szz, sxy, sxz, syz, lam, gam);
+            plastic_flow_delta<T, 3, DevParams>(P, (T)dt, sxx, syy, szz, sxy, sxz, syz, lam, gam);
         else
             plastic_flow<T>(P, (T)dt, sxx, syy, szz, sxy, sxz, syz, lam, gam);
         U[u + (o + 3) * plane] = sxx; U[u + (o + 4) * plane] = syy; U[u + (o + 5) * plane] = szz;

@@ -13,7 +13,7 @@
 //   transverse corrections, final face states, flux difference and update as in the tile
 //   kernels (LinElastPatchGodunov.cpp:101-129, :174-454; LinElastPhysics.cpp:135-179).
 //
-// Every value is the one the tile kernels and the oracle compute for that cell, by the same
+// In FP64 every value is the one the tile kernels and the oracle compute for that cell, by the same
 // expressions in the same order: a slope, face value or face state shared by two cells is
 // computed once, not twice (the face value of x + 1/2 is the same expression whether it is seen
 // as the hi face of cell x or the lo face of cell x + 1, FP additions being commutative).  The
@@ -174,8 +174,77 @@ struct MarchCarry {
     T h1v[2], h1s[2];      // predictor state of the lo y face of row r - 2
     T cpu[2];              // right characteristics of row r - 2's uncorrected W+ (y)
     T cpc[2];              // the same of its corrected W+
-    T f1v[2], f1s[2];      // final state of the lo y face of row r - 2 (FP32)
-    T fl[5];               // flux through the lo y face of row r - 2 (FP64)
+    T fl[5];               // flux through the lo y face of row r - 2
+};
+
+// The FP32 march carries characteristics.  A face's Riemann state needs one characteristic of each
+// cell beside it, the left-moving a = s + z v of the cell above and the right-moving b = s - z v of the
+// cell below (z = Z with the side's velocity sign), and everything up to it is linear in (v, s): the
+// predictor traces a and b from the limited increments, the transverse corrections add to them, and a
+// face keeps D = a - b and E = a + b, whose scales (v = D / (2 z), s = E / 2) go into the constants of
+// what reads them.  The limited increments come straight from the differences and half slopes, not
+// from a face value minus the cell's.  FP32 is bound by instruction issue where the level does not
+// outgrow the caches: a row without plasticity takes about 215 vector instructions for 270 in (v, s),
+// and 4 carried values fewer.  12 single-level scenarios 26.0 -> 23.6 ms for 200 steps, 1024 x 512
+// plastic 200 steps 17.3 -> 15.9 with its state read, the lens hierarchy's 12 coarse steps 60.1 ->
+// 58.3; 8192 x 4096 plastic, bound by memory, 103.5 -> 102.9.  Errors against 64 bits are the same
+// within 3 % (261 x 131, 400 steps: 1.2e-6 both; 1024 x 512, 200 steps: 1.7e-6 both).
+template <>
+struct MarchCarry<float> {
+    float w1[5], w2[5], w3[5];  // as above
+    float dly[4];
+    float dy2[4];               // half the y slopes of row r - 1
+    float fy[4];                // y increments of row r - 2: lo face value minus the cell's
+    float xa[2], xb[2];         // x predictor of row r - 2: a on its lo, b on its hi face, uncorrected
+    float h1d[2], h1e[2];       // predictor state of the lo y face of row r - 2
+    float cpu[2];               // b of row r - 2's uncorrected hi y face
+    float cpc[2];               // the same, corrected
+    float f1d[2], f1e[2];       // final state of the lo y face of row r - 2
+};
+
+// half the monotonized central slope: minmod(l, r, (l + r) / 4).  Half: one product fewer than
+// vl_limit_centred, the same value times 1/2
+__device__ __forceinline__ float half_slope(float l, float r)
+{
+    return __builtin_amdgcn_fmed3f(__builtin_amdgcn_fmed3f(l, r, 0.0f), 0.25f * (l + r), 0.0f);
+}
+
+// a uniform value in a scalar register
+__device__ __forceinline__ float uniform_f(float v) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v))); }
+
+// The FP32 march's constants (ppm_slot, transverse_side and cell_update_side folded for a, b, D, E); h
+// = 1 / (2 Z), r the velocity sign in y.  The signs of the two sweeps leave one set p, q for both
+// transverse corrections, and the flux differences of D need none (r^2 = 1).
+struct MarchConst32 {
+    float ta[2], tb[2];         // tracing: a = (s + ta ds_lo + tb ds_hi) + z (v + ta dv_lo + tb dv_hi)
+    float z[2], zy[2];          // Z, r Z
+    float p[2], q[2];           // transverse: a += p D_k + q E_k', b += p D_k - q E_k'
+    float kv, kl2, kl, kg, ry;  // update
+    template <typename M>
+    __device__ __forceinline__ MarchConst32(const M& m, float dtbydx, float scale, float sc, float r)
+    {
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const float sig = (k == 0 ? m.cp : m.cs) * dtbydx;
+            const float c1 = 0.5f * sig, c2 = c1 * (3.0f - 2.0f * sig);
+            ta[k] = uniform_f((1.0f - c1) - c2);
+            tb[k] = uniform_f(c1 - c2);
+            z[k] = m.Z(k);
+            zy[k] = uniform_f(r * m.Z(k));
+            p[k] = uniform_f(-(scale * (k == 0 ? m.lam : m.G)) * m.i2Z(k));
+            q[k] = uniform_f(-(0.5f * scale * m.irho) * (r * m.Z(k)));
+        }
+        kv = uniform_f(-(0.5f * sc * m.irho));
+        kl2 = uniform_f(-(sc * m.lam2G) * m.i2Zp);
+        kl = uniform_f(-(sc * m.lam) * m.i2Zp);
+        kg = uniform_f(-(sc * m.G) * m.i2Zs);
+        ry = r;
+    }
+};
+
+struct NoMarchConst {
+    template <typename... A>
+    __device__ __forceinline__ explicit NoMarchConst(const A&...) {}
 };
 
 // LDS floats of one wavefront's march: the ring, the plastic return's constants (16 floats), the
@@ -287,6 +356,7 @@ __device__ __forceinline__ void march_strip(const KArgs<T>& a, const Tile& tl, c
         return;
     }
     const bool plastic = PL && P.plast && a.plastic;
+    const std::conditional_t<sizeof(T) == sizeof(float), MarchConst32, NoMarchConst> C(m, dtbydx, scale, K.sc, rvy);
     const int o = 11 * sd;
     // stencil planes vx vy sxx syy sxy, read with the stencil (the in copies)
     constexpr int QC[5] = {0, 1, 3, 4, 6};
@@ -410,11 +480,16 @@ __device__ __forceinline__ void march_strip(const KArgs<T>& a, const Tile& tl, c
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             const T dry = w0[MQ_Y[q]] - A.w1[MQ_Y[q]];
-            const T dy1 = mc_slope(A.dly[q], dry);
-            const T fy1 = ppm_face(A.w2[MQ_Y[q]], A.w1[MQ_Y[q]], A.dy2[q], dy1);
+            if constexpr (f32) {
+                const float dy1 = half_slope(A.dly[q], dry);
+                A.fy[q] = fmaf(-0.5f, A.dly[q], (1.0f / 3.0f) * (A.dy2[q] - dy1));
+                A.dy2[q] = dy1;
+            } else {
+                const T dy1 = mc_slope(A.dly[q], dry);
+                A.fy[q] = ppm_face(A.w2[MQ_Y[q]], A.w1[MQ_Y[q]], A.dy2[q], dy1);
+                A.dy2[q] = dy1;
+            }
             A.dly[q] = dry;
-            A.dy2[q] = dy1;
-            A.fy[q] = fy1;
         }
 #pragma unroll
         for (int q = 0; q < 5; ++q) {
@@ -424,11 +499,18 @@ __device__ __forceinline__ void march_strip(const KArgs<T>& a, const Tile& tl, c
     }
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
-        A.xp.mv[k] = A.xp.ms[k] = A.xp.pv[k] = A.xp.ps[k] = (T)0;
-        A.h1v[k] = A.h1s[k] = A.cpu[k] = A.cpc[k] = A.f1v[k] = A.f1s[k] = (T)0;
+        if constexpr (f32) {
+            A.xa[k] = A.xb[k] = A.h1d[k] = A.h1e[k] = A.f1d[k] = A.f1e[k] = 0.0f;
+        } else {
+            A.xp.mv[k] = A.xp.ms[k] = A.xp.pv[k] = A.xp.ps[k] = (T)0;
+            A.h1v[k] = A.h1s[k] = (T)0;
+        }
+        A.cpu[k] = A.cpc[k] = (T)0;
     }
+    if constexpr (!f32) {
 #pragma unroll
-    for (int k = 0; k < 5; ++k) A.fl[k] = (T)0;
+        for (int k = 0; k < 5; ++k) A.fl[k] = (T)0;
+    }
     if constexpr (ring_fetch) {
 #pragma unroll
         for (int q = 1; q < RING; ++q) request(y0 + q);
@@ -437,6 +519,29 @@ __device__ __forceinline__ void march_strip(const KArgs<T>& a, const Tile& tl, c
 #pragma unroll
         for (int q = 0; q < 5; ++q) A.wn[q] = bld<T>(rin[q], off);
     }
+
+    // a cell's values before the update (side-local component index), and the stores of a row: every row
+    // of the strip issues exactly ROW_STORES stores (the ring's waits count them)
+    auto old_values = [](const MarchCarry<T>& c, T szz, T gam, T (&u)[11]) {
+        u[0] = c.w3[0];
+        u[1] = c.w3[1];
+        u[3] = c.w3[2];
+        u[4] = c.w3[3];
+        u[6] = c.w3[4];
+        u[2] = u[7] = u[8] = u[9] = (T)0;
+        u[5] = szz;
+        u[10] = gam;
+    };
+    auto store_row = [&](unsigned off3, const T (&u)[11]) {
+#pragma unroll
+        for (int q = 0; q < 5; ++q) bst<T>(rout[q], off3, u[QC[q]]);
+        bst<T>(rpw[0], off3, u[5]);
+        if constexpr (PL) {
+            const unsigned offl = plastic ? off3 : kDropOffset;
+            bst<T>(rpw[3], offl, u[9]);
+            bst<T>(rpw[4], offl, u[10]);
+        }
+    };
 
     // one row of the march: after loading row r, the predictors of row r - 2 and the update of
     // row r - 3, from what c carries in; n receives what the next row needs.  The first row
@@ -496,143 +601,248 @@ __device__ __forceinline__ void march_strip(const KArgs<T>& a, const Tile& tl, c
             szz = bld<T>(rpw[0], off3);
             gam = (T)0;
         }
-        // y: differences, slopes of row r - 1, face values at r - 3/2
-        T dry[4], dy1[4], fy1[4];
+        if constexpr (f32) {
+            // y: differences, half slopes of row r - 1, increments at the face r - 3/2 (the hi ones of row
+            // r - 2; the lo ones of row r - 1 are the next row's), then row r - 2's a on its lo y face, b on
+            // its hi one
+            float dy[4], gy[4], fl[4], fh[4];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            dry[q] = w0[MQ_Y[q]] - c.w1[MQ_Y[q]];
-            dy1[q] = mc_slope(c.dly[q], dry[q]);
-            fy1[q] = ppm_face(c.w2[MQ_Y[q]], c.w1[MQ_Y[q]], c.dy2[q], dy1[q]);
-        }
-        // y predictor of row r - 2 (its y faces r - 5/2 and r - 3/2)
-        Pred2<T> yp;
-#pragma unroll
-        for (int k = 0; k < 2; ++k) {
-            const T wv = c.w2[MQ_Y[k]], ws = c.w2[MQ_Y[2 + k]];
-            const T dvm = incr(c.fy[k], wv), dvp = incr(fy1[k], wv);
-            const T dsm = incr(c.fy[2 + k], ws), dsp = incr(fy1[2 + k], ws);
-            ppm_slot<T>(my, k, rvy, dtbydx, true, false, wv, ws, dvm, dvp, dsm, dsp, yp.mv[k], yp.ms[k], yp.pv[k],
-                        yp.ps[k]);
-        }
-        // x predictor of row r - 2: slopes and face values once per lane, neighbours by DPP
-        Pred2<T> xn;
-#pragma unroll
-        for (int k = 0; k < 2; ++k) {
-            T inc[2][2];  // [v|s][m|p]
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const T wc = c.w2[h == 0 ? MQ_XV[k] : MQ_XS[k]];
-                const T wr = dshift<DPP_FROM_NEXT>(wc);  // W(i + 1)
-                const T dr = wr - wc;
-                const T dl = dshift<DPP_FROM_PREV>(dr);  // W(i) - W(i - 1)
-                const T d0 = mc_slope(dl, dr);
-                const T fh = ppm_face(wc, wr, d0, dshift<DPP_FROM_NEXT>(d0));  // face value at i + 1/2
-                const T fl = dshift<DPP_FROM_PREV>(fh);                        // at i - 1/2
-                inc[h][0] = incr(fl, wc);
-                inc[h][1] = incr(fh, wc);
+            for (int q = 0; q < 4; ++q) {
+                dy[q] = w0[MQ_Y[q]] - c.w1[MQ_Y[q]];
+                gy[q] = half_slope(c.dly[q], dy[q]);
+                const float t = (1.0f / 3.0f) * (c.dy2[q] - gy[q]);
+                fl[q] = c.fy[q];
+                fh[q] = fmaf(0.5f, c.dly[q], t);
+                n.fy[q] = fmaf(-0.5f, c.dly[q], t);
+                n.dly[q] = dy[q];
+                n.dy2[q] = gy[q];
+                ppm_limit(fl[q], fh[q]);
             }
-            ppm_slot<T>(m, k, (T)1, dtbydx, true, false, c.w2[MQ_XV[k]], c.w2[MQ_XS[k]], inc[0][0], inc[0][1],
-                        inc[1][0], inc[1][1], xn.mv[k], xn.ms[k], xn.pv[k], xn.ps[k]);
-        }
-        // predictor state of the lo x face of row r - 2 (its left lane's W+ and its W-)
-        T h0v[2], h0s[2];
-        {
-            T cpx[2], wpL[2], wmR[2];
-            right_chars_side<T, 2>(m, (T)1, xn.pv, xn.ps, cpx);
+            // a on the lo face and b on the hi face of a cell from its values and limited increments
+            auto trace = [&](int k, float z, float wv, float ws, float vm, float vp, float sm, float sp, float& ca, float& cb) {
+                ca = fmaf(z, fmaf(C.tb[k], vp, fmaf(C.ta[k], vm, wv)), fmaf(C.tb[k], sp, fmaf(C.ta[k], sm, ws)));
+                cb = fmaf(-z, fmaf(C.tb[k], vm, fmaf(C.ta[k], vp, wv)), fmaf(C.tb[k], sm, fmaf(C.ta[k], sp, ws)));
+            };
+            float ya[2], yb[2];
 #pragma unroll
-            for (int k = 0; k < 2; ++k) wpL[k] = dshift<DPP_FROM_PREV>(cpx[k]);
-            left_chars_side<T, 2>(m, (T)1, xn.mv, xn.ms, wmR);
-            riemann_side<T, 2>(m, (T)1, wpL, wmR, h0v, h0s);
-        }
-        // predictor state of the lo y face of row r - 2 (row r - 3's uncorrected W+, its W-)
-        {
-            T wmR[2];
-            left_chars_side<T, 2>(my, rvy, yp.mv, yp.ms, wmR);
-            riemann_side<T, 2>(my, rvy, c.cpu, wmR, n.h1v, n.h1s);
-            right_chars_side<T, 2>(my, rvy, yp.pv, yp.ps, n.cpu);
-        }
-        // y predictor corrected with the x-face states of its cell (GETADWDXF, dir2 = x)
-        {
-            T hv[2], hs[2];
+            for (int k = 0; k < 2; ++k)
+                trace(k, C.zy[k], c.w2[MQ_Y[k]], c.w2[MQ_Y[2 + k]], fl[k], fh[k], fl[2 + k], fh[2 + k], ya[k], yb[k]);
+            // x: the same within row r - 2, once per lane, the neighbours' by DPP
 #pragma unroll
             for (int k = 0; k < 2; ++k) {
-                hv[k] = dshift<DPP_FROM_NEXT>(h0v[k]);
-                hs[k] = dshift<DPP_FROM_NEXT>(h0s[k]);
-            }
-            transverse_side<T, 2>(m, scale, h0v, h0s, hv, hs, yp.mv, yp.ms);
-            transverse_side<T, 2>(m, scale, h0v, h0s, hv, hs, yp.pv, yp.ps);
-        }
-        // final state of the lo y face of row r - 2 (row r - 3's corrected W+, its corrected W-)
-        {
-            T wmR[2];
-            left_chars_side<T, 2>(my, rvy, yp.mv, yp.ms, wmR);
-            riemann_side<T, 2>(my, rvy, c.cpc, wmR, n.f1v, n.f1s);
-            right_chars_side<T, 2>(my, rvy, yp.pv, yp.ps, n.cpc);
-        }
-        // FP64 carries the face's flux, which the row above it reads again: the reference's flux of a face
-        // is one expression wherever it is read from (FP32 differences the face states instead)
-        T fyh[7];
-        if constexpr (!regroup<T>()) {
-            face_flux_side<T, 2>(my, n.f1v, n.f1s, rvy, fyh);
+                float inc[2][2];  // [v|s][lo|hi]
 #pragma unroll
-            for (int k = 0; k < 5; ++k) n.fl[k] = fyh[k];
-        }
-        const int j2 = r - 2;
-        // flux registers (multi-level): the lo y face of row r - 2, the x faces of row r - 3
-        // (below); the lane's column, hidden from the compiler here, so that it builds each face's
-        // address in place rather than keeping a 64-bit per-lane address alive through the loop
-        if (flux1 && j2 >= y0 && fbit(1, j2 - y0)) {
-            int ix = i - fvlo0;
-            asm volatile("" : "+v"(ix));
-            put_face_flux<T, 2>(Fo1, (size_t)ix + (size_t)(j2 - fvlo1) * fvnx, (size_t)fvnx * (fvny + 1), my, 1, n.f1v,
-                                n.f1s, rvy, sd);
-        }
-        // row r - 3, a row of the strip: x predictor corrected with the y-face states below and
-        // above it, its final x-face state and its update
-        if (strip_row) {
-            T f0v[2], f0s[2];
-            Pred2<T> xp = c.xp;
-            transverse_side<T, 2>(m, scx, c.h1v, c.h1s, n.h1v, n.h1s, xp.mv, xp.ms);
-            transverse_side<T, 2>(m, scx, c.h1v, c.h1s, n.h1v, n.h1s, xp.pv, xp.ps);
-            T cpx[2], wpL[2], wmR[2];
-            right_chars_side<T, 2>(m, (T)1, xp.pv, xp.ps, cpx);
-#pragma unroll
-            for (int k = 0; k < 2; ++k) wpL[k] = dshift<DPP_FROM_PREV>(cpx[k]);
-            left_chars_side<T, 2>(m, (T)1, xp.mv, xp.ms, wmR);
-            riemann_side<T, 2>(m, (T)1, wpL, wmR, f0v, f0s);
-            if (flux0 && fbit(0, j3 - y0)) {
-                int ix = i - fvlo0;
-                asm volatile("" : "+v"(ix));
-                put_face_flux<T, 2>(Fo0, (size_t)ix + (size_t)(j3 - fvlo1) * (fvnx + 1), (size_t)(fvnx + 1) * fvny, m,
-                                    0, f0v, f0s, (T)1, sd);
+                for (int h = 0; h < 2; ++h) {
+                    const float wc = c.w2[h == 0 ? MQ_XV[k] : MQ_XS[k]];
+                    const float dr = dshift<DPP_FROM_NEXT>(wc) - wc;
+                    const float g = half_slope(dshift<DPP_FROM_PREV>(dr), dr);
+                    const float t = (1.0f / 3.0f) * (g - dshift<DPP_FROM_NEXT>(g));
+                    inc[h][0] = dshift<DPP_FROM_PREV>(fmaf(-0.5f, dr, t));
+                    inc[h][1] = fmaf(0.5f, dr, t);
+                    ppm_limit(inc[h][0], inc[h][1]);
+                }
+                trace(k, C.z[k], c.w2[MQ_XV[k]], c.w2[MQ_XS[k]], inc[0][0], inc[0][1], inc[1][0], inc[1][1], n.xa[k], n.xb[k]);
             }
-            // update of row r - 3: every row of the strip issues exactly ROW_STORES stores (the
-            // ring's waits count them)
-            // every lane runs the update (a lane outside the strip has off3 past the planes)
-            T u[11];
-            u[0] = c.w3[0];
-            u[1] = c.w3[1];
-            u[3] = c.w3[2];
-            u[4] = c.w3[3];
-            u[6] = c.w3[4];
-            u[2] = u[7] = u[8] = u[9] = (T)0;
-            u[5] = szz;
-            u[10] = gam;
-            if constexpr (f32) {
-                Faces1<T, 2> F;
+            // predictor states of the lo x face (the left lane's b and its a) and the lo y face (row r - 3's
+            // b and its a) of row r - 2
+            float h0d[2], h0e[2];
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                const float bl = dshift<DPP_FROM_PREV>(n.xb[k]);
+                h0d[k] = n.xa[k] - bl;
+                h0e[k] = n.xa[k] + bl;
+                n.h1d[k] = ya[k] - c.cpu[k];
+                n.h1e[k] = ya[k] + c.cpu[k];
+                n.cpu[k] = yb[k];
+            }
+            // y predictor corrected with the x-face states of its cell (GETADWDXF, dir2 = x), then the final
+            // state of the lo y face of row r - 2
+            {
+                float dd[2], de[2];
 #pragma unroll
                 for (int k = 0; k < 2; ++k) {
-                    F.xlv[k] = f0v[k];
-                    F.xls[k] = f0s[k];
-                    F.xhv[k] = dshift<DPP_FROM_NEXT>(f0v[k]);
-                    F.xhs[k] = dshift<DPP_FROM_NEXT>(f0s[k]);
-                    F.ylv[k] = c.f1v[k];
-                    F.yls[k] = c.f1s[k];
-                    F.yhv[k] = n.f1v[k];
-                    F.yhs[k] = n.f1s[k];
+                    dd[k] = dshift<DPP_FROM_NEXT>(h0d[k]) - h0d[k];
+                    de[k] = dshift<DPP_FROM_NEXT>(h0e[k]) - h0e[k];
                 }
-                cell_update_side<T, 2>(pc, m, dt, K.sc, plastic, rvy, F, u);
-            } else {
+#pragma unroll
+                for (int k = 0; k < 2; ++k) {
+                    const float ca = fmaf(C.q[k], de[1 - k], fmaf(C.p[k], dd[k], ya[k]));
+                    n.f1d[k] = ca - c.cpc[k];
+                    n.f1e[k] = ca + c.cpc[k];
+                    n.cpc[k] = fmaf(-C.q[k], de[1 - k], fmaf(C.p[k], dd[k], yb[k]));
+                }
+            }
+            // (v, s) of a face, for the flux registers
+            auto face_state = [&](float r, const float (&d)[2], const float (&e)[2], float (&v)[2], float (&sv)[2]) {
+#pragma unroll
+                for (int k = 0; k < 2; ++k) {
+                    v[k] = d[k] * (r * m.i2Z(k));
+                    sv[k] = 0.5f * e[k];
+                }
+            };
+            const int j2 = r - 2;
+            // flux registers (multi-level): the lo y face of row r - 2, the x faces of row r - 3 (below); the
+            // lane's column hidden from the compiler, as in the FP64 march
+            if (flux1 && j2 >= y0 && fbit(1, j2 - y0)) {
+                int ix = i - fvlo0;
+                asm volatile("" : "+v"(ix));
+                float v[2], sv[2];
+                face_state(rvy, n.f1d, n.f1e, v, sv);
+                put_face_flux<T, 2>(Fo1, (size_t)ix + (size_t)(j2 - fvlo1) * fvnx, (size_t)fvnx * (fvny + 1), m, 1, v, sv,
+                                    rvy, sd);
+            }
+            // row r - 3, a row of the strip: x predictor corrected with the y-face states below and above it,
+            // its final x-face state and its update
+            if (strip_row) {
+                float f0d[2], f0e[2];
+#pragma unroll
+                for (int k = 0; k < 2; ++k) {
+                    const float dd = n.h1d[k] - c.h1d[k], de = n.h1e[1 - k] - c.h1e[1 - k];
+                    const float ca = fmaf(C.q[k], de, fmaf(C.p[k], dd, c.xa[k]));
+                    const float bl = dshift<DPP_FROM_PREV>(fmaf(-C.q[k], de, fmaf(C.p[k], dd, c.xb[k])));
+                    f0d[k] = ca - bl;
+                    f0e[k] = ca + bl;
+                }
+                if (flux0 && fbit(0, j3 - y0)) {
+                    int ix = i - fvlo0;
+                    asm volatile("" : "+v"(ix));
+                    float v[2], sv[2];
+                    face_state(1.0f, f0d, f0e, v, sv);
+                    put_face_flux<T, 2>(Fo0, (size_t)ix + (size_t)(j3 - fvlo1) * (fvnx + 1), (size_t)(fvnx + 1) * fvny, m, 0,
+                                        v, sv, 1.0f, sd);
+                }
+                // every lane runs the update (a lane outside the strip has off3 past the planes); differences of
+                // the face states first, then one uniform coefficient per component (cell_update_side)
+                T u[11];
+                old_values(c, szz, gam, u);
+                const float xd0 = dshift<DPP_FROM_NEXT>(f0d[0]) - f0d[0], xd1 = dshift<DPP_FROM_NEXT>(f0d[1]) - f0d[1];
+                const float xe0 = dshift<DPP_FROM_NEXT>(f0e[0]) - f0e[0], xe1 = dshift<DPP_FROM_NEXT>(f0e[1]) - f0e[1];
+                const float yd0 = n.f1d[0] - c.f1d[0], yd1 = n.f1d[1] - c.f1d[1];
+                const float ye0 = n.f1e[0] - c.f1e[0], ye1 = n.f1e[1] - c.f1e[1];
+                u[0] = fmaf(C.kv, fmaf(C.ry, ye1, xe0), u[0]);
+                u[1] = fmaf(C.kv, fmaf(C.ry, ye0, xe1), u[1]);
+                u[3] = fmaf(C.kl2, xd0, fmaf(C.kl, yd0, u[3]));
+                u[4] = fmaf(C.kl, xd0, fmaf(C.kl2, yd0, u[4]));
+                u[5] = fmaf(C.kl, xd0 + yd0, u[5]);
+                u[6] = fmaf(C.kg, xd1 + yd1, u[6]);
+                if (plastic) plastic_flow_delta<T, 2, PlasticConstL>(pc, (T)dt, u[3], u[4], u[5], u[6], u[7], u[8], u[9], u[10]);
+                store_row(off3, u);
+            }
+        } else {
+            // y: differences, slopes of row r - 1, face values at r - 3/2
+            T dry[4], dy1[4], fy1[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                dry[q] = w0[MQ_Y[q]] - c.w1[MQ_Y[q]];
+                dy1[q] = mc_slope(c.dly[q], dry[q]);
+                fy1[q] = ppm_face(c.w2[MQ_Y[q]], c.w1[MQ_Y[q]], c.dy2[q], dy1[q]);
+            }
+            // y predictor of row r - 2 (its y faces r - 5/2 and r - 3/2)
+            Pred2<T> yp;
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                const T wv = c.w2[MQ_Y[k]], ws = c.w2[MQ_Y[2 + k]];
+                const T dvm = incr(c.fy[k], wv), dvp = incr(fy1[k], wv);
+                const T dsm = incr(c.fy[2 + k], ws), dsp = incr(fy1[2 + k], ws);
+                ppm_slot<T>(my, k, rvy, dtbydx, true, false, wv, ws, dvm, dvp, dsm, dsp, yp.mv[k], yp.ms[k], yp.pv[k],
+                            yp.ps[k]);
+            }
+            // x predictor of row r - 2: slopes and face values once per lane, neighbours by DPP
+            Pred2<T> xn;
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                T inc[2][2];  // [v|s][m|p]
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const T wc = c.w2[h == 0 ? MQ_XV[k] : MQ_XS[k]];
+                    const T wr = dshift<DPP_FROM_NEXT>(wc);  // W(i + 1)
+                    const T dr = wr - wc;
+                    const T dl = dshift<DPP_FROM_PREV>(dr);  // W(i) - W(i - 1)
+                    const T d0 = mc_slope(dl, dr);
+                    const T fh = ppm_face(wc, wr, d0, dshift<DPP_FROM_NEXT>(d0));  // face value at i + 1/2
+                    const T fl = dshift<DPP_FROM_PREV>(fh);                        // at i - 1/2
+                    inc[h][0] = incr(fl, wc);
+                    inc[h][1] = incr(fh, wc);
+                }
+                ppm_slot<T>(m, k, (T)1, dtbydx, true, false, c.w2[MQ_XV[k]], c.w2[MQ_XS[k]], inc[0][0], inc[0][1],
+                            inc[1][0], inc[1][1], xn.mv[k], xn.ms[k], xn.pv[k], xn.ps[k]);
+            }
+            // predictor state of the lo x face of row r - 2 (its left lane's W+ and its W-)
+            T h0v[2], h0s[2];
+            {
+                T cpx[2], wpL[2], wmR[2];
+                right_chars_side<T, 2>(m, (T)1, xn.pv, xn.ps, cpx);
+#pragma unroll
+                for (int k = 0; k < 2; ++k) wpL[k] = dshift<DPP_FROM_PREV>(cpx[k]);
+                left_chars_side<T, 2>(m, (T)1, xn.mv, xn.ms, wmR);
+                riemann_side<T, 2>(m, (T)1, wpL, wmR, h0v, h0s);
+            }
+            // predictor state of the lo y face of row r - 2 (row r - 3's uncorrected W+, its W-)
+            {
+                T wmR[2];
+                left_chars_side<T, 2>(my, rvy, yp.mv, yp.ms, wmR);
+                riemann_side<T, 2>(my, rvy, c.cpu, wmR, n.h1v, n.h1s);
+                right_chars_side<T, 2>(my, rvy, yp.pv, yp.ps, n.cpu);
+            }
+            // y predictor corrected with the x-face states of its cell (GETADWDXF, dir2 = x)
+            {
+                T hv[2], hs[2];
+#pragma unroll
+                for (int k = 0; k < 2; ++k) {
+                    hv[k] = dshift<DPP_FROM_NEXT>(h0v[k]);
+                    hs[k] = dshift<DPP_FROM_NEXT>(h0s[k]);
+                }
+                transverse_side<T, 2>(m, scale, h0v, h0s, hv, hs, yp.mv, yp.ms);
+                transverse_side<T, 2>(m, scale, h0v, h0s, hv, hs, yp.pv, yp.ps);
+            }
+            // final state of the lo y face of row r - 2 (row r - 3's corrected W+, its corrected W-)
+            T f1v[2], f1s[2];
+            {
+                T wmR[2];
+                left_chars_side<T, 2>(my, rvy, yp.mv, yp.ms, wmR);
+                riemann_side<T, 2>(my, rvy, c.cpc, wmR, f1v, f1s);
+                right_chars_side<T, 2>(my, rvy, yp.pv, yp.ps, n.cpc);
+            }
+            // the face's flux is carried too: the row above it reads it again, and the reference's flux of a
+            // face is one expression wherever it is read from
+            T fyh[7];
+            face_flux_side<T, 2>(my, f1v, f1s, rvy, fyh);
+#pragma unroll
+            for (int k = 0; k < 5; ++k) n.fl[k] = fyh[k];
+            const int j2 = r - 2;
+            // flux registers (multi-level): the lo y face of row r - 2, the x faces of row r - 3
+            // (below); the lane's column, hidden from the compiler here, so that it builds each face's
+            // address in place rather than keeping a 64-bit per-lane address alive through the loop
+            if (flux1 && j2 >= y0 && fbit(1, j2 - y0)) {
+                int ix = i - fvlo0;
+                asm volatile("" : "+v"(ix));
+                put_face_flux<T, 2>(Fo1, (size_t)ix + (size_t)(j2 - fvlo1) * fvnx, (size_t)fvnx * (fvny + 1), my, 1, f1v,
+                                    f1s, rvy, sd);
+            }
+            // row r - 3, a row of the strip: x predictor corrected with the y-face states below and
+            // above it, its final x-face state and its update
+            if (strip_row) {
+                T f0v[2], f0s[2];
+                Pred2<T> xp = c.xp;
+                transverse_side<T, 2>(m, scx, c.h1v, c.h1s, n.h1v, n.h1s, xp.mv, xp.ms);
+                transverse_side<T, 2>(m, scx, c.h1v, c.h1s, n.h1v, n.h1s, xp.pv, xp.ps);
+                T cpx[2], wpL[2], wmR[2];
+                right_chars_side<T, 2>(m, (T)1, xp.pv, xp.ps, cpx);
+#pragma unroll
+                for (int k = 0; k < 2; ++k) wpL[k] = dshift<DPP_FROM_PREV>(cpx[k]);
+                left_chars_side<T, 2>(m, (T)1, xp.mv, xp.ms, wmR);
+                riemann_side<T, 2>(m, (T)1, wpL, wmR, f0v, f0s);
+                if (flux0 && fbit(0, j3 - y0)) {
+                    int ix = i - fvlo0;
+                    asm volatile("" : "+v"(ix));
+                    put_face_flux<T, 2>(Fo0, (size_t)ix + (size_t)(j3 - fvlo1) * (fvnx + 1), (size_t)(fvnx + 1) * fvny, m,
+                                        0, f0v, f0s, (T)1, sd);
+                }
+                // update of row r - 3: every row of the strip issues exactly ROW_STORES stores (the
+                // ring's waits count them)
+                // every lane runs the update (a lane outside the strip has off3 past the planes)
+                T u[11];
+                old_values(c, szz, gam, u);
                 T fxl[7], fxh[7], fyl[7];
                 face_flux_side<T, 2>(m, f0v, f0s, (T)1, fxl);
 #pragma unroll
@@ -643,23 +853,15 @@ __device__ __forceinline__ void march_strip(const KArgs<T>& a, const Tile& tl, c
                 flux_update<T>(K.sc, fxl, fxh, fyl, fyh, u);
                 if (plastic)
                     plastic_flow<T, PlasticConstL64>(pc64, (T)dt, u[3], u[4], u[5], u[6], u[7], u[8], u[9], u[10]);
+                store_row(off3, u);
             }
+            n.xp = xn;
 #pragma unroll
-            for (int q = 0; q < 5; ++q) bst<T>(rout[q], off3, u[QC[q]]);
-            bst<T>(rpw[0], off3, u[5]);
-            if constexpr (PL) {
-                const unsigned offl = plastic ? off3 : kDropOffset;
-                bst<T>(rpw[3], offl, u[9]);
-                bst<T>(rpw[4], offl, u[10]);
+            for (int q = 0; q < 4; ++q) {
+                n.dly[q] = dry[q];
+                n.dy2[q] = dy1[q];
+                n.fy[q] = fy1[q];
             }
-        }
-        // carried to the next row
-        n.xp = xn;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            n.dly[q] = dry[q];
-            n.dy2[q] = dy1[q];
-            n.fy[q] = fy1[q];
         }
 #pragma unroll
         for (int q = 0; q < 5; ++q) {

@@ -982,34 +982,43 @@ __device__ __forceinline__ float plastic_pbg(const PlasticConstL& P, int k) { re
 __device__ __forceinline__ float plastic_pf(const PlasticConstL& P, int k) { return P.c[7 + k]; }
 __device__ __forceinline__ float plastic_G(const PlasticConstL& P) { return P.c[13]; }
 
-// PP: DevParams or PlasticConstL
-template <typename T, typename PP>
+// The deviator is free of trace, so J2 = (exx^2 + eyy^2 + ezz^2) / 2 + the shears.  The divisions are by
+// reciprocal (the hardware's, within an ulp, of tau): they scale increments far below the stresses.
+// PP: DevParams or PlasticConstL; NS = 2: mode II, whose anti-plane stresses are zero.
+template <typename T, int NS, typename PP>
 __device__ __forceinline__ void plastic_flow_delta(const PP& P, T dt, T& dxx, T& dyy, T& dzz, T& dxy, T& dxz,
                                                    T& dyz, T& plam, T& pgam)
 {
     const T md = (dxx + dyy + dzz) * (T)(1.0 / 3.0);
     const T exx = (dxx - md) + (T)plastic_pbg(P, 1), eyy = (dyy - md) + (T)plastic_pbg(P, 2), ezz = (dzz - md) + (T)plastic_pbg(P, 3);
-    const T sxy = dxy + (T)plastic_pbg(P, 4), sxz = dxz + (T)plastic_pbg(P, 5), syz = dyz + (T)plastic_pbg(P, 6);
+    const T sxy = dxy + (T)plastic_pbg(P, 4);
+    T sxz = (T)0, syz = (T)0;
     const T sigma = md + (T)plastic_pbg(P, 0);
-    const T a = exx - eyy, b = eyy - ezz, c = ezz - exx;
-    const T J2 = (a * a + b * b + c * c) * (T)(1.0 / 6.0) + sxy * sxy + sxz * sxz + syz * syz;
+    T J2 = (T)0.5 * (exx * exx + eyy * eyy + ezz * ezz) + sxy * sxy;
+    if constexpr (NS == 3) {
+        sxz = dxz + (T)plastic_pbg(P, 5);
+        syz = dyz + (T)plastic_pbg(P, 6);
+        J2 = J2 + sxz * sxz + syz * syz;
+    }
     const T bb = (T)plastic_pf(P, 1) + pgam * (T)plastic_pf(P, 2);
     const T ys = fmax(-(T)plastic_pf(P, 0) * sigma + bb, (T)0);
     // yield iff sqrt(J2) > ys >= 0, i.e. J2 > ys^2: the root only where the cell yields
     if (!(J2 > ys * ys)) { plam = (T)0; return; }
     const T tau = sqrt(J2);
     const T Y = tau - ys;
-    plam = Y / (dt * (T)plastic_pf(P, 3) + (T)plastic_pf(P, 4));
-    pgam = pgam + dt * plam;
-    const T dG = dt * plam * (T)plastic_G(P);
-    const T g = dG / tau;  // 1 - tau_new / (tau_new + dt lam G), tau_new = tau - dt lam G
-    const T dm = dt * plam * (T)plastic_pf(P, 5);
+    plam = Y * __builtin_amdgcn_rcpf(dt * (T)plastic_pf(P, 3) + (T)plastic_pf(P, 4));
+    const T dl = dt * plam;
+    pgam = pgam + dl;
+    const T g = dl * (T)plastic_G(P) * __builtin_amdgcn_rcpf(tau);  // 1 - tau_new / (tau_new + dt lam G), tau_new = tau - dt lam G
+    const T dm = dl * (T)plastic_pf(P, 5);
     dxx = dxx - (dm + g * exx);
     dyy = dyy - (dm + g * eyy);
     dzz = dzz - (dm + g * ezz);
     dxy = dxy - g * sxy;
-    dxz = dxz - g * sxz;
-    dyz = dyz - g * syz;
+    if constexpr (NS == 3) {
+        dxz = dxz - g * sxz;
+        dyz = dyz - g * syz;
+    }
 }
 
 }  // namespace tmk
