@@ -1,0 +1,65 @@
+"""Reading a box back (tmk_level_download): its planes come in pieces of 1 MiB through pinned slots, by
+one, two or four host threads, and FP32 levels add the background on the host.
+
+The sizes: one piece; pieces that end inside a plane; two and four threads with a short last piece;
+several boxes of one island; readers on several threads at once.  What is read is what was uploaded:
+FP64 bit for bit, FP32 the background plus the difference rounded to FP32, both exact in NumPy.
+"""
+import threading
+
+import numpy as np
+import pytest
+
+from tetemoko_amd import capi, scenarios
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(nx, ny, precision, maxbox=0, seed=1):
+    cfg = scenarios.config_c1(seed=seed, nx=nx, ny=ny, dx=25.0)
+    U, B = scenarios.level_arrays(cfg)
+    scenarios.perturb(U, seed=seed, amp_v=1.0, amp_s=5.0)
+    boxes = scenarios.split_boxes(nx, ny, maxbox) if maxbox else [(0, 0, nx - 1, ny - 1)]
+    ctx = capi.Context(cfg, precision)
+    lev = capi.Level(ctx, boxes)
+    for k, b in enumerate(boxes):
+        lev.upload(k, scenarios.box_view(U, b), scenarios.box_bview(B, b) if b[1] == 0 else None)
+    want = U
+    if precision == capi.PREC_FP32_BULK:
+        bg = scenarios.background_vector(cfg)[:, None, None]
+        want = (U - bg).astype(np.float32).astype(np.float64) + bg
+    ok = True
+    for k, b in enumerate(boxes):
+        Ub = np.full_like(scenarios.box_view(U, b), np.nan)
+        Bb = np.full_like(scenarios.box_bview(B, b), np.nan) if b[1] == 0 else None
+        lev.download(k, Ub, Bb)
+        g = scenarios.GHOST
+        ok = ok and np.array_equal(Ub[:, g:-g, g:-g], scenarios.box_view(want, b)[:, g:-g, g:-g])
+        if Bb is not None:
+            ok = ok and np.array_equal(Bb[:, g:-g], scenarios.box_bview(B, b)[:, g:-g])
+    lev.close()
+    ctx.close()
+    return ok
+
+
+@pytest.mark.parametrize("precision", [capi.PREC_FP64, capi.PREC_FP32_BULK])
+@pytest.mark.parametrize("nx,ny,maxbox", [(9, 8, 0), (101, 73, 0), (257, 201, 0), (401, 333, 0), (300, 190, 97)])
+def test_what_was_uploaded(nx, ny, maxbox, precision):
+    assert _check(nx, ny, precision, maxbox)
+
+
+def test_readers_on_several_threads():
+    got = [None] * 6
+
+    def run(t):
+        got[t] = all(_check(150 + 40 * t, 90 + 31 * t, capi.PREC_FP64 if t % 2 else capi.PREC_FP32_BULK, seed=t + 1)
+                     for _ in range(2))
+
+    th = [threading.Thread(target=run, args=(t,)) for t in range(6)]
+    for t in th:
+        t.start()
+    for t in th:
+        t.join()
+    assert got == [True] * 6
+    assert capi.lib().tmk_cache_trim() == 0
+    assert _check(120, 80, capi.PREC_FP64)
