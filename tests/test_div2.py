@@ -84,3 +84,14 @@ def test_signed_zero_and_sign():
     assert math.copysign(1.0, -0.0 * (1 / y) + -0.0) == -1.0
     for x in (3.7, -3.7, 1e-200, -1e-200):
         assert divr2(x, y) == x / y
+
+
+@pytest.mark.parametrize("y", [3.0, 6.0])
+def test_the_plastic_return_divides_exactly(y):
+    """div3, div6: the low words are exact and every quotient rounds as the division does."""
+    h, l = (1.0 / 3.0, 2.0 ** -54 / 3.0) if y == 3.0 else (0.5 / 3.0, 2.0 ** -55 / 3.0)
+    assert h == 1.0 / y and l == float(F(1) / F(y) - F(h))
+    assert not suspects(y)[1]
+    r = random.Random(11)
+    for x in [float(k) for k in range(-40, 41)] + [r.uniform(-1, 1) * 10.0 ** r.randint(-30, 12) for _ in range(20000)]:
+        assert divr2(x, y) == x / y

@@ -815,15 +815,15 @@ static void fill_dev_params(const tmk_params& h, DevParams& P)
     P.irho = 1.0 / P.rho;
     P.i2Zp = 0.5 * P.iZp;
     P.i2Zs = 0.5 * P.iZs;
-    P.lZp = recip_low(P.Zp, P.iZp);
-    P.lZs = recip_low(P.Zs, P.iZs);
+    P.l2Zp = 0.5 * recip_low(P.Zp, P.iZp);
+    P.l2Zs = 0.5 * recip_low(P.Zs, P.iZs);
     P.lrho = recip_low(P.rho, P.irho);
     P.div2 = div2_exact(P.Zp) && div2_exact(P.Zs) && div2_exact(P.rho);
     P.K = P.lam + 2.0 * h.G / 3.0;
     P.den = 2.0 * h.G + P.lam;
     P.lam2G = P.lam + 2.0 * h.G;
     P.frho = (float)P.rho; P.flam = (float)P.lam; P.fG = (float)P.G; P.fZp = (float)P.Zp; P.fZs = (float)P.Zs;
-    P.fden = (float)P.den; P.flam2G = (float)P.lam2G; P.fiZp = (float)P.iZp; P.fiZs = (float)P.iZs;
+    P.fden = (float)P.den; P.flam2G = (float)P.lam2G;
     P.firho = (float)P.irho; P.fi2Zp = (float)P.i2Zp; P.fi2Zs = (float)P.i2Zs;
     P.fcp = (float)P.cp; P.fcs = (float)P.cs;
     const double s9[9] = {0.0, 0.0, 0.0, h.sxx0, h.syy0, h.szz0, h.sxy0, h.sxz0, h.syz0};

@@ -278,7 +278,8 @@ template <typename T>
 __device__ __forceinline__ void flux_update(T sc, const T (&fxl)[7], const T (&fxh)[7], const T (&fyl)[7],
                                             const T (&fyh)[7], T (&u)[11])
 {
-    // dU = (0 + (Fx_hi - Fx_lo)) + (Fy_hi - Fy_lo); U += dU * (-dt/dx)
+    // dU = (0 + (Fx_hi - Fx_lo)) + (Fy_hi - Fy_lo); U += dU * (-dt/dx) (the sum with 0 only changes the
+    // sign of a zero and is left out)
     // x flux: vx<-F(vn) vy<-F(vt) sxx<-F(snn) syy,szz<-F(stt) sxy<-F(snt)
     // y flux: vy<-F(vn) vx<-F(vt) syy<-F(snn) sxx,szz<-F(stt) sxy<-F(snt)
     const T dvx_x = fxh[0] - fxl[0], dvx_y = fyh[2] - fyl[2];
@@ -287,12 +288,12 @@ __device__ __forceinline__ void flux_update(T sc, const T (&fxl)[7], const T (&f
     const T dsyy_x = fxh[4] - fxl[4], dsyy_y = fyh[1] - fyl[1];
     const T dszz_x = fxh[4] - fxl[4], dszz_y = fyh[4] - fyl[4];
     const T dsxy_x = fxh[3] - fxl[3], dsxy_y = fyh[3] - fyl[3];
-    u[0] = u[0] + (((T)0 + dvx_x) + dvx_y) * sc;
-    u[1] = u[1] + (((T)0 + dvy_x) + dvy_y) * sc;
-    u[3] = u[3] + (((T)0 + dsxx_x) + dsxx_y) * sc;
-    u[4] = u[4] + (((T)0 + dsyy_x) + dsyy_y) * sc;
-    u[5] = u[5] + (((T)0 + dszz_x) + dszz_y) * sc;
-    u[6] = u[6] + (((T)0 + dsxy_x) + dsxy_y) * sc;
+    u[0] = u[0] + (dvx_x + dvx_y) * sc;
+    u[1] = u[1] + (dvy_x + dvy_y) * sc;
+    u[3] = u[3] + (dsxx_x + dsxx_y) * sc;
+    u[4] = u[4] + (dsyy_x + dsyy_y) * sc;
+    u[5] = u[5] + (dszz_x + dszz_y) * sc;
+    u[6] = u[6] + (dsxy_x + dsxy_y) * sc;
 }
 
 // New values of one side's state of a valid cell from its old values u[0..10] (side-local

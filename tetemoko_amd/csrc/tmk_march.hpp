@@ -47,19 +47,27 @@ __device__ __forceinline__ bool march_interior(const Tile& t, const DevParams& P
            t.y1 + 3 <= P.dhi[1];
 }
 
-// the monotonized central slope of a cell from its two one-sided differences (vl_slope, side 0)
-template <typename T>
-__device__ __forceinline__ T mc_slope(T dl, T dr)
+// half the monotonized central slope of a cell from its two one-sided differences: min(|l|, |r|,
+// |l + r| / 4) with their sign, 0 at extrema (vl_slope, side 0; half: two products fewer, and halving is
+// exact).  FP32 from medians (vl_limit_centred).
+__device__ __forceinline__ float half_slope(float l, float r)
 {
-    return vl_limit_centred((T)0.5 * (dr + dl), dl, dr);
+    return __builtin_amdgcn_fmed3f(__builtin_amdgcn_fmed3f(l, r, 0.0f), 0.25f * (l + r), 0.0f);
+}
+__device__ __forceinline__ double half_slope(double l, double r)
+{
+    const double c = l + r;
+    double g = fmin(fmin(fabs(l), fabs(r)), 0.25 * fabs(c));
+    if (l * r < 0.0) g = 0.0;
+    return copysign(g, c);
 }
 
-// PPM face value between cells a (lo) and b (hi) with slopes da, db (ppm_incr's fl / fh)
-template <typename T>
-__device__ __forceinline__ T ppm_face(T wa, T wb, T da, T db)
+// PPM face value between cells a (lo) and b (hi) with half slopes ga, gb: (wb + wa) / 2 + (da - db) / 6
+// (ppm_incr's fl / fh); doubling the constant and halving in the fma are exact
+__device__ __forceinline__ double ppm_face(double wa, double wb, double ga, double gb)
 {
-    const T sixth = (T)(1.0 / 6.0);
-    return (T)0.5 * (wb + wa) + sixth * (da - db);
+    const double third = 2.0 * (1.0 / 6.0);
+    return fma(0.5, wb + wa, third * (ga - gb));
 }
 
 // Buffer descriptors over one state plane: the kernel addresses a plane with a 32-bit byte
@@ -168,7 +176,7 @@ struct MarchCarry {
     T wn[5];               // W of row r + 1 (requested ahead, without the ring)
     T w1[5], w2[5], w3[5]; // W of rows r, r - 1, r - 2 (the next row's r - 1, r - 2, r - 3)
     T dly[4];              // y differences W(r) - W(r - 1) of the y-sweep quantities
-    T dy2[4];              // y slopes of row r - 1
+    T dy2[4];              // half the y slopes of row r - 1
     T fy[4];               // y face values at r - 3/2
     Pred2<T> xp;           // x predictor of row r - 2, not yet transversely corrected
     T h1v[2], h1s[2];      // predictor state of the lo y face of row r - 2
@@ -193,7 +201,7 @@ template <>
 struct MarchCarry<float> {
     float w1[5], w2[5], w3[5];  // as above
     float dly[4];
-    float dy2[4];               // half the y slopes of row r - 1
+    float dy2[4];               // as above
     float fy[4];                // y increments of row r - 2: lo face value minus the cell's
     float xa[2], xb[2];         // x predictor of row r - 2: a on its lo, b on its hi face, uncorrected
     float h1d[2], h1e[2];       // predictor state of the lo y face of row r - 2
@@ -201,13 +209,6 @@ struct MarchCarry<float> {
     float cpc[2];               // the same, corrected
     float f1d[2], f1e[2];       // final state of the lo y face of row r - 2
 };
-
-// half the monotonized central slope: minmod(l, r, (l + r) / 4).  Half: one product fewer than
-// vl_limit_centred, the same value times 1/2
-__device__ __forceinline__ float half_slope(float l, float r)
-{
-    return __builtin_amdgcn_fmed3f(__builtin_amdgcn_fmed3f(l, r, 0.0f), 0.25f * (l + r), 0.0f);
-}
 
 // a uniform value in a scalar register
 __device__ __forceinline__ float uniform_f(float v) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v))); }
@@ -480,15 +481,10 @@ __device__ __forceinline__ void march_strip(const KArgs<T>& a, const Tile& tl, c
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             const T dry = w0[MQ_Y[q]] - A.w1[MQ_Y[q]];
-            if constexpr (f32) {
-                const float dy1 = half_slope(A.dly[q], dry);
-                A.fy[q] = fmaf(-0.5f, A.dly[q], (1.0f / 3.0f) * (A.dy2[q] - dy1));
-                A.dy2[q] = dy1;
-            } else {
-                const T dy1 = mc_slope(A.dly[q], dry);
-                A.fy[q] = ppm_face(A.w2[MQ_Y[q]], A.w1[MQ_Y[q]], A.dy2[q], dy1);
-                A.dy2[q] = dy1;
-            }
+            const T dy1 = half_slope(A.dly[q], dry);
+            if constexpr (f32) A.fy[q] = fmaf(-0.5f, A.dly[q], (1.0f / 3.0f) * (A.dy2[q] - dy1));
+            else A.fy[q] = ppm_face(A.w2[MQ_Y[q]], A.w1[MQ_Y[q]], A.dy2[q], dy1);
+            A.dy2[q] = dy1;
             A.dly[q] = dry;
         }
 #pragma unroll
@@ -734,7 +730,7 @@ __device__ __forceinline__ void march_strip(const KArgs<T>& a, const Tile& tl, c
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 dry[q] = w0[MQ_Y[q]] - c.w1[MQ_Y[q]];
-                dy1[q] = mc_slope(c.dly[q], dry[q]);
+                dy1[q] = half_slope(c.dly[q], dry[q]);
                 fy1[q] = ppm_face(c.w2[MQ_Y[q]], c.w1[MQ_Y[q]], c.dy2[q], dy1[q]);
             }
             // y predictor of row r - 2 (its y faces r - 5/2 and r - 3/2)
@@ -758,7 +754,7 @@ __device__ __forceinline__ void march_strip(const KArgs<T>& a, const Tile& tl, c
                     const T wr = dshift<DPP_FROM_NEXT>(wc);  // W(i + 1)
                     const T dr = wr - wc;
                     const T dl = dshift<DPP_FROM_PREV>(dr);  // W(i) - W(i - 1)
-                    const T d0 = mc_slope(dl, dr);
+                    const T d0 = half_slope(dl, dr);
                     const T fh = ppm_face(wc, wr, d0, dshift<DPP_FROM_NEXT>(d0));  // face value at i + 1/2
                     const T fl = dshift<DPP_FROM_PREV>(fh);                        // at i - 1/2
                     inc[h][0] = incr(fl, wc);

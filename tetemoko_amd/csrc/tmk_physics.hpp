@@ -58,10 +58,10 @@ struct DevParams {
     double cs, cp, G, rho, lam, K, Zp, Zs;
     double iZp, iZs, irho;  // correctly rounded reciprocals 1/Zp, 1/Zs, 1/rho
     double i2Zp, i2Zs;      // 1/(2 Zp), 1/(2 Zs): the reciprocals halved (exact)
-    double lZp, lZs, lrho;  // RN(1/Z - RN(1/Z)): the low words of the reciprocals
+    double l2Zp, l2Zs, lrho;  // the low words of 1/(2 Zp), 1/(2 Zs), 1/rho: RN(1/b - RN(1/b))
     int div2;               // Zp, Zs, rho divide exactly in two operations (div2_exact)
     // the same constants rounded to FP32 on the host, for the FP32-bulk kernels
-    float frho, flam, fG, fZp, fZs, fden, flam2G, fiZp, fiZs, firho, fi2Zp, fi2Zs, fcp, fcs;
+    float frho, flam, fG, fZp, fZs, fden, flam2G, firho, fi2Zp, fi2Zs, fcp, fcs;
     double den;    // 2G + lam   (LinElastPhysicsF.ChF:427 form)
     double lam2G;  // lam + 2G   (LinElastPhysicsF.ChF:318 form)
     double bg[22];  // the uniform background state (both sides alike)
@@ -112,14 +112,11 @@ __host__ __device__ constexpr bool regroup()
     return sizeof(T) == sizeof(float);
 }
 
-// f - w: the reference's (0 - w) + f in FP64
+// f - w: the reference's (0 - w) + f, the same value (a zero's sign aside)
 template <typename T>
 __device__ __forceinline__ T incr(T f, T w)
 {
-    if constexpr (regroup<T>())
-        return f - w;
-    else
-        return ((T)0 - w) + f;
+    return f - w;
 }
 
 template <typename T, int NS>
@@ -163,22 +160,24 @@ __device__ __forceinline__ T pick(double d, float f)
 // div2_exact tries those on the host, and constants that fail keep divr.  Two operations for six
 // (divr and its copysign): the sign of a zero dividend comes out by itself.  A cell side of the FP64
 // march divides 28 times; with the flux of a face computed once (march_strip) the 4096 x 2048 level
-// went from 522 to 461 us per step without plasticity and from 640 to 577 with it.
+// went from 522 to 461 us per step without plasticity and from 640 to 577 with it.  Halvings folded into
+// fmas and divisors, half slopes and the plastic return's early way out (div3, plastic_flow) took it on
+// from 505 to 480 with its reads (60 steps 30.3 -> 28.8 ms), 8192 x 4096 plastic from 2.42 to 2.33 ms.
 __device__ __forceinline__ double divr2(double a, double yh, double yl) { return fma(a, yh, a * yl); }
 
 // elastic constants in the bulk arithmetic type.  D2 (FP64): the constants divide by divr2.
 template <typename T, bool D2 = false>
 struct Mat {
     T rho, lam, G, Zp, Zs, den, lam2G;
-    T iZp, iZs, irho, i2Zp, i2Zs;  // reciprocals (1/(2Z) = (1/Z)/2 exactly)
-    T lZp, lZs, lrho;              // their low words (D2)
+    T irho, i2Zp, i2Zs;    // reciprocals of rho, 2 Zp, 2 Zs
+    T lrho, l2Zp, l2Zs;    // their low words (D2)
     T cp, cs;
     __device__ __forceinline__ explicit Mat(const DevParams& p)
         : rho(pick<T>(p.rho, p.frho)), lam(pick<T>(p.lam, p.flam)), G(pick<T>(p.G, p.fG)),
           Zp(pick<T>(p.Zp, p.fZp)), Zs(pick<T>(p.Zs, p.fZs)), den(pick<T>(p.den, p.fden)),
-          lam2G(pick<T>(p.lam2G, p.flam2G)), iZp(pick<T>(p.iZp, p.fiZp)), iZs(pick<T>(p.iZs, p.fiZs)),
-          irho(pick<T>(p.irho, p.firho)), i2Zp(pick<T>(p.i2Zp, p.fi2Zp)), i2Zs(pick<T>(p.i2Zs, p.fi2Zs)),
-          lZp((T)p.lZp), lZs((T)p.lZs), lrho((T)p.lrho), cp(pick<T>(p.cp, p.fcp)), cs(pick<T>(p.cs, p.fcs)) {}
+          lam2G(pick<T>(p.lam2G, p.flam2G)), irho(pick<T>(p.irho, p.firho)), i2Zp(pick<T>(p.i2Zp, p.fi2Zp)),
+          i2Zs(pick<T>(p.i2Zs, p.fi2Zs)), lrho((T)p.lrho), l2Zp((T)p.l2Zp), l2Zs((T)p.l2Zs),
+          cp(pick<T>(p.cp, p.fcp)), cs(pick<T>(p.cs, p.fcs)) {}
     // the same with every constant that the velocity sign of a side multiplies carrying that sign: side
     // 2 in y (sd = 1) then runs the expressions of side 1, and no product with the sign is left (FP64 with
     // D2, whose division takes either sign; negation is exact).  The sign goes in by integer arithmetic on uniform values: scalar registers.
@@ -190,20 +189,15 @@ struct Mat {
                 double, __builtin_bit_cast(unsigned long long, (double)v) ^ ((unsigned long long)sd << 63));
         };
         o.rho = s(rho); o.lam = s(lam); o.G = s(G); o.Zp = s(Zp); o.Zs = s(Zs); o.lam2G = s(lam2G);
-        o.iZp = s(iZp); o.iZs = s(iZs); o.irho = s(irho); o.i2Zp = s(i2Zp); o.i2Zs = s(i2Zs);
-        o.lZp = s(lZp); o.lZs = s(lZs); o.lrho = s(lrho);
+        o.irho = s(irho); o.i2Zp = s(i2Zp); o.i2Zs = s(i2Zs);
+        o.lrho = s(lrho); o.l2Zp = s(l2Zp); o.l2Zs = s(l2Zs);
         return o;
     }
     __device__ __forceinline__ T Z(int k) const { return k == 0 ? Zp : Zs; }
-    // x / Z(k), x / (2 Z(k)), x / rho, rounded like the division
-    __device__ __forceinline__ T divZ(T x, int k) const
-    {
-        if constexpr (D2) return k == 0 ? divr2(x, iZp, lZp) : divr2(x, iZs, lZs);
-        else return k == 0 ? divr(x, Zp, iZp) : divr(x, Zs, iZs);
-    }
+    // x / (2 Z(k)), x / rho, rounded like the division
     __device__ __forceinline__ T div2Z(T x, int k) const
     {
-        if constexpr (D2) return k == 0 ? divr2(x, i2Zp, (T)0.5 * lZp) : divr2(x, i2Zs, (T)0.5 * lZs);
+        if constexpr (D2) return k == 0 ? divr2(x, i2Zp, l2Zp) : divr2(x, i2Zs, l2Zs);
         else return k == 0 ? divr(x, (T)2 * Zp, i2Zp) : divr(x, (T)2 * Zs, i2Zs);
     }
     __device__ __forceinline__ T divrho(T x) const
@@ -369,24 +363,23 @@ __device__ __forceinline__ void ppm_slot(const Mat<T, D2>& m, int k, T rvs, T dt
         ppm_limit(cm_m, cm_p);
         ppm_limit(cp_m, cp_p);
     }
-    // PPM tracing: left-moving waves (lambda<0) on the lo face, right-moving on the hi face
+    // PPM tracing: left-moving waves (lambda<0) on the lo face, right-moving on the hi face.  Halving is
+    // exact, so a half before a sum goes into its fma and one before a division into the divisor
     const T sig = (k == 0 ? m.cp : m.cs) * dtbydx;
     {
         const T mm = cm_m, pp = cm_p;
-        cm_m = mm + sig * ((pp - mm) - (pp + mm) * ((T)3 - (T)2 * sig)) / (T)2;
+        cm_m = fma((T)0.5, sig * ((pp - mm) - (pp + mm) * ((T)3 - (T)2 * sig)), mm);
     }
     {
         const T mm = cp_m, pp = cp_p;
-        cp_p = pp + sig * ((mm - pp) - (pp + mm) * ((T)3 - (T)2 * sig)) / (T)2;
+        cp_p = fma((T)0.5, sig * ((mm - pp) - (pp + mm) * ((T)3 - (T)2 * sig)), pp);
     }
-    const T vmi = m.divZ(rvs * (cm_m - cp_m) / (T)2, k);
-    const T vpi = m.divZ(rvs * (cm_p - cp_p) / (T)2, k);
-    const T smi = (cm_m + cp_m) / (T)2;
-    const T spi = (cm_p + cp_p) / (T)2;
+    const T vmi = m.div2Z(rvs * (cm_m - cp_m), k);
+    const T vpi = m.div2Z(rvs * (cm_p - cp_p), k);
     Wmv = vmi + wv;
     Wpv = vpi + wv;
-    Wms = smi + ws;
-    Wps = spi + ws;
+    Wms = fma((T)0.5, cm_m + cp_m, ws);
+    Wps = fma((T)0.5, cm_p + cp_p, ws);
 }
 
 // ---------------------------------------------------------------------------
@@ -420,8 +413,8 @@ __device__ __forceinline__ void normal_pred_side(const DevParams& P, const Mat<T
     const bool charl = PK >= 0 ? false : P.char_lim != 0;
     // CHARSYNTHESISF (LinElastPhysicsF.ChF:526-550), then W+- = increment + W
     auto synth = [&](int k, T cm_m, T cp_m, T cm_p, T cp_p) {
-        const T vmi = m.divZ(rvs * (cm_m - cp_m) / (T)2, k);
-        const T vpi = m.divZ(rvs * (cm_p - cp_p) / (T)2, k);
+        const T vmi = m.div2Z(rvs * (cm_m - cp_m), k);
+        const T vpi = m.div2Z(rvs * (cm_p - cp_p), k);
         const T smi = (cm_m + cp_m) / (T)2;
         const T spi = (cm_p + cp_p) / (T)2;
         Wmv[k] = vmi + w[k][0][2];
@@ -535,7 +528,7 @@ __device__ __forceinline__ void riemann_side(const Mat<T, D2>& m, T rvs, const T
             v[k] = (wm[k] - wp[k]) * (rvs * m.i2Z(k));
             s[k] = (wm[k] + wp[k]) * (T)0.5;
         } else {
-            v[k] = m.divZ(rvs * (wm[k] - wp[k]) / (T)2, k);
+            v[k] = m.div2Z(rvs * (wm[k] - wp[k]), k);  // ((wm - wp) / 2) / Z: halving is exact
             s[k] = (wm[k] + wp[k]) / (T)2;
         }
     }
@@ -936,16 +929,26 @@ __device__ __forceinline__ double plastic_d(const DevParams& P, int k)
 }
 __device__ __forceinline__ double plastic_d(const PlasticConstL64& P, int k) { return P.c[k]; }
 
+// x / 3 and x / 6, rounded like the division (divr2: no quotient by 3 lies near a midpoint, the gap is a
+// multiple of 2^51 in its scale; tests/test_div2.py)
+__device__ __forceinline__ double div3(double x) { return divr2(x, 1.0 / 3.0, 0x1p-54 / 3.0); }
+__device__ __forceinline__ double div6(double x) { return divr2(x, 0.5 / 3.0, 0x1p-55 / 3.0); }
+
+// A cell that stays well inside the yield surface, J2 < ys^2 (1 - 2^-50), is left before the root: there
+// tau = RN(sqrt(J2)) <= ys.  A row of the 8192 x 4096 level's march took the root and two divisions by
+// constants, some 50 instructions of 700.
 template <typename T, typename PP>
 __device__ __forceinline__ void plastic_flow(const PP& P, T dt, T& sxx, T& syy, T& szz, T& sxy, T& sxz, T& syz,
                                              T& plam, T& pgam)
 {
-    T sigma = (sxx + syy + szz) / (T)3;
+    T sigma = div3(sxx + syy + szz);
     const T a = sxx - syy, b = syy - szz, c = szz - sxx;
-    const T J2 = (a * a + b * b + c * c) / (T)6 + sxy * sxy + sxz * sxz + syz * syz;
-    T tau = sqrt(J2);
+    const T J2 = div6(a * a + b * b + c * c) + sxy * sxy + sxz * sxz + syz * syz;
     const T bb = (T)plastic_d(P, PD_B) + pgam * (T)plastic_d(P, PD_H);
-    const T Y = tau - fmax(-(T)plastic_d(P, PD_MU) * sigma + bb, (T)0);
+    const T ys = fmax(-(T)plastic_d(P, PD_MU) * sigma + bb, (T)0);
+    if (J2 < ys * ys * (T)(1.0 - 0x1p-50)) { plam = (T)0; return; }
+    T tau = sqrt(J2);
+    const T Y = tau - ys;
     if (Y <= (T)0) { plam = (T)0; return; }
     const T G = (T)plastic_d(P, PD_G), K = (T)plastic_d(P, PD_K);
     plam = Y / (dt * ((T)plastic_d(P, PD_H) + G + (T)plastic_d(P, PD_MU) * (T)plastic_d(P, PD_BETA) * K) +
