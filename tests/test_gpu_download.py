@@ -63,3 +63,33 @@ def test_readers_on_several_threads():
     assert got == [True] * 6
     assert capi.lib().tmk_cache_trim() == 0
     assert _check(120, 80, capi.PREC_FP64)
+
+
+@pytest.mark.parametrize("precision", [capi.PREC_FP64, capi.PREC_FP32_BULK])
+@pytest.mark.parametrize("valid,flux", [((0, 0, 0, 0), True), ((5, 0, 37, 20), True), ((40, 17, 71, 50), False),
+                                        ((3, 1, 95, 61), True)])
+def test_drop_in_call_through_a_stage_and_by_copies(valid, flux, precision):
+    """tmk_patch_update_state moves its data through a pinned stage; the allocation-free call copies when
+    no stage is idle (tmk_cache_trim).  The same kernels on the same data: bit-identical, ghosts and
+    untouched planes included."""
+    g = scenarios.GHOST
+    cfg = scenarios.config_c1(seed=9, nx=110, ny=70, dx=25.0)
+    U, B = scenarios.level_arrays(cfg)
+    scenarios.perturb(U, seed=4, amp_v=1.0, amp_s=5.0)
+    x0, y0, x1, y1 = valid
+    ub, bb = (x0 - g, y0 - g, x1 + g, y1 + g), (x0 - g, 0, x1 + g, 0)
+    fault = y0 == 0
+    ctx = capi.Context(cfg, precision)
+    got = []
+    for copies in (False, True):
+        Ub = np.ascontiguousarray(U[:, y0:y1 + 2 * g + 1, x0:x1 + 2 * g + 1])
+        Bb = np.ascontiguousarray(B[:, x0:x1 + 2 * g + 1]) if fault else None
+        F = [np.full((22, y1 - y0 + 1, x1 - x0 + 2), np.nan), np.full((22, y1 - y0 + 2, x1 - x0 + 1), np.nan)]
+        if copies:
+            assert capi.lib().tmk_cache_trim() == 0
+        ctx.update_state(valid, Ub, ub, Bb, bb if fault else None, *(F if flux else (None, None)), time=0.3,
+                         dt=scenarios.dt_of(cfg), noalloc=copies)
+        got.append([Ub, Bb] + (F if flux else []))
+    ctx.close()
+    for a, b in zip(*got):
+        assert a is None and b is None or np.array_equal(a, b) and not np.isnan(a).any()

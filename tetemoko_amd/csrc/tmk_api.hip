@@ -13,6 +13,7 @@
 #include <cstdio>
 #include <cstring>
 #include <functional>
+#include <initializer_list>
 #include <map>
 #include <mutex>
 #include <new>
@@ -248,8 +249,9 @@ static void stage_free(HostStage* S)
     delete S;
 }
 
-// a stage of the current device (NULL: none to be had; the caller copies without)
-static HostStage* stage_take()
+// a stage of the current device (NULL: none to be had, the caller copies without; may_pin: one may be
+// made)
+static HostStage* stage_take(bool may_pin = true)
 {
     int dev = 0;
     hipError_t (*pin)(void**, size_t, unsigned) = hipHostMalloc;
@@ -264,6 +266,7 @@ static HostStage* stage_take()
                 return S;
             }
     }
+    if (!may_pin) return nullptr;
     HostStage* S = new (std::nothrow) HostStage;
     if (!S) return nullptr;
     S->dev = dev;
@@ -916,6 +919,7 @@ extern "C" int tmk_ctx_create(tmk_ctx** out, const tmk_params* p, int precision)
     // the allocation-free drop-in's scratch on this device; on failure only that entry point
     // is unavailable (it returns TMK_E_HIP)
     if (scratch_device_ptr(&c->noalloc_scratch) != TMK_OK) c->noalloc_scratch = nullptr;
+    stage_give(stage_take());  // one idle stage for the calls that may not allocate
     const double* fa[8] = {p->f_a, p->f_b, p->f_L, p->f_fs, p->f_fd, p->f_dc, p->f_syy, p->f_tau};
     const double** fd[8] = {&c->P.f_a, &c->P.f_b, &c->P.f_L, &c->P.f_fs, &c->P.f_fd, &c->P.f_dc, &c->P.f_syy,
                             &c->P.f_tau};
@@ -1544,11 +1548,81 @@ static PatchSizes patch_sizes(const tmk_box& valid, const tmk_box& ub, const dou
     return z;
 }
 
+// the level's stored form of a host value and back (FP32 bulk stores U - bg)
+template <typename T>
+__device__ __forceinline__ T to_stored(double v, double bg)
+{
+    if constexpr (stores_delta<T>()) return (T)(v - bg);
+    else return v;
+}
+template <typename T>
+__device__ __forceinline__ double from_stored(T v, double bg)
+{
+    if constexpr (stores_delta<T>()) return (double)v + bg;
+    else return v;
+}
+
+// A drop-in call's data between host and device in one launch each way, through a pinned stage.  In: the
+// state in the bulk's stored form into both copies (uin NULL: only uout), the fault data into both of
+// its copies, the launch tables.
+template <typename T>
+static __global__ void k_patch_in(const double* hu, T* uin, T* uout, size_t nu, size_t plane, StateVec bg, const double* hb,
+                                  double* b0, size_t nb, const unsigned* hm, unsigned* meta, size_t words)
+{
+    size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t < nu) {
+        const T v = to_stored<T>(hu[t], bg.c[t / plane]);
+        if (uin) uin[t] = v;
+        uout[t] = v;
+        return;
+    }
+    t -= nu;
+    if (t < nb) {
+        b0[t] = hb[t];
+        b0[nb + t] = hb[t];
+        return;
+    }
+    t -= nb;
+    if (t < words) meta[t] = hm[t];
+}
+
+// Out: of the state the box vx x vy at (x0, y0) of the planes listed (what the call can have changed;
+// FP32: all of it, its ghosts rounded as ever), the written fault data, the fluxes and the error word.
+struct PlaneList {
+    int n;
+    unsigned char c[TMK_NCOMP];
+};
+template <typename T>
+static __global__ void k_patch_out(const T* u, size_t plane, int unx, int x0, int y0, int vx, int vy, PlaneList pl,
+                                   StateVec bg, double* hu, const double* b, double* hb, size_t nb, const double* f,
+                                   double* hf, size_t nf, const int* err, int* herr)
+{
+    size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const size_t cells = (size_t)vx * vy, nu = cells * pl.n;
+    if (t == 0 && err) *herr = *err;
+    if (t < nu) {
+        const int q = (int)(t / cells);
+        const unsigned k = (unsigned)(t - (size_t)q * cells);
+        const unsigned y = k / (unsigned)vx, x = k - y * (unsigned)vx;
+        const int c = pl.c[q];
+        hu[t] = from_stored<T>(u[(size_t)(x + x0) + (size_t)(y + y0) * unx + c * plane], bg.c[c]);
+        return;
+    }
+    t -= nu;
+    if (t < nb) {
+        hb[t] = b[t];
+        return;
+    }
+    t -= nb;
+    if (t < nf) hf[t] = f[t];
+}
+
 // One drop-in call on the buffers of w.  tiles: the box's tiles (patch_tiles), nint interior.
+// S: a stage that holds the call's data either way (patch_staged), or NULL: copies.
 template <typename T>
 static int patch_update_t(tmk_ctx* c, tmk_box valid, double* U, tmk_box ub, double* F0, double* F1, double* B,
                           tmk_box bb, int nb, double time, double dt, bool plastic_only, const PatchWork<T>& w,
-                          const Tile* tiles, int ntiles, int nint)
+                          const Tile* tiles, int ntiles, int nint, HostStage* S)
 {
     const PatchSizes z = patch_sizes(valid, ub, F0, F1, B, bb, nb);
     const size_t unx = z.unx, plane = z.plane, nU = z.nU, bnx = z.bnx, nB = z.nB, nF0 = z.nF0, nF1 = z.nF1;
@@ -1560,7 +1634,52 @@ static int patch_update_t(tmk_ctx* c, tmk_box valid, double* U, tmk_box ub, doub
     double* Fd = w.Fd;
     const dim3 cvt_grid((unsigned)std::min<size_t>((plane + 255) / 256, 1024), TMK_NCOMP);
     std::vector<float> tmp;
-    if (sizeof(T) == sizeof(double)) {
+    const StateVec bg = background(c->P);
+    // the stage: state, fault data, tables on the way in; state, fault data, fluxes, error word out
+    double* const hu = S ? (double*)S->p : nullptr;
+    auto staged_in = [&](size_t mbytes) -> int {
+        memcpy(hu, U, nU * sizeof(double));
+        if (B) memcpy(hu + nU, B, nB * sizeof(double));
+        const size_t words = mbytes / sizeof(unsigned), n = nU + nB + words;
+        hipLaunchKernelGGL(k_patch_in<T>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, (const double*)hu,
+                           plastic_only ? (T*)nullptr : Uin, Uout, nU, plane, bg, (const double*)(hu + nU), Bd, nB,
+                           (const unsigned*)(hu + nU + nB), (unsigned*)w.meta, words);
+        return hipGetLastError() == hipSuccess ? TMK_OK : TMK_E_HIP;
+    };
+    // planes: those the call can have changed
+    auto staged_out = [&](std::initializer_list<int> planes, const int* err) -> int {
+        constexpr bool all = stores_delta<T>();
+        PlaneList pl;
+        pl.n = 0;
+        if (all) for (int k = 0; k < TMK_NCOMP; ++k) pl.c[pl.n++] = (unsigned char)k;
+        else
+            for (int sd = 0; sd < 2; ++sd)
+                for (int k : planes) pl.c[pl.n++] = (unsigned char)(11 * sd + k);
+        const tmk_box r = all ? ub : valid;
+        const int x0 = r.lo[0] - ub.lo[0], y0 = r.lo[1] - ub.lo[1];
+        const int vx = r.hi[0] - r.lo[0] + 1, vy = r.hi[1] - r.lo[1] + 1;
+        const size_t cells = (size_t)vx * vy, nu = cells * pl.n, nf = nF0 + nF1, n = nu + nB + nf;
+        double *const hb = hu + nu, *const hf = hb + nB;
+        int* const herr = (int*)(hf + nf);
+        hipLaunchKernelGGL(k_patch_out<T>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, (const T*)Uout, plane,
+                           (int)unx, x0, y0, vx, vy, pl, bg, hu, (const double*)(Bd + nB), hb, nB, (const double*)Fd, hf, nf,
+                           err, herr);
+        HIPCHK(hipGetLastError());
+        HIPCHK(hipStreamSynchronize(st));
+        if (err && *herr) return *herr;
+        if (B) memcpy(B, hb, nB * sizeof(double));
+        if (F0) memcpy(F0, hf, nF0 * sizeof(double));
+        if (F1) memcpy(F1, hf + nF0, nF1 * sizeof(double));
+        for (int q = 0; q < pl.n; ++q)
+            for (int y = 0; y < vy; ++y)
+                memcpy(U + pl.c[q] * plane + (size_t)(y + y0) * unx + x0, hu + q * cells + (size_t)y * vx,
+                       sizeof(double) * (size_t)vx);
+        return TMK_OK;
+    };
+    int e;
+    if (S) {
+        if (plastic_only && (e = staged_in(0))) return e;
+    } else if (sizeof(T) == sizeof(double)) {
         HIPCHK(hipMemcpyAsync(Uin, U, nU * sizeof(double), hipMemcpyHostToDevice, st));
     } else if (w.stage) {
         HIPCHK(hipMemcpyAsync(w.stage, U, nU * sizeof(double), hipMemcpyHostToDevice, st));
@@ -1572,15 +1691,16 @@ static int patch_update_t(tmk_ctx* c, tmk_box valid, double* U, tmk_box ub, doub
         to_stored_f32(U, tmp.data(), plane, c->P);
         HIPCHK(hipMemcpyAsync(Uin, tmp.data(), nU * sizeof(float), hipMemcpyHostToDevice, st));
     }
-    HIPCHK(hipMemcpyAsync(Uout, Uin, nU * sizeof(T), hipMemcpyDeviceToDevice, st));
+    if (!S) HIPCHK(hipMemcpyAsync(Uout, Uin, nU * sizeof(T), hipMemcpyDeviceToDevice, st));
     if (plastic_only) {
         const int vnx = valid.hi[0] - valid.lo[0] + 1, vny = valid.hi[1] - valid.lo[1] + 1;
         const int n = vnx * vny;
         hipLaunchKernelGGL(k_plastic<T>, dim3((n + 255) / 256), dim3(256), 0, st, c->P, Uout, ub.lo[0], ub.lo[1],
                            (int)unx, plane, valid.lo[0], valid.lo[1], vnx, vny, dt);
         HIPCHK(hipGetLastError());
+        if (S) return staged_out({3, 4, 5, 6, 7, 8, 9, 10}, nullptr);
     } else {
-        if (B) {
+        if (B && !S) {
             HIPCHK(hipMemcpyAsync(Bd, B, nB * sizeof(double), hipMemcpyHostToDevice, st));
             HIPCHK(hipMemcpyAsync(Bd + nB, Bd, nB * sizeof(double), hipMemcpyDeviceToDevice, st));
         }
@@ -1603,9 +1723,17 @@ static int patch_update_t(tmk_ctx* c, tmk_box valid, double* U, tmk_box ub, doub
         memset(&sc, 0, sizeof sc);
         sc.P = c->P;
         scen_set_clock(sc, time, dt);
-        HIPCHK(hipMemcpyAsync(meta, &pt, sizeof pt, hipMemcpyHostToDevice, st));
-        HIPCHK(hipMemcpyAsync(meta + off_t, tiles, sizeof(Tile) * ntiles, hipMemcpyHostToDevice, st));
-        HIPCHK(hipMemcpyAsync(meta + off_s, &sc, sizeof sc, hipMemcpyHostToDevice, st));
+        if (S) {
+            char* const m = (char*)(hu + nU + nB);  // the tables are laid out in the stage itself
+            memcpy(m, &pt, sizeof pt);
+            memcpy(m + off_t, tiles, sizeof(Tile) * ntiles);
+            memcpy(m + off_s, &sc, sizeof sc);
+            if ((e = staged_in(mbytes))) return e;
+        } else {
+            HIPCHK(hipMemcpyAsync(meta, &pt, sizeof pt, hipMemcpyHostToDevice, st));
+            HIPCHK(hipMemcpyAsync(meta + off_t, tiles, sizeof(Tile) * ntiles, hipMemcpyHostToDevice, st));
+            HIPCHK(hipMemcpyAsync(meta + off_s, &sc, sizeof sc, hipMemcpyHostToDevice, st));
+        }
         KArgs<T> a;
         a.scen = (Scen*)(meta + off_s);
         a.patches = (const Patch<T>*)meta;
@@ -1628,9 +1756,18 @@ static int patch_update_t(tmk_ctx* c, tmk_box valid, double* U, tmk_box ub, doub
                 }
             ns = zero ? 2 : 3;
         }
-        int e;
         if ((e = launch_update<T>(st, nullptr, nullptr, nullptr, ns, pred_kind(c->P), c->bx, c->by, a, nint, nullptr)))
             return e;
+        if (S) {
+            const int* const err = (const int*)(meta + off_s + offsetof(Scen, err));
+            e = ns == 2 ? staged_out({0, 1, 3, 4, 5, 6}, err) : staged_out({0, 1, 2, 3, 4, 5, 6, 7, 8}, err);
+            if (e) return e;
+            if (stores_delta<T>()) {
+                if (F0) add_bg_flux(c->P, 0, F0, nF0);
+                if (F1) add_bg_flux(c->P, 1, F1, nF1);
+            }
+            return TMK_OK;
+        }
         int herr = 0;
         HIPCHK(hipMemcpyAsync(&herr, meta + off_s + offsetof(Scen, err), sizeof(int), hipMemcpyDeviceToHost, st));
         HIPCHK(hipStreamSynchronize(st));
@@ -1661,6 +1798,17 @@ static int patch_update_t(tmk_ctx* c, tmk_box valid, double* U, tmk_box ub, doub
     return TMK_OK;
 }
 
+// The stage of a drop-in call whose data fits one, else NULL: a 32 x 32 call with fluxes took five copies
+// to the device, two on it and five back, each with a wait: 201 us, now 98 (93 x 61 FP32 and its plastic
+// return 462, now 363); calls beyond 8 MiB are bound by the link either way.
+template <typename T>
+static HostStage* patch_staged(const PatchSizes& z, size_t mbytes, bool may_pin)
+{
+    const size_t in = (z.nU + z.nB) * sizeof(double) + mbytes;
+    const size_t out = (z.nU + z.nB + z.nF0 + z.nF1) * sizeof(double) + 64;
+    return std::max(in, out) <= STAGE_SLOT * STAGE_SLOTS ? stage_take(may_pin) : nullptr;
+}
+
 // drop-in call on the context's grow-only buffers (allocated on first need)
 template <typename T>
 static int patch_update_bufs(tmk_ctx* c, tmk_box valid, double* U, tmk_box ub, double* F0, double* F1, double* B,
@@ -1689,8 +1837,12 @@ static int patch_update_bufs(tmk_ctx* c, tmk_box valid, double* U, tmk_box ub, d
     w.Bd = (double*)c->bufs[3].p;
     w.Fd = (double*)c->bufs[4].p;
     w.meta = (char*)c->bufs[5].p;
-    return patch_update_t<T>(c, valid, U, ub, F0, F1, B, bb, nb, time, dt, plastic_only, w, tiles.data(),
-                             (int)tiles.size(), nint);
+    HostStage* const S = patch_staged<T>(z, mbytes, true);
+    e = patch_update_t<T>(c, valid, U, ub, F0, F1, B, bb, nb, time, dt, plastic_only, w, tiles.data(), (int)tiles.size(),
+                          nint, S);
+    if (S && e) (void)hipStreamSynchronize(c->stream);  // a launch still queued may use the stage
+    stage_give(S);
+    return e;
 }
 
 // argument checks of tmk_patch_update_state (B is cleared when valid does not touch the fault)
@@ -1804,7 +1956,11 @@ static int patch_update_noalloc_t(tmk_ctx* c, tmk_box valid, double* U, tmk_box 
     w.Fd = (double*)(base + oF);
     w.stage = sizeof(T) == sizeof(double) ? nullptr : (double*)(base + oS);
     w.meta = base + oM;
-    return patch_update_t<T>(c, valid, U, ub, F0, F1, B, bb, nb, time, dt, false, w, tiles, ntiles, nint);
+    HostStage* const S = patch_staged<T>(z, mbytes, false);  // pinning allocates
+    const int e = patch_update_t<T>(c, valid, U, ub, F0, F1, B, bb, nb, time, dt, false, w, tiles, ntiles, nint, S);
+    if (S && e) (void)hipStreamSynchronize(c->stream);
+    stage_give(S);
+    return e;
 }
 
 extern "C" int tmk_patch_update_state_noalloc(tmk_ctx* c, tmk_box valid, double* U, tmk_box ub, int ncomp,
@@ -2155,20 +2311,6 @@ extern "C" int tmk_level_destroy(tmk_level* L)
     level_free_arrays(L);
     delete L;
     return TMK_OK;
-}
-
-// the level's stored form of a host value and back (FP32 bulk stores U - bg)
-template <typename T>
-__device__ __forceinline__ T to_stored(double v, double bg)
-{
-    if constexpr (stores_delta<T>()) return (T)(v - bg);
-    else return v;
-}
-template <typename T>
-__device__ __forceinline__ double from_stored(T v, double bg)
-{
-    if constexpr (stores_delta<T>()) return (double)v + bg;
-    else return v;
 }
 
 // a box's ghosted region <-> staging array (22 FP64 planes of the ghosted box, x fastest); put
