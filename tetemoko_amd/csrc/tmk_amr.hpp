@@ -135,12 +135,15 @@ __device__ __forceinline__ void amr_fill_state(const CfFill<T>& F, long long t)
     }
     T v[9];
     if (cc.flags & 32) {
-        // one plane pointer for the nine cells (a weight of 0 reads the second state too: a NaN or an
-        // infinity there reaches the ghost cell as in the general form)
+        // one plane pointer for the nine cells, and no second state where the weight is 0
         const __attribute__((address_space(1))) T* po = gmem(F.cold[cc.cpatch[4]].in[c]);
-        const __attribute__((address_space(1))) T* pn = gmem(F.cnew[cc.cpatch[4]].in[c]);
 #pragma unroll
-        for (int k = 0; k < 9; ++k) v[k] = time_interp<T>(po[cc.coff[k]], pn[cc.coff[k]], alpha);
+        for (int k = 0; k < 9; ++k) v[k] = po[cc.coff[k]];
+        if (alpha != 0.0) {
+            const __attribute__((address_space(1))) T* pn = gmem(F.cnew[cc.cpatch[4]].in[c]);
+#pragma unroll
+            for (int k = 0; k < 9; ++k) v[k] = time_interp<T>(v[k], pn[cc.coff[k]], alpha);
+        }
     } else {
 #pragma unroll
         for (int k = 0; k < 9; ++k) {
