@@ -563,6 +563,7 @@ struct Group {
     Tile* tiles_dev = nullptr;     // interior tiles first, then the boundary tiles
     int ntiles = 0;
     int nint = 0;                  // interior tiles (k_godunov_interior); the rest run k_godunov
+    int patch0 = -1;               // the patch of every tile (-1: they differ)
     long long cells_int = 0, cells_bnd = 0;
     hipStream_t side = nullptr;    // boundary tiles run here, concurrently with the interior launch
     hipEvent_t ev_fork = nullptr, ev_join = nullptr;
@@ -1160,6 +1161,7 @@ static int group_enqueue_step_t(Group& G, hipStream_t st, const StepTimers* tm =
     a.par = G.g;
     a.nint = G.nint;
     a.nscen = G.nscen;
+    a.patch0 = G.patch0;
     int e = G.march > 0 ? launch_step<T>(st, a, G.any_plast, G.div2, tm)
                         : launch_update<T>(st, G.side, G.ev_fork, G.ev_join, G.ns, G.pk, G.bx, G.by, a, G.nint, tm);
     if (e) return e;
@@ -1327,6 +1329,11 @@ static int group_build_t(Group& G, const std::vector<tmk_level*>& mem, const std
         G.nint = partition_tiles(
             tiles, [&](const Tile& t) { return tile_interior_host(t, sc[patch_scen[t.patch]].P, bx, by); },
             [&](const Tile& t) -> const DevParams& { return sc[patch_scen[t.patch]].P; }, G.xcd != 0);
+    }
+    G.patch0 = tiles.empty() ? -1 : tiles[0].patch;
+    for (Tile& t : tiles) {
+        t.scen = patch_scen[t.patch];
+        if (t.patch != G.patch0) G.patch0 = -1;
     }
     G.cells_int = G.cells_bnd = 0;
     for (size_t k = 0; k < tiles.size(); ++k)
@@ -1743,6 +1750,7 @@ static int patch_update_t(tmk_ctx* c, tmk_box valid, double* U, tmk_box ub, doub
         a.par = 0;
         a.nint = nint;
         a.nscen = 1;
+        a.patch0 = 0;
         // the anti-plane planes are skipped only when background and data are zero there
         int ns = 3;
         if (!c->antiplane) {

@@ -101,6 +101,7 @@ struct Tile {
     int patch;
     int x0, y0, x1, y1;  // valid cells of this tile (inclusive)
     int flux;            // marching strips of a hierarchy level: 0 when no face of the strip carries a register flux
+    int scen;            // marching steps: the patch's scenario (Patch::scen), one load earlier than the patch gives it
 };
 
 template <typename T>
@@ -113,6 +114,7 @@ struct KArgs {
     int par;       // clock parity of this launch (Scen::time)
     int nint;      // k_godunov_step: tiles [0, nint) are interior strips, the rest boundary pieces
     int nscen;     // k_godunov_step: the scenarios whose clocks it advances
+    int patch0;    // k_godunov_step: the patch of every tile, -1: they differ
 };
 
 __device__ __forceinline__ void report(int* err, int code)

@@ -43,8 +43,8 @@ constexpr int MARCH_ROW_STORES = 8;   // stores per row: 5 stencil planes, szz, 
 // a strip whose stencil lies in the domain (the same rule as tile_interior)
 __device__ __forceinline__ bool march_interior(const Tile& t, const DevParams& P)
 {
-    return t.x1 - t.x0 + 1 <= MARCH_COLS && t.x0 - 3 >= P.dlo[0] && t.x1 + 3 <= P.dhi[0] && t.y0 - 3 >= P.dlo[1] &&
-           t.y1 + 3 <= P.dhi[1];
+    return (t.x1 - t.x0 + 1 <= MARCH_COLS) & (t.x0 - 3 >= P.dlo[0]) & (t.x1 + 3 <= P.dhi[0]) & (t.y0 - 3 >= P.dlo[1]) &
+           (t.y1 + 3 <= P.dhi[1]);
 }
 
 // half the monotonized central slope of a cell from its two one-sided differences: min(|l|, |r|,
@@ -325,15 +325,13 @@ __global__ void __launch_bounds__(64) k_strip_flux(Tile* tiles, const Patch<T>* 
 // PL: the launch may hold scenarios with plasticity.  Without (PL false), a row neither reads gam
 // nor writes lam and gam, and a scenario with plasticity is an error.
 template <typename T, int PK, bool PL, bool D2>
-__device__ __forceinline__ void march_strip(const KArgs<T>& a, const Tile& tl, const int sd, const int lane,
-                                            float* const ring)
+__device__ __forceinline__ void march_strip(const KArgs<T>& a, const Tile& tl, const Patch<T>& pt, const Scen& S, int* const errp,
+                                            const int sd, const int lane, float* const ring)
 {
     static_assert(PK == PK_PPM_PRIM, "row marching carries PPM with primitive limiting");
-    const Patch<T>& pt = a.patches[tl.patch];
-    Scen& S = a.scen[pt.scen];
     const DevParams& P = S.P;
     if (!march_interior(tl, P)) {
-        if (lane == 0 && sd == 0) report(&S.err, TMK_E_BOX);
+        if (lane == 0 && sd == 0) report(errp, TMK_E_BOX);
         return;
     }
     const Mat<T, D2> m(P);
@@ -353,7 +351,7 @@ __device__ __forceinline__ void march_strip(const KArgs<T>& a, const Tile& tl, c
     const T rvy = sgn ? (T)1 : sd ? rv1 : (T)1;
     const T scx = sd ? rv1 * scale : scale;
     if (!PL && P.plast && a.plastic) {
-        if (lane == 0 && sd == 0) report(&S.err, TMK_E_ARG);
+        if (lane == 0 && sd == 0) report(errp, TMK_E_ARG);
         return;
     }
     const bool plastic = PL && P.plast && a.plastic;
@@ -423,7 +421,7 @@ __device__ __forceinline__ void march_strip(const KArgs<T>& a, const Tile& tl, c
     __attribute__((address_space(1))) double* const Fo0 = uniform_ptr(pt.F[0]);
     __attribute__((address_space(1))) double* const Fo1 = uniform_ptr(pt.F[1]);
     if ((flux0 || flux1) && y1 - y0 + 1 > 63) {  // the masks hold 64 rows of faces
-        if (lane == 0 && sd == 0) report(&S.err, TMK_E_BOX);
+        if (lane == 0 && sd == 0) report(errp, TMK_E_BOX);
         return;
     }
     if (flux0 || flux1) {
