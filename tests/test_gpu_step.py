@@ -111,3 +111,43 @@ def test_fp32_march_no_further_off_than_the_tiles(nx, ny, plastic):
         scale = np.maximum(np.abs(Ur).reshape(22, -1).max(axis=1), 1e-300)
         errs.append(np.abs(Ug - Ur).reshape(22, -1).max(axis=1) / scale)
     assert np.all(errs[0] <= 2.0 * errs[1] + NSTEPS * 2.0 ** -24), errs
+
+
+@pytest.mark.parametrize("fault", ["sw", "rs"])
+@pytest.mark.parametrize("ghosts", [3, 4])
+@pytest.mark.parametrize("valid", [(0, 0, 31, 31), (40, 0, 40, 0), (17, 0, 80, 70), (5, 3, 62, 20), (90, 60, 129, 79),
+                                   (60, 1, 63, 79), (3, 3, 126, 76)])
+def test_drop_in_call_marches_as_the_tiles(valid, ghosts, fault):
+    """An FP64 drop-in call takes the marching step; set_march(0) keeps it on the tile kernels.  State,
+    fluxes and slip-weakening fault data are the same bit for bit; boxes on edges and corners, of one
+    cell, of more than 63 rows, inside; arrays of 4 ghosts and of the least a call accepts (3, cut off
+    at the domain)."""
+    nx, ny = 130, 80
+    cfg = (scenarios.config_c0 if fault == "sw" else scenarios.config_c1)(seed=6, nx=nx, ny=ny, dx=50.0)
+    U, B = scenarios.level_arrays(cfg)
+    scenarios.perturb(U, seed=8, amp_v=1.0, amp_s=5.0)
+    x0, y0, x1, y1 = valid
+    ub = (x0 - ghosts, y0 - ghosts, x1 + ghosts, y1 + ghosts)
+    if ghosts == 3:
+        ub = (max(ub[0], 0), max(ub[1], 0), min(ub[2], nx - 1), min(ub[3], ny - 1))
+    g = 1 if ghosts == 3 else G
+    bb = (x0 - g, 0, x1 + g, 0)
+    got = []
+    for march in (None, 0):
+        ctx = capi.Context(cfg, capi.PREC_FP64)
+        if march is not None:
+            ctx.set_march(march)
+        Ub = np.ascontiguousarray(U[:, ub[1] + G:ub[3] + G + 1, ub[0] + G:ub[2] + G + 1])
+        Bb = np.ascontiguousarray(B[:, bb[0] + G:bb[2] + G + 1]) if y0 == 0 else None
+        F = [np.full((22, y1 - y0 + 1, x1 - x0 + 2), np.nan), np.full((22, y1 - y0 + 2, x1 - x0 + 1), np.nan)]
+        ctx.update_state(valid, Ub, ub, Bb, bb if y0 == 0 else None, F[0], F[1], time=0.2, dt=scenarios.dt_of(cfg))
+        ctx.close()
+        got.append([Ub, Bb] + F)
+    for k, (a, b) in enumerate(zip(*got)):
+        if a is None:
+            assert b is None
+        elif fault == "sw" or y0 > 0:
+            assert np.array_equal(a, b) and not np.isnan(a).any(), k
+        else:  # the two builds of the rate-and-state solve: 1e-13 of the largest value, as against the oracle
+            top = np.maximum(np.abs(b).reshape(b.shape[0], -1).max(axis=1), 1e-300)
+            assert np.all(np.abs(a - b).reshape(b.shape[0], -1).max(axis=1) <= 1e-13 * top), k

@@ -1624,12 +1624,51 @@ static __global__ void k_patch_out(const T* u, size_t plane, int unx, int x0, in
     if (t < nf) hf[t] = f[t];
 }
 
-// One drop-in call on the buffers of w.  tiles: the box's tiles (patch_tiles), nint interior.
+// the components a drop-in call carries: the anti-plane planes are skipped only when background and data
+// are zero there
+static int patch_ns(const tmk_ctx* c, const double* U, size_t plane)
+{
+    if (c->antiplane) return 3;
+    for (int s = 0; s < 2; ++s)
+        for (int cc : {2, 7, 8}) {
+            const double* q = U + (size_t)(11 * s + cc) * plane;
+            for (size_t k = 0; k < plane; ++k)
+                if (q[k] != 0.0) return 3;
+        }
+    return 2;
+}
+
+// An FP64 drop-in call marches by the rule a level marches by, in one launch: 32 x 32 with fluxes 98 -> 76
+// us.  FP32 calls keep the tile kernels: a flux between a strip and a boundary piece is stored by both, and
+// in FP32 the two round differently.  Its strips (nint of them, at most 63 rows, as on every level that
+// stores fluxes), then its boundary pieces.
+static bool patch_marches(const tmk_ctx* c, int ns)
+{
+    return c->precision == TMK_PREC_FP64 && c->march > 0 && ns == 2 && pred_kind(c->P) == PK_PPM_PRIM;
+}
+static std::vector<Tile> patch_strips(const tmk_ctx* c, const tmk_box& v, int* nint)
+{
+    Tile r;
+    memset(&r, 0, sizeof r);
+    r.x0 = v.lo[0]; r.y0 = v.lo[1]; r.x1 = v.hi[0]; r.y1 = v.hi[1];
+    auto params = [&](const Tile&) -> const DevParams& { return c->P; };
+    const int rows = c->march_auto ? march_height({r}, params, false, false) : c->march;
+    std::vector<Tile> strips, bf, bo;
+    march_rect(r, c->P, std::min(rows, 63), strips, bf, bo);
+    *nint = (int)strips.size();
+    strips.insert(strips.end(), bf.begin(), bf.end());
+    strips.insert(strips.end(), bo.begin(), bo.end());
+    for (Tile& t : strips) t.scen = 0;
+    return strips;
+}
+
+// One drop-in call on the buffers of w.  tiles: the box's tiles (patch_tiles; march: patch_strips), nint
+// interior.
 // S: a stage that holds the call's data either way (patch_staged), or NULL: copies.
 template <typename T>
 static int patch_update_t(tmk_ctx* c, tmk_box valid, double* U, tmk_box ub, double* F0, double* F1, double* B,
                           tmk_box bb, int nb, double time, double dt, bool plastic_only, const PatchWork<T>& w,
-                          const Tile* tiles, int ntiles, int nint, HostStage* S)
+                          const Tile* tiles, int ntiles, int nint, int ns, bool march, HostStage* S)
 {
     const PatchSizes z = patch_sizes(valid, ub, F0, F1, B, bb, nb);
     const size_t unx = z.unx, plane = z.plane, nU = z.nU, bnx = z.bnx, nB = z.nB, nF0 = z.nF0, nF1 = z.nF1;
@@ -1751,21 +1790,9 @@ static int patch_update_t(tmk_ctx* c, tmk_box valid, double* U, tmk_box ub, doub
         a.nint = nint;
         a.nscen = 1;
         a.patch0 = 0;
-        // the anti-plane planes are skipped only when background and data are zero there
-        int ns = 3;
-        if (!c->antiplane) {
-            bool zero = true;
-            for (int s = 0; s < 2 && zero; ++s)
-                for (int cc : {2, 7, 8}) {
-                    const double* q = U + (size_t)(11 * s + cc) * plane;
-                    for (size_t k = 0; k < plane; ++k)
-                        if (q[k] != 0.0) { zero = false; break; }
-                    if (!zero) break;
-                }
-            ns = zero ? 2 : 3;
-        }
-        if ((e = launch_update<T>(st, nullptr, nullptr, nullptr, ns, pred_kind(c->P), c->bx, c->by, a, nint, nullptr)))
-            return e;
+        e = march ? launch_step<T>(st, a, false, c->P.div2, nullptr)
+                  : launch_update<T>(st, nullptr, nullptr, nullptr, ns, pred_kind(c->P), c->bx, c->by, a, nint, nullptr);
+        if (e) return e;
         if (S) {
             const int* const err = (const int*)(meta + off_s + offsetof(Scen, err));
             e = ns == 2 ? staged_out({0, 1, 3, 4, 5, 6}, err) : staged_out({0, 1, 2, 3, 4, 5, 6, 7, 8}, err);
@@ -1826,7 +1853,11 @@ static int patch_update_bufs(tmk_ctx* c, tmk_box valid, double* U, tmk_box ub, d
     if (z.plane * sizeof(T) > kPlaneMaxBytes) return TMK_E_NOMEM;
     int nint = 0;
     std::vector<Tile> tiles;
-    if (!plastic_only) {
+    const int ns = plastic_only ? 3 : patch_ns(c, U, z.plane);
+    const bool march = !plastic_only && patch_marches(c, ns);
+    if (march) {
+        tiles = patch_strips(c, valid, &nint);
+    } else if (!plastic_only) {
         const int n = patch_tiles(valid, c->P, c->bx, c->by, nullptr, 0, &nint);
         tiles.resize(n);
         patch_tiles(valid, c->P, c->bx, c->by, tiles.data(), n, &nint);
@@ -1847,7 +1878,7 @@ static int patch_update_bufs(tmk_ctx* c, tmk_box valid, double* U, tmk_box ub, d
     w.meta = (char*)c->bufs[5].p;
     HostStage* const S = patch_staged<T>(z, mbytes, true);
     e = patch_update_t<T>(c, valid, U, ub, F0, F1, B, bb, nb, time, dt, plastic_only, w, tiles.data(), (int)tiles.size(),
-                          nint, S);
+                          nint, ns, march, S);
     if (S && e) (void)hipStreamSynchronize(c->stream);  // a launch still queued may use the stage
     stage_give(S);
     return e;
@@ -1954,8 +1985,25 @@ static int patch_update_noalloc_t(tmk_ctx* c, tmk_box valid, double* U, tmk_box 
     const size_t oS = oF + align256((z.nF0 + z.nF1) * sizeof(double));
     const size_t oM = oS + (sizeof(T) == sizeof(double) ? 0 : align256(z.nU * sizeof(double)));
     if (oM + mbytes > (size_t)TMK_NOALLOC_SCRATCH_BYTES) return TMK_E_SCRATCH;
+    // what fits by the tile kernels' list is accepted; its strips, where their list fits too
+    const int ns = patch_ns(c, U, z.plane);
     Tile tiles[kNoAllocMaxTiles];
-    patch_tiles(valid, c->P, c->bx, c->by, tiles, kNoAllocMaxTiles, &nint);
+    const Tile* list = tiles;
+    int nlist = ntiles;
+    std::vector<Tile> strips;
+    if (patch_marches(c, ns)) {
+        strips = patch_strips(c, valid, &nint);
+        patch_meta<T>((int)strips.size(), &off_t, &off_s, &mbytes);
+        if (strips.size() > (size_t)kNoAllocMaxTiles || oM + mbytes > (size_t)TMK_NOALLOC_SCRATCH_BYTES) strips.clear();
+    }
+    const bool march = !strips.empty();
+    if (march) {
+        list = strips.data();
+        nlist = (int)strips.size();
+    } else {
+        patch_tiles(valid, c->P, c->bx, c->by, tiles, kNoAllocMaxTiles, &nint);
+        patch_meta<T>(ntiles, &off_t, &off_s, &mbytes);
+    }
     char* base = (char*)c->noalloc_scratch;
     PatchWork<T> w;
     w.Uin = (T*)base;
@@ -1965,7 +2013,7 @@ static int patch_update_noalloc_t(tmk_ctx* c, tmk_box valid, double* U, tmk_box 
     w.stage = sizeof(T) == sizeof(double) ? nullptr : (double*)(base + oS);
     w.meta = base + oM;
     HostStage* const S = patch_staged<T>(z, mbytes, false);  // pinning allocates
-    const int e = patch_update_t<T>(c, valid, U, ub, F0, F1, B, bb, nb, time, dt, false, w, tiles, ntiles, nint, S);
+    const int e = patch_update_t<T>(c, valid, U, ub, F0, F1, B, bb, nb, time, dt, false, w, list, nlist, nint, ns, march, S);
     if (S && e) (void)hipStreamSynchronize(c->stream);
     stage_give(S);
     return e;
