@@ -488,20 +488,20 @@ void march_rect(const Tile& r, const DevParams& P, int rows, std::vector<Tile>& 
 }
 
 // Strip height of a launch over rectangles (their domains' parameters: params(r)) whose levels have
-// set none.  A wavefront marches rows + 3 rows (the two before its strip, and the first loads), and a
-// SIMD issues for its share of the wavefronts in turn, so a launch takes about ceil(wavefronts / 1024
-// SIMDs) (rows + 3) row times: short strips where the launch does not fill the chip (a 400 x 200 FP64
-// level: 32 rows 59 us per step, 4 rows 19; 1024 x 512: 65, 6 rows 49), tall ones where they repeat
-// less work (4096 x 2048: 48 rows 545 us, 16 rows 579, 6 rows 657).  FP32 moves half the bytes per
-// row and is bound by memory before issue, where tall strips cost: the halos that neighbouring strips
-// share drift out of L2 as their wavefronts drift apart.  With plasticity 8 rows stay the best up to
-// the largest level (4096 x 2048: 266 us, 16 rows 286, 32 rows 305), without it 12 to 16 (228; 8 rows
-// 239, 32 rows 239).
+// set none.  A wavefront marches rows + 3 rows (the two before its strip, and the first loads).  A SIMD
+// runs its n = ceil(wavefronts / 1024) FP64 wavefronts in pairs whose instructions interleave; a lone one
+// takes 3/4 of a pair's time.  The cost is half that and half the launch's mean work, plus a wavefront's
+// own latency.  Fitted to steps of 400 x 200 to 4096 x 2048 in 4 to 48 rows, it is within 1 % of the fastest
+// height on average and 4.5 % at most (counting n alike, lone or not: 4 % and 18 %; 1500 x 750 took 76 us in
+// strips of 48 rows, one wavefront on a SIMD, for 65 in 8).  FP32 moves half the bytes per row and is bound
+// by memory before issue, where tall strips cost: the halos that neighbouring strips share drift out of L2
+// as their wavefronts drift apart.  8 rows stay the best up to the largest level (4096 x 2048: 203 us, 12
+// rows 210, 16 rows 217; plastic 257, 272, 278), fewer where that does not fill the chip.
 template <typename P>
-int march_height(const std::vector<Tile>& rects, P params, bool fp32, bool plast)
+int march_height(const std::vector<Tile>& rects, P params, bool fp32)
 {
     static const int heights[] = {4, 6, 8, 12, 16, 24, 32, 48};
-    const int most = !fp32 ? 48 : plast ? 8 : 16;
+    const int most = fp32 ? 8 : 48;
     int best = heights[0];
     double least = 0.0;
     for (int rows : heights) {
@@ -519,8 +519,15 @@ int march_height(const std::vector<Tile>& rects, P params, bool fp32, bool plast
             tallest = std::max(tallest, std::min(h, rows));
         }
         if (strips == 0) return rows;
-        const double mean = (double)lines / (double)strips + 3.0;
-        const double cost = std::max((double)((2 * strips + 1023) / 1024) * mean, tallest + 3.0);
+        double cost;
+        if (fp32) {
+            const double mean = (double)lines / (double)strips + 3.0;
+            cost = std::max((double)((2 * strips + 1023) / 1024) * mean, tallest + 3.0);
+        } else {
+            const long long n = (2 * strips + 1023) / 1024;
+            const double whole = (double)(n / 2 * 2) + (n % 2 ? 1.5 : 0.0);
+            cost = ((double)lines / (double)strips + 5.0) * (0.5 * whole + (double)strips / 1024.0 + 0.4);
+        }
         if (least == 0.0 || cost < least) {
             least = cost;
             best = rows;
@@ -1317,7 +1324,7 @@ static int group_build_t(Group& G, const std::vector<tmk_level*>& mem, const std
         auto params = [&](const Tile& t) -> const DevParams& { return sc[patch_scen[t.patch]].P; };
         bool chosen = false;  // some member's level has a height of its own
         for (tmk_level* L : mem) chosen = chosen || !L->march_auto;
-        if (!chosen) G.march = march_height(tiles, params, sizeof(T) == sizeof(float), G.plastic && G.any_plast);
+        if (!chosen) G.march = march_height(tiles, params, sizeof(T) == sizeof(float));
         const int rows = fluxes ? std::min(G.march, 63) : G.march;
         for (const Tile& r : tiles) march_rect(r, params(r), rows, strips, bf, bo);
         if (G.xcd) xcd_order(strips, STEP_WAVES / 2);
@@ -1652,7 +1659,7 @@ static std::vector<Tile> patch_strips(const tmk_ctx* c, const tmk_box& v, int* n
     memset(&r, 0, sizeof r);
     r.x0 = v.lo[0]; r.y0 = v.lo[1]; r.x1 = v.hi[0]; r.y1 = v.hi[1];
     auto params = [&](const Tile&) -> const DevParams& { return c->P; };
-    const int rows = c->march_auto ? march_height({r}, params, false, false) : c->march;
+    const int rows = c->march_auto ? march_height({r}, params, false) : c->march;
     std::vector<Tile> strips, bf, bo;
     march_rect(r, c->P, std::min(rows, 63), strips, bf, bo);
     *nint = (int)strips.size();
