@@ -54,6 +54,15 @@ struct StateVec {
     double c[22];
 };
 
+// The FP32 march's constants (ppm_slot, transverse_side and cell_update_side folded for a, b, D, E of
+// tmk_march.hpp), each rounded once from FP64.  z is the rounded impedance the march works with, so that
+// (a - b) / (2 z) gives back a velocity exactly and only dissipation feels its rounding.
+struct MarchK32 {
+    float ta[2], tb[2];     // tracing: a = (s + ta ds_lo + tb ds_hi) + z (v + ta dv_lo + tb dv_hi)
+    float p[2], q[2];       // transverse: a += p D_k + r q E_k', b += p D_k - r q E_k'
+    float kv, kl2, kl, kg;  // update
+};
+
 // one scenario's parameters, clock and error word; device resident so that
 // boxes of several scenarios can share one launch
 struct Scen {
@@ -66,6 +75,7 @@ struct Scen {
     // dt/dx, -(1/2) dt/dx (transverse correction), -dt/dx (flux difference), and in FP32
     double dtdx, hdtdx, mdtdx;
     float fdtdx, fhdtdx, fmdtdx;
+    MarchK32 m32;
     int err;      // first error reported by any launch (0 = none)
     int pad;
 };
@@ -81,6 +91,19 @@ __host__ inline void scen_set_clock(Scen& s, double time, double dt)
     s.fdtdx = (float)s.dtdx;
     s.fhdtdx = (float)s.hdtdx;
     s.fmdtdx = (float)s.mdtdx;
+    const double z[2] = {(double)s.P.fZp, (double)s.P.fZs}, c[2] = {s.P.cp, s.P.cs}, m[2] = {s.P.lam, s.P.G};
+    MarchK32& K = s.m32;
+    for (int k = 0; k < 2; ++k) {
+        const double sig = c[k] * s.dtdx, c1 = 0.5 * sig, c2 = c1 * (3.0 - 2.0 * sig);
+        K.ta[k] = (float)(1.0 - c1 - c2);
+        K.tb[k] = (float)(c1 - c2);
+        K.p[k] = (float)(-s.hdtdx * m[k] / (2.0 * z[k]));
+        K.q[k] = (float)(-0.5 * s.hdtdx / s.P.rho * z[k]);
+    }
+    K.kv = (float)(-0.5 * s.mdtdx / s.P.rho);
+    K.kl2 = (float)(-s.mdtdx * s.P.lam2G / (2.0 * z[0]));
+    K.kl = (float)(-s.mdtdx * s.P.lam / (2.0 * z[0]));
+    K.kg = (float)(-s.mdtdx * s.P.G / (2.0 * z[1]));
 }
 
 // step constants in the bulk arithmetic type

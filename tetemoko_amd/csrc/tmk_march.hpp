@@ -213,36 +213,22 @@ struct MarchCarry<float> {
 // a uniform value in a scalar register
 __device__ __forceinline__ float uniform_f(float v) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v))); }
 
-// The FP32 march's constants (ppm_slot, transverse_side and cell_update_side folded for a, b, D, E); h
-// = 1 / (2 Z), r the velocity sign in y.  The signs of the two sweeps leave one set p, q for both
-// transverse corrections, and the flux differences of D need none (r^2 = 1).
-struct MarchConst32 {
-    float ta[2], tb[2];         // tracing: a = (s + ta ds_lo + tb ds_hi) + z (v + ta dv_lo + tb dv_hi)
-    float z[2], zy[2];          // Z, r Z
-    float p[2], q[2];           // transverse: a += p D_k + q E_k', b += p D_k - q E_k'
-    float kv, kl2, kl, kg, ry;  // update
+// MarchK32 with the impedances, and the velocity sign r in y where it does not drop out: the signs of the
+// two sweeps leave one set p, q for both transverse corrections, and the flux differences of D need none
+// (r^2 = 1)
+struct MarchConst32 : MarchK32 {
+    float z[2], zy[2], ry;  // Z, r Z, r
     template <typename M>
-    __device__ __forceinline__ MarchConst32(const M& m, float dtbydx, float scale, float sc, float r)
+    __device__ __forceinline__ MarchConst32(const M& m, const MarchK32& K, float r) : MarchK32(K), ry(r)
     {
 #pragma unroll
         for (int k = 0; k < 2; ++k) {
-            const float sig = (k == 0 ? m.cp : m.cs) * dtbydx;
-            const float c1 = 0.5f * sig, c2 = c1 * (3.0f - 2.0f * sig);
-            ta[k] = uniform_f((1.0f - c1) - c2);
-            tb[k] = uniform_f(c1 - c2);
             z[k] = m.Z(k);
             zy[k] = uniform_f(r * m.Z(k));
-            p[k] = uniform_f(-(scale * (k == 0 ? m.lam : m.G)) * m.i2Z(k));
-            q[k] = uniform_f(-(0.5f * scale * m.irho) * (r * m.Z(k)));
+            q[k] = uniform_f(r * K.q[k]);
         }
-        kv = uniform_f(-(0.5f * sc * m.irho));
-        kl2 = uniform_f(-(sc * m.lam2G) * m.i2Zp);
-        kl = uniform_f(-(sc * m.lam) * m.i2Zp);
-        kg = uniform_f(-(sc * m.G) * m.i2Zs);
-        ry = r;
     }
 };
-
 struct NoMarchConst {
     template <typename... A>
     __device__ __forceinline__ explicit NoMarchConst(const A&...) {}
@@ -355,7 +341,7 @@ __device__ __forceinline__ void march_strip(const KArgs<T>& a, const Tile& tl, c
         return;
     }
     const bool plastic = PL && P.plast && a.plastic;
-    const std::conditional_t<sizeof(T) == sizeof(float), MarchConst32, NoMarchConst> C(m, dtbydx, scale, K.sc, rvy);
+    const std::conditional_t<sizeof(T) == sizeof(float), MarchConst32, NoMarchConst> C(m, S.m32, rvy);
     const int o = 11 * sd;
     // stencil planes vx vy sxx syy sxy, read with the stencil (the in copies)
     constexpr int QC[5] = {0, 1, 3, 4, 6};
