@@ -1187,7 +1187,7 @@ static int group_enqueue_step_t(Group& G, hipStream_t st, const StepTimers* tm =
         if (hipGetLastError() != hipSuccess) return TMK_E_HIP;
     }
     if (G.stations) {
-        hipLaunchKernelGGL(k_station_record<T>, dim3(1), dim3(256), 0, st, pn, G.scen_dev, G.g ^ 1, *G.stations);
+        hipLaunchKernelGGL(k_station_record<T>, dim3(1), dim3(1024), 0, st, pn, G.scen_dev, G.g ^ 1, *G.stations);
         if (hipGetLastError() != hipSuccess) return TMK_E_HIP;
     }
     G.g ^= 1;

@@ -956,13 +956,16 @@ __global__ void k_station_record(const Patch<T>* patches, const Scen* scen, int 
         if (threadIdx.x == 0) s.count[1] = 1;
         return;
     }
-    for (int k = threadIdx.x; k < s.n; k += blockDim.x) {
+    // a thread per entry: one per station took its components' loads one after another, 10 us a step
+    const int w = 1 + s.nb;
+    for (int t = threadIdx.x; t < s.n * w; t += blockDim.x) {
+        const int k = t / w, c = t - k * w - 1;
         const Patch<T>& p = patches[s.patch[k]];
         const size_t i = (size_t)(s.face[k] - p.blo0), bp = (size_t)p.bnx;
         const double d = s.d[k];
-        double* r = s.rec + ((size_t)b * s.n + k) * (size_t)(1 + s.nb);
-        r[0] = scen[p.scen].time[par];
-        for (int c = 0; c < s.nb; ++c) r[1 + c] = gmem(p.bout)[i + c * bp] * (1.0 - d) + gmem(p.bout)[i + 1 + c * bp] * d;
+        double* r = s.rec + ((size_t)b * s.n + k) * (size_t)w + 1 + c;
+        if (c < 0) *r = scen[p.scen].time[par];
+        else *r = gmem(p.bout)[i + c * bp] * (1.0 - d) + gmem(p.bout)[i + 1 + c * bp] * d;
     }
     __syncthreads();
     if (threadIdx.x == 0) s.count[0] = b + 1;
