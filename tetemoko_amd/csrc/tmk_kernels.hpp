@@ -55,8 +55,10 @@ struct StateVec {
 };
 
 // The FP32 march's constants (ppm_slot, transverse_side and cell_update_side folded for a, b, D, E of
-// tmk_march.hpp), each rounded once from FP64.  z is the rounded impedance the march works with, so that
-// (a - b) / (2 z) gives back a velocity exactly and only dissipation feels its rounding.
+// tmk_march.hpp): of the predictor rounded once from FP64, of the update those of cell_update_side to the
+// bit.  Boundary pieces and strips share faces; a flux that differs between them by a constant's rounding,
+// always the same way, is a stress between the two that acts on the fault (4000 steps: slip 4e-7 off for
+// 9e-8).
 struct MarchK32 {
     float ta[2], tb[2];     // tracing: a = (s + ta ds_lo + tb ds_hi) + z (v + ta dv_lo + tb dv_hi)
     float p[2], q[2];       // transverse: a += p D_k + r q E_k', b += p D_k - r q E_k'
@@ -100,10 +102,10 @@ __host__ inline void scen_set_clock(Scen& s, double time, double dt)
         K.p[k] = (float)(-s.hdtdx * m[k] / (2.0 * z[k]));
         K.q[k] = (float)(-0.5 * s.hdtdx / s.P.rho * z[k]);
     }
-    K.kv = (float)(-0.5 * s.mdtdx / s.P.rho);
-    K.kl2 = (float)(-s.mdtdx * s.P.lam2G / (2.0 * z[0]));
-    K.kl = (float)(-s.mdtdx * s.P.lam / (2.0 * z[0]));
-    K.kg = (float)(-s.mdtdx * s.P.G / (2.0 * z[1]));
+    K.kv = 0.5f * -(s.fmdtdx * s.P.firho);
+    K.kl2 = -(s.fmdtdx * s.P.flam2G);
+    K.kl = -(s.fmdtdx * s.P.flam);
+    K.kg = -(s.fmdtdx * s.P.fG);
 }
 
 // step constants in the bulk arithmetic type

@@ -190,7 +190,7 @@ struct MarchCarry {
 // cell below (z = Z with the side's velocity sign), and everything up to it is linear in (v, s): the
 // predictor traces a and b from the limited increments, the transverse corrections add to them, and a
 // face keeps D = a - b and E = a + b, whose scales (v = D / (2 z), s = E / 2) go into the constants of
-// what reads them.  The limited increments come straight from the differences and half slopes, not
+// what reads them; final faces keep v, as the boundary pieces do that share them (MarchK32).  The limited increments come straight from the differences and half slopes, not
 // from a face value minus the cell's.  FP32 is bound by instruction issue where the level does not
 // outgrow the caches: a row without plasticity takes about 215 vector instructions for 270 in (v, s),
 // and 4 carried values fewer.  12 single-level scenarios 26.0 -> 23.6 ms for 200 steps, 1024 x 512
@@ -207,7 +207,7 @@ struct MarchCarry<float> {
     float h1d[2], h1e[2];       // predictor state of the lo y face of row r - 2
     float cpu[2];               // b of row r - 2's uncorrected hi y face
     float cpc[2];               // the same, corrected
-    float f1d[2], f1e[2];       // final state of the lo y face of row r - 2
+    float f1d[2], f1e[2];       // final state of the lo y face of row r - 2: D / (2 Z) (r v) and E
 };
 
 // a uniform value in a scalar register
@@ -647,7 +647,7 @@ __device__ __forceinline__ void march_strip(const KArgs<T>& a, const Tile& tl, c
 #pragma unroll
                 for (int k = 0; k < 2; ++k) {
                     const float ca = fmaf(C.q[k], de[1 - k], fmaf(C.p[k], dd[k], ya[k]));
-                    n.f1d[k] = ca - c.cpc[k];
+                    n.f1d[k] = (ca - c.cpc[k]) * m.i2Z(k);
                     n.f1e[k] = ca + c.cpc[k];
                     n.cpc[k] = fmaf(-C.q[k], de[1 - k], fmaf(C.p[k], dd[k], yb[k]));
                 }
@@ -656,7 +656,7 @@ __device__ __forceinline__ void march_strip(const KArgs<T>& a, const Tile& tl, c
             auto face_state = [&](float r, const float (&d)[2], const float (&e)[2], float (&v)[2], float (&sv)[2]) {
 #pragma unroll
                 for (int k = 0; k < 2; ++k) {
-                    v[k] = d[k] * (r * m.i2Z(k));
+                    v[k] = r * d[k];
                     sv[k] = 0.5f * e[k];
                 }
             };
@@ -680,7 +680,7 @@ __device__ __forceinline__ void march_strip(const KArgs<T>& a, const Tile& tl, c
                     const float dd = n.h1d[k] - c.h1d[k], de = n.h1e[1 - k] - c.h1e[1 - k];
                     const float ca = fmaf(C.q[k], de, fmaf(C.p[k], dd, c.xa[k]));
                     const float bl = dshift<DPP_FROM_PREV>(fmaf(-C.q[k], de, fmaf(C.p[k], dd, c.xb[k])));
-                    f0d[k] = ca - bl;
+                    f0d[k] = (ca - bl) * m.i2Z(k);
                     f0e[k] = ca + bl;
                 }
                 if (flux0 && fbit(0, j3 - y0)) {
