@@ -1,0 +1,158 @@
+// Host code of libtetemoko_hip checked from the inside: this file is the library's main source with a
+// driver below it, built host only with the sanitizers and run against the host-memory stand-in of the HIP
+// runtime (hip_host_stand_in.cpp), so that tables a launch would read are plain host memory.  No kernel
+// runs.  Usage: host_library CHECK (see main).
+#include "../../tetemoko_amd/csrc/tmk_api.hip"
+
+#include <cstdlib>
+#include <set>
+#include <utility>
+
+static void fail(const char* what, int line)
+{
+    fprintf(stderr, "host_library.cpp:%d: %s\n", line, what);
+    exit(1);
+}
+#define EXPECT(x)                                   \
+    do {                                            \
+        if (!(x)) fail(#x, __LINE__);               \
+    } while (0)
+
+static tmk_params params(int nx, int ny, double dx)
+{
+    tmk_params p{};
+    const double cs = 3464.0, cp = 6000.0;
+    p.cs = cs; p.cp = cp; p.G = 2.67e-3 * cs * cs;
+    p.sxx0 = p.syy0 = p.szz0 = -120.0; p.sxy0 = 70.0;
+    p.fault_kind = TMK_FAULT_SW;
+    p.fs = 0.677; p.fd = 0.525; p.dw = 0.4; p.sw_rupture_thr = 1e-3;
+    p.num_patches = 1; p.xc[0] = nx * dx / 2; p.xw[0] = 1500.0; p.tau_p[0] = 81.6;
+    p.fric_width[0] = 1e40; p.fric_width[1] = 1e40; p.outside_f = 10.0; p.ramp_w = 1e40;
+    p.normal_pred = TMK_PRED_PPM; p.fourth_order = 1; p.prim_limiting = 1;
+    p.dx = dx;
+    p.domain.hi[0] = nx - 1; p.domain.hi[1] = ny - 1;
+    return p;
+}
+
+// ---------------------------------------------------------------------------
+// register faces: every entry a hierarchy's registers read is stored by one workgroup of the launch
+// ---------------------------------------------------------------------------
+typedef std::map<std::pair<const double*, int>, int> Writers;
+
+// the faces that the workgroups of a level's launch compute and store: of a tile, a strip or a boundary
+// piece, the lo x faces of its cells and of the column beyond, the lo y faces of its cells and of the row
+// beyond (the kernels' conditions on lx, ly)
+template <typename T>
+static void writers_of(const Group& G, bool all, Writers& w)
+{
+    const Patch<T>* pts = (const Patch<T>*)G.patches_dev[0];
+    for (int q = 0; q < G.ntiles; ++q) {
+        const Tile& t = G.tiles_dev[q];
+        const Patch<T>& p = pts[t.patch];
+        const int mw = p.vhi0 - p.vlo0 + 3;
+        for (int d = 0; d < 2; ++d)
+            for (int j = t.y0; j <= t.y1 + (d == 1); ++j)
+                for (int i = t.x0; i <= t.x1 + (d == 0); ++i) {
+                    const unsigned char* mk = p.fmask + (size_t)(i - p.vlo0 + 1) + (size_t)(j - p.vlo1 + 1) * mw;
+                    const bool lo = all || (d == 0 ? i > t.x0 : j > t.y0), hi = all || (d == 0 ? i <= t.x1 : j <= t.y1);
+                    if (!register_face(d == 0 ? mk[-1] : mk[-mw], *mk, lo, hi)) continue;
+                    const int fnx = p.vhi0 - p.vlo0 + 1 + (d == 0);
+                    ++w[{p.F[d], (i - p.vlo0) + (j - p.vlo1) * fnx}];
+                }
+    }
+}
+
+template <typename T>
+static int registers_case(const std::vector<std::vector<tmk_box>>& boxes, int nx, int ny, int r, int march)
+{
+    const int prec = sizeof(T) == sizeof(double) ? TMK_PREC_FP64 : TMK_PREC_FP32_BULK;
+    std::vector<tmk_ctx*> ctx;
+    std::vector<tmk_level*> lev;
+    int lnx = nx, lny = ny;
+    double dx = 100.0;
+    for (const auto& b : boxes) {
+        const tmk_params p = params(lnx, lny, dx);
+        tmk_ctx* c = nullptr;
+        tmk_level* L = nullptr;
+        EXPECT(tmk_ctx_create(&c, &p, prec) == TMK_OK);
+        if (march >= 0) EXPECT(tmk_set_march(c, march) == TMK_OK);
+        EXPECT(tmk_level_create(c, (int)b.size(), b.data(), &L) == TMK_OK);
+        ctx.push_back(c);
+        lev.push_back(L);
+        lnx *= r; lny *= r; dx /= r;
+    }
+    tmk_amr* A = nullptr;
+    EXPECT(tmk_amr_create((int)lev.size(), lev.data(), r, &A) == TMK_OK);
+    EXPECT(tmk_amr_run(A, 1, 0.0, 1e-3) == TMK_OK);
+    int shared = 0;
+    std::vector<Writers> w(lev.size());
+    for (int l = 0; l < A->nlev; ++l) {
+        writers_of<T>(A->lv[l].grp, false, w[l]);
+        for (const auto& f : w[l]) EXPECT(f.second == 1);
+        Writers both;
+        writers_of<T>(A->lv[l].grp, true, both);
+        EXPECT(both.size() == w[l].size());  // no register face goes without its writer
+        for (const auto& f : both) shared += f.second > 1;
+    }
+    for (int l = 0; l + 1 < A->nlev; ++l) {
+        const AmrLevel& a = A->lv[l];
+        const Patch<T>* crs = (const Patch<T>*)a.grp.patches_dev[0];
+        const Patch<T>* fine = (const Patch<T>*)A->lv[l + 1].grp.patches_dev[0];
+        EXPECT(a.nreg > 0);
+        for (int k = 0; k < a.nreg; ++k) {
+            const RegFace& f = ((const RegFace*)a.regf.p)[k];
+            EXPECT(w[l].count({crs[f.cpatch].F[f.d], f.cface}) == 1);
+            for (int m = 0; m < r; ++m) EXPECT(w[l + 1].count({fine[f.fpatch].F[f.d], f.fface[m]}) == 1);
+        }
+    }
+    EXPECT(tmk_amr_destroy(A) == TMK_OK);
+    for (tmk_level* L : lev) EXPECT(tmk_level_destroy(L) == TMK_OK);
+    for (tmk_ctx* c : ctx) EXPECT(tmk_ctx_destroy(c) == TMK_OK);
+    return shared;
+}
+
+static tmk_box box(int x0, int y0, int x1, int y1)
+{
+    tmk_box b;
+    b.lo[0] = x0; b.lo[1] = y0; b.hi[0] = x1; b.hi[1] = y1;
+    return b;
+}
+
+static void registers()
+{
+    const int nx = 72, ny = 40;
+    const std::vector<tmk_box> whole = {box(0, 0, nx - 1, ny - 1)};
+    // refined regions whose edges lie 3 coarse cells from the fault and from the other edges, inside and
+    // out, at a strip's 58th column, and one that spans the domain; a third level inside one of them
+    const std::vector<std::vector<tmk_box>> refined = {
+        {box(12, 0, 27, 2)}, {box(12, 3, 27, 9)},         // covered below row 3, from row 3 on
+        {box(3, 12, 20, 20)}, {box(0, 12, 2, 20)},        // column 3, both ways
+        {box(30, 12, nx - 4, 20)}, {box(nx - 3, 12, nx - 1, 20)},
+        {box(20, 20, 60, ny - 4)}, {box(20, ny - 3, 60, ny - 1)},
+        {box(50, 10, 60, 20), box(61, 10, 64, 20)},
+        {box(0, 0, nx - 1, 2)},
+    };
+    int shared = 0;
+    for (int r : {2, 4})
+        for (const auto& c : refined) {
+            std::vector<std::vector<tmk_box>> b = {whole, {}};
+            for (const tmk_box& q : c)
+                b[1].push_back(box(q.lo[0] * r, q.lo[1] * r, (q.hi[0] + 1) * r - 1, (q.hi[1] + 1) * r - 1));
+            for (int march : {-1, 0, 4, 63}) {
+                shared += registers_case<float>(b, nx, ny, r, march);
+                shared += registers_case<double>(b, nx, ny, r, march);
+            }
+        }
+    const std::vector<std::vector<tmk_box>> three = {whole, {box(24, 0, 87, 31)}, {box(64, 0, 159, 5)}};
+    shared += registers_case<float>(three, nx, ny, 2, -1);
+    EXPECT(shared > 0);  // faces that two workgroups of a launch compute
+}
+
+int main(int argc, char** argv)
+{
+    const char* const what = argc > 1 ? argv[1] : "";
+    if (!strcmp(what, "registers")) registers();
+    else fail("no such check", __LINE__);
+    printf("%s ok\n", what);
+    return 0;
+}

@@ -539,3 +539,48 @@ def test_c2_three_levels_ratio_four_rate_and_state_plastic_tagged_regrid():
         assert np.count_nonzero((U[9] > 0) & lev.valid) + np.count_nonzero((U[20] > 0) & lev.valid) > 0
         assert np.count_nonzero(lev.B[9, G:-G][lev.fvalid] != SENTINEL) >= 8
     H.close()
+
+
+@pytest.mark.parametrize("r,fine", [
+    (2, [(24, 0, 55, 5)]),            # the refined region ends 3 coarse cells above the fault
+    (2, [(6, 24, 41, 41)]),           # begins 3 coarse cells from the left edge
+    (4, [(12, 40, 83, 87)]),
+    (2, [(60, 20, 121, 57)]),         # ends 3 coarse cells below the upper edge, in a strip's last columns
+    (4, [(184, 0, 251, 11), (252, 0, 275, 11)]),  # 3 cells from the right edge and from the fault
+])
+def test_register_faces_between_strips_and_boundary_pieces(r, fine):
+    """A register face 3 coarse cells from an edge lies between a strip and a boundary piece, which compute
+    its flux apart.  FP64: every level bit for bit the oracle's.  FP32, where the two round differently: one
+    of them stores it, so two runs and two strip heights give the same bits; and the levels stay within
+    1e-4 of the oracle, as the FP32 hierarchy's slip above."""
+    nx, ny = 72, 32
+    cfg = scenarios.config_c0(seed=8, nx=nx, ny=ny, dx=100.0)
+    boxes = [[(0, 0, nx - 1, ny - 1)], fine]
+    cfgs = _cfgs(cfg, 2, r)
+    x0, y0, x1, y1 = fine[0]
+    arrays = _bump_arrays(cfgs, 0.5 * (x0 + x1 + 1) * cfgs[1]["dx"], 0.5 * (y0 + y1 + 1) * cfgs[1]["dx"],
+                          0.6 * max(x1 - x0, y1 - y0) * cfgs[1]["dx"])
+    h = _compare(cfg, boxes, r, 3, arrays, exact=True)
+    got = []
+    for rows in (0, 0, 5):  # 0: the height the launch chooses
+        ctxs, levels = amr.make_levels(cfg, boxes, r, capi.PREC_FP32_BULK)
+        for l, lev in enumerate(levels):
+            U, B = arrays(l)
+            for k, b in enumerate(boxes[l]):
+                lev.upload(k, scenarios.box_view(U, b), scenarios.box_bview(B, b) if b[1] == 0 else None)
+            if rows:
+                lev.set_update_shape(rows)
+        A = capi.Amr(levels, r)
+        A.run(3, 0.0, scenarios.dt_of(cfg))
+        A.sync()
+        A.close()
+        got.append(_download_levels(levels, boxes, cfgs))
+        for o in levels + ctxs:
+            o.close()
+    for l, lev in enumerate(h.levels):
+        for other in got[1:]:
+            for a, b in zip(got[0][l], other[l]):
+                assert np.array_equal(np.nan_to_num(a, nan=7.0), np.nan_to_num(b, nan=7.0)), l
+        Ur, Ug = lev.U[:, G:-G, G:-G][:, lev.valid], got[0][l][0][:, G:-G, G:-G][:, lev.valid]
+        for c in range(scenarios.NCOMP):
+            assert np.max(np.abs(Ug[c] - Ur[c])) <= 1e-4 * max(np.max(np.abs(Ur[c])), 1e-300), (l, c)

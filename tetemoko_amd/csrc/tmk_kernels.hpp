@@ -224,15 +224,19 @@ __device__ __forceinline__ void fault_output(const DevParams& P, const FaultOut&
 // the 11 flux components of side sd from face state (v, s) on the lo d-face of cell (i, j) into
 // the flux register array of direction d (surroundingNodes(valid box, d)).  With stores_delta
 // this is the flux of U - bg: flux registers only ever difference fluxes of one precision, and
-// the drop-in path adds the background's flux (bg_flux) on the host.
-// whether a face between cells with face-mask bits a and b carries a register flux: a face of
-// the level's boundary (exactly one side a cell of the level), or, between two cells of the
-// level, a face around the finer level (exactly one side covered by it)
-__device__ __forceinline__ bool register_face(unsigned a, unsigned b)
+// the drop-in path adds the background's flux (bg_flux) on the host.  lo, hi: the workgroup updates the
+// cell below / above the face (register_face; without a mask every face is stored).
+// whether a workgroup stores the register flux of a face between cells with face-mask bits a (lo) and b
+// (hi); lo, hi: it updates that cell.  A face of the level's boundary (one side a cell of the level, the
+// fine side of a register) belongs to that cell, a face around the finer level (between two cells of the
+// level, one of them covered) to the uncovered one, the cell that reflux corrects.  One workgroup updates
+// that cell, so every register entry has one writer, and the flux it takes is the one the cell's own
+// update used: a strip and a boundary piece round the flux of a face between them differently in FP32,
+// and with a store by each the entry depended on their order.
+__host__ __device__ __forceinline__ bool register_face(unsigned a, unsigned b, bool lo, bool hi)
 {
-    const bool edge = ((a ^ b) & 1) != 0;           // level boundary (fine side)
-    const bool cf = (a & b & 1) && ((a ^ b) & 2);  // around the finer level (coarse side)
-    return edge || cf;
+    if ((a ^ b) & 1) return (a & 1) ? lo : hi;
+    return (a & 1) && ((a ^ b) & 2) && ((a & 2) ? hi : lo);
 }
 
 // the 11 components of side sd of the face flux in direction d at index fi of the flux array
@@ -272,14 +276,14 @@ __device__ __forceinline__ void put_face_flux(__attribute__((address_space(1))) 
 
 template <typename T, int NS, bool D2>
 __device__ __forceinline__ void store_flux_side(const Patch<T>& pt, const Mat<T, D2>& m, int d, const T (&v)[NS],
-                                                const T (&sv)[NS], T r, int i, int j, int sd)
+                                                const T (&sv)[NS], T r, int i, int j, int sd, bool lo, bool hi)
 {
     const int fnx = pt.vhi0 - pt.vlo0 + 1 + (d == 0), fny = pt.vhi1 - pt.vlo1 + 1 + (d == 1);
     if (pt.fmask) {
         const int mw = pt.vhi0 - pt.vlo0 + 3;
         const __attribute__((address_space(1))) unsigned char* mk =
             gmem(pt.fmask) + (size_t)(i - pt.vlo0 + 1) + (size_t)(j - pt.vlo1 + 1) * mw;
-        if (!register_face(d == 0 ? mk[-1] : mk[-mw], *mk)) return;
+        if (!register_face(d == 0 ? mk[-1] : mk[-mw], *mk, lo, hi)) return;
     }
     const size_t fp = (size_t)fnx * fny;
     const size_t fi = (size_t)(i - pt.vlo0) + (size_t)(j - pt.vlo1) * fnx;
@@ -288,10 +292,10 @@ __device__ __forceinline__ void store_flux_side(const Patch<T>& pt, const Mat<T,
 
 template <typename T, int NS, bool D2>
 __device__ __forceinline__ void store_flux(const Patch<T>& pt, const Mat<T, D2>& m, int d, const Slots<T, NS>& Fs, T rv,
-                                           int i, int j)
+                                           int i, int j, bool lo, bool hi)
 {
-    store_flux_side<T, NS>(pt, m, d, Fs.v[0], Fs.s[0], (T)1, i, j, 0);
-    store_flux_side<T, NS>(pt, m, d, Fs.v[1], Fs.s[1], rv, i, j, 1);
+    store_flux_side<T, NS>(pt, m, d, Fs.v[0], Fs.s[0], (T)1, i, j, 0, lo, hi);
+    store_flux_side<T, NS>(pt, m, d, Fs.v[1], Fs.s[1], rv, i, j, 1, lo, hi);
 }
 
 // face states of one side on the four faces of a cell: lo/hi x face, lo/hi y face
@@ -812,8 +816,10 @@ __device__ __forceinline__ void godunov_tile(const KArgs<T>& a, const Tile& tl, 
             }
         __syncthreads();
         // optional flux output for flux registers (LinElastPatchGodunov.cpp:117-118, LinElastPhysics.cpp:153)
-        if (pt.F[0] && lx >= 1 && lx <= tnx + 1 && ly >= 1 && ly <= tny) store_flux<T, NS>(pt, m, 0, F0, (T)1, i, j);
-        if (pt.F[1] && ly >= 1 && ly <= tny + 1 && lx >= 1 && lx <= tnx) store_flux<T, NS>(pt, m, 1, F1, rv1, i, j);
+        if (pt.F[0] && lx >= 1 && lx <= tnx + 1 && ly >= 1 && ly <= tny)
+            store_flux<T, NS>(pt, m, 0, F0, (T)1, i, j, lx > 1, lx <= tnx);
+        if (pt.F[1] && ly >= 1 && ly <= tny + 1 && lx >= 1 && lx <= tnx)
+            store_flux<T, NS>(pt, m, 1, F1, rv1, i, j, ly > 1, ly <= tny);
         if (valid) {
             Slots<T, NS> F0h, F1h;
 #pragma unroll

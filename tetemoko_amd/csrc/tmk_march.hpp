@@ -258,10 +258,10 @@ struct MarchRing {
     static constexpr int LDS_FLOATS = RING_FLOATS + 16 + 4 * 64;
 };
 
-// The faces of strip tl that carry a register flux, from the level's face masks (Patch::fmask): bit
-// j - y0 of m0 for this lane's lo x face on row j, of m1 for its lo y face (row y1 + 1 too).  One mask
-// byte is loaded per row, four rows at a time; the left neighbour's comes by a lane shift and the lower
-// one's from the row before.
+// The faces of strip tl whose register flux the strip stores (register_face), from the level's face masks
+// (Patch::fmask): bit j - y0 of m0 for this lane's lo x face on row j, of m1 for its lo y face (row y1 + 1
+// too).  One mask byte is loaded per row, four rows at a time; the left neighbour's comes by a lane shift
+// and the lower one's from the row before.
 template <typename T>
 __device__ __forceinline__ void march_faces(const Patch<T>& pt, const Tile& tl, int lane, unsigned long long& m0,
                                             unsigned long long& m1)
@@ -271,6 +271,7 @@ __device__ __forceinline__ void march_faces(const Patch<T>& pt, const Tile& tl, 
     const int mw = pt.vhi0 - pt.vlo0 + 3;  // the masks cover the descriptor's valid box grown by one
     const int i = tl.x0 - 3 + min(max(lane, 2), tnx + 3);
     const size_t at = (size_t)(i - pt.vlo0 + 1) + (size_t)(y0 - pt.vlo1 + 1) * mw;
+    const bool left_in = lane >= 4, here_in = lane <= tnx + 2;  // the left and this lane's column: of the strip
     unsigned below = mk[at - mw];
     for (int k = 0; k <= rows; k += 4) {
         unsigned b[4];
@@ -279,8 +280,8 @@ __device__ __forceinline__ void march_faces(const Patch<T>& pt, const Tile& tl, 
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             const unsigned left = (unsigned)__builtin_amdgcn_update_dpp(0, (int)b[q], DPP_FROM_PREV, 0xF, 0xF, true);
-            if (k + q < rows && register_face(left, b[q])) m0 |= 1ull << (k + q);
-            if (k + q <= rows && register_face(below, b[q])) m1 |= 1ull << (k + q);
+            if (k + q < rows && register_face(left, b[q], left_in, here_in)) m0 |= 1ull << (k + q);
+            if (k + q <= rows && register_face(below, b[q], k + q > 0, k + q < rows)) m1 |= 1ull << (k + q);
             below = b[q];
         }
     }

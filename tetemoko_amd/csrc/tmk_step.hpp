@@ -268,8 +268,9 @@ __device__ __forceinline__ void bnd_piece(const KArgs<T>& a, const Tile& tl, con
     }
     // flux registers (hierarchy levels)
     if (pt.F[0] && lx >= 1 && lx <= tnx + 1 && ly >= 1 && ly <= tny)
-        store_flux_side<T, 2>(pt, m, 0, xv, xs, (T)1, i, j, sd);
-    if (pt.F[1] && ly >= 1 && ly <= tny + 1 && lx >= 1 && lx <= tnx) store_flux_side<T, 2>(pt, m, 1, yv, ys, ry, i, j, sd);
+        store_flux_side<T, 2>(pt, m, 0, xv, xs, (T)1, i, j, sd, lx > 1, lx <= tnx);
+    if (pt.F[1] && ly >= 1 && ly <= tny + 1 && lx >= 1 && lx <= tnx)
+        store_flux_side<T, 2>(pt, m, 1, yv, ys, ry, i, j, sd, ly > 1, ly <= tny);
     if (valid) {
         Faces1<T, 2> F;
 #pragma unroll
