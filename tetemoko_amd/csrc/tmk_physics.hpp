@@ -985,8 +985,7 @@ __device__ __forceinline__ float plastic_pbg(const PlasticConstL& P, int k) { re
 __device__ __forceinline__ float plastic_pf(const PlasticConstL& P, int k) { return P.c[7 + k]; }
 __device__ __forceinline__ float plastic_G(const PlasticConstL& P) { return P.c[13]; }
 
-// The deviator is free of trace, so J2 = (exx^2 + eyy^2 + ezz^2) / 2 + the shears.  g is formed
-// with the hardware's reciprocal of tau (within an ulp): it scales increments far below the stresses.
+// The deviator is free of trace, so J2 = (exx^2 + eyy^2 + ezz^2) / 2 + the shears.
 // PP: DevParams or PlasticConstL; NS = 2: mode II, whose anti-plane stresses are zero.
 template <typename T, int NS, typename PP>
 __device__ __forceinline__ void plastic_flow_delta(const PP& P, T dt, T& dxx, T& dyy, T& dzz, T& dxy, T& dxz,
@@ -1012,7 +1011,7 @@ __device__ __forceinline__ void plastic_flow_delta(const PP& P, T dt, T& dxx, T&
     plam = Y / (dt * (T)plastic_pf(P, 3) + (T)plastic_pf(P, 4));
     const T dl = dt * plam;
     pgam = pgam + dl;
-    const T g = dl * (T)plastic_G(P) * __builtin_amdgcn_rcpf(tau);  // 1 - tau_new / (tau_new + dt lam G), tau_new = tau - dt lam G
+    const T g = dl * (T)plastic_G(P) / tau;  // 1 - tau_new / (tau_new + dt lam G), tau_new = tau - dt lam G
     const T dm = dl * (T)plastic_pf(P, 5);
     dxx = dxx - (dm + g * exx);
     dyy = dyy - (dm + g * eyy);
