@@ -138,10 +138,10 @@ int tmk_patch_update_state(tmk_ctx *ctx, tmk_box valid, double *U, tmk_box U_box
  * loops, harnesses that forbid hipMalloc).  Same arguments, checks, results and error codes as
  * tmk_patch_update_state (the same kernels on the same tiles), but every device buffer of the
  * call -- both state copies, the fault data, the fluxes, the FP64 staging of the FP32 bulk and the
- * launch tables -- lives in one fixed array of TMK_NOALLOC_SCRATCH_BYTES per device, held from
- * the first context created on that device until the process ends.  TMK_E_SCRATCH when the call
- * needs more than that (for FP64 with both fluxes, boxes up to about 128 x 128 cells fit) or
- * more than 1024 tiles.  Every call on a device shares that array: calls that overlap on one
+ * launch tables -- lives in one fixed array per device, held from the first context created on
+ * that device until the process ends.  TMK_E_SCRATCH when the call needs more than
+ * TMK_NOALLOC_SCRATCH_BYTES of it (for FP64 with both fluxes, boxes up to about 128 x 128 cells
+ * fit) or more than 1024 tiles.  Every call on a device shares that array: calls that overlap on one
  * device (from several threads, or contexts used concurrently) race and must be serialised by
  * the caller. */
 #define TMK_NOALLOC_SCRATCH_BYTES (16u << 20)

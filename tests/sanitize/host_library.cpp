@@ -148,10 +148,55 @@ static void registers()
     EXPECT(shared > 0);  // faces that two workgroups of a launch compute
 }
 
+// ---------------------------------------------------------------------------
+// which calls fit the allocation-free call's scratch
+// ---------------------------------------------------------------------------
+// The rule the limit was set with: two copies of the state, the FP64 image of an FP32 one, the fluxes and
+// the tables (a descriptor of 512 bytes, 20 bytes a tile, a scenario block of 1048), each part from a
+// multiple of 256 bytes, within TMK_NOALLOC_SCRATCH_BYTES.
+static void scratch_limit()
+{
+    for (int prec : {TMK_PREC_FP64, TMK_PREC_FP32_BULK})
+        for (bool flux : {false, true}) {
+            const int nx = 1000, ny = 240;
+            const tmk_params p = params(nx, ny, 25.0);
+            tmk_ctx* c = nullptr;
+            EXPECT(tmk_ctx_create(&c, &p, prec) == TMK_OK);
+            const size_t ts = prec == TMK_PREC_FP64 ? sizeof(double) : sizeof(float);
+            int fits = 0, refused = 0, close = 0;
+            for (int vny = 24; vny <= 200; ++vny)
+                for (int vnx = 100; vnx < 900; ++vnx) {
+                    const tmk_box v = box(8, 8, 8 + vnx - 1, 8 + vny - 1);
+                    const tmk_box ub = box(v.lo[0] - 4, v.lo[1] - 4, v.hi[0] + 4, v.hi[1] + 4);
+                    const size_t plane = (size_t)(vnx + 8) * (vny + 8), nU = plane * TMK_NCOMP;
+                    const size_t n0 = (size_t)(vnx + 1) * vny * TMK_NCOMP, n1 = (size_t)vnx * (vny + 1) * TMK_NCOMP;
+                    auto up = [](size_t b) { return (b + 255) / 256 * 256; };
+                    size_t need = 2 * up(nU * ts) + (flux ? up((n0 + n1) * sizeof(double)) : 0);
+                    if (prec != TMK_PREC_FP64) need += up(nU * sizeof(double));
+                    int nint = 0;
+                    const int nt = patch_tiles(v, c->P, c->bx, c->by, nullptr, 0, &nint);
+                    need += 512 + up(20 * (size_t)nt) + 1048;
+                    if (need + 8192 < TMK_NOALLOC_SCRATCH_BYTES || need > TMK_NOALLOC_SCRATCH_BYTES + 8192) continue;
+                    const bool ok = need <= TMK_NOALLOC_SCRATCH_BYTES && nt <= 1024;
+                    std::vector<double> U(nU, 0.0), F0(flux ? n0 : 0), F1(flux ? n1 : 0);
+                    double mws = 0.0;
+                    const int e = tmk_patch_update_state_noalloc(c, v, U.data(), ub, TMK_NCOMP, flux ? F0.data() : nullptr,
+                                                                 flux ? F1.data() : nullptr, nullptr, ub, 0, 0.0, 1e-3, &mws);
+                    EXPECT(e == (ok ? TMK_OK : TMK_E_SCRATCH));
+                    fits += ok;
+                    refused += !ok;
+                    close += ok && need + 2048 > TMK_NOALLOC_SCRATCH_BYTES;
+                }
+            EXPECT(fits > 0 && refused > 0 && close > 0);
+            EXPECT(tmk_ctx_destroy(c) == TMK_OK);
+        }
+}
+
 int main(int argc, char** argv)
 {
     const char* const what = argc > 1 ? argv[1] : "";
     if (!strcmp(what, "registers")) registers();
+    else if (!strcmp(what, "scratch_limit")) scratch_limit();
     else fail("no such check", __LINE__);
     printf("%s ok\n", what);
     return 0;

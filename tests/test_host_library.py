@@ -5,6 +5,8 @@ host-memory stand-in of the HIP runtime, so that the tables a launch would read 
 registers: of every face that a hierarchy's flux registers read, exactly one workgroup of the level's
 launch stores the flux, with regions that end 3 coarse cells from the fault and from the other edges,
 where strips and boundary pieces meet.
+scratch_limit: the allocation-free drop-in call takes and refuses the boxes it always did, by bytes near
+its limit.
 """
 import os
 import shutil
@@ -24,7 +26,7 @@ def driver():
     return os.path.join(HERE, "_build", "host_library")
 
 
-@pytest.mark.parametrize("check", ["registers"])
+@pytest.mark.parametrize("check", ["registers", "scratch_limit"])
 def test_host_library(driver, check):
     r = subprocess.run([driver, check], cwd=HERE, capture_output=True, text=True, timeout=300)
     assert r.returncode == 0 and check + " ok" in r.stdout, r.stdout[-4000:] + r.stderr[-8000:]

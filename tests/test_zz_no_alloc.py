@@ -85,3 +85,22 @@ def test_noalloc_refuses_a_box_beyond_its_scratch():
             assert np.array_equal(a, b)
     finally:
         ctx.close()
+
+
+def test_noalloc_takes_a_box_at_its_scratch_limit():
+    """389 x 112 cells without fluxes: all but 7680 of the scratch's bytes are state, of which the launch
+    tables count 6680."""
+    cfg = scenarios.config_c1(seed=6, nx=420, ny=130, dx=25.0)
+    dt = scenarios.dt_of(cfg)
+    valid = (10, 6, 398, 117)
+    Ub, ubox, _, _ = _inputs(cfg, valid, 33)
+    ctx = capi.Context(cfg, capi.PREC_FP64)
+    try:
+        got = []
+        for noalloc in (False, True):
+            U = Ub.copy()
+            ctx.update_state(valid, U, ubox, None, None, time=0.2, dt=dt, noalloc=noalloc)
+            got.append(U)
+        assert np.array_equal(got[0], got[1]) and not np.array_equal(got[0], Ub)
+    finally:
+        ctx.close()

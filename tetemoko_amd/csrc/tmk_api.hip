@@ -1536,11 +1536,13 @@ struct PatchWork {
     char* meta = nullptr;
 };
 
+static constexpr size_t align256(size_t b) { return ((b + 255) / 256) * 256; }
+
 template <typename T>
 static void patch_meta(int ntiles, size_t* off_t, size_t* off_s, size_t* bytes)
 {
-    *off_t = ((sizeof(Patch<T>) + 255) / 256) * 256;
-    *off_s = *off_t + ((sizeof(Tile) * (size_t)ntiles + 255) / 256) * 256;
+    *off_t = align256(sizeof(Patch<T>));
+    *off_s = *off_t + align256(sizeof(Tile) * (size_t)ntiles);
     *bytes = *off_s + sizeof(Scen);
 }
 
@@ -1939,16 +1941,25 @@ extern "C" int tmk_patch_plastic_update(tmk_ctx* c, tmk_box valid, double* U, tm
 // ---------------------------------------------------------------------------
 // allocation-free drop-in
 // ---------------------------------------------------------------------------
+// the most tiles one allocation-free call launches (they are listed in a stack array)
+static constexpr int kNoAllocMaxTiles = 1024;
+
+// The launch tables of an allocation-free call lie behind the TMK_NOALLOC_SCRATCH_BYTES of its data.  What
+// they count toward that limit is fixed, at the sizes their entries had when the limit was set (a patch
+// descriptor of 512 bytes, 20 bytes a tile, a scenario block of 1048): which calls fit does not move with
+// the tables' layout.
+static constexpr size_t kNoAllocTables =
+    align256(sizeof(Patch<double>)) + align256(sizeof(Tile) * kNoAllocMaxTiles) + align256(sizeof(Scen));
+static_assert(sizeof(Patch<float>) == sizeof(Patch<double>), "one table size for both precisions");
+static size_t noalloc_counted(int ntiles) { return 512 + align256(20 * (size_t)ntiles) + 1048; }
+
 // Device scratch of tmk_patch_update_state_noalloc: the two state copies, the fault data (read
-// and written copies), the fluxes, the FP64 staging of the FP32 bulk and the launch tables of
-// one call.  One array per device for the life of the process; every call on a device shares
+// and written copies), the fluxes and the FP64 staging of the FP32 bulk of one call, then its launch
+// tables.  One array per device for the life of the process; every call on a device shares
 // it, so calls that overlap on one device race.  Host code never passes this name to a kernel
 // or a copy: it is a host-side stand-in, and the device address comes from
 // hipGetSymbolAddress (scratch_device_ptr).
-static __device__ __align__(256) unsigned char scratch[TMK_NOALLOC_SCRATCH_BYTES];
-
-// the most tiles one allocation-free call launches (they are listed in a stack array)
-static constexpr int kNoAllocMaxTiles = 1024;
+static __device__ __align__(256) unsigned char scratch[TMK_NOALLOC_SCRATCH_BYTES + kNoAllocTables];
 
 static std::mutex g_scratch_mu;
 static void* g_scratch_ptr[64];  // per device ordinal, resolved once
@@ -1972,8 +1983,6 @@ static int scratch_device_ptr(void** out)
     return TMK_OK;
 }
 
-static size_t align256(size_t b) { return ((b + 255) / 256) * 256; }
-
 template <typename T>
 static int patch_update_noalloc_t(tmk_ctx* c, tmk_box valid, double* U, tmk_box ub, double* F0, double* F1,
                                   double* B, tmk_box bb, int nb, double time, double dt)
@@ -1985,13 +1994,13 @@ static int patch_update_noalloc_t(tmk_ctx* c, tmk_box valid, double* U, tmk_box 
     if (ntiles > kNoAllocMaxTiles) return TMK_E_SCRATCH;
     size_t off_t, off_s, mbytes;
     patch_meta<T>(ntiles, &off_t, &off_s, &mbytes);
-    // layout: Uin, Uout, fault data (2 copies), fluxes, FP64 staging (FP32 bulk only), tables
+    // layout: Uin, Uout, fault data (2 copies), fluxes, FP64 staging (FP32 bulk only); the tables behind
     const size_t oUout = align256(z.nU * sizeof(T));
     const size_t oB = oUout + align256(z.nU * sizeof(T));
     const size_t oF = oB + align256(2 * z.nB * sizeof(double));
     const size_t oS = oF + align256((z.nF0 + z.nF1) * sizeof(double));
     const size_t oM = oS + (sizeof(T) == sizeof(double) ? 0 : align256(z.nU * sizeof(double)));
-    if (oM + mbytes > (size_t)TMK_NOALLOC_SCRATCH_BYTES) return TMK_E_SCRATCH;
+    if (oM + noalloc_counted(ntiles) > (size_t)TMK_NOALLOC_SCRATCH_BYTES) return TMK_E_SCRATCH;
     // what fits by the tile kernels' list is accepted; its strips, where their list fits too
     const int ns = patch_ns(c, U, z.plane);
     Tile tiles[kNoAllocMaxTiles];
@@ -2001,7 +2010,7 @@ static int patch_update_noalloc_t(tmk_ctx* c, tmk_box valid, double* U, tmk_box 
     if (patch_marches(c, ns)) {
         strips = patch_strips(c, valid, &nint);
         patch_meta<T>((int)strips.size(), &off_t, &off_s, &mbytes);
-        if (strips.size() > (size_t)kNoAllocMaxTiles || oM + mbytes > (size_t)TMK_NOALLOC_SCRATCH_BYTES) strips.clear();
+        if (strips.size() > (size_t)kNoAllocMaxTiles) strips.clear();
     }
     const bool march = !strips.empty();
     if (march) {
@@ -2018,7 +2027,7 @@ static int patch_update_noalloc_t(tmk_ctx* c, tmk_box valid, double* U, tmk_box 
     w.Bd = (double*)(base + oB);
     w.Fd = (double*)(base + oF);
     w.stage = sizeof(T) == sizeof(double) ? nullptr : (double*)(base + oS);
-    w.meta = base + oM;
+    w.meta = base + TMK_NOALLOC_SCRATCH_BYTES;
     HostStage* const S = patch_staged<T>(z, mbytes, false);  // pinning allocates
     const int e = patch_update_t<T>(c, valid, U, ub, F0, F1, B, bb, nb, time, dt, false, w, list, nlist, nint, ns, march, S);
     if (S && e) (void)hipStreamSynchronize(c->stream);
