@@ -192,11 +192,47 @@ static void scratch_limit()
         }
 }
 
+// ---------------------------------------------------------------------------
+// the allocation-free call's list: every FP64 box that fits the scratch has its strips and pieces
+// ---------------------------------------------------------------------------
+static void strip_lists()
+{
+    size_t longest = 0;
+    for (int w : {1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 14, 30, 64, 130})
+        for (int tall : {0, 1}) {
+            // the longest box of this width that fits, in a domain of its own width and in a wider one
+            for (int margin : {0, 1, 5}) {
+                const int n = 47662 / (w + 2 * std::min(margin, 3)) - (margin ? 6 : 0);
+                const int nx = tall ? w + 2 * margin : n + 2 * margin, ny = tall ? n + 2 * margin : w + 2 * margin;
+                if (std::min(nx, ny) < 4) continue;  // the smallest domain
+                const tmk_params p = params(nx, ny, 25.0);
+                tmk_ctx* c = nullptr;
+                EXPECT(tmk_ctx_create(&c, &p, TMK_PREC_FP64) == TMK_OK);
+                const tmk_box v = tall ? box(margin, margin, margin + w - 1, margin + n - 1)
+                                       : box(margin, margin, margin + n - 1, margin + w - 1);
+                for (int rows : {0, 1, 4, 63}) {  // 0: the height the call chooses
+                    if (rows) EXPECT(tmk_set_march(c, rows) == TMK_OK);
+                    EXPECT(patch_marches(c, 2));
+                    int nint = 0;
+                    const std::vector<Tile> t = patch_strips(c, v, &nint, kNoAllocMaxStrips);
+                    EXPECT(t.size() <= (size_t)kNoAllocMaxStrips);
+                    longest = std::max(longest, t.size());
+                    long long cells = 0;
+                    for (const Tile& q : t) cells += (long long)(q.x1 - q.x0 + 1) * (q.y1 - q.y0 + 1);
+                    EXPECT(cells == (long long)n * w);
+                }
+                EXPECT(tmk_ctx_destroy(c) == TMK_OK);
+            }
+        }
+    EXPECT(longest > 1024);
+}
+
 int main(int argc, char** argv)
 {
     const char* const what = argc > 1 ? argv[1] : "";
     if (!strcmp(what, "registers")) registers();
     else if (!strcmp(what, "scratch_limit")) scratch_limit();
+    else if (!strcmp(what, "strip_lists")) strip_lists();
     else fail("no such check", __LINE__);
     printf("%s ok\n", what);
     return 0;

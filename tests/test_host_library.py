@@ -7,6 +7,7 @@ launch stores the flux, with regions that end 3 coarse cells from the fault and 
 where strips and boundary pieces meet.
 scratch_limit: the allocation-free drop-in call takes and refuses the boxes it always did, by bytes near
 its limit.
+strip_lists: the strips and boundary pieces of every FP64 box that call takes fit its list.
 """
 import os
 import shutil
@@ -26,7 +27,7 @@ def driver():
     return os.path.join(HERE, "_build", "host_library")
 
 
-@pytest.mark.parametrize("check", ["registers", "scratch_limit"])
+@pytest.mark.parametrize("check", ["registers", "scratch_limit", "strip_lists"])
 def test_host_library(driver, check):
     r = subprocess.run([driver, check], cwd=HERE, capture_output=True, text=True, timeout=300)
     assert r.returncode == 0 and check + " ok" in r.stdout, r.stdout[-4000:] + r.stderr[-8000:]

@@ -104,3 +104,23 @@ def test_noalloc_takes_a_box_at_its_scratch_limit():
         assert np.array_equal(got[0], got[1]) and not np.array_equal(got[0], Ub)
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("rows", [None, 1])
+def test_noalloc_takes_the_same_kernels_on_a_long_list(rows):
+    """9 x 2300 rate-and-state cells on the fault: in strips of one row a list beyond the 1024 tiles of the
+    other kernels."""
+    cfg = scenarios.config_c1(seed=7, nx=40, ny=2310, dx=25.0)
+    dt = scenarios.dt_of(cfg)
+    valid = (12, 0, 20, 2299)
+    Ub, ubox, Bb, bbox = _inputs(cfg, valid, 34)
+    ctx = capi.Context(cfg, capi.PREC_FP64)
+    try:
+        if rows:
+            ctx.set_march(rows)
+        ref = _call(ctx, valid, Ub, ubox, Bb, bbox, False, dt)
+        U, B = Ub.copy(), Bb.copy()
+        ctx.update_state(valid, U, ubox, B, bbox, time=0.41, dt=dt, noalloc=True)
+        assert np.array_equal(U, ref[1]) and np.array_equal(B, ref[2])
+    finally:
+        ctx.close()

@@ -10,6 +10,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstdint>
 #include <cstdio>
 #include <cstring>
 #include <functional>
@@ -1650,20 +1651,25 @@ static int patch_ns(const tmk_ctx* c, const double* U, size_t plane)
 // An FP64 drop-in call marches by the rule a level marches by, in one launch: 32 x 32 with fluxes 98 -> 76
 // us.  FP32 calls keep the tile kernels: a flux between a strip and a boundary piece is stored by both, and
 // in FP32 the two round differently.  Its strips (nint of them, at most 63 rows, as on every level that
-// stores fluxes), then its boundary pieces.
+// stores fluxes), then its boundary pieces; at most most of both, by taller strips where the height chosen
+// makes more (FP64 values do not depend on it).
 static bool patch_marches(const tmk_ctx* c, int ns)
 {
     return c->precision == TMK_PREC_FP64 && c->march > 0 && ns == 2 && pred_kind(c->P) == PK_PPM_PRIM;
 }
-static std::vector<Tile> patch_strips(const tmk_ctx* c, const tmk_box& v, int* nint)
+static std::vector<Tile> patch_strips(const tmk_ctx* c, const tmk_box& v, int* nint, size_t most = SIZE_MAX)
 {
     Tile r;
     memset(&r, 0, sizeof r);
     r.x0 = v.lo[0]; r.y0 = v.lo[1]; r.x1 = v.hi[0]; r.y1 = v.hi[1];
     auto params = [&](const Tile&) -> const DevParams& { return c->P; };
-    const int rows = c->march_auto ? march_height({r}, params, false) : c->march;
+    int rows = std::min(c->march_auto ? march_height({r}, params, false) : c->march, 63);
     std::vector<Tile> strips, bf, bo;
-    march_rect(r, c->P, std::min(rows, 63), strips, bf, bo);
+    for (;; rows = std::min(2 * rows, 63)) {
+        march_rect(r, c->P, rows, strips, bf, bo);
+        if (rows == 63 || strips.size() + bf.size() + bo.size() <= most) break;
+        strips.clear(); bf.clear(); bo.clear();
+    }
     *nint = (int)strips.size();
     strips.insert(strips.end(), bf.begin(), bf.end());
     strips.insert(strips.end(), bo.begin(), bo.end());
@@ -1943,13 +1949,18 @@ extern "C" int tmk_patch_plastic_update(tmk_ctx* c, tmk_box valid, double* U, tm
 // ---------------------------------------------------------------------------
 // the most tiles one allocation-free call launches (they are listed in a stack array)
 static constexpr int kNoAllocMaxTiles = 1024;
+// and the most strips and boundary pieces, where it marches: a list that every call fits.  The state of
+// TMK_NOALLOC_SCRATCH_BYTES has at most 47662 cells; a piece covers at least 12 of them (4 columns of a
+// domain too narrow for strips, in pieces of 23 x 3), 23 beside strips, and patch_strips takes taller
+// strips before they are many.
+static constexpr int kNoAllocMaxStrips = 4096;
 
 // The launch tables of an allocation-free call lie behind the TMK_NOALLOC_SCRATCH_BYTES of its data.  What
 // they count toward that limit is fixed, at the sizes their entries had when the limit was set (a patch
 // descriptor of 512 bytes, 20 bytes a tile, a scenario block of 1048): which calls fit does not move with
 // the tables' layout.
 static constexpr size_t kNoAllocTables =
-    align256(sizeof(Patch<double>)) + align256(sizeof(Tile) * kNoAllocMaxTiles) + align256(sizeof(Scen));
+    align256(sizeof(Patch<double>)) + align256(sizeof(Tile) * kNoAllocMaxStrips) + align256(sizeof(Scen));
 static_assert(sizeof(Patch<float>) == sizeof(Patch<double>), "one table size for both precisions");
 static size_t noalloc_counted(int ntiles) { return 512 + align256(20 * (size_t)ntiles) + 1048; }
 
@@ -1992,8 +2003,6 @@ static int patch_update_noalloc_t(tmk_ctx* c, tmk_box valid, double* U, tmk_box 
     int nint = 0;
     const int ntiles = patch_tiles(valid, c->P, c->bx, c->by, nullptr, 0, &nint);
     if (ntiles > kNoAllocMaxTiles) return TMK_E_SCRATCH;
-    size_t off_t, off_s, mbytes;
-    patch_meta<T>(ntiles, &off_t, &off_s, &mbytes);
     // layout: Uin, Uout, fault data (2 copies), fluxes, FP64 staging (FP32 bulk only); the tables behind
     const size_t oUout = align256(z.nU * sizeof(T));
     const size_t oB = oUout + align256(z.nU * sizeof(T));
@@ -2001,25 +2010,26 @@ static int patch_update_noalloc_t(tmk_ctx* c, tmk_box valid, double* U, tmk_box 
     const size_t oS = oF + align256((z.nF0 + z.nF1) * sizeof(double));
     const size_t oM = oS + (sizeof(T) == sizeof(double) ? 0 : align256(z.nU * sizeof(double)));
     if (oM + noalloc_counted(ntiles) > (size_t)TMK_NOALLOC_SCRATCH_BYTES) return TMK_E_SCRATCH;
-    // what fits by the tile kernels' list is accepted; its strips, where their list fits too
+    // what fits by the tile kernels' list is accepted; the call takes the kernels that
+    // tmk_patch_update_state takes
     const int ns = patch_ns(c, U, z.plane);
+    const bool march = patch_marches(c, ns);
     Tile tiles[kNoAllocMaxTiles];
-    const Tile* list = tiles;
-    int nlist = ntiles;
     std::vector<Tile> strips;
-    if (patch_marches(c, ns)) {
-        strips = patch_strips(c, valid, &nint);
-        patch_meta<T>((int)strips.size(), &off_t, &off_s, &mbytes);
-        if (strips.size() > (size_t)kNoAllocMaxTiles) strips.clear();
-    }
-    const bool march = !strips.empty();
     if (march) {
-        list = strips.data();
-        nlist = (int)strips.size();
+        try {
+            strips = patch_strips(c, valid, &nint, kNoAllocMaxStrips);
+        } catch (const std::bad_alloc&) {
+            return TMK_E_NOMEM;
+        }
+        if (strips.size() > (size_t)kNoAllocMaxStrips) return TMK_E_SCRATCH;
     } else {
         patch_tiles(valid, c->P, c->bx, c->by, tiles, kNoAllocMaxTiles, &nint);
-        patch_meta<T>(ntiles, &off_t, &off_s, &mbytes);
     }
+    const Tile* const list = march ? strips.data() : tiles;
+    const int nlist = march ? (int)strips.size() : ntiles;
+    size_t off_t, off_s, mbytes;
+    patch_meta<T>(nlist, &off_t, &off_s, &mbytes);
     char* base = (char*)c->noalloc_scratch;
     PatchWork<T> w;
     w.Uin = (T*)base;
