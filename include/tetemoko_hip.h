@@ -117,7 +117,7 @@ int tmk_mem_info(size_t *free_bytes, size_t *total_bytes);
  * cached bytes per device (default 32 GiB); tmk_cache_set_limit sets that limit and frees idle
  * blocks above it on every device (0 turns caching off); tmk_cache_trim frees every idle block
  * of the current device, and the idle pinned buffers that downloads and drop-in calls go
- * through (8 MiB each, at most 4 kept in a process). */
+ * through (8 MiB each, at most 16 a device). */
 int tmk_cache_info(size_t *cached_bytes, size_t *live_bytes, size_t *limit_bytes);
 int tmk_cache_set_limit(size_t bytes);
 int tmk_cache_trim(void);

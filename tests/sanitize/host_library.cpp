@@ -4,9 +4,34 @@
 // runs.  Usage: host_library CHECK (see main).
 #include "../../tetemoko_amd/csrc/tmk_api.hip"
 
+#include <atomic>
 #include <cstdlib>
-#include <set>
 #include <utility>
+
+// the pinned-memory calls, counted (out of memory until a check turns them on: with a stage, a drop-in
+// call's error word comes from a kernel), and the current device of a thread (the stand-in's own is weak here)
+static std::atomic<int> g_pinned{0}, g_pins{0}, g_frees{0};
+static bool g_pin_on = false;
+static thread_local int g_dev = 0;
+extern "C" {
+hipError_t hipHostMalloc(void** p, size_t n, unsigned)
+{
+    if (!g_pin_on) return hipErrorOutOfMemory;
+    *p = std::calloc(n, 1);
+    ++g_pins;
+    ++g_pinned;
+    return hipSuccess;
+}
+hipError_t hipHostFree(void* p)
+{
+    std::free(p);
+    ++g_frees;
+    --g_pinned;
+    return hipSuccess;
+}
+hipError_t hipSetDevice(int dev) { g_dev = dev; return hipSuccess; }
+hipError_t hipGetDevice(int* dev) { *dev = g_dev; return hipSuccess; }
+}
 
 static void fail(const char* what, int line)
 {
@@ -227,12 +252,80 @@ static void strip_lists()
     EXPECT(longest > 1024);
 }
 
+// ---------------------------------------------------------------------------
+// the pinned stages of downloads and drop-in calls
+// ---------------------------------------------------------------------------
+static void stages()
+{
+    g_pin_on = true;
+    const int nx = 40, ny = 30;
+    const tmk_params p = params(nx, ny, 25.0);
+    const tmk_box v = box(0, 0, nx - 1, ny - 1), ub = box(-4, -4, nx + 3, ny + 3), bb = box(-4, 0, nx + 3, 0);
+    const size_t nU = (size_t)(nx + 8) * (ny + 8) * TMK_NCOMP, nB = (size_t)(nx + 8) * TMK_NBDRY_SW;
+    auto calls = [&](int dev, int precision) {
+        EXPECT(hipSetDevice(dev) == hipSuccess);
+        tmk_ctx* c = nullptr;
+        tmk_level* L = nullptr;
+        EXPECT(tmk_ctx_create(&c, &p, precision) == TMK_OK);
+        EXPECT(tmk_level_create(c, 1, &v, &L) == TMK_OK);
+        std::vector<double> U(nU, 0.0), B(nB, 0.0);
+        double mws = 0.0;
+        for (int k = 0; k < 20; ++k) {
+            EXPECT(tmk_level_download(L, 0, U.data(), B.data()) == TMK_OK);
+            std::fill(U.begin(), U.end(), 0.0);
+            (void)tmk_patch_update_state_noalloc(c, v, U.data(), ub, TMK_NCOMP, nullptr, nullptr, B.data(), bb,
+                                                 TMK_NBDRY_SW, 0.0, 1e-3, &mws);
+        }
+        EXPECT(tmk_level_destroy(L) == TMK_OK);
+        EXPECT(tmk_ctx_destroy(c) == TMK_OK);
+    };
+    // ten devices from one process: each context leaves its device an idle stage, and none is made or freed again
+    for (int round = 0; round < 2; ++round)
+        for (int dev = 0; dev < 10; ++dev) {
+            calls(dev, dev % 2 ? TMK_PREC_FP64 : TMK_PREC_FP32_BULK);
+            EXPECT(stage_pool().idle[dev] != nullptr);
+            EXPECT(g_pins == (round ? 10 : dev + 1) && g_frees == 0);
+        }
+    // forty readers of one device at once: at most STAGE_MOST stages of it, none freed
+    std::vector<std::thread> th;
+    std::atomic<int> ready{0};
+    for (int t = 0; t < 40; ++t)
+        th.emplace_back([&, t] {
+            ++ready;
+            while (ready < 40) std::this_thread::yield();
+            calls(3, t % 2 ? TMK_PREC_FP64 : TMK_PREC_FP32_BULK);
+        });
+    for (std::thread& t : th) t.join();
+    EXPECT(g_pins <= 9 + STAGE_MOST && g_frees == 0 && stage_pool().live[3] <= STAGE_MOST);
+    // all stages of a device in use: calls copy, and pin nothing
+    EXPECT(hipSetDevice(2) == hipSuccess);
+    std::vector<HostStage*> held;
+    while (HostStage* S = stage_take()) held.push_back(S);
+    EXPECT(held.size() == (size_t)STAGE_MOST);
+    const int pins = g_pins;
+    calls(2, TMK_PREC_FP64);
+    calls(2, TMK_PREC_FP32_BULK);
+    EXPECT(g_pins == pins && g_frees == 0);
+    for (HostStage* S : held) stage_give(S);
+    // trimming frees the current device's, no other's
+    const int before = g_pinned;
+    EXPECT(tmk_cache_trim() == TMK_OK);
+    EXPECT(g_pinned == before - STAGE_MOST && !stage_pool().idle[2] && stage_pool().live[2] == 0);
+    EXPECT(stage_pool().idle[1] && stage_pool().idle[3]);
+    for (int dev = 0; dev < 10; ++dev) {
+        EXPECT(hipSetDevice(dev) == hipSuccess);
+        EXPECT(tmk_cache_trim() == TMK_OK);
+    }
+    EXPECT(g_pinned == 0);
+}
+
 int main(int argc, char** argv)
 {
     const char* const what = argc > 1 ? argv[1] : "";
     if (!strcmp(what, "registers")) registers();
     else if (!strcmp(what, "scratch_limit")) scratch_limit();
     else if (!strcmp(what, "strip_lists")) strip_lists();
+    else if (!strcmp(what, "stages")) stages();
     else fail("no such check", __LINE__);
     printf("%s ok\n", what);
     return 0;

@@ -93,3 +93,23 @@ def test_drop_in_call_through_a_stage_and_by_copies(valid, flux, precision):
     ctx.close()
     for a, b in zip(*got):
         assert a is None and b is None or np.array_equal(a, b) and not np.isnan(a).any()
+
+
+def test_more_readers_than_pinned_buffers():
+    """24 readers at once on one device, which has 16 pinned buffers: those that find none copy through
+    device memory (1 and 2 such pieces), with the same values."""
+    n = 24
+    got = [None] * n
+    start = threading.Barrier(n)
+
+    def run(t):
+        precision = capi.PREC_FP64 if t % 2 else capi.PREC_FP32_BULK
+        start.wait()
+        got[t] = all(_check(90 + 11 * t, 70 + 7 * t, precision, seed=t + 1) for _ in range(3))
+
+    th = [threading.Thread(target=run, args=(t,)) for t in range(n)]
+    for t in th:
+        t.start()
+    for t in th:
+        t.join()
+    assert got == [True] * n

@@ -16,6 +16,7 @@
 #include <functional>
 #include <initializer_list>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <new>
 #include <system_error>
@@ -214,9 +215,10 @@ static void dev_free(void* p)
 }
 
 // Pinned host memory that kernels write results of a level into, STAGE_SLOTS slots with an event each,
-// for one reader at a time.  Contexts come and go, and pinning takes milliseconds: up to STAGE_KEEP
-// idle stages per process (8 MiB each) wait for the next reader; tmk_cache_trim frees the current
-// device's.
+// for one reader at a time.  Contexts come and go, and pinning takes milliseconds: a stage (8 MiB) stays
+// for the next reader until tmk_cache_trim frees the current device's idle ones.  A device has at most
+// STAGE_MOST, idle and in use; a reader that finds them all in use copies without one, so no call pins or
+// frees over and over, however many threads read or devices a process drives.
 // Weak references: the host-only sanitizer build links a stand-in of the HIP runtime without these
 // calls, and takes the path of a machine that has no pinned memory left.
 extern "C" {
@@ -224,17 +226,19 @@ hipError_t hipHostMalloc(void** p, size_t n, unsigned flags) __attribute__((weak
 hipError_t hipHostFree(void* p) __attribute__((weak));
 hipError_t hipSetDevice(int dev) __attribute__((weak));
 }
-constexpr int STAGE_SLOTS = 8, STAGE_KEEP = 4;
+constexpr int STAGE_SLOTS = 8, STAGE_MOST = 16, STAGE_DEVICES = 64;
 constexpr size_t STAGE_SLOT = (size_t)1 << 20;
 struct HostStage {
     int dev = 0;
     char* p = nullptr;
     hipEvent_t ev[STAGE_SLOTS] = {};
+    HostStage* next = nullptr;  // in the pool's list
     char* slot(int k) const { return p + STAGE_SLOT * (size_t)k; }
 };
 struct StagePool {
     std::mutex mu;
-    std::vector<HostStage*> idle;
+    HostStage* idle[STAGE_DEVICES] = {};
+    int live[STAGE_DEVICES] = {};  // idle and in use
 };
 static StagePool& stage_pool()
 {
@@ -256,28 +260,30 @@ static HostStage* stage_take(bool may_pin = true)
 {
     int dev = 0;
     hipError_t (*pin)(void**, size_t, unsigned) = hipHostMalloc;
-    if (!pin || hipGetDevice(&dev) != hipSuccess) return nullptr;
+    if (!pin || hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= STAGE_DEVICES) return nullptr;
     StagePool& C = stage_pool();
     {
         std::lock_guard<std::mutex> lk(C.mu);
-        for (size_t k = 0; k < C.idle.size(); ++k)
-            if (C.idle[k]->dev == dev) {
-                HostStage* S = C.idle[k];
-                C.idle.erase(C.idle.begin() + (long)k);
-                return S;
-            }
+        if (HostStage* S = C.idle[dev]) {
+            C.idle[dev] = S->next;
+            return S;
+        }
+        if (!may_pin || C.live[dev] >= STAGE_MOST) return nullptr;
+        ++C.live[dev];
     }
-    if (!may_pin) return nullptr;
     HostStage* S = new (std::nothrow) HostStage;
-    if (!S) return nullptr;
-    S->dev = dev;
-    bool ok = pin((void**)&S->p, STAGE_SLOT * STAGE_SLOTS, hipHostMallocDefault) == hipSuccess;
-    if (!ok) S->p = nullptr;
-    for (hipEvent_t& e : S->ev)
-        if (ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) { e = nullptr; ok = false; }
+    bool ok = S && pin((void**)&S->p, STAGE_SLOT * STAGE_SLOTS, hipHostMallocDefault) == hipSuccess;
+    if (S) {
+        S->dev = dev;
+        if (!ok) S->p = nullptr;
+        for (hipEvent_t& e : S->ev)
+            if (ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) { e = nullptr; ok = false; }
+    }
     if (ok) return S;
     (void)hipGetLastError();
-    stage_free(S);
+    if (S) stage_free(S);
+    std::lock_guard<std::mutex> lk(C.mu);
+    --C.live[dev];
     return nullptr;
 }
 
@@ -286,29 +292,26 @@ static void stage_give(HostStage* S)
 {
     if (!S) return;
     StagePool& C = stage_pool();
-    {
-        std::lock_guard<std::mutex> lk(C.mu);
-        if (C.idle.size() < (size_t)STAGE_KEEP) {
-            C.idle.push_back(S);
-            return;
-        }
-    }
-    stage_free(S);
+    std::lock_guard<std::mutex> lk(C.mu);
+    S->next = C.idle[S->dev];
+    C.idle[S->dev] = S;
 }
 
 static void stage_trim(int dev)
 {
+    if (dev < 0 || dev >= STAGE_DEVICES) return;
     StagePool& C = stage_pool();
-    std::vector<HostStage*> drop;
+    HostStage* drop = nullptr;
     {
         std::lock_guard<std::mutex> lk(C.mu);
-        for (size_t k = C.idle.size(); k-- > 0;)
-            if (C.idle[k]->dev == dev) {
-                drop.push_back(C.idle[k]);
-                C.idle.erase(C.idle.begin() + (long)k);
-            }
+        std::swap(drop, C.idle[dev]);
+        for (HostStage* S = drop; S; S = S->next) --C.live[dev];
     }
-    for (HostStage* S : drop) stage_free(S);
+    while (drop) {
+        HostStage* S = drop;
+        drop = S->next;
+        stage_free(S);
+    }
 }
 
 // A DevBuf's block comes from the block cache; it grows or goes back only when no queued work
@@ -2544,14 +2547,19 @@ static int level_get_box(tmk_level* L, int b, double* U, hipStream_t st)
     HIPCHK(hipGetDevice(&R.dev));
     R.S = stage_take();
     int e = TMK_OK;
-    if (!R.S) {  // no pinned memory: a piece at a time through device memory
-        std::vector<T> tmp(std::min(R.piece, R.total));
-        if ((e = c->bufs[7].ensure(tmp.size() * sizeof(T)))) return e;
+    if (!R.S) {  // none to be had: through device memory, a stage's bytes at a time
+        R.piece *= STAGE_SLOTS;
+        R.npieces = (R.total + R.piece - 1) / R.piece;
+        constexpr bool direct = sizeof(T) == sizeof(double);
+        const size_t most = std::min(R.piece, R.total);
+        std::unique_ptr<T[]> tmp(direct ? nullptr : new (std::nothrow) T[most]);
+        if (!direct && !tmp) return TMK_E_NOMEM;
+        if ((e = c->bufs[7].ensure(most * sizeof(T)))) return e;
         for (size_t k = 0; k < R.npieces; ++k) {
             if ((e = box_piece_start<T>(R, k, (T*)c->bufs[7].p))) return e;
-            HIPCHK(copy_on(st, tmp.data(), c->bufs[7].p, std::min(R.piece, R.total - k * R.piece) * sizeof(T),
-                           hipMemcpyDeviceToHost));
-            box_piece_end<T>(R, k, tmp.data());
+            T* const to = direct ? (T*)(U + k * R.piece) : tmp.get();
+            HIPCHK(copy_on(st, to, c->bufs[7].p, std::min(R.piece, R.total - k * R.piece) * sizeof(T), hipMemcpyDeviceToHost));
+            if (!direct) box_piece_end<T>(R, k, to);
         }
         return TMK_OK;
     }
