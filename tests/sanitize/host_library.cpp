@@ -319,6 +319,29 @@ static void stages()
     EXPECT(g_pinned == 0);
 }
 
+// ---------------------------------------------------------------------------
+// device memory that an upload stages through
+// ---------------------------------------------------------------------------
+static void upload_staging()
+{
+    const int nx = 50, ny = 40;
+    const tmk_params p = params(nx, ny, 25.0);
+    const tmk_box v = box(0, 0, nx - 1, ny - 1);
+    const size_t nU = (size_t)(nx + 8) * (ny + 8) * TMK_NCOMP, nB = (size_t)(nx + 8) * TMK_NBDRY_SW;
+    for (int prec : {TMK_PREC_FP64, TMK_PREC_FP32_BULK}) {
+        tmk_ctx* c = nullptr;
+        tmk_level* L = nullptr;
+        EXPECT(tmk_ctx_create(&c, &p, prec) == TMK_OK);
+        EXPECT(tmk_level_create(c, 1, &v, &L) == TMK_OK);
+        std::vector<double> U(nU, 0.0), B(nB, 0.0);
+        EXPECT(tmk_level_upload(L, 0, U.data(), B.data()) == TMK_OK);
+        // no more than the box's planes in the level's own type
+        EXPECT(c->bufs[7].n == nU * (prec == TMK_PREC_FP64 ? sizeof(double) : sizeof(float)));
+        EXPECT(tmk_level_destroy(L) == TMK_OK);
+        EXPECT(tmk_ctx_destroy(c) == TMK_OK);
+    }
+}
+
 int main(int argc, char** argv)
 {
     const char* const what = argc > 1 ? argv[1] : "";
@@ -326,6 +349,7 @@ int main(int argc, char** argv)
     else if (!strcmp(what, "scratch_limit")) scratch_limit();
     else if (!strcmp(what, "strip_lists")) strip_lists();
     else if (!strcmp(what, "stages")) stages();
+    else if (!strcmp(what, "upload_staging")) upload_staging();
     else fail("no such check", __LINE__);
     printf("%s ok\n", what);
     return 0;

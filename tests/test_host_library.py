@@ -10,6 +10,7 @@ its limit.
 strip_lists: the strips and boundary pieces of every FP64 box that call takes fit its list.
 stages: the pinned buffers of downloads and drop-in calls: bounded for each device, never pinned and freed
 over and over, by ten devices or forty readers, and none needed.
+upload_staging: an upload takes no more device memory than the box's planes in the level's type.
 """
 import os
 import shutil
@@ -29,7 +30,7 @@ def driver():
     return os.path.join(HERE, "_build", "host_library")
 
 
-@pytest.mark.parametrize("check", ["registers", "scratch_limit", "strip_lists", "stages"])
+@pytest.mark.parametrize("check", ["registers", "scratch_limit", "strip_lists", "stages", "upload_staging"])
 def test_host_library(driver, check):
     r = subprocess.run([driver, check], cwd=HERE, capture_output=True, text=True, timeout=300)
     assert r.returncode == 0 and check + " ok" in r.stdout, r.stdout[-4000:] + r.stderr[-8000:]
