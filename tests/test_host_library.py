@@ -11,6 +11,8 @@ strip_lists: the strips and boundary pieces of every FP64 box that call takes fi
 stages: the pinned buffers of downloads and drop-in calls: bounded for each device, never pinned and freed
 over and over, by ten devices or forty readers, and none needed.
 upload_staging: an upload takes no more device memory than the box's planes in the level's type.
+reader_threads: a download whose threads cannot be started for want of host memory carries its pieces on
+by itself.
 """
 import os
 import shutil
@@ -30,7 +32,7 @@ def driver():
     return os.path.join(HERE, "_build", "host_library")
 
 
-@pytest.mark.parametrize("check", ["registers", "scratch_limit", "strip_lists", "stages", "upload_staging"])
+@pytest.mark.parametrize("check", ["registers", "scratch_limit", "strip_lists", "stages", "upload_staging", "reader_threads"])
 def test_host_library(driver, check):
     r = subprocess.run([driver, check], cwd=HERE, capture_output=True, text=True, timeout=300)
     assert r.returncode == 0 and check + " ok" in r.stdout, r.stdout[-4000:] + r.stderr[-8000:]

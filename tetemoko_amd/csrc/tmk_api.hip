@@ -13,13 +13,13 @@
 #include <cstdint>
 #include <cstdio>
 #include <cstring>
+#include <exception>
 #include <functional>
 #include <initializer_list>
 #include <map>
 #include <memory>
 #include <mutex>
 #include <new>
-#include <system_error>
 #include <thread>
 #include <unordered_map>
 #include <vector>
@@ -2574,7 +2574,7 @@ static int level_get_box(tmk_level* L, int b, double* U, hipStream_t st)
         try {
             th[t] = std::thread([&R, &es, t] { es[t] = box_read_share<T>(R, t); });
             on[t] = true;
-        } catch (const std::system_error&) {  // no more threads: this one takes the share
+        } catch (const std::exception&) {  // no more threads, or no memory for one: this one takes the share
         }
     }
     for (int t = 0; t < R.nthreads; ++t)
