@@ -366,7 +366,10 @@ int tmk_set_march(tmk_ctx *ctx, int rows);
 /* A level's own update shape (no reference counterpart; levels start with their context's):
  * march_rows as tmk_set_march, (bx, by) as tmk_set_tile.  Not while the level is in a batch or
  * hierarchy; members of one batch or hierarchy level need equal shapes.  get reports the
- * shape the update runs (march_rows 0 where the numerics keep the tile kernels). */
+ * shape the update runs (march_rows 0 where the numerics keep the tile kernels); for a level
+ * that has set no height, the one its own launches take.  Such a level joins others that have
+ * set none, the nominal 32 rows and the height it takes alone; a launch with a member that has
+ * set one takes that member's, else one that suits all its members' sizes. */
 int tmk_level_set_update_shape(tmk_level *lev, int march_rows, int bx, int by);
 int tmk_level_get_update_shape(const tmk_level *lev, int *march_rows, int *bx, int *by);
 /* The order of a level's interior workgroups (no reference counterpart, whose box loop is

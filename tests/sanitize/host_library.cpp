@@ -389,6 +389,57 @@ static void reader_threads()
     EXPECT(tmk_cache_trim() == TMK_OK);
 }
 
+// ---------------------------------------------------------------------------
+// strip heights: what a level reports is what its launches take, alone and in a batch
+// ---------------------------------------------------------------------------
+static void strip_heights()
+{
+    const int sizes[][2] = {{60, 40}, {261, 131}, {300, 150}, {1021, 509}, {1500, 750}, {4096, 2048}};
+    for (int prec : {TMK_PREC_FP64, TMK_PREC_FP32_BULK}) {
+        bool other = false;  // some level takes another height than the nominal one
+        for (const auto& n : sizes) {
+            const tmk_params p = params(n[0], n[1], 25.0);
+            const tmk_box v = box(0, 0, n[0] - 1, n[1] - 1);
+            tmk_ctx* c = nullptr;
+            EXPECT(tmk_ctx_create(&c, &p, prec) == TMK_OK);
+            tmk_level* L[3] = {};
+            for (tmk_level*& l : L) {
+                EXPECT(tmk_level_create(c, 1, &v, &l) == TMK_OK);
+                if (n[0] == 4096) break;  // (one is large enough)
+            }
+            int rows = 0, bx = 0, by = 0, r2 = 0, x2 = 0, y2 = 0;
+            EXPECT(tmk_level_get_update_shape(L[0], &rows, &bx, &by) == TMK_OK);
+            EXPECT(group_build(L[0]->own, {L[0]}, {0}, 1) == TMK_OK);
+            EXPECT(L[0]->own.march == rows);
+            other = other || rows != 32;
+            if (L[1]) {
+                // the shape of one level set on another: the same launches, and the two share them; so does
+                // the nominal height, and no other
+                EXPECT(tmk_level_set_update_shape(L[1], rows, bx, by) == TMK_OK);
+                EXPECT(tmk_level_get_update_shape(L[1], &r2, &x2, &y2) == TMK_OK);
+                EXPECT(r2 == rows && x2 == bx && y2 == by);
+                for (int set : {rows, 32, 20}) {
+                    EXPECT(tmk_level_set_update_shape(L[2], set, bx, by) == TMK_OK);
+                    for (int first : {0, 2}) {
+                        tmk_batch* B = nullptr;
+                        EXPECT(tmk_batch_create(&B) == TMK_OK);
+                        EXPECT(tmk_batch_add(B, L[first], 0.0, 1e-3) == TMK_OK);
+                        const int e = tmk_batch_add(B, L[2 - first], 0.0, 1e-3);
+                        EXPECT(e == (set == 20 && rows != 20 ? TMK_E_ARG : TMK_OK));
+                        EXPECT(tmk_batch_run(B, 1) == TMK_OK);
+                        EXPECT(B->grp.march == (e == TMK_OK ? set : first ? set : rows));
+                        EXPECT(tmk_batch_destroy(B) == TMK_OK);
+                    }
+                }
+            }
+            for (tmk_level* l : L)
+                if (l) EXPECT(tmk_level_destroy(l) == TMK_OK);
+            EXPECT(tmk_ctx_destroy(c) == TMK_OK);
+        }
+        EXPECT(other);
+    }
+}
+
 int main(int argc, char** argv)
 {
     const char* const what = argc > 1 ? argv[1] : "";
@@ -398,6 +449,7 @@ int main(int argc, char** argv)
     else if (!strcmp(what, "stages")) stages();
     else if (!strcmp(what, "upload_staging")) upload_staging();
     else if (!strcmp(what, "reader_threads")) reader_threads();
+    else if (!strcmp(what, "strip_heights")) strip_heights();
     else fail("no such check", __LINE__);
     printf("%s ok\n", what);
     return 0;

@@ -13,6 +13,8 @@ over and over, by ten devices or forty readers, and none needed.
 upload_staging: an upload takes no more device memory than the box's planes in the level's type.
 reader_threads: a download whose threads cannot be started for want of host memory carries its pieces on
 by itself.
+strip_heights: the height a level reports is the one its launches take, and levels that report the same
+share launches.
 """
 import os
 import shutil
@@ -32,7 +34,7 @@ def driver():
     return os.path.join(HERE, "_build", "host_library")
 
 
-@pytest.mark.parametrize("check", ["registers", "scratch_limit", "strip_lists", "stages", "upload_staging", "reader_threads"])
+@pytest.mark.parametrize("check", ["registers", "scratch_limit", "strip_lists", "stages", "upload_staging", "reader_threads", "strip_heights"])
 def test_host_library(driver, check):
     r = subprocess.run([driver, check], cwd=HERE, capture_output=True, text=True, timeout=300)
     assert r.returncode == 0 and check + " ok" in r.stdout, r.stdout[-4000:] + r.stderr[-8000:]

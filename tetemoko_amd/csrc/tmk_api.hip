@@ -1326,9 +1326,10 @@ static int group_build_t(Group& G, const std::vector<tmk_level*>& mem, const std
         // strips of levels with flux registers hold at most 63 rows (the kernel's face masks)
         for (const Patch<T>& p : pts[0]) fluxes = fluxes || p.F[0] || p.F[1];
         auto params = [&](const Tile& t) -> const DevParams& { return sc[patch_scen[t.patch]].P; };
-        bool chosen = false;  // some member's level has a height of its own
-        for (tmk_level* L : mem) chosen = chosen || !L->march_auto;
-        if (!chosen) G.march = march_height(tiles, params, sizeof(T) == sizeof(float));
+        const tmk_level* set = nullptr;  // a member whose level has a height of its own
+        for (const tmk_level* L : mem)
+            if (!set && !L->march_auto) set = L;
+        G.march = set ? set->march : march_height(tiles, params, sizeof(T) == sizeof(float));
         const int rows = fluxes ? std::min(G.march, 63) : G.march;
         for (const Tile& r : tiles) march_rect(r, params(r), rows, strips, bf, bo);
         if (G.xcd) xcd_order(strips, STEP_WAVES / 2);
@@ -3021,11 +3022,29 @@ extern "C" int tmk_level_set_tile_order(tmk_level* L, int xcd)
     return TMK_OK;
 }
 
+// the strip height of the level's own launches (0: the tile kernels)
+static int level_march_rows(const tmk_level* L)
+{
+    if (L->march <= 0 || L->ns != 2 || pred_kind(L->ctx->P) != PK_PPM_PRIM) return 0;
+    if (!L->march_auto) return L->march;
+    return march_height(L->urects, [L](const Tile&) -> const DevParams& { return L->ctx->P; },
+                        L->tsize == sizeof(float));
+}
+
+// whether levels a and b may share launches by their strip heights: equal ones, or a's and b's both left to
+// the launch; one that is left to it also joins the nominal height and the one it takes alone
+static bool same_march(const tmk_level* a, const tmk_level* b)
+{
+    if (a->march == b->march) return true;
+    if (a->march_auto == b->march_auto) return false;
+    const tmk_level *set = a->march_auto ? b : a, *free = a->march_auto ? a : b;
+    return set->march > 0 && set->march == level_march_rows(free);
+}
+
 extern "C" int tmk_level_get_update_shape(const tmk_level* L, int* march_rows, int* bx, int* by)
 {
     if (!L || !march_rows || !bx || !by) return TMK_E_ARG;
-    const bool m = L->march > 0 && L->ns == 2 && pred_kind(L->ctx->P) == PK_PPM_PRIM;
-    *march_rows = m ? L->march : 0;
+    *march_rows = level_march_rows(L);
     *bx = L->bx;
     *by = L->by;
     return TMK_OK;
@@ -3242,8 +3261,9 @@ extern "C" int tmk_batch_add(tmk_batch* B, tmk_level* L, double time, double dt)
     if (!B || !L || L->batch || L->amr_stream) return TMK_E_ARG;
     if (!B->members.empty()) {
         tmk_level* L0 = B->members[0];
-        if (L0->tsize != L->tsize || L0->ns != L->ns || L0->bx != L->bx || L0->by != L->by || L0->march != L->march)
-            return TMK_E_ARG;
+        if (L0->tsize != L->tsize || L0->ns != L->ns || L0->bx != L->bx || L0->by != L->by) return TMK_E_ARG;
+        for (const tmk_level* M : B->members)
+            if (!same_march(M, L)) return TMK_E_ARG;
     }
     HIPCHK(hipStreamSynchronize(L->ctx->stream));
     int e = batch_detach_all(B);
@@ -4082,8 +4102,9 @@ extern "C" int tmk_amr_add(tmk_amr* A, tmk_level* const* levels, double time, do
         for (int l = 0; l < A->nlev; ++l) {
             const tmk_level* a = A->mem[0]->L[l];
             const tmk_level* b = levels[l];
-            if (a->tsize != b->tsize || a->ns != b->ns || a->bx != b->bx || a->by != b->by || a->march != b->march)
-                return TMK_E_ARG;
+            if (a->tsize != b->tsize || a->ns != b->ns || a->bx != b->bx || a->by != b->by) return TMK_E_ARG;
+            for (const AmrMember* M : A->mem)
+                if (!same_march(M->L[l], b)) return TMK_E_ARG;
         }
     }
     {   // level 0 covers its domain
