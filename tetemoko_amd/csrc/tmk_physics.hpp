@@ -817,7 +817,7 @@ __device__ __forceinline__ void rs_fault(const DevParams& P, const FaultFace& f,
     const double phi_yz = 0.5 * (wpyz2 - wpyz1) + tau_yz_0;
     const double phi = sqrt(phi_xy * phi_xy + phi_yz * phi_yz);
     const double syy = -((wpyy1 - wpyy2) / 2.0);
-    const double vy = -divr((wpyy1 + wpyy2) / 2.0, Zp, P.iZp);
+    const double vy = -((wpyy1 + wpyy2) / 2.0 / Zp);
     const double dvx = in.vx[0] - in.vx[1], dvz = in.vz[0] - in.vz[1];
     double V = sqrt(dvx * dvx + dvz * dvz);
     double sn = -syy;
@@ -827,8 +827,8 @@ __device__ __forceinline__ void rs_fault(const DevParams& P, const FaultFace& f,
     const double syz = (phi_yz / phi) * tau - tau_yz_0;
     const double Vx = (phi_xy / phi) * V;
     const double Vz = (phi_yz / phi) * V;
-    const double vx1 = -divr(sxy + wpxy1, Zs, P.iZs);
-    const double vz1 = -divr(syz + wpyz1, Zs, P.iZs);
+    const double vx1 = -((sxy + wpxy1) / Zs);
+    const double vz1 = -((syz + wpyz1) / Zs);
     o.vx[0] = vx1; o.vy[0] = vy; o.vz[0] = vz1; o.syy[0] = syy; o.sxy[0] = sxy; o.syz[0] = syz;
     o.vx[1] = vx1 - Vx; o.vy[1] = vy; o.vz[1] = vz1 - Vz; o.syy[1] = syy; o.sxy[1] = sxy; o.syz[1] = syz;
 }
@@ -868,7 +868,7 @@ __device__ __forceinline__ void sw_fault(const DevParams& P, int i, const FaultF
     const double tb = 0.5 * (wpyz2 - wpyz1);
     const double tau_lock = sqrt(ta * ta + tb * tb);
     const double syy = -((wpyy1 - wpyy2) / 2.0);
-    const double vy = -divr((wpyy1 + wpyy2) / 2.0, Zp, P.iZp);
+    const double vy = -((wpyy1 + wpyy2) / 2.0 / Zp);
     const double valx = (fabs(x) >= P.fric_w0) ? 0.0 : 1.0;
     double fric = f.a * valx + (1.0 - valx) * P.outside_f;
     fric = fric - (fric - f.b) * fmin(1.0, slip / f.L);
@@ -880,11 +880,11 @@ __device__ __forceinline__ void sw_fault(const DevParams& P, int i, const FaultF
     const double phi = sqrt(phi_xy * phi_xy + phi_yz * phi_yz);
     const double sxy = (phi_xy / phi) * tau;
     const double syz = (phi_yz / phi) * tau;
-    o.vx[0] = -divr(sxy + wpxy1, Zs, P.iZs);
-    o.vz[0] = -divr(syz + wpyz1, Zs, P.iZs);
+    o.vx[0] = -((sxy + wpxy1) / Zs);
+    o.vz[0] = -((syz + wpyz1) / Zs);
     o.vy[0] = vy; o.syy[0] = syy; o.sxy[0] = sxy; o.syz[0] = syz;
-    o.vx[1] = divr(sxy - wpxy2, Zs, P.iZs);
-    o.vz[1] = divr(syz - wpyz2, Zs, P.iZs);
+    o.vx[1] = (sxy - wpxy2) / Zs;
+    o.vz[1] = (syz - wpyz2) / Zs;
     o.vy[1] = vy; o.syy[1] = syy; o.sxy[1] = sxy; o.syz[1] = syz;
 }
 
