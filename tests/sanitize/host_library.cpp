@@ -440,6 +440,39 @@ static void strip_heights()
     }
 }
 
+// ---------------------------------------------------------------------------
+// divisions in two operations: what the host decides for a divisor, and what the functions give
+// ---------------------------------------------------------------------------
+// stdin: lines "div B N x1 .. xN" -> "flag yh yl, then divr2(x) divr(x) each"; "par cs cp G" -> the material's
+// flag, rho Zp Zs and their low words; "third N x1 .. xN" -> div3(x) div6(x) each; hexadecimal floats
+static void division()
+{
+    char kind[16];
+    while (scanf("%15s", kind) == 1) {
+        if (!strcmp(kind, "div")) {
+            double b;
+            int n;
+            EXPECT(scanf("%la %d", &b, &n) == 2);
+            const double y = 1.0 / b, yl = recip_low(b, y);
+            printf("%d %a %a", (int)div2_exact(b), y, yl);
+            for (double x; n > 0 && scanf("%la", &x) == 1; --n) printf(" %a %a", divr2(x, y, yl), divr(x, b, y));
+        } else if (!strcmp(kind, "par")) {
+            tmk_params p = params(32, 32, 1.0);
+            EXPECT(scanf("%la %la %la", &p.cs, &p.cp, &p.G) == 3);
+            DevParams P;
+            fill_dev_params(p, P);
+            printf("%d %a %a %a %a %a %a", P.div2, P.rho, P.Zp, P.Zs, P.lrho, P.l2Zp, P.l2Zs);
+        } else if (!strcmp(kind, "third")) {
+            int n;
+            EXPECT(scanf("%d", &n) == 1);
+            for (double x; n > 0 && scanf("%la", &x) == 1; --n) printf("%a %a ", div3(x), div6(x));
+        } else {
+            fail("division: no such line", __LINE__);
+        }
+        printf("\n");
+    }
+}
+
 int main(int argc, char** argv)
 {
     const char* const what = argc > 1 ? argv[1] : "";
@@ -450,6 +483,7 @@ int main(int argc, char** argv)
     else if (!strcmp(what, "upload_staging")) upload_staging();
     else if (!strcmp(what, "reader_threads")) reader_threads();
     else if (!strcmp(what, "strip_heights")) strip_heights();
+    else if (!strcmp(what, "division")) division();
     else fail("no such check", __LINE__);
     printf("%s ok\n", what);
     return 0;

@@ -784,7 +784,8 @@ extern "C" int tmk_cache_trim(void)
 // RN(1/b - y) for y = RN(1/b): the remainder 1 - b y is exact in one fma
 static double recip_low(double b, double y) { return std::fma(-b, y, 1.0) / b; }
 
-// whether divr2 by b gives the IEEE quotient for every dividend.  With b and the dividend scaled to
+// whether divr2 by b gives the IEEE quotient for every finite dividend whose product with the low word is
+// normal.  With b and the dividend scaled to
 // 53-bit integers Y, X and the quotient next to the midpoint (2Q + 1) / 2^p (p = 53 for X >= Y, else 54),
 // 2^p X - (2Q + 1) Y = N is a nonzero integer, and the sum under divr2's last rounding, within 2^-105 of
 // a / b, can lie on the other side of the midpoint only if |N| <= 2^(p-105) X < 4.  For each such N

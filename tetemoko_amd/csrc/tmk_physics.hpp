@@ -133,7 +133,7 @@ struct Slots {
 // in one fma.  copysign keeps the sign of a zero dividend.  The result equals the IEEE quotient
 // bit for bit, at five fma/mul instead of the 10-instruction scaled division sequence.
 // FP32 (bulk arithmetic of the reduced-precision mode): a y, within 1.5 ulps.
-__device__ __forceinline__ double divr(double a, double b, double y)
+__host__ __device__ __forceinline__ double divr(double a, double b, double y)
 {
     double q = a * y;
     double r = fma(-q, b, a);
@@ -157,13 +157,16 @@ __device__ __forceinline__ T pick(double d, float f)
 // The sum under the last rounding is a / b to within 2^-105, so the result is the IEEE quotient
 // unless a / b lies that close to a midpoint of two floating-point numbers, which for a given b a few
 // dividends at most do (Brisebarre, Muller and Raina, IEEE Trans. Comput. 53 (2004) 1069-1072);
-// div2_exact tries those on the host, and constants that fail keep divr.  Two operations for six
-// (divr and its copysign): the sign of a zero dividend comes out by itself.  A cell side of the FP64
+// div2_exact tries those on the host, and constants that fail keep divr.  That holds for finite dividends
+// whose a yl is a normal number, |a| above 1e-289 for the impedances and densities of rock; below, the low
+// word loses bits and the result may be an ulp off (divr's remainder does there too), and an infinite
+// dividend gives infinity or NaN (divr: NaN).  Two operations for six (divr and its copysign): the sign of a
+// zero dividend comes out by itself where yl is positive.  A cell side of the FP64
 // march divides 28 times; with the flux of a face computed once (march_strip) the 4096 x 2048 level
 // went from 522 to 461 us per step without plasticity and from 640 to 577 with it.  Halvings folded into
 // fmas and divisors, half slopes and the plastic return's early way out (div3, plastic_flow) took it on
 // from 505 to 480 with its reads (60 steps 30.3 -> 28.8 ms), 8192 x 4096 plastic from 2.42 to 2.33 ms.
-__device__ __forceinline__ double divr2(double a, double yh, double yl) { return fma(a, yh, a * yl); }
+__host__ __device__ __forceinline__ double divr2(double a, double yh, double yl) { return fma(a, yh, a * yl); }
 
 // elastic constants in the bulk arithmetic type.  D2 (FP64): the constants divide by divr2.
 template <typename T, bool D2 = false>
@@ -930,9 +933,9 @@ __device__ __forceinline__ double plastic_d(const DevParams& P, int k)
 __device__ __forceinline__ double plastic_d(const PlasticConstL64& P, int k) { return P.c[k]; }
 
 // x / 3 and x / 6, rounded like the division (divr2: no quotient by 3 lies near a midpoint, the gap is a
-// multiple of 2^51 in its scale; tests/test_div2.py)
-__device__ __forceinline__ double div3(double x) { return divr2(x, 1.0 / 3.0, 0x1p-54 / 3.0); }
-__device__ __forceinline__ double div6(double x) { return divr2(x, 0.5 / 3.0, 0x1p-55 / 3.0); }
+// multiple of 2^51 in its scale; tests/test_div2.py) above 1e-290; infinities and zeros keep their signs
+__host__ __device__ __forceinline__ double div3(double x) { return divr2(x, 1.0 / 3.0, 0x1p-54 / 3.0); }
+__host__ __device__ __forceinline__ double div6(double x) { return divr2(x, 0.5 / 3.0, 0x1p-55 / 3.0); }
 
 // A cell that stays well inside the yield surface, J2 < ys^2 (1 - 2^-50), is left before the root: there
 // tau = RN(sqrt(J2)) <= ys.  A row of the 8192 x 4096 level's march took the root and two divisions by
