@@ -74,7 +74,7 @@ def parse():
 
 
 def measured_traffic(workload, precision, shape):
-    """HBM bytes per launch of the interior update kernel from the committed counter runs
+    """HBM bytes per launch of the update kernel from the committed counter runs
     (profiles/traffic_*.json: FETCH_SIZE and WRITE_SIZE per dispatch, each scaled by the
     copy-kernel calibration), if one was taken on this workload, precision and update shape
     ("march32", "tile32x16", ...)."""
@@ -130,9 +130,8 @@ TUNE = True  # autotune each level's update shape before it is timed
 def timed_leg(cfg, precision, boxes, warmup, steps):
     """The level's update shape autotuned from its initial state (tmk_level_autotune: every
     strip height and tile shape timed, then the fastest with the other workgroup order, the level
-    returned to that state), then W untimed
-    graph-replayed steps, then exactly K graph-replayed steps bracketed by HIP events on the
-    level's stream (after a device synchronisation), then per-launch durations of the update
+    returned to that state), then W untimed steps, then exactly K steps bracketed by HIP events on
+    the level's stream (after a device synchronisation), then per-launch durations of the update
     kernels inside a replayed graph (stamps on each kernel's stream)."""
     ctx, lev = make_level(cfg, precision, boxes)
     dt = scenarios.dt_of(cfg)

@@ -136,7 +136,7 @@ int tmk_patch_update_state(tmk_ctx *ctx, tmk_box valid, double *U, tmk_box U_box
 /* tmk_patch_update_state with no device allocation: no counterpart in the reference.  For
  * callers that cannot allocate device memory (code under HIP graph capture, tight serving
  * loops, harnesses that forbid hipMalloc).  Same arguments, checks, results and error codes as
- * tmk_patch_update_state (the same kernels on the same tiles), but every device buffer of the
+ * tmk_patch_update_state (the same kernels; its strips may be taller), but every device buffer of the
  * call -- both state copies, the fault data, the fluxes, the FP64 staging of the FP32 bulk and the
  * launch tables -- lives in one fixed array per device, held from the first context created on
  * that device until the process ends.  TMK_E_SCRATCH when the call needs more than
@@ -181,7 +181,8 @@ int tmk_level_download_fault(tmk_level *lev, int ibox, double *B);
  * same-level ghost exchange, one launch over every box of the level, fault data
  * update.  dt_new = dx / max(cs,cp) (LinElastLevelGodunov.cpp:377). */
 int tmk_level_step(tmk_level *lev, double time, double dt, double *dt_new);
-/* nsteps level steps with time advancing by dt, captured once as a hipGraph */
+/* nsteps level steps with time advancing by dt.  A level that marches (tmk_set_march) enqueues
+ * one launch a step; on the tile kernels two steps are captured once as a hipGraph and replayed */
 int tmk_level_run(tmk_level *lev, int nsteps, double time, double dt);
 /* tmk_level_run bracketed by HIP events recorded on the level's own stream;
  * waits for completion and returns the elapsed milliseconds in *ms */
@@ -260,7 +261,7 @@ int tmk_batch_member_error(tmk_batch *b, tmk_level *lev, int *code);
  * centre): face i = floor(x/dx - 0.5), weight d = x - (i + 0.5) dx.  After every level step of
  * tmk_level_step/run the device appends one record per station -- the new time, then
  * B[i] (1 - d) + B[i+1] d for each fault-data component, the reference's expression with d in
- * metres -- inside captured step graphs as well.  capacity = records kept between reads.
+ * metres -- in captured steps as well.  capacity = records kept between reads.
  * Stations of a level that is in a batch record nothing.  A station whose face lies on no
  * fault box is TMK_E_ARG. */
 typedef struct tmk_stations tmk_stations;
@@ -356,9 +357,9 @@ int tmk_set_tile(tmk_ctx *ctx, int bx, int by);
 /* Row-marching interior update (autotuner hook; no reference counterpart: the reference updates
  * box by box, LinElastLevelGodunov.cpp:284-358).  rows > 0: levels created from this context
  * update the cells whose +-3 stencil lies inside the domain in strips of 58 columns x rows,
- * one wavefront per strip and side marching up the rows with no LDS (mode II, PPM with primitive
- * limiting; other numerics keep the tile kernels); the cells along the domain boundary run the
- * general kernel.  0 = the tile kernels of tmk_set_tile.  Results are those of the tile kernels
+ * one wavefront per strip and side marching up the rows, which come through an LDS ring of its own
+ * (mode II, PPM with primitive limiting; other numerics keep the tile kernels); the cells along the
+ * domain boundary run as boundary pieces of the same launch.  0 = the tile kernels of tmk_set_tile.  Results are those of the tile kernels
  * (bit-identical in FP64).  New contexts start at 32 rows, a nominal height: until a height is set
  * here or by tmk_level_set_update_shape, each launch takes one that suits its size. */
 int tmk_set_march(tmk_ctx *ctx, int rows);
@@ -381,7 +382,7 @@ int tmk_level_get_update_shape(const tmk_level *lev, int *march_rows, int *bx, i
 int tmk_level_set_tile_order(tmk_level *lev, int xcd);
 
 /* Autotuning of a level's update shape (no reference counterpart).  Times nsteps
- * graph-replayed steps from (time, dt), after two untimed ones, for every strip height of the
+ * steps as tmk_level_run makes them from (time, dt), after two untimed ones, for every strip height of the
  * row-marching update (4 .. 64 rows, where the numerics allow it) and every tile shape, each
  * from the level's current state, then the fastest of them with the other order of the
  * interior workgroups (tmk_level_set_tile_order); sets the fastest shape and order and returns

@@ -5,7 +5,7 @@ by default, 8-64 cells per side on refined AMR levels).  Here every box of a lev
 same two update launches, with a ghost exchange between boxes each step.  This measures the
 cost of a box layout: a 1024 x 512 rate-and-state level as one box and as boxes of 64, 32, 16
 and 8 cells per side, FP64 and FP32 bulk.  Times come from HIP events on the level's stream
-(graph-replayed steps); the per-kernel split from tmk_level_profile_kernels.
+(tmk_level_run_timed); the per-kernel split from tmk_level_profile_kernels.
 """
 import argparse
 import json

@@ -1393,7 +1393,7 @@ static int group_build(Group& G, const std::vector<tmk_level*>& mem, const std::
                                            : group_build_t<float>(G, mem, phase, plastic);
 }
 
-// the clock and step constants (Scen fields time .. fmdtdx) of member m
+// the clock and step constants (Scen fields time .. m32) of member m
 static int group_set_clock(Group& G, hipStream_t st, int m, double time, double dt, const DevParams& P)
 {
     Scen s;
@@ -2566,7 +2566,8 @@ static int level_get_box(tmk_level* L, int b, double* U, hipStream_t st)
         }
         return TMK_OK;
     }
-    // a thread costs about as long to start as half a piece to copy: one per 4 pieces, up to 4
+    // two threads from 8 pieces on, four from 16 (three would not divide the slots).  A thread costs about
+    // as long to start as half a piece to copy, so fewer pieces could pay as well: not measured
     R.nthreads = (int)std::min<size_t>(4, std::max<size_t>(1, R.npieces / 4));
     if (R.nthreads == 3) R.nthreads = 2;
     int es[4] = {TMK_OK, TMK_OK, TMK_OK, TMK_OK};

@@ -190,13 +190,14 @@ struct MarchCarry {
 // cell below (z = Z with the side's velocity sign), and everything up to it is linear in (v, s): the
 // predictor traces a and b from the limited increments, the transverse corrections add to them, and a
 // face keeps D = a - b and E = a + b, whose scales (v = D / (2 z), s = E / 2) go into the constants of
-// what reads them; final faces keep v, as the boundary pieces do that share them (MarchK32).  The limited increments come straight from the differences and half slopes, not
-// from a face value minus the cell's.  FP32 is bound by instruction issue where the level does not
-// outgrow the caches: a row without plasticity takes about 215 vector instructions for 270 in (v, s),
+// what reads them; final faces keep v, as the boundary pieces do that share them (MarchK32).  The limited
+// increments come straight from the differences and half slopes, not from a face value minus the cell's.
+// FP32 is bound by instruction issue above all where the level does not outgrow the caches (12 scenarios:
+// 67 % of the issue rate): a row without plasticity takes about 215 vector instructions for 270 in (v, s),
 // and 4 carried values fewer.  12 single-level scenarios 26.0 -> 23.6 ms for 200 steps, 1024 x 512
 // plastic 200 steps 17.3 -> 15.9 with its state read, the lens hierarchy's 12 coarse steps 60.1 ->
-// 58.3; 8192 x 4096 plastic, bound by memory, 103.5 -> 102.9.  Errors against 64 bits are the same
-// within 3 % (261 x 131, 400 steps: 1.2e-6 both; 1024 x 512, 200 steps: 1.7e-6 both).
+// 58.3; 8192 x 4096 plastic, bound by memory, 103.5 -> 102.9.  Errors against 64 bits on one set of
+// inputs, in (v, s) and now: 261 x 131, 400 steps 5.5e-7 and 5.2e-7; 1024 x 512, 200 steps 3.2e-6 and 3.1e-6.
 template <>
 struct MarchCarry<float> {
     float w1[5], w2[5], w3[5];  // as above
