@@ -45,8 +45,8 @@ struct Patch {
     int vlo0, vlo1, vhi0, vhi1; // valid box
     int scen;          // index of the scenario (parameters, time, step) this box belongs to
     // with F: per-cell flags over the valid box grown by 1 (bit 0: a cell of the level, bit 1:
-    // covered by the next finer level); NULL keeps every face, else only the faces between a
-    // cell of the level and one outside it, or between covered and uncovered cells of the level
+    // covered by the next finer level); NULL keeps every face, else only the register faces: between
+    // an uncovered cell of the level and a covered one or one outside (register_face)
     const unsigned char* fmask;
 };
 
@@ -224,19 +224,18 @@ __device__ __forceinline__ void fault_output(const DevParams& P, const FaultOut&
 // the 11 flux components of side sd from face state (v, s) on the lo d-face of cell (i, j) into
 // the flux register array of direction d (surroundingNodes(valid box, d)).  With stores_delta
 // this is the flux of U - bg: flux registers only ever difference fluxes of one precision, and
-// the drop-in path adds the background's flux (bg_flux) on the host.  lo, hi: the workgroup updates the
-// cell below / above the face (register_face; without a mask every face is stored).
+// the drop-in path adds the background's flux (bg_flux) on the host.
 // whether a workgroup stores the register flux of a face between cells with face-mask bits a (lo) and b
-// (hi); lo, hi: it updates that cell.  A face of the level's boundary (one side a cell of the level, the
-// fine side of a register) belongs to that cell, a face around the finer level (between two cells of the
-// level, one of them covered) to the uncovered one, the cell that reflux corrects.  One workgroup updates
-// that cell, so every register entry has one writer, and the flux it takes is the one the cell's own
-// update used: a strip and a boundary piece round the flux of a face between them differently in FP32,
-// and with a store by each the entry depended on their order.
+// (hi); lo, hi: it updates that cell.  A register face has an uncovered cell of the level (bits 1) on
+// one side only: outside is the coarser level (the fine side of a register; covered cells do not touch the
+// level's boundary, proper nesting) or a covered cell (the coarse side, whose uncovered cell reflux
+// corrects).  One workgroup updates that cell, so every register entry has one writer, and the flux it takes
+// is the one the cell's own update used: a strip and a boundary piece round the flux of a face between
+// them differently in FP32, and with a store by each the entry depended on their order.
 __host__ __device__ __forceinline__ bool register_face(unsigned a, unsigned b, bool lo, bool hi)
 {
-    if ((a ^ b) & 1) return (a & 1) ? lo : hi;
-    return (a & 1) && ((a ^ b) & 2) && ((a & 2) ? hi : lo);
+    const bool ua = a == 1, ub = b == 1;
+    return (ua != ub) & (ua ? lo : hi);
 }
 
 // the 11 components of side sd of the face flux in direction d at index fi of the flux array
@@ -274,28 +273,42 @@ __device__ __forceinline__ void put_face_flux(__attribute__((address_space(1))) 
     Fo[fi + (o + 10) * fp] = 0.0;
 }
 
+// whether a workgroup stores the register flux of the lo d-face of cell (i, j): lo, hi: it updates the cell
+// below / above the face (register_face); without a mask every face is stored
+template <typename T>
+__device__ __forceinline__ bool stores_flux(const Patch<T>& pt, int d, int i, int j, bool lo, bool hi)
+{
+    if (!pt.fmask) return true;
+    const int mw = pt.vhi0 - pt.vlo0 + 3;
+    const __attribute__((address_space(1))) unsigned char* mk =
+        gmem(pt.fmask) + (size_t)(i - pt.vlo0 + 1) + (size_t)(j - pt.vlo1 + 1) * mw;
+    return register_face(d == 0 ? mk[-1] : mk[-mw], *mk, lo, hi);
+}
+
 template <typename T, int NS, bool D2>
-__device__ __forceinline__ void store_flux_side(const Patch<T>& pt, const Mat<T, D2>& m, int d, const T (&v)[NS],
-                                                const T (&sv)[NS], T r, int i, int j, int sd, bool lo, bool hi)
+__device__ __forceinline__ void put_flux_side(const Patch<T>& pt, const Mat<T, D2>& m, int d, const T (&v)[NS],
+                                              const T (&sv)[NS], T r, int i, int j, int sd)
 {
     const int fnx = pt.vhi0 - pt.vlo0 + 1 + (d == 0), fny = pt.vhi1 - pt.vlo1 + 1 + (d == 1);
-    if (pt.fmask) {
-        const int mw = pt.vhi0 - pt.vlo0 + 3;
-        const __attribute__((address_space(1))) unsigned char* mk =
-            gmem(pt.fmask) + (size_t)(i - pt.vlo0 + 1) + (size_t)(j - pt.vlo1 + 1) * mw;
-        if (!register_face(d == 0 ? mk[-1] : mk[-mw], *mk, lo, hi)) return;
-    }
     const size_t fp = (size_t)fnx * fny;
     const size_t fi = (size_t)(i - pt.vlo0) + (size_t)(j - pt.vlo1) * fnx;
     put_face_flux<T, NS>(gmem(pt.F[d]), fi, fp, m, d, v, sv, r, sd);
 }
 
 template <typename T, int NS, bool D2>
+__device__ __forceinline__ void store_flux_side(const Patch<T>& pt, const Mat<T, D2>& m, int d, const T (&v)[NS],
+                                                const T (&sv)[NS], T r, int i, int j, int sd, bool lo, bool hi)
+{
+    if (stores_flux(pt, d, i, j, lo, hi)) put_flux_side<T, NS>(pt, m, d, v, sv, r, i, j, sd);
+}
+
+template <typename T, int NS, bool D2>
 __device__ __forceinline__ void store_flux(const Patch<T>& pt, const Mat<T, D2>& m, int d, const Slots<T, NS>& Fs, T rv,
                                            int i, int j, bool lo, bool hi)
 {
-    store_flux_side<T, NS>(pt, m, d, Fs.v[0], Fs.s[0], (T)1, i, j, 0, lo, hi);
-    store_flux_side<T, NS>(pt, m, d, Fs.v[1], Fs.s[1], rv, i, j, 1, lo, hi);
+    if (!stores_flux(pt, d, i, j, lo, hi)) return;
+    put_flux_side<T, NS>(pt, m, d, Fs.v[0], Fs.s[0], (T)1, i, j, 0);
+    put_flux_side<T, NS>(pt, m, d, Fs.v[1], Fs.s[1], rv, i, j, 1);
 }
 
 // face states of one side on the four faces of a cell: lo/hi x face, lo/hi y face
