@@ -10,7 +10,8 @@ its limit.
 strip_lists: the strips and boundary pieces of every FP64 box that call takes fit its list.
 stages: the pinned buffers of downloads and drop-in calls: bounded for each device, never pinned and freed
 over and over, by ten devices or forty readers, and none needed.
-upload_staging: an upload takes no more device memory than the box's planes in the level's type.
+upload_staging: an upload takes no more device memory than the box's planes in the level's type, small
+boxes aside.
 reader_threads: a download whose threads cannot be started for want of host memory carries its pieces on
 by itself.
 strip_heights: the height a level reports is the one its launches take, and levels that report the same

@@ -2401,13 +2401,13 @@ extern "C" int tmk_level_destroy(tmk_level* L)
 }
 
 // a box's ghosted region <-> staging array (FP64 planes of the ghosted box, x fastest); put
-// writes planes [c0, c0 + nc), the cells the box owns and the island's ghost cells, never another box's
+// writes planes [c0, c0 + NC), the cells the box owns and the island's ghost cells, never another box's
 // cells.  The FP32
 // bulk's conversion is done here, on values already in flight: on the host it took one thread and a
 // second array, 13 of the 18 ms of a 200-step pass over a 1024 x 512 level that reads its state.
-template <typename T>
+template <typename T, int NC>
 static __global__ void k_box_put(T* u0, T* u1, T* w, const int* owner, int aunx, size_t aplane, int ox, int oy,
-                                 const double* src, int c0, int nc, StateVec bg, int gnx, int gny, int box)
+                                 const double* src, int c0, StateVec bg, int gnx, int gny, int box)
 {
     const size_t n = (size_t)gnx * gny;
     const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -2416,8 +2416,11 @@ static __global__ void k_box_put(T* u0, T* u1, T* w, const int* owner, int aunx,
     const size_t a = (size_t)(x + ox) + (size_t)(y + oy) * aunx;
     const int o = owner[a];
     if (o != box && o != -1) return;
-    for (int c = c0; c < c0 + nc; ++c) {
-        const T v = to_stored<T>(src[t + (c - c0) * n], bg.c[c]);
+    u0 += c0 * aplane;
+    u1 += c0 * aplane;
+    w += c0 * aplane;
+    for (int c = 0; c < NC; ++c) {
+        const T v = to_stored<T>(src[t + c * n], bg.c[c0 + c]);
         u0[a + c * aplane] = v;
         u1[a + c * aplane] = v;
         w[a + c * aplane] = v;
@@ -2670,9 +2673,11 @@ extern "C" int tmk_level_upload(tmk_level* L, int b, const double* U, const doub
     if (L->has_b[b] && !B) return TMK_E_NO_BDRY;
     HIPCHK(hipStreamSynchronize(c->stream));
     int e;
-    // staged in the bytes that the planes take on the device: FP32 levels a side at a time
-    if ((e = c->bufs[7].ensure(nU * L->tsize))) return e;
-    const int nc = (int)(TMK_NCOMP * L->tsize / sizeof(double));
+    // staged in the bytes that the planes take on the device: FP32 levels a side at a time, but boxes of up
+    // to 8 MiB at once (64 x 48: 90 us, 110 in two)
+    const bool sides = L->tsize != sizeof(double) && nU * sizeof(double) > STAGE_SLOT * STAGE_SLOTS;
+    const int nc = sides ? TMK_NCOMP / 2 : TMK_NCOMP;
+    if ((e = c->bufs[7].ensure(nc * plane * sizeof(double)))) return e;
     const StateVec bg = background(c->P);
     const Island& I = L->isl[L->box_isl[b]];
     const int ox = ub.lo[0] - I.abox.lo[0], oy = ub.lo[1] - I.abox.lo[1];
@@ -2682,11 +2687,14 @@ extern "C" int tmk_level_upload(tmk_level* L, int b, const double* U, const doub
         // (in the stream's order: the copy waits for the kernel that reads the side before)
         HIPCHK(copy_on(c->stream, c->bufs[7].p, U + c0 * plane, nc * plane * sizeof(double), hipMemcpyHostToDevice));
         if (L->tsize == sizeof(double))
-            hipLaunchKernelGGL(k_box_put<double>, grid, dim3(256), 0, c->stream, (double*)I.u[0], (double*)I.u[1],
-                               (double*)I.w, I.owner, I.unx(), I.plane(), ox, oy, src, c0, nc, bg, gnx, gny, b);
+            hipLaunchKernelGGL((k_box_put<double, TMK_NCOMP>), grid, dim3(256), 0, c->stream, (double*)I.u[0],
+                               (double*)I.u[1], (double*)I.w, I.owner, I.unx(), I.plane(), ox, oy, src, 0, bg, gnx, gny, b);
+        else if (!sides)
+            hipLaunchKernelGGL((k_box_put<float, TMK_NCOMP>), grid, dim3(256), 0, c->stream, (float*)I.u[0],
+                               (float*)I.u[1], (float*)I.w, I.owner, I.unx(), I.plane(), ox, oy, src, 0, bg, gnx, gny, b);
         else
-            hipLaunchKernelGGL(k_box_put<float>, grid, dim3(256), 0, c->stream, (float*)I.u[0], (float*)I.u[1],
-                               (float*)I.w, I.owner, I.unx(), I.plane(), ox, oy, src, c0, nc, bg, gnx, gny, b);
+            hipLaunchKernelGGL((k_box_put<float, TMK_NCOMP / 2>), grid, dim3(256), 0, c->stream, (float*)I.u[0],
+                               (float*)I.u[1], (float*)I.w, I.owner, I.unx(), I.plane(), ox, oy, src, c0, bg, gnx, gny, b);
         HIPCHK(hipGetLastError());
     }
     HIPCHK(hipStreamSynchronize(c->stream));
