@@ -256,7 +256,7 @@ static void strip_lists()
                                        : box(margin, margin, margin + n - 1, margin + w - 1);
                 for (int rows : {0, 1, 4, 63}) {  // 0: the height the call chooses
                     if (rows) EXPECT(tmk_set_march(c, rows) == TMK_OK);
-                    EXPECT(patch_marches(c, 2));
+                    EXPECT(patch_may_march(c));
                     int nint = 0;
                     const std::vector<Tile> t = patch_strips(c, v, &nint, kNoAllocMaxStrips);
                     EXPECT(t.size() <= (size_t)kNoAllocMaxStrips);

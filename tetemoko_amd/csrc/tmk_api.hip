@@ -1640,15 +1640,20 @@ static __global__ void k_patch_out(const T* u, size_t plane, int unx, int x0, in
 }
 
 // the components a drop-in call carries: the anti-plane planes are skipped only when background and data
-// are zero there
+// are zero there.  A call whose route depends on it scans before anything is queued (patch_may_march), the
+// others behind their copies; blocks without an early way out let the compiler take several values at once.
 static int patch_ns(const tmk_ctx* c, const double* U, size_t plane)
 {
     if (c->antiplane) return 3;
     for (int s = 0; s < 2; ++s)
         for (int cc : {2, 7, 8}) {
             const double* q = U + (size_t)(11 * s + cc) * plane;
-            for (size_t k = 0; k < plane; ++k)
-                if (q[k] != 0.0) return 3;
+            for (size_t k = 0; k < plane; k += 256) {
+                const size_t n = std::min<size_t>(256, plane - k);
+                int some = 0;
+                for (size_t t = 0; t < n; ++t) some |= q[k + t] != 0.0;
+                if (some) return 3;
+            }
         }
     return 2;
 }
@@ -1658,9 +1663,9 @@ static int patch_ns(const tmk_ctx* c, const double* U, size_t plane)
 // in FP32 the two round differently.  Its strips (nint of them, at most 63 rows, as on every level that
 // stores fluxes), then its boundary pieces; at most most of both, by taller strips where the height chosen
 // makes more (FP64 values do not depend on it).
-static bool patch_marches(const tmk_ctx* c, int ns)
+static bool patch_may_march(const tmk_ctx* c)
 {
-    return c->precision == TMK_PREC_FP64 && c->march > 0 && ns == 2 && pred_kind(c->P) == PK_PPM_PRIM;
+    return c->precision == TMK_PREC_FP64 && c->march > 0 && !c->antiplane && pred_kind(c->P) == PK_PPM_PRIM;
 }
 static std::vector<Tile> patch_strips(const tmk_ctx* c, const tmk_box& v, int* nint, size_t most = SIZE_MAX)
 {
@@ -1683,7 +1688,7 @@ static std::vector<Tile> patch_strips(const tmk_ctx* c, const tmk_box& v, int* n
 }
 
 // One drop-in call on the buffers of w.  tiles: the box's tiles (patch_tiles; march: patch_strips), nint
-// interior.
+// interior.  ns: patch_ns, or 0: not known yet.
 // S: a stage that holds the call's data either way (patch_staged), or NULL: copies.
 template <typename T>
 static int patch_update_t(tmk_ctx* c, tmk_box valid, double* U, tmk_box ub, double* F0, double* F1, double* B,
@@ -1810,6 +1815,7 @@ static int patch_update_t(tmk_ctx* c, tmk_box valid, double* U, tmk_box ub, doub
         a.nint = nint;
         a.nscen = 1;
         a.patch0 = 0;
+        if (!ns) ns = patch_ns(c, U, plane);
         e = march ? launch_step<T>(st, a, false, c->P.div2, nullptr)
                   : launch_update<T>(st, nullptr, nullptr, nullptr, ns, pred_kind(c->P), c->bx, c->by, a, nint, nullptr);
         if (e) return e;
@@ -1873,8 +1879,8 @@ static int patch_update_bufs(tmk_ctx* c, tmk_box valid, double* U, tmk_box ub, d
     if (z.plane * sizeof(T) > kPlaneMaxBytes) return TMK_E_NOMEM;
     int nint = 0;
     std::vector<Tile> tiles;
-    const int ns = plastic_only ? 3 : patch_ns(c, U, z.plane);
-    const bool march = !plastic_only && patch_marches(c, ns);
+    const int ns = !plastic_only && patch_may_march(c) ? patch_ns(c, U, z.plane) : 0;
+    const bool march = ns == 2;
     if (march) {
         tiles = patch_strips(c, valid, &nint);
     } else if (!plastic_only) {
@@ -2017,8 +2023,8 @@ static int patch_update_noalloc_t(tmk_ctx* c, tmk_box valid, double* U, tmk_box 
     if (oM + noalloc_counted(ntiles) > (size_t)TMK_NOALLOC_SCRATCH_BYTES) return TMK_E_SCRATCH;
     // what fits by the tile kernels' list is accepted; the call takes the kernels that
     // tmk_patch_update_state takes
-    const int ns = patch_ns(c, U, z.plane);
-    const bool march = patch_marches(c, ns);
+    const int ns = patch_may_march(c) ? patch_ns(c, U, z.plane) : 0;
+    const bool march = ns == 2;
     Tile tiles[kNoAllocMaxTiles];
     std::vector<Tile> strips;
     if (march) {
