@@ -113,3 +113,33 @@ def test_more_readers_than_pinned_buffers():
     for t in th:
         t.join()
     assert got == [True] * n
+
+
+@pytest.mark.parametrize("n", [40, 62, 66, 90])
+def test_fp32_calls_on_both_sides_of_the_stage_limits(n):
+    """FP32 calls without fault data and fluxes copy beyond 1 MiB of state, the plastic return beyond 5/8 MiB;
+    the allocation-free call stages them: bit-identical, and so is a return through a stage and by copies."""
+    g = scenarios.GHOST
+    cfg = scenarios.config_c1(seed=9, nx=140, ny=120, dx=25.0)
+    cfg.update(plasticity=1, p_mu=0.6, p_beta=0.3, p_eta=0.03 * scenarios.G_MPA, p_b=1.0)
+    U, _ = scenarios.level_arrays(cfg)
+    scenarios.perturb(U, seed=4, amp_v=1.0, amp_s=60.0)
+    x0, y0, x1, y1 = 9, 8, 9 + n - 1, 8 + n - 1
+    ub = (x0 - g, y0 - g, x1 + g, y1 + g)
+    U0 = np.ascontiguousarray(U[:, y0:y1 + 2 * g + 1, x0:x1 + 2 * g + 1])
+    dt = scenarios.dt_of(cfg)
+    ctx = capi.Context(cfg, capi.PREC_FP32_BULK)
+    a, b = U0.copy(), U0.copy()
+    ctx.update_state((x0, y0, x1, y1), a, ub, time=0.3, dt=dt)
+    ctx.update_state((x0, y0, x1, y1), b, ub, time=0.3, dt=dt, noalloc=True)
+    assert np.array_equal(a, b) and not np.array_equal(a, U0)
+    whole, parts = a.copy(), a.copy()
+    ctx.plastic_update((x0, y0, x1, y1), whole, ub, dt)
+    for y in range(y0, y1 + 1, 20):  # boxes small enough for a stage
+        yt = min(y + 19, y1)
+        sub = np.ascontiguousarray(parts[:, y - ub[1]:yt - ub[1] + 1])
+        ctx.plastic_update((x0, y, x1, yt), sub, (ub[0], y, ub[2], yt), dt)
+        parts[:, y - ub[1]:yt - ub[1] + 1] = sub
+    ctx.close()
+    s = (slice(None), slice(g, -g), slice(g, -g))
+    assert np.array_equal(whole[s], parts[s]) and not np.array_equal(whole[s], a[s])

@@ -1859,15 +1859,28 @@ static int patch_update_t(tmk_ctx* c, tmk_box valid, double* U, tmk_box ub, doub
     return TMK_OK;
 }
 
-// The stage of a drop-in call whose data fits one, else NULL: a 32 x 32 call with fluxes took five copies
-// to the device, two on it and five back, each with a wait: 201 us, now 98 (93 x 61 FP32 and its plastic
-// return 462, now 363); calls beyond 8 MiB are bound by the link either way.
-template <typename T>
-static HostStage* patch_staged(const PatchSizes& z, size_t mbytes, bool may_pin)
+// a stage where the call's data fits one either way
+static HostStage* patch_stage_fits(const PatchSizes& z, size_t mbytes, bool may_pin)
 {
     const size_t in = (z.nU + z.nB) * sizeof(double) + mbytes;
     const size_t out = (z.nU + z.nB + z.nF0 + z.nF1) * sizeof(double) + 64;
     return std::max(in, out) <= STAGE_SLOT * STAGE_SLOTS ? stage_take(may_pin) : nullptr;
+}
+
+// The stage of a drop-in call, NULL where it does not fit one or copies are faster.  A 32 x 32 call with
+// fluxes took five copies to the device, two on it and five back, each with a wait: 201 us, now 98; calls
+// beyond 8 MiB are bound by the link either way.  An FP32 call with neither fault
+// data nor fluxes copies twice only, in FP32, where the stage carries every plane in FP64: it wins up to 1
+// MiB (64 x 64 112 us, 117 by copies; 80 x 80 154, 147; 96 x 96 200, 183), the plastic return, whose
+// kernel hides less, up to 5/8 MiB (48 x 48 67, 70; 64 x 64 102, 92; 96 x 96 209, 159).  The allocation-free
+// call, whose copies go through FP64 on the device, stages whatever fits (128 x 128 326, 408).
+template <typename T>
+static HostStage* patch_staged(const PatchSizes& z, size_t mbytes, bool plastic_only)
+{
+    if (sizeof(T) != sizeof(double) && z.nB + z.nF0 + z.nF1 == 0 &&
+        z.nU * sizeof(double) > (plastic_only ? STAGE_SLOT * 5 / 8 : STAGE_SLOT))
+        return nullptr;
+    return patch_stage_fits(z, mbytes, true);
 }
 
 // drop-in call on the context's grow-only buffers (allocated on first need)
@@ -1902,7 +1915,7 @@ static int patch_update_bufs(tmk_ctx* c, tmk_box valid, double* U, tmk_box ub, d
     w.Bd = (double*)c->bufs[3].p;
     w.Fd = (double*)c->bufs[4].p;
     w.meta = (char*)c->bufs[5].p;
-    HostStage* const S = patch_staged<T>(z, mbytes, true);
+    HostStage* const S = patch_staged<T>(z, mbytes, plastic_only);
     e = patch_update_t<T>(c, valid, U, ub, F0, F1, B, bb, nb, time, dt, plastic_only, w, tiles.data(), (int)tiles.size(),
                           nint, ns, march, S);
     if (S && e) (void)hipStreamSynchronize(c->stream);  // a launch still queued may use the stage
@@ -2049,7 +2062,7 @@ static int patch_update_noalloc_t(tmk_ctx* c, tmk_box valid, double* U, tmk_box 
     w.Fd = (double*)(base + oF);
     w.stage = sizeof(T) == sizeof(double) ? nullptr : (double*)(base + oS);
     w.meta = base + TMK_NOALLOC_SCRATCH_BYTES;
-    HostStage* const S = patch_staged<T>(z, mbytes, false);  // pinning allocates
+    HostStage* const S = patch_stage_fits(z, mbytes, false);  // pinning allocates
     const int e = patch_update_t<T>(c, valid, U, ub, F0, F1, B, bb, nb, time, dt, false, w, list, nlist, nint, ns, march, S);
     if (S && e) (void)hipStreamSynchronize(c->stream);
     stage_give(S);
