@@ -1689,11 +1689,12 @@ static std::vector<Tile> patch_strips(const tmk_ctx* c, const tmk_box& v, int* n
 
 // One drop-in call on the buffers of w.  tiles: the box's tiles (patch_tiles; march: patch_strips), nint
 // interior.  ns: patch_ns, or 0: not known yet.
-// S: a stage that holds the call's data either way (patch_staged), or NULL: copies.
+// S: a stage that holds the call's data either way (patch_staged), or NULL: copies (queued: the state's
+// has been).
 template <typename T>
 static int patch_update_t(tmk_ctx* c, tmk_box valid, double* U, tmk_box ub, double* F0, double* F1, double* B,
                           tmk_box bb, int nb, double time, double dt, bool plastic_only, const PatchWork<T>& w,
-                          const Tile* tiles, int ntiles, int nint, int ns, bool march, HostStage* S)
+                          const Tile* tiles, int ntiles, int nint, int ns, bool march, HostStage* S, bool queued)
 {
     const PatchSizes z = patch_sizes(valid, ub, F0, F1, B, bb, nb);
     const size_t unx = z.unx, plane = z.plane, nU = z.nU, bnx = z.bnx, nB = z.nB, nF0 = z.nF0, nF1 = z.nF1;
@@ -1751,7 +1752,7 @@ static int patch_update_t(tmk_ctx* c, tmk_box valid, double* U, tmk_box ub, doub
     if (S) {
         if (plastic_only && (e = staged_in(0))) return e;
     } else if (sizeof(T) == sizeof(double)) {
-        HIPCHK(hipMemcpyAsync(Uin, U, nU * sizeof(double), hipMemcpyHostToDevice, st));
+        if (!queued) HIPCHK(hipMemcpyAsync(Uin, U, nU * sizeof(double), hipMemcpyHostToDevice, st));
     } else if (w.stage) {
         HIPCHK(hipMemcpyAsync(w.stage, U, nU * sizeof(double), hipMemcpyHostToDevice, st));
         hipLaunchKernelGGL(k_to_f32, cvt_grid, dim3(256), 0, st, (const double*)w.stage, (float*)Uin, plane,
@@ -1859,12 +1860,16 @@ static int patch_update_t(tmk_ctx* c, tmk_box valid, double* U, tmk_box ub, doub
     return TMK_OK;
 }
 
-// a stage where the call's data fits one either way
-static HostStage* patch_stage_fits(const PatchSizes& z, size_t mbytes, bool may_pin)
+// whether the call's data fits a stage either way, and one where it does
+static bool patch_fits(const PatchSizes& z, size_t mbytes)
 {
     const size_t in = (z.nU + z.nB) * sizeof(double) + mbytes;
     const size_t out = (z.nU + z.nB + z.nF0 + z.nF1) * sizeof(double) + 64;
-    return std::max(in, out) <= STAGE_SLOT * STAGE_SLOTS ? stage_take(may_pin) : nullptr;
+    return std::max(in, out) <= STAGE_SLOT * STAGE_SLOTS;
+}
+static HostStage* patch_stage_fits(const PatchSizes& z, size_t mbytes, bool may_pin)
+{
+    return patch_fits(z, mbytes) ? stage_take(may_pin) : nullptr;
 }
 
 // The stage of a drop-in call, NULL where it does not fit one or copies are faster.  A 32 x 32 call with
@@ -1890,9 +1895,15 @@ static int patch_update_bufs(tmk_ctx* c, tmk_box valid, double* U, tmk_box ub, d
 {
     const PatchSizes z = patch_sizes(valid, ub, F0, F1, B, bb, nb);
     if (z.plane * sizeof(T) > kPlaneMaxBytes) return TMK_E_NOMEM;
-    int nint = 0;
+    int nint = 0, e;
     std::vector<Tile> tiles;
-    const int ns = !plastic_only && patch_may_march(c) ? patch_ns(c, U, z.plane) : 0;
+    const bool may_march = !plastic_only && patch_may_march(c);
+    // a call beyond a stage that may march (FP64) queues its state ahead of the scan that decides
+    const bool queued = may_march && !patch_fits(z, 0);
+    if ((e = c->bufs[1].ensure(z.nU * sizeof(T)))) return e;
+    if ((e = c->bufs[2].ensure(z.nU * sizeof(T)))) return e;
+    if (queued) HIPCHK(hipMemcpyAsync(c->bufs[1].p, U, z.nU * sizeof(T), hipMemcpyHostToDevice, c->stream));
+    const int ns = may_march ? patch_ns(c, U, z.plane) : 0;
     const bool march = ns == 2;
     if (march) {
         tiles = patch_strips(c, valid, &nint);
@@ -1903,12 +1914,11 @@ static int patch_update_bufs(tmk_ctx* c, tmk_box valid, double* U, tmk_box ub, d
     }
     size_t off_t, off_s, mbytes;
     patch_meta<T>((int)tiles.size(), &off_t, &off_s, &mbytes);
-    int e;
-    if ((e = c->bufs[1].ensure(z.nU * sizeof(T)))) return e;
-    if ((e = c->bufs[2].ensure(z.nU * sizeof(T)))) return e;
-    if ((e = c->bufs[3].ensure(std::max<size_t>(2 * z.nB, 1) * sizeof(double)))) return e;
-    if ((e = c->bufs[4].ensure(std::max<size_t>(z.nF0 + z.nF1, 1) * sizeof(double)))) return e;
-    if ((e = c->bufs[5].ensure(mbytes))) return e;
+    if ((e = c->bufs[3].ensure(std::max<size_t>(2 * z.nB, 1) * sizeof(double))) ||
+        (e = c->bufs[4].ensure(std::max<size_t>(z.nF0 + z.nF1, 1) * sizeof(double))) || (e = c->bufs[5].ensure(mbytes))) {
+        if (queued) (void)hipStreamSynchronize(c->stream);  // the caller's memory is free again
+        return e;
+    }
     PatchWork<T> w;
     w.Uin = (T*)c->bufs[1].p;
     w.Uout = (T*)c->bufs[2].p;
@@ -1917,7 +1927,7 @@ static int patch_update_bufs(tmk_ctx* c, tmk_box valid, double* U, tmk_box ub, d
     w.meta = (char*)c->bufs[5].p;
     HostStage* const S = patch_staged<T>(z, mbytes, plastic_only);
     e = patch_update_t<T>(c, valid, U, ub, F0, F1, B, bb, nb, time, dt, plastic_only, w, tiles.data(), (int)tiles.size(),
-                          nint, ns, march, S);
+                          nint, ns, march, S, queued);
     if (S && e) (void)hipStreamSynchronize(c->stream);  // a launch still queued may use the stage
     stage_give(S);
     return e;
@@ -2063,7 +2073,7 @@ static int patch_update_noalloc_t(tmk_ctx* c, tmk_box valid, double* U, tmk_box 
     w.stage = sizeof(T) == sizeof(double) ? nullptr : (double*)(base + oS);
     w.meta = base + TMK_NOALLOC_SCRATCH_BYTES;
     HostStage* const S = patch_stage_fits(z, mbytes, false);  // pinning allocates
-    const int e = patch_update_t<T>(c, valid, U, ub, F0, F1, B, bb, nb, time, dt, false, w, list, nlist, nint, ns, march, S);
+    const int e = patch_update_t<T>(c, valid, U, ub, F0, F1, B, bb, nb, time, dt, false, w, list, nlist, nint, ns, march, S, false);
     if (S && e) (void)hipStreamSynchronize(c->stream);
     stage_give(S);
     return e;
