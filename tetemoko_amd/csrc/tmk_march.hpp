@@ -261,8 +261,11 @@ struct MarchRing {
 
 // The faces of strip tl whose register flux the strip stores (register_face), from the level's face masks
 // (Patch::fmask): bit j - y0 of m0 for this lane's lo x face on row j, of m1 for its lo y face (row y1 + 1
-// too).  One mask byte is loaded per row, four rows at a time; what a row's cells are is one word of a bit
-// per lane, the same in every lane, so the rule runs on scalars.
+// too).  One mask byte is loaded per row, four rows at a time.  FP64: a lane's own bytes, the left
+// neighbour's by a lane shift, the lower one's from the row before.  FP32: what a row's cells are is one word
+// of a bit per lane, the same in every lane, so the rule runs on scalars; FP64 has none to spare (94 scalar
+// registers spilled for 102: 1021 x 509 steps 35.6 us for 36.0), FP32's vector registers are the scarcer
+// (1021 x 509 with plasticity 21.6 us for 21.9).
 template <typename T>
 __device__ __forceinline__ void march_faces(const Patch<T>& pt, const Tile& tl, int lane, unsigned long long& m0,
                                             unsigned long long& m1)
@@ -272,25 +275,36 @@ __device__ __forceinline__ void march_faces(const Patch<T>& pt, const Tile& tl, 
     const int mw = pt.vhi0 - pt.vlo0 + 3;  // the masks cover the descriptor's valid box grown by one
     const int i = tl.x0 - 3 + min(max(lane, 2), tnx + 3);
     const size_t at = (size_t)(i - pt.vlo0 + 1) + (size_t)(y0 - pt.vlo1 + 1) * mw;
-    const unsigned long long cols = ((1ull << tnx) - 1) << 3;  // the lanes of the strip's columns
-    unsigned long long below = __builtin_amdgcn_ballot_w64(mk[at - mw] == 1);
+    const bool left_in = lane >= 4, here_in = lane <= tnx + 2;          // the left and this lane's column: of the strip
+    const unsigned long long cols = ((1ull << tnx) - 1) << 3;           // the lanes of its columns
+    unsigned below = mk[at - mw];
+    unsigned long long ubelow = __builtin_amdgcn_ballot_w64(below == 1);  // the row's uncovered cells of the level
     for (int k = 0; k <= rows; k += 4) {
         unsigned b[4];
 #pragma unroll
         for (int q = 0; q < 4; ++q) b[q] = mk[at + (size_t)min(k + q, rows) * mw];
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            const unsigned long long here = __builtin_amdgcn_ballot_w64(b[q] == 1), left = here << 1;
-            const bool up = k + q < rows;  // the row belongs to the strip; row k + q - 1 does from the second on
-            const unsigned long long x = up ? (cols & here & ~left) | (cols << 1 & left & ~here) : 0ull;
-            const unsigned long long y = cols & ((up ? here & ~below : 0ull) | (k + q > 0 ? below & ~here : 0ull));
-            if (k + q <= rows) {
-                m0 |= (unsigned long long)((x >> lane) & 1) << (k + q);
-                m1 |= (unsigned long long)((y >> lane) & 1) << (k + q);
+            const bool down = k + q > 0, up = k + q < rows;  // the row below and this one: of the strip
+            if constexpr (sizeof(T) == sizeof(float)) {
+                const unsigned long long u = __builtin_amdgcn_ballot_w64(b[q] == 1), left = u << 1;
+                const unsigned long long x = up ? (cols & u & ~left) | (cols << 1 & left & ~u) : 0ull;
+                const unsigned long long y = cols & ((up ? u & ~ubelow : 0ull) | (down ? ubelow & ~u : 0ull));
+                if (k + q <= rows) {
+                    m0 |= (unsigned long long)((x >> lane) & 1) << (k + q);
+                    m1 |= (unsigned long long)((y >> lane) & 1) << (k + q);
+                }
+                ubelow = u;
+            } else {
+                const unsigned left = (unsigned)__builtin_amdgcn_update_dpp(0, (int)b[q], DPP_FROM_PREV, 0xF, 0xF, true);
+                if (up && register_face(left, b[q], left_in, here_in)) m0 |= 1ull << (k + q);
+                if (k + q <= rows && register_face(below, b[q], down, up)) m1 |= 1ull << (k + q);
+                below = b[q];
             }
-            below = here;
         }
     }
+    if (lane < 3 || lane > tnx + 3) m0 = 0;
+    if (lane < 3 || lane > tnx + 2) m1 = 0;
 }
 
 // marks the strips tiles[0, n) of a hierarchy level that touch a face of its registers (one wavefront
